@@ -26,7 +26,8 @@ using namespace eolc_cd;
 namespace eolc {
 hipError_t cd_prep(eolc_ctx *c, double thr, double *xj, double *fn, double *aabb_part, double *aabb);
 hipError_t cd_grid_build(eolc_ctx *c, const CdGrid &gp, const double *xj, unsigned *bcnt, unsigned *bstart,
-                         unsigned *cursor, int *entries, unsigned *nalways, int *always, unsigned *total, bool fill);
+                         unsigned *cursor, int *entries, unsigned *nalways, int *always, unsigned *sums, unsigned *total,
+                         bool fill);
 hipError_t cd_query(eolc_ctx *c, const CdGrid &gp, int Q, const double *qpts, const double *qnrm, double thr,
                     const double *aabb, const double *xj, const double *fn, const unsigned *bstart, const unsigned *bcnt,
                     const int *entries, const unsigned *nalways, const int *always, int *face, eolc_collision *rec);
@@ -36,9 +37,10 @@ hipError_t cd_eolpts(eolc_ctx *c, int P, double thr, const double *pts, const do
                      eolc_collision *rec);
 hipError_t cd_ee(eolc_ctx *c, int pass, double thr, const BoxGeom *box, const double *xj, unsigned *counts,
                  const unsigned *offsets, int *ambig, eolc_collision *out);
-hipError_t cd_compact(eolc_ctx *c, int n, const int *flag, unsigned *u32, unsigned *offs, unsigned *total,
-                      const eolc_collision *rec, eolc_collision *out, bool write);
-hipError_t cd_scan(eolc_ctx *c, unsigned n, const unsigned *in, unsigned *out, unsigned *total);
+hipError_t cd_compact(eolc_ctx *c, int n, const int *flag, unsigned *u32, unsigned *offs, unsigned *sums,
+                      unsigned *total, const eolc_collision *rec, eolc_collision *out, bool write);
+size_t cd_scan_words(size_t n);
+hipError_t cd_scan(eolc_ctx *c, unsigned n, const unsigned *in, unsigned *out, unsigned *sums, unsigned *total);
 }  // namespace eolc
 
 namespace {
@@ -301,15 +303,17 @@ int collide_impl(eolc_ctx *c, Workspace &ws, double thr, int P, const double *pt
     EOLC_HIP(ws.get(&total, 1));
     EOLC_HIP(ws.get(&nalways, 1));
     EOLC_HIP(ws.get(&always, (size_t)F));
+    unsigned *sums = nullptr;
+    EOLC_HIP(ws.get(&sums, eolc::cd_scan_words(std::max<size_t>({tbl, (size_t)N, (size_t)c->n_cedges}))));
     EOLC_HIP(hipMemsetAsync(bcnt, 0, tbl * sizeof(unsigned), c->stream));
     EOLC_HIP(hipMemsetAsync(cursor, 0, tbl * sizeof(unsigned), c->stream));
     EOLC_HIP(hipMemsetAsync(nalways, 0, sizeof(unsigned), c->stream));
-    EOLC_HIP(eolc::cd_grid_build(c, g, xj, bcnt, bstart, cursor, nullptr, nalways, always, total, false));
+    EOLC_HIP(eolc::cd_grid_build(c, g, xj, bcnt, bstart, cursor, nullptr, nalways, always, sums, total, false));
     unsigned nentries = 0;
     EOLC_HIP(hipMemcpyAsync(&nentries, total, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
     EOLC_HIP(hipStreamSynchronize(c->stream));
     EOLC_HIP(ws.get(&entries, nentries));
-    EOLC_HIP(eolc::cd_grid_build(c, g, xj, bcnt, bstart, cursor, entries, nalways, always, total, true));
+    EOLC_HIP(eolc::cd_grid_build(c, g, xj, bcnt, bstart, cursor, entries, nalways, always, sums, total, true));
     // ---- point / corner queries against the faces
     const int Q = P + 8 * B;
     std::vector<double> hq(3 * (size_t)std::max(Q, 1)), hn(3 * (size_t)std::max(Q, 1));
@@ -346,7 +350,7 @@ int collide_impl(eolc_ctx *c, Workspace &ws, double thr, int P, const double *pt
     EOLC_HIP(ws.get(&err, 1));
     EOLC_HIP(hipMemsetAsync(err, 0, sizeof(int), c->stream));
     auto per_vertex_records = [&](std::vector<eolc_collision> &dst) -> int {
-        EOLC_HIP(eolc::cd_compact(c, N, flag, u32, offs, total, nullptr, nullptr, false));
+        EOLC_HIP(eolc::cd_compact(c, N, flag, u32, offs, sums, total, nullptr, nullptr, false));
         unsigned cnt = 0;
         EOLC_HIP(hipMemcpyAsync(&cnt, total, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
         EOLC_HIP(hipStreamSynchronize(c->stream));
@@ -355,7 +359,7 @@ int collide_impl(eolc_ctx *c, Workspace &ws, double thr, int P, const double *pt
             const size_t m = ws.mark();
             eolc_collision *o = nullptr;
             EOLC_HIP(ws.get(&o, cnt));
-            EOLC_HIP(eolc::cd_compact(c, N, flag, u32, offs, total, vrec, o, true));
+            EOLC_HIP(eolc::cd_compact(c, N, flag, u32, offs, sums, total, vrec, o, true));
             EOLC_HIP(hipMemcpyAsync(dst.data(), o, sizeof(eolc_collision) * cnt, hipMemcpyDeviceToHost, c->stream));
             EOLC_HIP(hipStreamSynchronize(c->stream));
             ws.release(m);
@@ -423,7 +427,7 @@ int collide_impl(eolc_ctx *c, Workspace &ws, double thr, int P, const double *pt
         // E2-E1
         if (E > 0) {
             EOLC_HIP(eolc::cd_ee(c, 0, thr, dbox, xj, ecnt, nullptr, eamb, nullptr));
-            EOLC_HIP(eolc::cd_scan(c, (unsigned)E, ecnt, eoff, total));
+            EOLC_HIP(eolc::cd_scan(c, (unsigned)E, ecnt, eoff, sums, total));
             unsigned ne = 0;
             EOLC_HIP(hipMemcpyAsync(&ne, total, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
             std::vector<int> amb((size_t)E);

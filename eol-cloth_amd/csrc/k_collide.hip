@@ -27,6 +27,7 @@
 //   k_cd_eolpts     one thread per cloth vertex (pointTri EOL branch)
 // Variable-length outputs are compacted in reference order by count -> scan ->
 // write passes (no atomics on record positions).
+#include <algorithm>
 #include <mutex>
 
 #include "eolc_internal.h"
@@ -82,16 +83,24 @@ __global__ void __launch_bounds__(256) k_cd_aabb(int N, const double *__restrict
         for (int k = 0; k < 6; ++k) part[6 * blockIdx.x + k] = s[k][0];
 }
 
-__global__ void k_cd_aabb_final(int nb, const double *__restrict__ part, double *__restrict__ out)
+// One workgroup of kAabbParts threads, one partial box each (min and max are order-free).
+// A single thread walking the 256 partials took 51-57 us, as long as the query itself.
+constexpr int kAabbParts = 256;
+__global__ void __launch_bounds__(kAabbParts) k_cd_aabb_final(const double *__restrict__ part, double *__restrict__ out)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double r[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    for (int b = 0; b < nb; ++b)
-        for (int k = 0; k < 3; ++k) {
-            r[k] = fmin(r[k], part[6 * b + k]);
-            r[3 + k] = fmax(r[3 + k], part[6 * b + 3 + k]);
-        }
-    for (int k = 0; k < 6; ++k) out[k] = r[k];
+    __shared__ double s[6][kAabbParts];
+    const int t = threadIdx.x;
+    for (int k = 0; k < 6; ++k) s[k][t] = part[6 * t + k];
+    __syncthreads();
+    for (int o = kAabbParts / 2; o > 0; o >>= 1) {
+        if (t < o)
+            for (int k = 0; k < 3; ++k) {
+                s[k][t] = fmin(s[k][t], s[k][t + o]);
+                s[3 + k][t] = fmax(s[3 + k][t], s[3 + k][t + o]);
+            }
+        __syncthreads();
+    }
+    if (t < 6) out[t] = s[t][0];
 }
 
 // ---------------------------------------------------------------------------
@@ -165,31 +174,91 @@ __global__ void k_grid_insert(int F, int pass, GridParams g, const double *__res
             }
 }
 
-// exclusive scan of the bucket counts (single workgroup, sequential chunks)
-__global__ void __launch_bounds__(1024) k_scan_u32(unsigned n, const unsigned *__restrict__ in,
-                                                   unsigned *__restrict__ out, unsigned *__restrict__ total)
+// Exclusive scan of n counts in two launches, kScanItems per workgroup: the sums of
+// the workgroups' pieces, then every workgroup adds the sums before its own and scans
+// its piece (integers: the order does not matter).  A single workgroup walking the
+// array took 1.8 ms for the 2^20 buckets of a 512^2 sheet; this is one read of it,
+// another and one write.
+constexpr int kScanWG = 512, kScanPer = 16, kScanItems = kScanWG * kScanPer;
+
+__device__ __forceinline__ unsigned scan_wave_sum(unsigned v)
 {
-    __shared__ unsigned s[1024];
-    __shared__ unsigned carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (unsigned base = 0; base < n; base += 1024) {
-        unsigned i = base + threadIdx.x;
-        unsigned v = i < n ? in[i] : 0u;
-        s[threadIdx.x] = v;
-        __syncthreads();
-        for (unsigned o = 1; o < 1024; o <<= 1) {
-            unsigned t = threadIdx.x >= o ? s[threadIdx.x - o] : 0u;
-            __syncthreads();
-            s[threadIdx.x] += t;
-            __syncthreads();
-        }
-        if (i < n) out[i] = carry + s[threadIdx.x] - v;
-        __syncthreads();
-        if (threadIdx.x == 1023) carry += s[1023];
-        __syncthreads();
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
+__global__ void __launch_bounds__(kScanWG) k_scan_sums(unsigned n, const unsigned *__restrict__ in,
+                                                       unsigned *__restrict__ sums)
+{
+    __shared__ unsigned w[kScanWG / 64];
+    const unsigned base = blockIdx.x * kScanItems;
+    unsigned v = 0;
+#pragma unroll
+    for (int k = 0; k < kScanPer; ++k) {
+        const unsigned i = base + k * kScanWG + threadIdx.x;
+        v += i < n ? in[i] : 0u;
     }
-    if (threadIdx.x == 0) *total = carry;
+    v = scan_wave_sum(v);
+    if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned s = 0;
+        for (int k = 0; k < kScanWG / 64; ++k) s += w[k];
+        sums[blockIdx.x] = s;
+    }
+}
+
+__global__ void __launch_bounds__(kScanWG) k_scan_write(unsigned n, const unsigned *__restrict__ in,
+                                                        const unsigned *__restrict__ sums, unsigned *__restrict__ out,
+                                                        unsigned *__restrict__ total)
+{
+    constexpr int NW = kScanWG / 64;
+    __shared__ unsigned w[NW], piece[kScanItems + kScanItems / 32];   // one word of padding per 32: a lane's 16 items
+    const unsigned base = blockIdx.x * kScanItems;
+    const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+    auto at = [](int i) { return i + (i >> 5); };
+    unsigned before = 0;
+    for (unsigned b = t; b < blockIdx.x; b += kScanWG) before += sums[b];
+    before = scan_wave_sum(before);
+    if (lane == 0) w[wid] = before;
+#pragma unroll
+    for (int k = 0; k < kScanPer; ++k) {
+        const unsigned i = base + k * kScanWG + t;
+        piece[at(k * kScanWG + t)] = i < n ? in[i] : 0u;
+    }
+    __syncthreads();
+    before = 0;
+    for (int k = 0; k < NW; ++k) before += w[k];
+    __syncthreads();
+    // each thread its own kScanPer consecutive items, then the wavefront and the workgroup
+    unsigned mine = 0;
+#pragma unroll
+    for (int k = 0; k < kScanPer; ++k) mine += piece[at(t * kScanPer + k)];
+    unsigned inc = mine;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned u = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += u;
+    }
+    if (lane == 63) w[wid] = inc;
+    __syncthreads();
+    unsigned run = before + inc - mine;
+    for (int k = 0; k < wid; ++k) run += w[k];
+#pragma unroll
+    for (int k = 0; k < kScanPer; ++k) {
+        const unsigned v = piece[at(t * kScanPer + k)];
+        piece[at(t * kScanPer + k)] = run;
+        run += v;
+    }
+    // the last thread's running sum is the sum of everything up to this piece's end
+    if (total && t == kScanWG - 1 && blockIdx.x == gridDim.x - 1) *total = run;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kScanPer; ++k) {
+        const unsigned i = base + k * kScanWG + t;
+        if (i < n) out[i] = piece[at(k * kScanWG + t)];
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -506,20 +575,25 @@ hipError_t cd_prep(eolc_ctx *c, double thr, double *xj, double *fn, double *aabb
     hipLaunchKernelGGL(k_cd_prep, dim3(blocks_for(3 * N)), dim3(256), 0, c->stream, N, F, thr, c->x, c->cd_unit,
                        c->tri, xj, fn);
     hipLaunchKernelGGL(k_cd_fnormals, dim3(blocks_for(F)), dim3(256), 0, c->stream, F, xj, c->tri, fn);
-    const int nb = 256;
-    hipLaunchKernelGGL(k_cd_aabb, dim3(nb), dim3(256), 0, c->stream, N, xj, aabb_part);
-    hipLaunchKernelGGL(k_cd_aabb_final, dim3(1), dim3(64), 0, c->stream, nb, aabb_part, aabb);
+    hipLaunchKernelGGL(k_cd_aabb, dim3(kAabbParts), dim3(256), 0, c->stream, N, xj, aabb_part);
+    hipLaunchKernelGGL(k_cd_aabb_final, dim3(1), dim3(kAabbParts), 0, c->stream, aabb_part, aabb);
     return hipGetLastError();
 }
 
-hipError_t cd_scan(eolc_ctx *c, unsigned n, const unsigned *in, unsigned *out, unsigned *total)
+size_t cd_scan_words(size_t n) { return (n + kScanItems - 1) / kScanItems; }
+
+// Exclusive scan of in[0..n) into out, the sum into *total; sums: cd_scan_words(n).
+hipError_t cd_scan(eolc_ctx *c, unsigned n, const unsigned *in, unsigned *out, unsigned *sums, unsigned *total)
 {
-    hipLaunchKernelGGL(k_scan_u32, dim3(1), dim3(1024), 0, c->stream, n, in, out, total);
+    const int nb = (int)std::max<size_t>(cd_scan_words(n), 1);
+    hipLaunchKernelGGL(k_scan_sums, dim3(nb), dim3(kScanWG), 0, c->stream, n, in, sums);
+    hipLaunchKernelGGL(k_scan_write, dim3(nb), dim3(kScanWG), 0, c->stream, n, in, sums, out, total);
     return hipGetLastError();
 }
 
 hipError_t cd_grid_build(eolc_ctx *c, const eolc_cd::CdGrid &gp, const double *xj, unsigned *bcnt, unsigned *bstart,
-                         unsigned *cursor, int *entries, unsigned *nalways, int *always, unsigned *total, bool fill)
+                         unsigned *cursor, int *entries, unsigned *nalways, int *always, unsigned *sums, unsigned *total,
+                         bool fill)
 {
     const int F = c->topo.F;
     GridParams g;
@@ -531,7 +605,8 @@ hipError_t cd_grid_build(eolc_ctx *c, const eolc_cd::CdGrid &gp, const double *x
     if (!fill) {
         hipLaunchKernelGGL(k_grid_insert, dim3(blocks_for(F)), dim3(256), 0, c->stream, F, 0, g, xj, c->tri, bcnt,
                            bstart, cursor, entries, nalways, always);
-        hipLaunchKernelGGL(k_scan_u32, dim3(1), dim3(1024), 0, c->stream, gp.mask + 1, bcnt, bstart, total);
+        const hipError_t e = cd_scan(c, gp.mask + 1, bcnt, bstart, sums, total);
+        if (e != hipSuccess) return e;
     } else {
         hipLaunchKernelGGL(k_grid_insert, dim3(blocks_for(F)), dim3(256), 0, c->stream, F, 1, g, xj, c->tri, bcnt,
                            bstart, cursor, entries, nalways, always);
@@ -584,12 +659,13 @@ hipError_t cd_ee(eolc_ctx *c, int pass, double thr, const BoxGeom *box, const do
     return hipGetLastError();
 }
 
-hipError_t cd_compact(eolc_ctx *c, int n, const int *flag, unsigned *u32, unsigned *offs, unsigned *total,
-                      const eolc_collision *rec, eolc_collision *out, bool write)
+hipError_t cd_compact(eolc_ctx *c, int n, const int *flag, unsigned *u32, unsigned *offs, unsigned *sums,
+                      unsigned *total, const eolc_collision *rec, eolc_collision *out, bool write)
 {
     if (!write) {
         hipLaunchKernelGGL(k_flag_to_u32, dim3(blocks_for(n)), dim3(256), 0, c->stream, n, flag, u32);
-        hipLaunchKernelGGL(k_scan_u32, dim3(1), dim3(1024), 0, c->stream, (unsigned)n, u32, offs, total);
+        const hipError_t e = cd_scan(c, (unsigned)n, u32, offs, sums, total);
+        if (e != hipSuccess) return e;
     } else {
         hipLaunchKernelGGL(k_compact, dim3(blocks_for(n)), dim3(256), 0, c->stream, n, flag, offs, rec, out);
     }

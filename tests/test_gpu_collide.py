@@ -189,3 +189,12 @@ def test_closed_form_scenes(ctx, name):
         v2 = S.jittered(verts, O.mt19937_uniform)
         exp = exp_fn(v2)
         S.compare(g[: len(exp)] if eol else g, exp)
+
+
+@pytest.mark.parametrize("n", [51, 52, 64, 74])
+def test_counts_at_the_scan_pieces(ctx, n):
+    """Record offsets come from scans over the edges and the grid's buckets in pieces of
+    8,192 counts: 7,905 and 8,216 edges (one piece, one and a remainder), 8,192 faces
+    (16,384 buckets, two whole pieces) and 16,576 edges; every record bit for bit."""
+    sc, pts, nrm, whd, E = thin_box_scene(n, 1e-3)
+    assert compare(ctx, sc, sc.x0, 2e-3, pts, nrm, whd, E)
