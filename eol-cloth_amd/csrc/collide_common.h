@@ -44,6 +44,13 @@ struct BoxGeom {
     double aabb[6];
 };
 
+// Faces worse shaped than this (|v0|^2 |v1|^2 over the barycentric denominator) are
+// tested against every query; a query that a better one accepts lies within
+// grid_margin of its box: |x - projection| and the barycentric rounding, L the cloth's
+// largest extent.
+constexpr double kGridCondMax = 1e6;
+CDQ double grid_margin(double thr, double L) { return 5.0 * thr * (1.0 + 1e-6) + 1e-7 * L + 1e-12; }
+
 struct CdGrid {
     double org[3];
     double inv_cell;
@@ -187,19 +194,24 @@ CDQ void rec_init(eolc_collision *c)
     c->edge2 = -1;
 }
 
-// E2-E1 test of one cloth edge against the 12 box edges (boxTriCollision.cpp:848-1017).
+// One cloth edge of the E2-E1 test: its ends, direction, length, normal and box.
 // cedges: (v0, v1, face0, face1 or -1) per edge in createEdges order; x the
-// un-jittered positions (edge normals), xj the jittered ones.  Writes the records
-// to out (when not null), returns their count; bit k1 of *ambig is set when an
-// angle comparison for box edge k1 fell within `band` of its threshold.
-CDQ int ee_edge(int k2, double thr, const BoxGeom &box, const int *cedges, const double *x, const double *xj,
-                const int *tri, eolc_collision *out, int *ambig, double band)
+// un-jittered positions (edge normals), xj the jittered ones.
+struct ClothEdge {
+    int v0, v1;
+    double a[3], b[3], dx[3], nor[3], len, aabb[6];
+};
+
+CDQ void cloth_edge(int k2, const int *cedges, const double *x, const double *xj, const int *tri, ClothEdge &ce)
 {
     const int *e2 = cedges + 4 * k2;
-    const double *x2a = xj + 3 * e2[0], *x2b = xj + 3 * e2[1];
-    double dx2[3], nor2[3], t[3], n0[3], n1[3] = {0.0, 0.0, 0.0};
-    v_sub(x2b, x2a, dx2);
-    const double len2 = v_norm(dx2);
+    ce.v0 = e2[0];
+    ce.v1 = e2[1];
+    v_copy(xj + 3 * e2[0], ce.a);
+    v_copy(xj + 3 * e2[1], ce.b);
+    double t[3], n0[3], n1[3] = {0.0, 0.0, 0.0};
+    v_sub(ce.b, ce.a, ce.dx);
+    ce.len = v_norm(ce.dx);
     {
         const int f0 = e2[2];
         double d1[3], d2[3], c[3];
@@ -216,98 +228,119 @@ CDQ int ee_edge(int k2, double thr, const BoxGeom &box, const int *cedges, const
         }
     }
     v_add(n0, n1, t);
-    v_normalized(t, nor2);
-    double aabbE[6];
+    v_normalized(t, ce.nor);
     for (int i = 0; i < 3; ++i) {
-        double lo = x2a[i], hi = x2a[i];
-        lo = (lo < x2b[i]) ? lo : x2b[i];
-        hi = (x2b[i] < hi) ? hi : x2b[i];
-        aabbE[i] = lo; aabbE[i + 3] = hi;
+        double lo = ce.a[i], hi = ce.a[i];
+        lo = (lo < ce.b[i]) ? lo : ce.b[i];
+        hi = (ce.b[i] < hi) ? hi : ce.b[i];
+        ce.aabb[i] = lo; ce.aabb[i + 3] = hi;
     }
+}
+
+// E2-E1 test of cloth edge k2 (ce) against box edge k1 (boxTriCollision.cpp:848-1017).
+// Returns 1 and writes the record (when out is not null) if they meet; sets *ambig when
+// an angle comparison fell within `band` of its threshold.
+CDQ int ee_pair(int k2, int k1, double thr, const BoxGeom &box, const ClothEdge &ce, eolc_collision *out, int *ambig,
+                double band)
+{
+    const double *x2a = ce.a, *x2b = ce.b, *dx2 = ce.dx, *nor2 = ce.nor;
+    const double len2 = ce.len;
     const double threshAng = 2.0 * kPi / 180.0;
+    if (box.eangle[k1] < kPi / 6.0) return 0;
+    if (!check_aabb(box.faabb[kBoxEdgeFaces[k1][0]], ce.aabb) && !check_aabb(box.faabb[kBoxEdgeFaces[k1][1]], ce.aabb))
+        return 0;
+    const double *x1a = box.v[kBoxEdgeVerts[k1][0]], *x1b = box.v[kBoxEdgeVerts[k1][1]];
+    double dx1[3], tan1[3];
+    v_sub(x1b, x1a, dx1);
+    const double len1 = v_norm(dx1);
+    for (int i = 0; i < 3; ++i) tan1[i] = dx1[i] / len1;
+    double angle = acos(v_dot(tan1, nor2));
+    if (fabs(fabs(angle) - threshAng) < band || fabs(fabs(kPi - angle) - threshAng) < band) *ambig = 1;
+    if (fabs(angle) < threshAng || fabs(kPi - angle) < threshAng) return 0;
+    angle = acos(v_dot(tan1, dx2) / len2);
+    if (fabs(fabs(angle) - threshAng) < band || fabs(fabs(kPi - angle) - threshAng) < band) *ambig = 1;
+    if (fabs(angle) < threshAng || fabs(kPi - angle) < threshAng) return 0;
+    double nor[3], c[3];
+    v_cross(dx1, dx2, c);
+    v_normalized(c, nor);
+    const double *x1c = box.v[kBoxEdgeVerts[k1][2]], *x1d = box.v[kBoxEdgeVerts[k1][3]];
+    const double *n1c = box.en[k1][0], *n1d = box.en[k1][1];
+    double nor1[3];
+    v_add(n1c, n1d, nor1);
+    v_normalized(nor1, nor1);
+    if (v_dot(nor, nor1) < 0.0) v_neg(nor);
+    double angleCD = acos(v_dot(n1c, n1d));
+    double angleCN = acos(v_dot(n1c, nor));
+    if (angleCD < 0.0) { angleCD = -angleCD; angleCN = -angleCN; }
+    if (fabs(angleCN + threshAng) < band || fabs(angleCN - angleCD - threshAng) < band) *ambig = 1;
+    if (angleCN < -threshAng || angleCN - angleCD > threshAng) return 0;
+    double u2c = 0, u2d = 0;
+    int i2c = intersect_square(x2a, dx2, x1a, x1b, x1c, &u2c);
+    int i2d = intersect_square(x2a, dx2, x1b, x1a, x1d, &u2d);
+    i2c = i2c && (0.0 <= u2c && u2c <= 1.0);
+    i2d = i2d && (0.0 <= u2d && u2d <= 1.0);
+    double u1, u2;
+    lineline(&u1, &u2, x1a, x1b, x2a, x2b);
+    const double thresh1 = 1.0 * thr / len1, thresh2 = 1.0 * thr / len2;
+    if (u1 < -thresh1 || u1 > 1.0 + thresh1 || u2 < -thresh2 || u2 > 1.0 + thresh2) return 0;
+    double x1[3], x2[3], dx[3];
+    if (i2c && i2d) {
+        for (int i = 0; i < 3; ++i) {
+            x1[i] = (1.0 - u1) * x1a[i] + u1 * x1b[i];
+            x2[i] = (1.0 - u2) * x2a[i] + u2 * x2b[i];
+        }
+    } else if (i2c && !i2d) {
+        v_sub(x2a, x1a, dx);
+        if (v_dot(dx, n1c) < 0.0) { double m = (u2 < u2c) ? u2 : u2c; u2 = (0.0 < m) ? m : 0.0; }
+        else { double m = (u2 < 1.0) ? u2 : 1.0; u2 = (u2c < m) ? m : u2c; }
+        for (int i = 0; i < 3; ++i) x2[i] = (1.0 - u2) * x2a[i] + u2 * x2b[i];
+        u1 = linepoint(x1a, x1b, x2);
+        for (int i = 0; i < 3; ++i) x1[i] = (1.0 - u1) * x1a[i] + u1 * x1b[i];
+    } else if (!i2c && i2d) {
+        v_sub(x2a, x1b, dx);
+        if (v_dot(dx, n1d) < 0.0) { double m = (u2 < u2d) ? u2 : u2d; u2 = (0.0 < m) ? m : 0.0; }
+        else { double m = (u2 < 1.0) ? u2 : 1.0; u2 = (u2d < m) ? m : u2d; }
+        for (int i = 0; i < 3; ++i) x2[i] = (1.0 - u2) * x2a[i] + u2 * x2b[i];
+        u1 = linepoint(x1a, x1b, x2);
+        for (int i = 0; i < 3; ++i) x1[i] = (1.0 - u1) * x1a[i] + u1 * x1b[i];
+    } else {
+        return 0;
+    }
+    if (u1 < -thresh1 || u1 > 1.0 + thresh1 || u2 < -thresh2 || u2 > 1.0 + thresh2) return 0;
+    v_sub(x2, x1, dx);
+    const double th = 2.0 * thr;
+    if (v_dot(dx, dx) > th * th) return 0;
+    if (out) {
+        eolc_collision cc;
+        rec_init(&cc);
+        cc.dist = v_norm(dx);
+        v_copy(nor1, cc.nor1); v_copy(nor, cc.nor2);
+        v_copy(x1, cc.pos1); v_copy(x2, cc.pos2);
+        cc.count1 = 2; cc.count2 = 2;
+        cc.verts1[0] = kBoxEdgeVerts[k1][0]; cc.verts1[1] = kBoxEdgeVerts[k1][1]; cc.verts1[2] = -1;
+        cc.verts2[0] = ce.v0; cc.verts2[1] = ce.v1; cc.verts2[2] = -1;
+        cc.weights1[0] = 1.0 - u1; cc.weights1[1] = u1;
+        cc.weights2[0] = 1.0 - u2; cc.weights2[1] = u2;
+        cc.nedge1 = 1; cc.edge1[0] = k1;
+        cc.edge2 = k2;
+        v_copy(tan1, cc.edgeDir);
+        *out = cc;
+    }
+    return 1;
+}
+
+// Cloth edge k2 against the 12 box edges in order: the records' count; bit k1 of *ambig
+// as ee_pair sets it.
+CDQ int ee_edge(int k2, double thr, const BoxGeom &box, const int *cedges, const double *x, const double *xj,
+                const int *tri, eolc_collision *out, int *ambig, double band)
+{
+    ClothEdge ce;
+    cloth_edge(k2, cedges, x, xj, tri, ce);
     int cnt = 0;
     for (int k1 = 0; k1 < 12; ++k1) {
-        if (box.eangle[k1] < kPi / 6.0) continue;
-        if (!check_aabb(box.faabb[kBoxEdgeFaces[k1][0]], aabbE) && !check_aabb(box.faabb[kBoxEdgeFaces[k1][1]], aabbE))
-            continue;
-        const double *x1a = box.v[kBoxEdgeVerts[k1][0]], *x1b = box.v[kBoxEdgeVerts[k1][1]];
-        double dx1[3], tan1[3];
-        v_sub(x1b, x1a, dx1);
-        const double len1 = v_norm(dx1);
-        for (int i = 0; i < 3; ++i) tan1[i] = dx1[i] / len1;
-        double angle = acos(v_dot(tan1, nor2));
-        if (fabs(fabs(angle) - threshAng) < band || fabs(fabs(kPi - angle) - threshAng) < band) *ambig |= 1 << k1;
-        if (fabs(angle) < threshAng || fabs(kPi - angle) < threshAng) continue;
-        angle = acos(v_dot(tan1, dx2) / len2);
-        if (fabs(fabs(angle) - threshAng) < band || fabs(fabs(kPi - angle) - threshAng) < band) *ambig |= 1 << k1;
-        if (fabs(angle) < threshAng || fabs(kPi - angle) < threshAng) continue;
-        double nor[3], c[3];
-        v_cross(dx1, dx2, c);
-        v_normalized(c, nor);
-        const double *x1c = box.v[kBoxEdgeVerts[k1][2]], *x1d = box.v[kBoxEdgeVerts[k1][3]];
-        const double *n1c = box.en[k1][0], *n1d = box.en[k1][1];
-        double nor1[3];
-        v_add(n1c, n1d, nor1);
-        v_normalized(nor1, nor1);
-        if (v_dot(nor, nor1) < 0.0) v_neg(nor);
-        double angleCD = acos(v_dot(n1c, n1d));
-        double angleCN = acos(v_dot(n1c, nor));
-        if (angleCD < 0.0) { angleCD = -angleCD; angleCN = -angleCN; }
-        if (fabs(angleCN + threshAng) < band || fabs(angleCN - angleCD - threshAng) < band) *ambig |= 1 << k1;
-        if (angleCN < -threshAng || angleCN - angleCD > threshAng) continue;
-        double u2c = 0, u2d = 0;
-        int i2c = intersect_square(x2a, dx2, x1a, x1b, x1c, &u2c);
-        int i2d = intersect_square(x2a, dx2, x1b, x1a, x1d, &u2d);
-        i2c = i2c && (0.0 <= u2c && u2c <= 1.0);
-        i2d = i2d && (0.0 <= u2d && u2d <= 1.0);
-        double u1, u2;
-        lineline(&u1, &u2, x1a, x1b, x2a, x2b);
-        const double thresh1 = 1.0 * thr / len1, thresh2 = 1.0 * thr / len2;
-        if (u1 < -thresh1 || u1 > 1.0 + thresh1 || u2 < -thresh2 || u2 > 1.0 + thresh2) continue;
-        double x1[3], x2[3], dx[3];
-        if (i2c && i2d) {
-            for (int i = 0; i < 3; ++i) {
-                x1[i] = (1.0 - u1) * x1a[i] + u1 * x1b[i];
-                x2[i] = (1.0 - u2) * x2a[i] + u2 * x2b[i];
-            }
-        } else if (i2c && !i2d) {
-            v_sub(x2a, x1a, dx);
-            if (v_dot(dx, n1c) < 0.0) { double m = (u2 < u2c) ? u2 : u2c; u2 = (0.0 < m) ? m : 0.0; }
-            else { double m = (u2 < 1.0) ? u2 : 1.0; u2 = (u2c < m) ? m : u2c; }
-            for (int i = 0; i < 3; ++i) x2[i] = (1.0 - u2) * x2a[i] + u2 * x2b[i];
-            u1 = linepoint(x1a, x1b, x2);
-            for (int i = 0; i < 3; ++i) x1[i] = (1.0 - u1) * x1a[i] + u1 * x1b[i];
-        } else if (!i2c && i2d) {
-            v_sub(x2a, x1b, dx);
-            if (v_dot(dx, n1d) < 0.0) { double m = (u2 < u2d) ? u2 : u2d; u2 = (0.0 < m) ? m : 0.0; }
-            else { double m = (u2 < 1.0) ? u2 : 1.0; u2 = (u2d < m) ? m : u2d; }
-            for (int i = 0; i < 3; ++i) x2[i] = (1.0 - u2) * x2a[i] + u2 * x2b[i];
-            u1 = linepoint(x1a, x1b, x2);
-            for (int i = 0; i < 3; ++i) x1[i] = (1.0 - u1) * x1a[i] + u1 * x1b[i];
-        } else {
-            continue;
-        }
-        if (u1 < -thresh1 || u1 > 1.0 + thresh1 || u2 < -thresh2 || u2 > 1.0 + thresh2) continue;
-        v_sub(x2, x1, dx);
-        const double th = 2.0 * thr;
-        if (v_dot(dx, dx) > th * th) continue;
-        if (out) {
-            eolc_collision cc;
-            rec_init(&cc);
-            cc.dist = v_norm(dx);
-            v_copy(nor1, cc.nor1); v_copy(nor, cc.nor2);
-            v_copy(x1, cc.pos1); v_copy(x2, cc.pos2);
-            cc.count1 = 2; cc.count2 = 2;
-            cc.verts1[0] = kBoxEdgeVerts[k1][0]; cc.verts1[1] = kBoxEdgeVerts[k1][1]; cc.verts1[2] = -1;
-            cc.verts2[0] = e2[0]; cc.verts2[1] = e2[1]; cc.verts2[2] = -1;
-            cc.weights1[0] = 1.0 - u1; cc.weights1[1] = u1;
-            cc.weights2[0] = 1.0 - u2; cc.weights2[1] = u2;
-            cc.nedge1 = 1; cc.edge1[0] = k1;
-            cc.edge2 = k2;
-            v_copy(tan1, cc.edgeDir);
-            out[cnt] = cc;
-        }
-        ++cnt;
+        int amb = 0;
+        cnt += ee_pair(k2, k1, thr, box, ce, out ? out + cnt : nullptr, &amb, band);
+        if (amb) *ambig |= 1 << k1;
     }
     return cnt;
 }

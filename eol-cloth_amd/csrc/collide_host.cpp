@@ -12,6 +12,7 @@
 //  - records are assembled in the reference's order: point records, then per box
 //    V2-T1, V1-T2, E2-E1, corner de-duplication and the pos1_ snap.
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <random>
@@ -30,15 +31,16 @@ hipError_t cd_grid_build(eolc_ctx *c, const CdGrid &gp, const double *xj, unsign
                          bool fill);
 hipError_t cd_query(eolc_ctx *c, const CdGrid &gp, int Q, const double *qpts, const double *qnrm, double thr,
                     const double *aabb, const double *xj, const double *fn, const unsigned *bstart, const unsigned *bcnt,
-                    const int *entries, const unsigned *nalways, const int *always, int *face, eolc_collision *rec);
-hipError_t cd_v2t1(eolc_ctx *c, double thr, const BoxGeom *box, const double *xj, const double *fn, int *flag,
-                   eolc_collision *rec, int *err);
-hipError_t cd_eolpts(eolc_ctx *c, int P, double thr, const double *pts, const double *nrm, const double *xj, int *flag,
-                     eolc_collision *rec);
-hipError_t cd_ee(eolc_ctx *c, int pass, double thr, const BoxGeom *box, const double *xj, unsigned *counts,
-                 const unsigned *offsets, int *ambig, eolc_collision *out);
-hipError_t cd_compact(eolc_ctx *c, int n, const int *flag, unsigned *u32, unsigned *offs, unsigned *sums,
-                      unsigned *total, const eolc_collision *rec, eolc_collision *out, bool write);
+                    const int *entries, const unsigned *nalways, const int *always, eolc_collision *rec);
+hipError_t cd_sweep(eolc_ctx *c, int Q, const double *qpts, const double *qnrm, double thr, const double *aabb,
+                    const double *xj, const double *fn, unsigned *ncand, void *cand, eolc_collision *rec);
+hipError_t cd_eolpts(eolc_ctx *c, int P, double thr, const double *pts, const double *nrm, const double *xj,
+                     unsigned *cnt, const unsigned *offs, eolc_collision *out);
+hipError_t cd_boxes(eolc_ctx *c, int b0, int b1, double thr, const BoxGeom *boxes, const double *xj, const double *fn,
+                    unsigned *cnt, const unsigned *offs, unsigned *npairs, unsigned *pairs, unsigned *nambig,
+                    unsigned *err, eolc_collision *out);
+hipError_t cd_ambiguous(eolc_ctx *c, double thr, const BoxGeom *box, const double *xj, int *ambig);
+hipError_t cd_first(eolc_ctx *c, int nb, const unsigned *offs, unsigned *first);
 size_t cd_scan_words(size_t n);
 hipError_t cd_scan(eolc_ctx *c, unsigned n, const unsigned *in, unsigned *out, unsigned *sums, unsigned *total);
 }  // namespace eolc
@@ -245,8 +247,9 @@ unsigned grid_table_size(int F)
     return tbl;
 }
 
-// Device bytes a collide call needs before the data-dependent buffers (the grid's
-// entry list and the record outputs), alignment included.
+// A bound of the device bytes of a collide call before the data-dependent buffers (the
+// grid's entry list and the record outputs), alignment included; what
+// eolc_collide_noalloc refuses a query by.
 size_t collide_fixed_bytes(const eolc_ctx *c, int P, int B)
 {
     const size_t N = (size_t)c->topo.N, F = (size_t)c->topo.F, E = (size_t)c->n_cedges;
@@ -257,27 +260,29 @@ size_t collide_fixed_bytes(const eolc_ctx *c, int P, int B)
     return bytes + 256 * 32;
 }
 
-int collide_impl(eolc_ctx *c, Workspace &ws, double thr, int P, const double *pts, const double *nrm, int B,
-                 const double *whd, const double *Eb, int eol_points, int box_npts, int box_nedges,
-                 std::vector<eolc_collision> &out)
+// Up to this many queries are swept over all faces; more build the grid.  The sweep costs
+// F x Q box tests, the grid two passes of atomics over the faces' cells, a scan and a
+// host read whatever Q is.
+constexpr int kCdSweepQueries = 2048;
+
+// What the first read-back of a call holds, before the query records.
+struct CdStatus {
+    unsigned ncand, err;
+    unsigned npairs, nambig[eolc::kCdBoxes];   // cleared per group of boxes
+    unsigned first[2 * eolc::kCdBoxes + 1];
+};
+
+// The queries against the uniform grid over the cloth faces.
+int query_grid(eolc_ctx *c, Workspace &ws, double thr, int Q, const double *qpts, const double *qnrm, const double *xj,
+               const double *fn, const double *aabb, eolc_collision *qrec)
 {
-    const int N = c->topo.N, F = c->topo.F;
-    double *xj = nullptr, *fn = nullptr, *aabb_part = nullptr, *aabb = nullptr;
-    EOLC_HIP(ws.get(&xj, 3 * (size_t)N));
-    EOLC_HIP(ws.get(&fn, 3 * (size_t)F));
-    EOLC_HIP(ws.get(&aabb_part, 6 * 256));
-    EOLC_HIP(ws.get(&aabb, 6));
-    EOLC_HIP(eolc::cd_prep(c, thr, xj, fn, aabb_part, aabb));
+    const int F = c->topo.F;
     double hab[6];
     EOLC_HIP(hipMemcpyAsync(hab, aabb, sizeof(hab), hipMemcpyDeviceToHost, c->stream));
     EOLC_HIP(hipStreamSynchronize(c->stream));
-    // boxes
-    std::vector<BoxGeom> boxes((size_t)B);
-    for (int b = 0; b < B; ++b) make_box(boxes[b], whd + 3 * b, Eb + 16 * b);
-    // ---- uniform grid over the cloth faces
     CdGrid g;
     const double L = std::max({hab[3] - hab[0], hab[4] - hab[1], hab[5] - hab[2], 1e-300});
-    g.margin = 5.0 * thr * (1.0 + 1e-6) + 1e-7 * L + 1e-12;
+    g.margin = grid_margin(thr, L);
     const double area = std::max((hab[3] - hab[0]) * (hab[4] - hab[1]), 1e-300);
     double cell = std::max(2.0 * g.margin, std::sqrt(area / std::max(F, 1)) * 4.0);
     int dims[3];
@@ -294,8 +299,9 @@ int collide_impl(eolc_ctx *c, Workspace &ws, double thr, int P, const double *pt
     g.inv_cell = 1.0 / cell;
     const unsigned tbl = grid_table_size(F);
     g.mask = tbl - 1;
-    g.cond_max = 1e6;
-    unsigned *bcnt = nullptr, *bstart = nullptr, *cursor = nullptr, *total = nullptr, *nalways = nullptr;
+    g.cond_max = kGridCondMax;
+    const size_t m = ws.mark();
+    unsigned *bcnt = nullptr, *bstart = nullptr, *cursor = nullptr, *total = nullptr, *nalways = nullptr, *sums = nullptr;
     int *always = nullptr, *entries = nullptr;
     EOLC_HIP(ws.get(&bcnt, tbl));
     EOLC_HIP(ws.get(&bstart, tbl));
@@ -303,8 +309,7 @@ int collide_impl(eolc_ctx *c, Workspace &ws, double thr, int P, const double *pt
     EOLC_HIP(ws.get(&total, 1));
     EOLC_HIP(ws.get(&nalways, 1));
     EOLC_HIP(ws.get(&always, (size_t)F));
-    unsigned *sums = nullptr;
-    EOLC_HIP(ws.get(&sums, eolc::cd_scan_words(std::max<size_t>({tbl, (size_t)N, (size_t)c->n_cedges}))));
+    EOLC_HIP(ws.get(&sums, eolc::cd_scan_words(tbl)));
     EOLC_HIP(hipMemsetAsync(bcnt, 0, tbl * sizeof(unsigned), c->stream));
     EOLC_HIP(hipMemsetAsync(cursor, 0, tbl * sizeof(unsigned), c->stream));
     EOLC_HIP(hipMemsetAsync(nalways, 0, sizeof(unsigned), c->stream));
@@ -314,9 +319,27 @@ int collide_impl(eolc_ctx *c, Workspace &ws, double thr, int P, const double *pt
     EOLC_HIP(hipStreamSynchronize(c->stream));
     EOLC_HIP(ws.get(&entries, nentries));
     EOLC_HIP(eolc::cd_grid_build(c, g, xj, bcnt, bstart, cursor, entries, nalways, always, sums, total, true));
-    // ---- point / corner queries against the faces
-    const int Q = P + 8 * B;
-    std::vector<double> hq(3 * (size_t)std::max(Q, 1)), hn(3 * (size_t)std::max(Q, 1));
+    EOLC_HIP(eolc::cd_query(c, g, Q, qpts, qnrm, thr, aabb, xj, fn, bstart, bcnt, entries, nalways, always, qrec));
+    if (ws.base) ws.release(m);   // (the kernels of this stream are done with it before the next ones start)
+    return EOLC_OK;
+}
+
+int collide_impl(eolc_ctx *c, Workspace &ws, double thr, int P, const double *pts, const double *nrm, int B,
+                 const double *whd, const double *Eb, int eol_points, int box_npts, int box_nedges,
+                 std::vector<eolc_collision> &out)
+{
+    const int N = c->topo.N, F = c->topo.F, E = c->n_cedges;
+    const size_t NE = (size_t)N + E;
+    // boxes per launch: their counts are numbered with 31 bits
+    const int group = std::max(1, (int)std::min<size_t>(eolc::kCdBoxes, INT_MAX / NE));
+    const int Q = P + 8 * B, nbg = std::min(B, group);
+    // ---- queries and boxes in one upload: points and corners, their normals, the boxes
+    std::vector<BoxGeom> boxes((size_t)B);
+    for (int b = 0; b < B; ++b) make_box(boxes[b], whd + 3 * b, Eb + 16 * b);
+    const size_t nbox = sizeof(BoxGeom) / sizeof(double);
+    static_assert(sizeof(BoxGeom) % sizeof(double) == 0, "boxes are packed behind the queries");
+    std::vector<double> hin(6 * (size_t)Q + nbox * (size_t)B);
+    double *hq = hin.data(), *hn = hq + 3 * (size_t)Q;
     for (int i = 0; i < 3 * P; ++i) { hq[i] = pts[i]; hn[i] = nrm[i]; }
     for (int b = 0; b < B; ++b)
         for (int i1 = 0; i1 < 8; ++i1)
@@ -324,197 +347,219 @@ int collide_impl(eolc_ctx *c, Workspace &ws, double thr, int P, const double *pt
                 hq[3 * (P + 8 * b + i1) + k] = boxes[b].v[i1][k];
                 hn[3 * (P + 8 * b + i1) + k] = boxes[b].vn[i1][k];
             }
-    double *qpts = nullptr, *qnrm = nullptr;
-    int *qface = nullptr;
-    eolc_collision *qrec = nullptr;
-    EOLC_HIP(ws.get(&qpts, hq.size()));
-    EOLC_HIP(ws.get(&qnrm, hn.size()));
-    EOLC_HIP(ws.get(&qface, std::max(Q, 1)));
-    EOLC_HIP(ws.get(&qrec, std::max(Q, 1)));
-    std::vector<eolc_collision> qres((size_t)std::max(Q, 1));
-    if (Q > 0) {
-        EOLC_HIP(hipMemcpyAsync(qpts, hq.data(), hq.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
-        EOLC_HIP(hipMemcpyAsync(qnrm, hn.data(), hn.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
-        EOLC_HIP(eolc::cd_query(c, g, Q, qpts, qnrm, thr, aabb, xj, fn, bstart, bcnt, entries, nalways, always, qface,
-                                qrec));
-        EOLC_HIP(hipMemcpyAsync(qres.data(), qrec, sizeof(eolc_collision) * Q, hipMemcpyDeviceToHost, c->stream));
+    if (B) std::memcpy(hn + 3 * (size_t)Q, boxes.data(), sizeof(BoxGeom) * B);
+    double *xj = nullptr, *fn = nullptr, *aabb_part = nullptr, *aabb = nullptr, *din = nullptr;
+    char *dst = nullptr, *cand = nullptr;
+    unsigned *cnt = nullptr, *offs = nullptr, *sums = nullptr, *pairs = nullptr;
+    const size_t nst = sizeof(CdStatus) + sizeof(eolc_collision) * (size_t)Q;
+    const size_t ncnt = std::max(NE * nbg, eol_points && P > 0 ? (size_t)N : 0);
+    EOLC_HIP(ws.get(&xj, 3 * (size_t)N));
+    EOLC_HIP(ws.get(&fn, 3 * (size_t)F));
+    EOLC_HIP(ws.get(&aabb_part, 6 * 256));
+    EOLC_HIP(ws.get(&aabb, 6));
+    EOLC_HIP(ws.get(&din, hin.size()));
+    EOLC_HIP(ws.get(&dst, nst));
+    EOLC_HIP(ws.get(&cnt, ncnt));
+    EOLC_HIP(ws.get(&offs, ncnt + 1));
+    EOLC_HIP(ws.get(&sums, eolc::cd_scan_words(ncnt)));
+    EOLC_HIP(ws.get(&pairs, (size_t)E * nbg));
+    CdStatus *dstat = reinterpret_cast<CdStatus *>(dst);
+    eolc_collision *qrec = reinterpret_cast<eolc_collision *>(dst + sizeof(CdStatus));
+    static_assert(sizeof(CdStatus) % 8 == 0, "records follow the status");
+    const double *qpts = din, *qnrm = din + 3 * (size_t)Q;
+    const BoxGeom *dbox = reinterpret_cast<const BoxGeom *>(din + 6 * (size_t)Q);
+    if (!hin.empty())
+        EOLC_HIP(hipMemcpyAsync(din, hin.data(), hin.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    EOLC_HIP(hipMemsetAsync(dst, 0, sizeof(CdStatus), c->stream));
+    EOLC_HIP(eolc::cd_prep(c, thr, xj, fn, aabb_part, aabb));
+    // ---- point / corner queries against the faces
+    const bool sweep = Q > 0 && Q <= kCdSweepQueries;
+    if (sweep) {
+        EOLC_HIP(ws.get(&cand, 16 * (size_t)eolc::kCdCandidates));
+        EOLC_HIP(eolc::cd_sweep(c, Q, qpts, qnrm, thr, aabb, xj, fn, &dstat->ncand, cand, qrec));
+    } else if (Q > 0) {
+        const int rc = query_grid(c, ws, thr, Q, qpts, qnrm, xj, fn, aabb, qrec);
+        if (rc) return rc;
     }
-    // ---- per-vertex passes (EOL points and V2-T1) share flag/record buffers
-    int *flag = nullptr, *err = nullptr;
-    eolc_collision *vrec = nullptr;
-    unsigned *u32 = nullptr, *offs = nullptr;
-    EOLC_HIP(ws.get(&flag, (size_t)N));
-    EOLC_HIP(ws.get(&vrec, (size_t)N));
-    EOLC_HIP(ws.get(&u32, (size_t)N));
-    EOLC_HIP(ws.get(&offs, (size_t)N));
-    EOLC_HIP(ws.get(&err, 1));
-    EOLC_HIP(hipMemsetAsync(err, 0, sizeof(int), c->stream));
-    auto per_vertex_records = [&](std::vector<eolc_collision> &dst) -> int {
-        EOLC_HIP(eolc::cd_compact(c, N, flag, u32, offs, sums, total, nullptr, nullptr, false));
-        unsigned cnt = 0;
-        EOLC_HIP(hipMemcpyAsync(&cnt, total, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
-        EOLC_HIP(hipStreamSynchronize(c->stream));
-        dst.resize(cnt);
-        if (cnt) {
-            const size_t m = ws.mark();
-            eolc_collision *o = nullptr;
-            EOLC_HIP(ws.get(&o, cnt));
-            EOLC_HIP(eolc::cd_compact(c, N, flag, u32, offs, sums, total, vrec, o, true));
-            EOLC_HIP(hipMemcpyAsync(dst.data(), o, sizeof(eolc_collision) * cnt, hipMemcpyDeviceToHost, c->stream));
-            EOLC_HIP(hipStreamSynchronize(c->stream));
-            ws.release(m);
-        }
+    std::vector<char> hst(nst);
+    auto status = [&]() -> const CdStatus & { return *reinterpret_cast<const CdStatus *>(hst.data()); };
+    auto qres = [&](int q) {
+        eolc_collision r;
+        std::memcpy(&r, hst.data() + sizeof(CdStatus) + sizeof(eolc_collision) * (size_t)q, sizeof(r));
+        return r;
+    };
+    // counts, offsets and read-back of one group of boxes
+    auto count_boxes = [&](int g0, int nb) -> int {
+        EOLC_HIP(eolc::cd_boxes(c, 0, nb, thr, dbox + g0, xj, fn, cnt, nullptr, &dstat->npairs, pairs, dstat->nambig,
+                                &dstat->err, nullptr));
+        EOLC_HIP(eolc::cd_scan(c, (unsigned)(NE * nb), cnt, offs, sums, offs + NE * nb));
+        EOLC_HIP(eolc::cd_first(c, nb, offs, dstat->first));
         return EOLC_OK;
     };
+    auto read_status = [&](size_t bytes) -> int {
+        EOLC_HIP(hipMemcpyAsync(hst.data(), dst, bytes, hipMemcpyDeviceToHost, c->stream));
+        EOLC_HIP(hipStreamSynchronize(c->stream));
+        return EOLC_OK;
+    };
+    int rc = EOLC_OK;
+    const bool eol_pass = eol_points && P > 0;
+    if (!eol_pass && nbg && (rc = count_boxes(0, nbg))) return rc;   // (the EOL pass uses the counts first)
+    if ((rc = read_status(nst))) return rc;
+    if (sweep && status().ncand > eolc::kCdCandidates) {
+        if ((rc = query_grid(c, ws, thr, Q, qpts, qnrm, xj, fn, aabb, qrec))) return rc;
+        if ((rc = read_status(nst))) return rc;
+    }
     const double snap = 0.1 * thr;
     auto snap_all = [&](std::vector<eolc_collision> &v, size_t from) {
         for (size_t k = from; k < v.size(); ++k)
             for (int i = 0; i < 3; ++i) v[k].pos1_[i] = v[k].pos1[i] - snap * v[k].nor1[i];
     };
     // ---- pointTriCollision
-    if (eol_points && P > 0) {
-        double *dpts = nullptr, *dnrm = nullptr;
-        EOLC_HIP(ws.get(&dpts, 3 * (size_t)P));
-        EOLC_HIP(ws.get(&dnrm, 3 * (size_t)P));
-        EOLC_HIP(hipMemcpyAsync(dpts, pts, 3 * (size_t)P * sizeof(double), hipMemcpyHostToDevice, c->stream));
-        EOLC_HIP(hipMemcpyAsync(dnrm, nrm, 3 * (size_t)P * sizeof(double), hipMemcpyHostToDevice, c->stream));
-        EOLC_HIP(eolc::cd_eolpts(c, P, thr, dpts, dnrm, xj, flag, vrec));
-        std::vector<eolc_collision> ev;
-        int rc = per_vertex_records(ev);
-        if (rc) return rc;
-        out.insert(out.end(), ev.begin(), ev.end());
-    } else {
+    if (eol_pass) {
+        // (P <= Q: the points and their normals are the first of the queries)
+        EOLC_HIP(eolc::cd_eolpts(c, P, thr, qpts, qnrm, xj, cnt, nullptr, nullptr));
+        EOLC_HIP(eolc::cd_scan(c, (unsigned)N, cnt, offs, sums, offs + N));
+        unsigned ne = 0;
+        EOLC_HIP(hipMemcpyAsync(&ne, offs + N, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
         EOLC_HIP(hipStreamSynchronize(c->stream));
+        if (ne) {
+            const size_t m = ws.mark();
+            eolc_collision *o = nullptr;
+            EOLC_HIP(ws.get(&o, ne));
+            out.resize(ne);
+            EOLC_HIP(eolc::cd_eolpts(c, P, thr, qpts, qnrm, xj, cnt, offs, o));
+            EOLC_HIP(hipMemcpyAsync(out.data(), o, sizeof(eolc_collision) * ne, hipMemcpyDeviceToHost, c->stream));
+            EOLC_HIP(hipStreamSynchronize(c->stream));
+            ws.release(m);
+        }
     }
     for (int i1 = 0; i1 < P; ++i1) {
-        eolc_collision r = qres[i1];
+        eolc_collision r = qres(i1);
         if (r.count1 == 0) continue;
         r.verts1[0] = i1;
         out.push_back(r);
     }
     snap_all(out, 0);
-    // ---- boxTriCollision per box
-    BoxGeom *dbox = nullptr;
-    unsigned *ecnt = nullptr, *eoff = nullptr;
-    int *eamb = nullptr;
-    EOLC_HIP(ws.get(&dbox, 1));
-    const int E = c->n_cedges;
-    EOLC_HIP(ws.get(&ecnt, (size_t)E));
-    EOLC_HIP(ws.get(&eoff, (size_t)E));
-    EOLC_HIP(ws.get(&eamb, (size_t)E));
+    // ---- boxTriCollision per box, a group of boxes at a time
     std::vector<double> hx, hxj;   // host copies, only if an acos decision must be re-made
-    const size_t base_after_points = out.size();
-    for (int b = 0; b < B; ++b) {
-        std::vector<eolc_collision> clst;
-        EOLC_HIP(hipMemcpyAsync(dbox, &boxes[b], sizeof(BoxGeom), hipMemcpyHostToDevice, c->stream));
-        // V2-T1
-        EOLC_HIP(eolc::cd_v2t1(c, thr, dbox, xj, fn, flag, vrec, err));
-        {
-            std::vector<eolc_collision> vv;
-            int rc = per_vertex_records(vv);
-            if (rc) return rc;
-            clst.insert(clst.end(), vv.begin(), vv.end());
+    std::vector<eolc_collision> recs, clst;
+    for (int g0 = 0; g0 < B; g0 += group) {
+        const int nb = std::min(B - g0, group);
+        if (g0 > 0 || eol_pass) {
+            EOLC_HIP(hipMemsetAsync(&dstat->npairs, 0, sizeof(unsigned) * (1 + eolc::kCdBoxes), c->stream));
+            if ((rc = count_boxes(g0, nb)) || (rc = read_status(sizeof(CdStatus)))) return rc;
         }
-        // V1-T2
-        for (int i1 = 0; i1 < 8; ++i1) {
-            eolc_collision r = qres[P + 8 * b + i1];
-            if (r.count1 == 0) continue;
-            r.verts1[0] = i1;
-            r.nedge1 = 3;
-            for (int i = 0; i < 3; ++i) r.edge1[i] = kBoxVertEdges[i1][i];
-            clst.push_back(r);
+        const CdStatus st = status();
+        if (st.err) {
+            c->err = "collide: a cloth vertex with index >= face count reached the face-normal lookup of V2-T1 "
+                     "(boxTriCollision.cpp:731 indexes face normals by vertex index)";
+            return EOLC_ERR_INVALID;
         }
-        // E2-E1
-        if (E > 0) {
-            EOLC_HIP(eolc::cd_ee(c, 0, thr, dbox, xj, ecnt, nullptr, eamb, nullptr));
-            EOLC_HIP(eolc::cd_scan(c, (unsigned)E, ecnt, eoff, sums, total));
-            unsigned ne = 0;
-            EOLC_HIP(hipMemcpyAsync(&ne, total, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
-            std::vector<int> amb((size_t)E);
-            EOLC_HIP(hipMemcpyAsync(amb.data(), eamb, sizeof(int) * E, hipMemcpyDeviceToHost, c->stream));
+        // the group's records, box after box, vertices before edges: in one piece, or box by
+        // box where a fixed workspace has no room for all
+        recs.resize(st.first[2 * nb]);
+        const size_t m = ws.mark();
+        eolc_collision *o = nullptr;
+        const bool whole = recs.empty() || ws.get(&o, recs.size()) == hipSuccess;
+        if (!whole && !ws.base) EOLC_HIP(hipErrorOutOfMemory);
+        if (!whole) ws.exhausted = false;
+        for (int b = 0; b < nb; b += whole ? nb : 1) {
+            const int b1 = whole ? nb : b + 1;
+            const size_t r0 = st.first[2 * b], n = st.first[2 * b1] - r0;
+            if (!n) continue;
+            if (!whole) EOLC_HIP(ws.get(&o, n));
+            EOLC_HIP(eolc::cd_boxes(c, b, b1, thr, dbox + g0, xj, fn, cnt, offs, &dstat->npairs, pairs, nullptr,
+                                    &dstat->err, o));
+            EOLC_HIP(hipMemcpyAsync(recs.data() + r0, o, sizeof(eolc_collision) * n, hipMemcpyDeviceToHost, c->stream));
             EOLC_HIP(hipStreamSynchronize(c->stream));
-            std::vector<eolc_collision> ee(ne);
-            if (ne) {
-                const size_t m = ws.mark();
-                eolc_collision *o = nullptr;
-                EOLC_HIP(ws.get(&o, ne));
-                EOLC_HIP(eolc::cd_ee(c, 1, thr, dbox, xj, ecnt, eoff, eamb, o));
-                EOLC_HIP(hipMemcpyAsync(ee.data(), o, sizeof(eolc_collision) * ne, hipMemcpyDeviceToHost, c->stream));
-                EOLC_HIP(hipStreamSynchronize(c->stream));
-                ws.release(m);
+            if (!whole) ws.release(m);
+        }
+        if (whole) ws.release(m);
+        for (int bg = 0; bg < nb; ++bg) {
+            const int b = g0 + bg;
+            const auto v0 = recs.begin() + st.first[2 * bg], v1 = recs.begin() + st.first[2 * bg + 1],
+                       e1 = recs.begin() + st.first[2 * bg + 2];
+            // V2-T1
+            clst.assign(v0, v1);
+            // V1-T2
+            for (int i1 = 0; i1 < 8; ++i1) {
+                eolc_collision r = qres(P + 8 * b + i1);
+                if (r.count1 == 0) continue;
+                r.verts1[0] = i1;
+                r.nedge1 = 3;
+                for (int i = 0; i < 3; ++i) r.edge1[i] = kBoxVertEdges[i1][i];
+                clst.push_back(r);
             }
-            // re-decide edges whose angle tests were within the band, with the C library acos
-            bool any = std::any_of(amb.begin(), amb.end(), [](int m) { return m != 0; });
-            if (any) {
+            // E2-E1; edges whose angle tests were within the band are re-decided with the C
+            // library's acos
+            if (!st.nambig[bg]) {
+                clst.insert(clst.end(), v1, e1);
+            } else {
+                std::vector<int> amb((size_t)E);
+                int *eamb = nullptr;
+                const size_t ma = ws.mark();
+                EOLC_HIP(ws.get(&eamb, (size_t)E));
+                EOLC_HIP(eolc::cd_ambiguous(c, thr, dbox + b, xj, eamb));
+                EOLC_HIP(hipMemcpyAsync(amb.data(), eamb, sizeof(int) * (size_t)E, hipMemcpyDeviceToHost, c->stream));
                 if (hx.empty()) {
                     hx.resize(3 * (size_t)N);
                     hxj.resize(3 * (size_t)N);
-                    EOLC_HIP(hipMemcpy(hx.data(), c->x, hx.size() * sizeof(double), hipMemcpyDeviceToHost));
-                    EOLC_HIP(hipMemcpy(hxj.data(), xj, hxj.size() * sizeof(double), hipMemcpyDeviceToHost));
+                    EOLC_HIP(hipMemcpyAsync(hx.data(), c->x, hx.size() * sizeof(double), hipMemcpyDeviceToHost,
+                                            c->stream));
+                    EOLC_HIP(hipMemcpyAsync(hxj.data(), xj, hxj.size() * sizeof(double), hipMemcpyDeviceToHost,
+                                            c->stream));
                 }
-                std::vector<eolc_collision> fixed;
-                size_t pos = 0;
+                EOLC_HIP(hipStreamSynchronize(c->stream));
+                ws.release(ma);
+                auto pos = v1;
                 for (int k2 = 0; k2 < E; ++k2) {
                     // records of edge k2 are contiguous and ordered by k2
-                    size_t end = pos;
-                    while (end < ee.size() && ee[end].edge2 == k2) ++end;
+                    auto end = pos;
+                    while (end != e1 && end->edge2 == k2) ++end;
                     if (amb[k2]) {
                         eolc_collision tmp[12];
                         int mask = 0;
-                        int n = ee_edge(k2, thr, boxes[b], c->h_cedges.data(), hx.data(), hxj.data(),
-                                        c->topo_tri.data(), tmp, &mask, 0.0);
-                        fixed.insert(fixed.end(), tmp, tmp + n);
+                        const int n = ee_edge(k2, thr, boxes[b], c->h_cedges.data(), hx.data(), hxj.data(),
+                                              c->topo_tri.data(), tmp, &mask, 0.0);
+                        clst.insert(clst.end(), tmp, tmp + n);
                     } else {
-                        fixed.insert(fixed.end(), ee.begin() + pos, ee.begin() + end);
+                        clst.insert(clst.end(), pos, end);
                     }
                     pos = end;
                 }
-                ee.swap(fixed);
                 c->cd_host_decisions += 1;
             }
-            clst.insert(clst.end(), ee.begin(), ee.end());
-        }
-        // corner de-duplication (boxTriCollision.cpp:1020-1052)
-        for (int i1 = 0; i1 < 8; ++i1) {
-            int kmin = -1;
-            double dmin = 1e9;
-            for (size_t k = 0; k < clst.size(); ++k)
-                if (clst[k].count1 == 1 && clst[k].verts1[0] == i1) {
-                    double dx[3];
-                    v_sub(clst[k].pos2, boxes[b].v[i1], dx);
-                    double d = v_dot(dx, dx);
-                    if (d < dmin) { kmin = (int)k; dmin = d; }
-                }
-            if (kmin != -1) {
-                std::vector<size_t> dl;
+            // corner de-duplication (boxTriCollision.cpp:1020-1052)
+            for (int i1 = 0; i1 < 8; ++i1) {
+                int kmin = -1;
+                double dmin = 1e9;
                 for (size_t k = 0; k < clst.size(); ++k)
-                    if (clst[k].count1 == 1 && clst[k].verts1[0] == i1 && (int)k != kmin) dl.push_back(k);
-                for (size_t kd : dl) {
-                    clst[kd] = clst.back();
-                    clst.pop_back();
+                    if (clst[k].count1 == 1 && clst[k].verts1[0] == i1) {
+                        double dx[3];
+                        v_sub(clst[k].pos2, boxes[b].v[i1], dx);
+                        double d = v_dot(dx, dx);
+                        if (d < dmin) { kmin = (int)k; dmin = d; }
+                    }
+                if (kmin != -1) {
+                    std::vector<size_t> dl;
+                    for (size_t k = 0; k < clst.size(); ++k)
+                        if (clst[k].count1 == 1 && clst[k].verts1[0] == i1 && (int)k != kmin) dl.push_back(k);
+                    for (size_t kd : dl) {
+                        clst[kd] = clst.back();
+                        clst.pop_back();
+                    }
                 }
             }
+            snap_all(clst, 0);
+            if (eol_points)
+                // CD: box feature indices shifted per obstacle (Collisions.cpp:38-49)
+                for (eolc_collision &r : clst) {
+                    const int base = P + b * box_npts + b * box_nedges;
+                    if (r.count1 == 1 && r.count2 == 3) r.verts1[0] = base + r.verts1[0];
+                    for (int e = 0; e < r.nedge1; ++e) r.edge1[e] = base + (box_npts + r.edge1[e]);
+                }
+            out.insert(out.end(), clst.begin(), clst.end());
         }
-        snap_all(clst, 0);
-        out.insert(out.end(), clst.begin(), clst.end());
-        if (eol_points) {
-            // CD: box feature indices shifted per obstacle (Collisions.cpp:38-49)
-            const size_t start = out.size() - clst.size();
-            for (size_t k = start; k < out.size(); ++k) {
-                eolc_collision &r = out[k];
-                const int base = P + b * box_npts + b * box_nedges;
-                if (r.count1 == 1 && r.count2 == 3) r.verts1[0] = base + r.verts1[0];
-                for (int e = 0; e < r.nedge1; ++e) r.edge1[e] = base + (box_npts + r.edge1[e]);
-            }
-        }
-    }
-    (void)base_after_points;
-    int herr = 0;
-    EOLC_HIP(hipMemcpy(&herr, err, sizeof(int), hipMemcpyDeviceToHost));
-    if (herr) {
-        c->err = "collide: a cloth vertex with index >= face count reached the face-normal lookup of V2-T1 "
-                 "(boxTriCollision.cpp:731 indexes face normals by vertex index)";
-        return EOLC_ERR_INVALID;
     }
     return EOLC_OK;
 }

@@ -21,12 +21,17 @@
 //                   face the brute-force loop would accept, and the lexicographic
 //                   minimum (dist, face index) reproduces the reference's
 //                   "strictly closer wins, first wins ties".
-//   k_cd_query      one workgroup per query (point obstacle or box corner)
-//   k_cd_v2t1       one thread per cloth vertex (box V2-T1)
-//   k_cd_ee         one thread per cloth edge, 12 box edges each (box E2-E1)
+//   k_cd_query      one workgroup per query (point obstacle or box corner), on the grid
+//   k_cd_sweep      one thread per face against every query, and k_cd_nearest, the
+//                   nearest of a query's candidates: what up to kCdSweepQueries queries
+//                   take instead of the grid, which is built anew for every call
+//   k_cd_boxes      one thread per cloth vertex (V2-T1) and per cloth edge (which boxes'
+//                   faces it reaches), for up to kCdBoxes boxes in one launch
+//   k_cd_pairs      E2-E1 of the edges and boxes left, 12 lanes each
 //   k_cd_eolpts     one thread per cloth vertex (pointTri EOL branch)
-// Variable-length outputs are compacted in reference order by count -> scan ->
-// write passes (no atomics on record positions).
+// Variable-length outputs come in the reference's order by count -> scan -> write
+// passes (no atomics on record positions); the write pass forms a record anew
+// instead of keeping room for one per vertex.
 #include <algorithm>
 #include <mutex>
 
@@ -269,9 +274,10 @@ struct Best {
     int face;
 };
 
-__device__ __forceinline__ void consider(const double *x1, const double *nor1, double thr, int j2,
-                                         const double *__restrict__ xj, const int *__restrict__ tri,
-                                         const double *__restrict__ fn, Best &best)
+// The reference's tests of one query against one face; its distance when they pass.
+__device__ __forceinline__ bool accepts(const double *x1, const double *nor1, double thr, int j2,
+                                        const double *__restrict__ xj, const int *__restrict__ tri,
+                                        const double *__restrict__ fn, double &dist)
 {
     const int *f2 = tri + 3 * j2;
     double nor2[3], dx[3], x2[3];
@@ -279,19 +285,32 @@ __device__ __forceinline__ void consider(const double *x1, const double *nor1, d
     if (v_dot(nor1, nor2) < 0.0) v_neg(nor2);
     v_sub(x1, xj + 3 * f2[0], dx);
     double proj = v_dot(dx, nor2);
-    if (proj < 0.0) return;
+    if (proj < 0.0) return false;
     for (int i = 0; i < 3; ++i) x2[i] = x1[i] - proj * nor2[i];
     v_sub(x2, x1, dx);
-    double dist = v_norm(dx);
-    if (dist > 5.0 * thr) return;
+    dist = v_norm(dx);
+    if (dist > 5.0 * thr) return false;
     double u, v;
     barycentric(&u, &v, xj + 3 * f2[0], xj + 3 * f2[1], xj + 3 * f2[2], x1);
     double w = 1.0 - u - v;
-    if (u < 0.0 || 1.0 < u || v < 0.0 || 1.0 < v || w < 0.0 || 1.0 < w) return;
+    if (u < 0.0 || 1.0 < u || v < 0.0 || 1.0 < v || w < 0.0 || 1.0 < w) return false;
+    return true;
+}
+
+__device__ __forceinline__ void take(Best &best, double dist, int j2)
+{
     if (best.face < 0 || dist < best.dist || (dist == best.dist && j2 < best.face)) {
         best.dist = dist;
         best.face = j2;
     }
+}
+
+__device__ __forceinline__ void consider(const double *x1, const double *nor1, double thr, int j2,
+                                         const double *__restrict__ xj, const int *__restrict__ tri,
+                                         const double *__restrict__ fn, Best &best)
+{
+    double dist;
+    if (accepts(x1, nor1, thr, j2, xj, tri, fn, dist)) take(best, dist, j2);
 }
 
 __device__ __forceinline__ Best best_min(Best a, Best b)
@@ -302,13 +321,115 @@ __device__ __forceinline__ Best best_min(Best a, Best b)
     return a;
 }
 
-// qpts/qnrm: query points and their normals; out_face[q] = winning face or -1.
+// Record of a query that found a face (V1-T2 / point-triangle), recomputed from the
+// winner exactly as the reference builds it; an empty record without one.
+__device__ void query_record(int q, int j2, const double *x1, const double *nor1, const double *__restrict__ xj,
+                             const int *__restrict__ tri, const double *__restrict__ fn,
+                             eolc_collision *__restrict__ out)
+{
+    eolc_collision c;
+    rec_init(&c);
+    if (j2 >= 0) {
+        double nor2[3], dx[3], x2[3];
+        const int *f2 = tri + 3 * j2;
+        ld(fn + 3 * j2, nor2);
+        if (v_dot(nor1, nor2) < 0.0) v_neg(nor2);
+        v_sub(x1, xj + 3 * f2[0], dx);
+        double proj = v_dot(dx, nor2);
+        for (int i = 0; i < 3; ++i) x2[i] = x1[i] - proj * nor2[i];
+        v_sub(x2, x1, dx);
+        double u, v;
+        barycentric(&u, &v, xj + 3 * f2[0], xj + 3 * f2[1], xj + 3 * f2[2], x1);
+        c.dist = v_norm(dx);
+        v_copy(nor1, c.nor1); v_copy(nor2, c.nor2);
+        v_copy(x1, c.pos1); v_copy(x2, c.pos2);
+        c.count1 = 1; c.count2 = 3;
+        c.verts1[0] = q; c.verts1[1] = -1; c.verts1[2] = -1;
+        c.verts2[0] = f2[0]; c.verts2[1] = f2[1]; c.verts2[2] = f2[2];
+        c.weights1[0] = 1.0;
+        c.weights2[0] = u; c.weights2[1] = v; c.weights2[2] = 1.0 - u - v;
+        c.tri2 = j2;
+    }
+    out[q] = c;
+}
+
+// Few queries: every face against every query.  A query that lies outside a face's box,
+// grown by the grid's margin, cannot pass its tests (face_cells' bound), so a face
+// and a query cost six compares, with the query in scalar registers; what passes goes
+// to a list (any order: the nearest is taken lexicographically) that k_cd_nearest
+// reduces.  Faces too ill-shaped for the bound are tested against all.  A thread takes
+// kSweepChunk queries (blockIdx.y the chunk): walking 2,048 took 0.35 ms on a 64^2
+// sheet, whose 8,192 faces fill an eighth of the chip.
+constexpr int kSweepChunk = 128;
+struct Candidate {
+    double dist;
+    int query, face;
+};
+
+__global__ void __launch_bounds__(256)
+k_cd_sweep(int F, int Q, const double *__restrict__ qpts, const double *__restrict__ qnrm, double thr, double cond_max,
+           const double *__restrict__ clothaabb, const double *__restrict__ xj, const int *__restrict__ tri,
+           const double *__restrict__ fn, unsigned cap, unsigned *__restrict__ ncand, Candidate *__restrict__ cand)
+{
+    const int f = blockIdx.x * blockDim.x + threadIdx.x;
+    if (f >= F) return;
+    const double *a = xj + 3 * tri[3 * f], *b = xj + 3 * tri[3 * f + 1], *c = xj + 3 * tri[3 * f + 2];
+    const double L = fmax(fmax(clothaabb[3] - clothaabb[0], clothaabb[4] - clothaabb[1]),
+                          fmax(clothaabb[5] - clothaabb[2], 1e-300));
+    GridParams g;
+    g.margin = grid_margin(thr, L);
+    g.cond_max = cond_max;
+    const bool ill = ill_shaped(g, a, b, c);
+    double lo[3], hi[3];
+    for (int k = 0; k < 3; ++k) {
+        lo[k] = ill ? -INFINITY : fmin(a[k], fmin(b[k], c[k])) - g.margin;
+        hi[k] = ill ? INFINITY : fmax(a[k], fmax(b[k], c[k])) + g.margin;
+    }
+    const int q0 = blockIdx.y * kSweepChunk, q1 = min(q0 + kSweepChunk, Q);
+#pragma unroll 4
+    for (int q = q0; q < q1; ++q) {
+        const double *x1 = qpts + 3 * q;
+        if (!(x1[0] >= lo[0] && x1[0] <= hi[0] && x1[1] >= lo[1] && x1[1] <= hi[1] && x1[2] >= lo[2] && x1[2] <= hi[2]))
+            continue;
+        const double pt[6] = {x1[0], x1[1], x1[2], x1[0], x1[1], x1[2]};
+        double dist;
+        if (!check_aabb(pt, clothaabb) || !accepts(x1, qnrm + 3 * q, thr, f, xj, tri, fn, dist)) continue;
+        const unsigned p = atomicAdd(ncand, 1u);
+        if (p < cap) cand[p] = Candidate{dist, q, f};
+    }
+}
+
+// One wavefront per query over the candidate list.
+__global__ void __launch_bounds__(64)
+k_cd_nearest(const double *__restrict__ qpts, const double *__restrict__ qnrm, const double *__restrict__ xj,
+             const int *__restrict__ tri, const double *__restrict__ fn, unsigned cap,
+             const unsigned *__restrict__ ncand, const Candidate *__restrict__ cand, eolc_collision *__restrict__ out)
+{
+    const int q = blockIdx.x;
+    const unsigned n = min(*ncand, cap);
+    Best best{0.0, -1};
+    for (unsigned e = threadIdx.x; e < n; e += 64)
+        if (cand[e].query == q) take(best, cand[e].dist, cand[e].face);
+    for (int o = 32; o > 0; o >>= 1) {
+        const double d = __shfl_xor(best.dist, o, 64);
+        const int f = __shfl_xor(best.face, o, 64);
+        if (f >= 0) take(best, d, f);
+    }
+    if (threadIdx.x == 0) {
+        double x1[3], n1[3];
+        ld(qpts + 3 * q, x1);
+        ld(qnrm + 3 * q, n1);
+        query_record(q, best.face, x1, n1, xj, tri, fn, out);
+    }
+}
+
+// qpts/qnrm: query points and their normals; out[q] = the winning face's record.
 __global__ void __launch_bounds__(256)
 k_cd_query(int Q, GridParams g, const double *__restrict__ qpts, const double *__restrict__ qnrm, double thr,
            const double *__restrict__ clothaabb, const double *__restrict__ xj, const int *__restrict__ tri,
            const double *__restrict__ fn, const unsigned *__restrict__ bstart, const unsigned *__restrict__ bcnt,
            const int *__restrict__ entries, const unsigned *__restrict__ nalways, const int *__restrict__ always,
-           int *__restrict__ out_face)
+           eolc_collision *__restrict__ out)
 {
     __shared__ double sd[256];
     __shared__ int sf[256];
@@ -341,65 +462,21 @@ k_cd_query(int Q, GridParams g, const double *__restrict__ qpts, const double *_
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) out_face[q] = sf[0];
-}
-
-// Record of a query that found a face (V1-T2 / point-triangle), recomputed from the
-// winner exactly as the reference builds it.
-__global__ void k_cd_query_records(int Q, double thr, const double *__restrict__ qpts, const double *__restrict__ qnrm,
-                                   const int *__restrict__ face, const double *__restrict__ xj,
-                                   const int *__restrict__ tri, const double *__restrict__ fn,
-                                   eolc_collision *__restrict__ out)
-{
-    int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= Q) return;
-    eolc_collision c;
-    rec_init(&c);
-    int j2 = face[q];
-    if (j2 >= 0) {
-        double x1[3], nor1[3], nor2[3], dx[3], x2[3];
-        ld(qpts + 3 * q, x1);
-        ld(qnrm + 3 * q, nor1);
-        const int *f2 = tri + 3 * j2;
-        ld(fn + 3 * j2, nor2);
-        if (v_dot(nor1, nor2) < 0.0) v_neg(nor2);
-        v_sub(x1, xj + 3 * f2[0], dx);
-        double proj = v_dot(dx, nor2);
-        for (int i = 0; i < 3; ++i) x2[i] = x1[i] - proj * nor2[i];
-        v_sub(x2, x1, dx);
-        double u, v;
-        barycentric(&u, &v, xj + 3 * f2[0], xj + 3 * f2[1], xj + 3 * f2[2], x1);
-        c.dist = v_norm(dx);
-        v_copy(nor1, c.nor1); v_copy(nor2, c.nor2);
-        v_copy(x1, c.pos1); v_copy(x2, c.pos2);
-        c.count1 = 1; c.count2 = 3;
-        c.verts1[0] = q; c.verts1[1] = -1; c.verts1[2] = -1;
-        c.verts2[0] = f2[0]; c.verts2[1] = f2[1]; c.verts2[2] = f2[2];
-        c.weights1[0] = 1.0;
-        c.weights2[0] = u; c.weights2[1] = v; c.weights2[2] = 1.0 - u - v;
-        c.tri2 = j2;
-    }
-    out[q] = c;
+    if (threadIdx.x == 0) query_record(q, sf[0], x1, n1, xj, tri, fn, out);
 }
 
 // ---------------------------------------------------------------------------
-// Box V2-T1 (boxTriCollision.cpp:675-764): one thread per cloth vertex.
-__global__ void __launch_bounds__(256)
-k_cd_v2t1(int N, int F, double thr, const BoxGeom *__restrict__ boxp, const double *__restrict__ xj, const double *__restrict__ fn,
-          int *__restrict__ flag, eolc_collision *__restrict__ rec, int *__restrict__ err)
+// Box V2-T1 (boxTriCollision.cpp:675-764) of one cloth vertex at x2, whose record is
+// written to rec when it is not null.
+__device__ bool v2t1(int i2, int F, double thr, const BoxGeom &box, const double *x2, const double *__restrict__ fn,
+                     eolc_collision *__restrict__ rec, unsigned *__restrict__ err)
 {
-    int i2 = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i2 >= N) return;
-    flag[i2] = 0;
-    const BoxGeom &box = *boxp;
-    double x2[3];
-    ld(xj + 3 * i2, x2);
-    double pt[6] = {x2[0], x2[1], x2[2], x2[0], x2[1], x2[2]};
-    if (!check_aabb(pt, box.aabb)) return;
+    const double pt[6] = {x2[0], x2[1], x2[2], x2[0], x2[1], x2[2]};
+    if (!check_aabb(pt, box.aabb)) return false;
     for (int j1 = 0; j1 < 24; ++j1) {
         double dx[3];
         v_sub(x2, box.v[kBoxFaces[j1][0]], dx);
-        if (v_dot(box.fn[j1], dx) > 0.0) return;
+        if (v_dot(box.fn[j1], dx) > 0.0) return false;
     }
     eolc_collision best;
     int found = 0;
@@ -419,7 +496,7 @@ k_cd_v2t1(int N, int F, double thr, const BoxGeom *__restrict__ boxp, const doub
         double w = 1.0 - u - v;
         if (u < 0.0 || 1.0 < u || v < 0.0 || 1.0 < v || w < 0.0 || 1.0 < w) continue;
         if (i2 >= F) {   // faceNors2.col(i2) would read past the face normals
-            atomicOr(err, 1);
+            atomicOr(err, 1u);
             continue;
         }
         double nor2[3];
@@ -439,20 +516,20 @@ k_cd_v2t1(int N, int F, double thr, const BoxGeom *__restrict__ boxp, const doub
             found = 1;
         }
     }
-    if (found) {
-        flag[i2] = 1;
-        rec[i2] = best;
-    }
+    if (found && rec) *rec = best;
+    return found != 0;
 }
 
 // pointTri EOL branch (boxTriCollision.cpp:1099-1139): nearest point within thr.
+// offs null: count (0 or 1 per vertex); else write the records at their offsets.
 __global__ void __launch_bounds__(256)
 k_cd_eolpts(int N, int P, double thr, const double *__restrict__ pts, const double *__restrict__ nrm,
-            const double *__restrict__ xj, int *__restrict__ flag, eolc_collision *__restrict__ rec)
+            const double *__restrict__ xj, unsigned *__restrict__ cnt, const unsigned *__restrict__ offs,
+            eolc_collision *__restrict__ out)
 {
     int i2 = blockIdx.x * blockDim.x + threadIdx.x;
     if (i2 >= N) return;
-    flag[i2] = 0;
+    if (offs && !cnt[i2]) return;
     double x2[3];
     ld(xj + 3 * i2, x2);
     int bi = -1;
@@ -463,7 +540,10 @@ k_cd_eolpts(int N, int P, double thr, const double *__restrict__ pts, const doub
         double dist = v_norm(dx);
         if (dist < thr && (bi < 0 || dist < bd)) { bi = i1; bd = dist; }
     }
-    if (bi < 0) return;
+    if (!offs) {
+        cnt[i2] = bi >= 0;
+        return;
+    }
     eolc_collision c;
     rec_init(&c);
     c.dist = bd;
@@ -473,24 +553,44 @@ k_cd_eolpts(int N, int P, double thr, const double *__restrict__ pts, const doub
     c.verts1[0] = bi; c.verts1[1] = -1; c.verts1[2] = -1;
     c.verts2[0] = i2; c.verts2[1] = -1; c.verts2[2] = -1;
     c.weights1[0] = 1.0; c.weights2[0] = 1.0;
-    flag[i2] = 1;
-    rec[i2] = c;
+    out[offs[i2]] = c;
 }
 
 // ---------------------------------------------------------------------------
-// Box E2-E1: one thread per cloth edge (ee_edge in collide_common.h); pass 0
-// counts the records and flags acos-ambiguous pairs, pass 1 writes the records
-// at their prefix-sum offsets.
-__global__ void __launch_bounds__(256)
-k_cd_ee(int E, int pass, double thr, const BoxGeom *__restrict__ boxp, const int *__restrict__ cedges, const double *__restrict__ x,
-        const double *__restrict__ xj, const int *__restrict__ tri, unsigned *__restrict__ counts,
-        const unsigned *__restrict__ offsets, int *__restrict__ ambig, eolc_collision *__restrict__ out)
+// The boxes b0 .. b1-1 of a group.  Box b's counts are cnt[b (N + E) ..], vertices then
+// edges: one scan gives every record's place.  Count passes:
+//   k_cd_boxes  V2-T1 of every cloth vertex (the first blocks_for(N) workgroups, one
+//               thread each); every cloth edge (the others) is read once, and where it
+//               reaches one of a box's 24 faces' bounds, which ee_pair requires of a box
+//               edge's two, it goes to the list of pairs (any order)
+//   k_cd_pairs  E2-E1 of the listed pairs, 12 lanes each, a lane per box edge
+// With offs both write the records of the non-zero counts, from box b0's first on.
+// A pair's tests are a long chain of dependent FP64 work that few edges need: a thread
+// walking the 12 box edges of its own edge took 40 us a pass for one box at 64^2 and
+// 240 us for four at 512^2, with the chip idle.
+constexpr int kBoxWG = 256;
+__global__ void __launch_bounds__(kBoxWG)
+k_cd_boxes(int N, int E, int F, int b0, int b1, double thr, const BoxGeom *__restrict__ boxes,
+           const int *__restrict__ cedges, const double *__restrict__ xj, const double *__restrict__ fn,
+           unsigned *__restrict__ cnt, const unsigned *__restrict__ offs, unsigned *__restrict__ npairs,
+           unsigned *__restrict__ pairs, unsigned *__restrict__ err, eolc_collision *__restrict__ out)
 {
-    int k2 = blockIdx.x * blockDim.x + threadIdx.x;
+    const int NE = N + E, vblocks = (N + kBoxWG - 1) / kBoxWG;
+    if ((int)blockIdx.x < vblocks) {
+        const int i = blockIdx.x * kBoxWG + threadIdx.x;
+        if (i >= N) return;
+        double x2[3];
+        ld(xj + 3 * i, x2);
+        const unsigned o0 = offs ? offs[(size_t)b0 * NE] : 0u;
+        for (int b = b0; b < b1; ++b) {
+            const size_t k = (size_t)b * NE + i;
+            if (!offs) cnt[k] = v2t1(i, F, thr, boxes[b], x2, fn, nullptr, err) ? 1u : 0u;
+            else if (cnt[k]) v2t1(i, F, thr, boxes[b], x2, fn, out + (offs[k] - o0), err);
+        }
+        return;
+    }
+    const int k2 = ((int)blockIdx.x - vblocks) * kBoxWG + threadIdx.x;
     if (k2 >= E) return;
-    const BoxGeom &box = *boxp;
-    int mask = 0;
-    // AABB quick reject against the box (the per-edge test below pads by 1e-3 too)
     const int *e2 = cedges + 4 * k2;
     double aabbE[6];
     for (int i = 0; i < 3; ++i) {
@@ -498,31 +598,75 @@ k_cd_ee(int E, int pass, double thr, const BoxGeom *__restrict__ boxp, const int
         aabbE[i] = a < b ? a : b;
         aabbE[i + 3] = a < b ? b : a;
     }
-    if (!check_aabb(box.aabb, aabbE)) {
-        if (pass == 0) { counts[k2] = 0; ambig[k2] = 0; }
-        return;
-    }
-    if (pass == 0) {
-        counts[k2] = (unsigned)ee_edge(k2, thr, box, cedges, x, xj, tri, nullptr, &mask, kAcosBand);
-        ambig[k2] = mask;
-    } else {
-        ee_edge(k2, thr, box, cedges, x, xj, tri, out + offsets[k2], &mask, kAcosBand);
+    for (int b = b0; b < b1; ++b) {
+        const unsigned k = (unsigned)b * (unsigned)NE + (unsigned)(N + k2);
+        cnt[k] = 0;
+        if (!check_aabb(boxes[b].aabb, aabbE)) continue;
+        bool near = false;
+        for (int f = 0; f < 24; ++f) near = near || check_aabb(boxes[b].faabb[f], aabbE);
+        if (near) pairs[atomicAdd(npairs, 1u)] = k;
     }
 }
 
-// compaction of per-vertex flagged records in vertex order
-__global__ void k_compact(int n, const int *__restrict__ flag, const unsigned *__restrict__ offs,
-                          const eolc_collision *__restrict__ rec, eolc_collision *__restrict__ out)
+// Workgroups stride over the listed pairs of the boxes b0 .. b1-1, five to a wavefront.
+constexpr int kPairGrid = 1024;
+__global__ void __launch_bounds__(64)
+k_cd_pairs(int N, int E, int b0, int b1, double thr, const BoxGeom *__restrict__ boxes, const int *__restrict__ cedges,
+           const double *__restrict__ x, const double *__restrict__ xj, const int *__restrict__ tri,
+           unsigned *__restrict__ cnt, const unsigned *__restrict__ offs, const unsigned *__restrict__ npairs,
+           const unsigned *__restrict__ pairs, unsigned *__restrict__ nambig, eolc_collision *__restrict__ out)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || !flag[i]) return;
-    out[offs[i]] = rec[i];
+    const unsigned NE = (unsigned)(N + E), n = *npairs;
+    const int lane = threadIdx.x, grp = lane / 12, k1 = lane % 12;
+    for (unsigned p0 = 5 * blockIdx.x; p0 < n; p0 += 5 * gridDim.x) {   // uniform in the wavefront
+        bool on = grp < 5 && p0 + grp < n;
+        const unsigned k = on ? pairs[p0 + grp] : 0u;
+        const int b = (int)(k / NE), e = (int)(k % NE) - N;
+        if (offs) on = on && b >= b0 && b < b1 && cnt[k];
+        ClothEdge ce;
+        int hit = 0, amb = 0;
+        if (on) {
+            cloth_edge(e, cedges, x, xj, tri, ce);
+            hit = ee_pair(e, k1, thr, boxes[b], ce, nullptr, &amb, kAcosBand);
+        }
+        const unsigned bits = (unsigned)(__ballot(hit) >> (12 * grp)) & 0xfffu;
+        if (!on) continue;
+        if (!offs) {
+            if (k1 == 0) cnt[k] = __popc(bits);
+            if (amb) atomicOr(&nambig[b], 1u);
+        } else if (hit) {
+            ee_pair(e, k1, thr, boxes[b], ce,
+                    out + (offs[k] - offs[(size_t)b0 * NE]) + __popc(bits & ((1u << k1) - 1)), &amb, kAcosBand);
+        }
+    }
 }
 
-__global__ void k_flag_to_u32(int n, const int *__restrict__ flag, unsigned *__restrict__ out)
+// The acos-ambiguous pairs of one box, per edge (only when k_cd_boxes saw one).
+__global__ void __launch_bounds__(256)
+k_cd_ambiguous(int E, double thr, const BoxGeom *__restrict__ box, const int *__restrict__ cedges,
+               const double *__restrict__ x, const double *__restrict__ xj, const int *__restrict__ tri,
+               int *__restrict__ ambig)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = flag[i] ? 1u : 0u;
+    const int k2 = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k2 >= E) return;
+    const int *e2 = cedges + 4 * k2;
+    double aabbE[6];
+    for (int i = 0; i < 3; ++i) {
+        double a = xj[3 * e2[0] + i], b = xj[3 * e2[1] + i];
+        aabbE[i] = a < b ? a : b;
+        aabbE[i + 3] = a < b ? b : a;
+    }
+    int mask = 0;
+    if (check_aabb(box->aabb, aabbE)) ee_edge(k2, thr, *box, cedges, x, xj, tri, nullptr, &mask, kAcosBand);
+    ambig[k2] = mask;
+}
+
+// first[2 b], first[2 b + 1]: the offsets of box b's vertex and edge records; first[2 nb]:
+// their number (the scan leaves it behind the last offset)
+__global__ void k_cd_first(int nb, int N, int NE, const unsigned *__restrict__ offs, unsigned *__restrict__ first)
+{
+    const int t = threadIdx.x;
+    if (t <= 2 * nb) first[t] = offs[(size_t)(t >> 1) * NE + ((t & 1) ? N : 0)];
 }
 
 inline int blocks_for(int64_t n, int t = 256) { return (int)((n + t - 1) / t); }
@@ -616,7 +760,7 @@ hipError_t cd_grid_build(eolc_ctx *c, const eolc_cd::CdGrid &gp, const double *x
 
 hipError_t cd_query(eolc_ctx *c, const eolc_cd::CdGrid &gp, int Q, const double *qpts, const double *qnrm, double thr,
                     const double *aabb, const double *xj, const double *fn, const unsigned *bstart, const unsigned *bcnt,
-                    const int *entries, const unsigned *nalways, const int *always, int *face, eolc_collision *rec)
+                    const int *entries, const unsigned *nalways, const int *always, eolc_collision *rec)
 {
     if (Q <= 0) return hipSuccess;
     GridParams g;
@@ -626,49 +770,62 @@ hipError_t cd_query(eolc_ctx *c, const eolc_cd::CdGrid &gp, int Q, const double 
     g.margin = gp.margin;
     g.cond_max = gp.cond_max;
     hipLaunchKernelGGL(k_cd_query, dim3(Q), dim3(256), 0, c->stream, Q, g, qpts, qnrm, thr, aabb, xj, c->tri, fn,
-                       bstart, bcnt, entries, nalways, always, face);
-    hipLaunchKernelGGL(k_cd_query_records, dim3(blocks_for(Q)), dim3(256), 0, c->stream, Q, thr, qpts, qnrm, face, xj,
-                       c->tri, fn, rec);
+                       bstart, bcnt, entries, nalways, always, rec);
     return hipGetLastError();
 }
 
-hipError_t cd_v2t1(eolc_ctx *c, double thr, const BoxGeom *box, const double *xj, const double *fn, int *flag,
-                   eolc_collision *rec, int *err)
+hipError_t cd_sweep(eolc_ctx *c, int Q, const double *qpts, const double *qnrm, double thr, const double *aabb,
+                    const double *xj, const double *fn, unsigned *ncand, void *cand, eolc_collision *rec)
+{
+    if (Q <= 0) return hipSuccess;
+    const int F = c->topo.F;
+    Candidate *cd = static_cast<Candidate *>(cand);
+    if (F > 0)
+        hipLaunchKernelGGL(k_cd_sweep, dim3(blocks_for(F), blocks_for(Q, kSweepChunk)), dim3(256), 0, c->stream, F, Q, qpts, qnrm, thr,
+                           eolc_cd::kGridCondMax, aabb, xj, c->tri, fn, kCdCandidates, ncand, cd);
+    hipLaunchKernelGGL(k_cd_nearest, dim3(Q), dim3(64), 0, c->stream, qpts, qnrm, xj, c->tri, fn, kCdCandidates, ncand,
+                       cd, rec);
+    return hipGetLastError();
+}
+
+hipError_t cd_eolpts(eolc_ctx *c, int P, double thr, const double *pts, const double *nrm, const double *xj,
+                     unsigned *cnt, const unsigned *offs, eolc_collision *out)
 {
     const int N = c->topo.N;
-    hipLaunchKernelGGL(k_cd_v2t1, dim3(blocks_for(N)), dim3(256), 0, c->stream, N, c->topo.F, thr, box, xj, fn, flag,
-                       rec, err);
+    hipLaunchKernelGGL(k_cd_eolpts, dim3(blocks_for(N)), dim3(256), 0, c->stream, N, P, thr, pts, nrm, xj, cnt, offs,
+                       out);
     return hipGetLastError();
 }
 
-hipError_t cd_eolpts(eolc_ctx *c, int P, double thr, const double *pts, const double *nrm, const double *xj, int *flag,
-                     eolc_collision *rec)
+hipError_t cd_boxes(eolc_ctx *c, int b0, int b1, double thr, const eolc_cd::BoxGeom *boxes, const double *xj,
+                    const double *fn, unsigned *cnt, const unsigned *offs, unsigned *npairs, unsigned *pairs,
+                    unsigned *nambig, unsigned *err, eolc_collision *out)
 {
-    const int N = c->topo.N;
-    hipLaunchKernelGGL(k_cd_eolpts, dim3(blocks_for(N)), dim3(256), 0, c->stream, N, P, thr, pts, nrm, xj, flag, rec);
+    const int N = c->topo.N, E = c->n_cedges;
+    // the record pass reads the edges from the list alone
+    const int blocks = blocks_for(N, kBoxWG) + (offs ? 0 : blocks_for(E, kBoxWG));
+    hipLaunchKernelGGL(k_cd_boxes, dim3(blocks), dim3(kBoxWG), 0, c->stream, N, E, c->topo.F, b0, b1, thr, boxes,
+                       c->cedges, xj, fn, cnt, offs, npairs, pairs, err, out);
+    if (E > 0)
+        hipLaunchKernelGGL(k_cd_pairs, dim3(kPairGrid), dim3(64), 0, c->stream, N, E, b0, b1, thr, boxes, c->cedges,
+                           c->x, xj, c->tri, cnt, offs, npairs, pairs, nambig, out);
     return hipGetLastError();
 }
 
-hipError_t cd_ee(eolc_ctx *c, int pass, double thr, const BoxGeom *box, const double *xj, unsigned *counts,
-                 const unsigned *offsets, int *ambig, eolc_collision *out)
+hipError_t cd_ambiguous(eolc_ctx *c, double thr, const eolc_cd::BoxGeom *box, const double *xj, int *ambig)
 {
     const int E = c->n_cedges;
     if (E == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_cd_ee, dim3(blocks_for(E)), dim3(256), 0, c->stream, E, pass, thr, box, c->cedges, c->x, xj,
-                       c->tri, counts, offsets, ambig, out);
+    hipLaunchKernelGGL(k_cd_ambiguous, dim3(blocks_for(E)), dim3(256), 0, c->stream, E, thr, box, c->cedges, c->x, xj,
+                       c->tri, ambig);
     return hipGetLastError();
 }
 
-hipError_t cd_compact(eolc_ctx *c, int n, const int *flag, unsigned *u32, unsigned *offs, unsigned *sums,
-                      unsigned *total, const eolc_collision *rec, eolc_collision *out, bool write)
+hipError_t cd_first(eolc_ctx *c, int nb, const unsigned *offs, unsigned *first)
 {
-    if (!write) {
-        hipLaunchKernelGGL(k_flag_to_u32, dim3(blocks_for(n)), dim3(256), 0, c->stream, n, flag, u32);
-        const hipError_t e = cd_scan(c, (unsigned)n, u32, offs, sums, total);
-        if (e != hipSuccess) return e;
-    } else {
-        hipLaunchKernelGGL(k_compact, dim3(blocks_for(n)), dim3(256), 0, c->stream, n, flag, offs, rec, out);
-    }
+    static_assert(2 * kCdBoxes < 64, "one wavefront");
+    hipLaunchKernelGGL(k_cd_first, dim3(1), dim3(64), 0, c->stream, nb, c->topo.N, c->topo.N + c->n_cedges, offs,
+                       first);
     return hipGetLastError();
 }
 

@@ -198,3 +198,43 @@ def test_counts_at_the_scan_pieces(ctx, n):
     (16,384 buckets, two whole pieces) and 16,576 edges; every record bit for bit."""
     sc, pts, nrm, whd, E = thin_box_scene(n, 1e-3)
     assert compare(ctx, sc, sc.x0, 2e-3, pts, nrm, whd, E)
+
+
+@pytest.mark.parametrize("P,B", [(2048, 0), (2049, 0), (1, 9), (0, 8)])
+def test_query_and_box_group_edges(ctx, P, B):
+    """Up to 2,048 queries are swept over all faces, more take the grid; boxes run eight to
+    a launch.  Both sides of each, with faces too ill-shaped for the box reject (a third
+    of the sheet flattened to a line), record for record."""
+    sc = scene.Scene(23, sigma_x=1e-3)
+    pts, nrm, whd, E = scene.obstacles(seed=40 + P + B, P=P, B=max(B, 1))
+    x = sc.x0.reshape(-1, 3).copy()
+    x[: sc.N // 3, 1:] = 0.0
+    if B:
+        compare(ctx, sc, x.reshape(-1), 2e-3, pts, nrm, whd, E)
+    else:
+        assert compare(ctx, sc, x.reshape(-1), 2e-3, pts, nrm, np.zeros((0, 3)), [])
+
+
+def test_sweep_list_overflow_takes_the_grid(ctx):
+    """More candidates than the sweep keeps (65,536): 1,500 points over 128 faces stacked
+    on each other, every point within the band of half of them."""
+    k = 64
+    X = np.zeros((4 * k, 2))
+    tri = np.zeros((2 * k, 3), dtype=np.int32)
+    x = np.zeros((4 * k, 3))
+    for s in range(k):
+        X[4 * s:4 * s + 4] = np.array([[0, 0], [1, 0], [0, 1], [1, 1]]) + [2.0 * s, 0.0]
+        x[4 * s:4 * s + 4, :2] = [[0, 0], [1, 0], [0, 1], [1, 1]]
+        x[4 * s:4 * s + 4, 2] = 1e-7 * s
+        tri[2 * s:2 * s + 2] = np.array([[0, 1, 2], [1, 3, 2]]) + 4 * s
+    rng = np.random.default_rng(3)
+    P = 1500
+    pts = np.concatenate([rng.uniform(0.05, 0.95, size=(P, 2)), np.full((P, 1), 2e-3)], axis=1)
+    nrm = np.tile([0.0, 0.0, 1.0], (P, 1))
+    ctx.set_topology(X, tri, np.zeros((0, 4), dtype=np.int32))
+    ctx.upload_state(x.reshape(-1), np.zeros(x.size))
+    g = ctx.collide(1e-3, pts, nrm)
+    o = oracle_cd(1e-3, pts, nrm, np.zeros((0, 3)), [], x.reshape(-1), tri)
+    print(f"{len(g)} records", flush=True)
+    assert len(g) == len(o) == P
+    assert all(rec_tuple(a) == rec_tuple(b) for a, b in zip(g, o))
