@@ -1273,8 +1273,8 @@ static int forces_fill_async(eolc_ctx *c, const double grav[3], double h, bool w
     EOLC_HIP(eolc::launch_face_eval(c, h, grav));
     EOLC_HIP(eolc::launch_hinge_eval(c, h));
     c->h_last = h;   // (the assembly's stiff threshold scales with h^2)
-    EOLC_HIP(eolc::launch_assemble(c, (want32 ? eolc::fp32_layout(c->spmv_variant[0]) : 0) |
-                                          eolc::fp64_layout(c->spmv_variant[1])));
+    EOLC_HIP(eolc::launch_assemble(c, (want32 ? eolc::fp32_layout(eolc::spmv_runs(c->topo, true, c->spmv_variant[0])) : 0) |
+                                          eolc::fp64_layout(eolc::spmv_runs(c->topo, false, c->spmv_variant[1]))));
     c->have_forces = true;
     return EOLC_OK;
 }

@@ -15,6 +15,7 @@ namespace eolc {
 // Rows of the 3x3 BSR matrix handled by one workgroup pass of the PCG kernels:
 // 16 lanes per block row, 256 threads per workgroup.
 constexpr int kPcgWG = 1024;        // threads per workgroup of the PCG row kernels
+constexpr int kVecWG = 256;         // the same of its vector kernels on small meshes (vec_wg)
 constexpr int kPcgGrid = 512;       // maximum workgroups of the PCG row kernels
 constexpr int kMaxPartials = 16384; // stride of one partial-sum array (max PCG workgroups)
 
@@ -455,6 +456,8 @@ hipError_t launch_rhs(eolc_ctx *c, double h);
 hipError_t launch_update_x(eolc_ctx *c, double h);
 
 int pcg_grid(int N);
+int vec_wg(int N);          // workgroup size and workgroups of the PCG's vector kernels
+int vec_grid(int N);
 int pcg_grid_phys(int G);   // physical workgroups of the row kernels with a second logical one
 hipError_t pcg_setup(eolc_ctx *c, bool mixed, int precond_kind, bool ml_linear = true);
 hipError_t pcg_init(eolc_ctx *c, bool mixed);
@@ -484,6 +487,10 @@ bool spmv_patch(int variant);    // the variant reads the patch layout
 // the patch layout was built), else spmv_fallback(variant) gives the same bits
 bool spmv_usable(const Topology &t, int variant);
 int spmv_fallback(int variant);
+// what runs for the variant on this topology (a variant, or the split kernel, which reads
+// the SoA arrays)
+constexpr int kSpmvSplit = kSpmvVariants;
+int spmv_runs(const Topology &t, bool mixed, int variant);
 hipError_t time_spmv(eolc_ctx *c, bool mixed, int variant, int reps, float *ms);
 hipError_t stream_copy(eolc_ctx *c, size_t bytes, int reps, float *ms, int read_only);
 // learned preconditioner (k_learned.hip); buffers allocated by the API layer

@@ -226,14 +226,14 @@ static hipError_t ensure_layout(eolc_ctx *c, int need)
     return e;
 }
 
-// (a variant this mesh cannot run is replaced by its twin, as the SpMV launch does)
+// (the variant that the SpMV launch runs)
 hipError_t ensure_fp32_layout(eolc_ctx *c, int variant)
 {
-    return ensure_layout(c, fp32_layout(spmv_usable(c->topo, variant) ? variant : spmv_fallback(variant)));
+    return ensure_layout(c, fp32_layout(spmv_runs(c->topo, true, variant)));
 }
 hipError_t ensure_fp64_layout(eolc_ctx *c, int variant)
 {
-    return ensure_layout(c, fp64_layout(spmv_usable(c->topo, variant) ? variant : spmv_fallback(variant)));
+    return ensure_layout(c, fp64_layout(spmv_runs(c->topo, false, variant)));
 }
 
 hipError_t launch_rhs(eolc_ctx *c, double h)

@@ -41,6 +41,8 @@
 // from which the coarse kernel gets every level >= 3 by the exact change of
 // centroid and radius; the prolongation evaluates the level-3 field at each vertex.
 // The batched solve keeps the translations on every level.
+#include <type_traits>
+
 #include "eolc_internal.h"
 #include "pcg_device.h"
 
@@ -823,15 +825,15 @@ __global__ void __launch_bounds__(kCoarse9WG) k_ml_coarse9(MLLevels lv, const in
 // arrive accumulated in C_3.
 // FINE = false: the coarse corrections alone (z_i = C(a_i) + C_3), for the learned
 // blocks' training loss, whose fine term is the network's.
-template <class T, bool FINE = true, class TD = T>
-__global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8, 8)))
+template <class T, bool FINE, int W>
+__global__ void __launch_bounds__(W) __attribute__((amdgpu_waves_per_eu(8, 8)))
 k_ml_prolong(int parity, int N, MLLevels lv, const int *__restrict__ agg1, const int *__restrict__ anc3,
              const double *__restrict__ Dinv, const double *__restrict__ R, const double *__restrict__ C,
-             const TD *__restrict__ D, const T *__restrict__ r, T *__restrict__ z,
+             const T *__restrict__ D, const T *__restrict__ r, T *__restrict__ z,
              const unsigned char *__restrict__ fixmask, const SolverScalars *scal, double *partials, int check_done,
              const double *__restrict__ feat3, const double *__restrict__ C9)
 {
-    __shared__ double lds[2 * (WG / 64) + 2];
+    __shared__ double lds[2 * (W / 64) + 2];
     int rb, re;
     wg_rows(N, &rb, &re);
     const int i0 = rb + (int)threadIdx.x;
@@ -844,7 +846,7 @@ k_ml_prolong(int parity, int N, MLLevels lv, const int *__restrict__ agg1, const
     }
     if (check_done && scal->done) return;
     double srz = 0.0;
-    for (int i = i0; i < re; i += WG) {
+    for (int i = i0; i < re; i += W) {
         if (i != i0) {
             a = agg1[i];
             if (lv.L >= 3) u = anc3[i];
@@ -871,8 +873,8 @@ k_ml_prolong(int parity, int N, MLLevels lv, const int *__restrict__ agg1, const
         const T r0 = r[3 * i], r1 = r[3 * i + 1], r2 = r[3 * i + 2];
         double g0 = 0.0, g1 = 0.0, g2 = 0.0;
         if constexpr (FINE) {
-            TD f0, f1, f2;
-            eolc::apply_sym3<TD>(D + i, N, (TD)r0, (TD)r1, (TD)r2, f0, f1, f2);
+            T f0, f1, f2;
+            eolc::apply_sym3<T>(D + i, N, r0, r1, r2, f0, f1, f2);
             g0 = (double)f0; g1 = (double)f1; g2 = (double)f2;
         }
         const unsigned fm = fixmask[i];
@@ -883,7 +885,7 @@ k_ml_prolong(int parity, int N, MLLevels lv, const int *__restrict__ agg1, const
         srz += ((double)r0 * (double)z0 + (double)r1 * (double)z1) + (double)r2 * (double)z2;
     }
     double v[1] = {srz};
-    write_partials<1>(v, PB(partials, parity), lds);
+    write_partials<1, W>(v, PB(partials, parity), lds);
 }
 
 inline int blocks_for(int64_t n, int t = 256) { return (int)((n + t - 1) / t); }
@@ -948,38 +950,37 @@ static void ml_coarse_chain(eolc_ctx *c, bool mixed, int check_done)
                            c->scal, check_done);
 }
 
-hipError_t ml_apply(eolc_ctx *c, bool mixed, int parity, int check_done)
+// The prolongation on the vector kernels' grid (vec_wg, vec_grid).
+template <class T, bool FINE>
+static void launch_prolong(eolc_ctx *c, int parity, const T *D, const T *r, T *z, int check_done)
 {
     const MLState &m = c->ml;
     const MLLevels &lv = m.lv;
     const int N = c->topo.N;
-    const int G = pcg_grid(N);
-    ml_coarse_chain(c, mixed, check_done);
     const double *c9 = (m.lin_on && lv.L >= kMLLinFrom) ? m.C9 : nullptr;
-    if (mixed) {
-        hipLaunchKernelGGL(k_ml_prolong<float>, dim3(G), dim3(WG), 0, c->stream, parity, N, lv, m.agg1, m.anc3, m.Dinv,
-                           m.R, m.C, c->D32, c->r32, c->z32, c->fixmask, c->scal, c->partials, check_done, m.feat3,
-                           c9);
-    } else {
-        hipLaunchKernelGGL(k_ml_prolong<double>, dim3(G), dim3(WG), 0, c->stream, parity, N, lv, m.agg1, m.anc3,
-                           m.Dinv, m.R, m.C, c->D64, c->r64, c->z64, c->fixmask, c->scal, c->partials, check_done,
-                           m.feat3, c9);
-    }
+    auto go = [&](auto w) {
+        constexpr int W = decltype(w)::value;
+        hipLaunchKernelGGL((k_ml_prolong<T, FINE, W>), dim3(vec_grid(N)), dim3(W), 0, c->stream, parity, N, lv, m.agg1,
+                           m.anc3, m.Dinv, m.R, m.C, D, r, z, c->fixmask, c->scal, c->partials, check_done, m.feat3, c9);
+    };
+    if (vec_wg(N) == kVecWG) go(std::integral_constant<int, kVecWG>());
+    else go(std::integral_constant<int, WG>());
+}
+
+hipError_t ml_apply(eolc_ctx *c, bool mixed, int parity, int check_done)
+{
+    ml_coarse_chain(c, mixed, check_done);
+    if (mixed) launch_prolong<float, true>(c, parity, c->D32, c->r32, c->z32, check_done);
+    else launch_prolong<double, true>(c, parity, c->D64, c->r64, c->z64, check_done);
     return hipGetLastError();
 }
 
 // z64 = the coarse corrections of r64 alone (no fine blocks), FP64, fixed DOFs zero.
 hipError_t ml_coarse64(eolc_ctx *c)
 {
-    const MLState &m = c->ml;
-    const MLLevels &lv = m.lv;
-    const int N = c->topo.N;
-    const int G = pcg_grid(N);
-    if (lv.L <= 0) return hipMemsetAsync(c->z64, 0, sizeof(double) * 3 * (size_t)N, c->stream);
+    if (c->ml.lv.L <= 0) return hipMemsetAsync(c->z64, 0, sizeof(double) * 3 * (size_t)c->topo.N, c->stream);
     ml_coarse_chain(c, false, 0);
-    const double *c9 = (m.lin_on && lv.L >= kMLLinFrom) ? m.C9 : nullptr;
-    hipLaunchKernelGGL((k_ml_prolong<double, false>), dim3(G), dim3(WG), 0, c->stream, 0, N, lv, m.agg1, m.anc3, m.Dinv,
-                       m.R, m.C, c->D64, c->r64, c->z64, c->fixmask, c->scal, c->partials, 0, m.feat3, c9);
+    launch_prolong<double, false>(c, 0, c->D64, c->r64, c->z64, 0);
     return hipGetLastError();
 }
 

@@ -158,7 +158,7 @@ k_pcg_spmv(int k, int N, int nslices, const int *__restrict__ slice_off, const i
            const int *__restrict__ slen, const int *__restrict__ scol, const T *__restrict__ A,
            const T *__restrict__ Mm, int64_t nbs, const unsigned char *__restrict__ fixmask, const T *__restrict__ z,
            const T *__restrict__ pold, T *__restrict__ pnew, T *__restrict__ q, SolverScalars *scal, double *partials,
-           SymLayout sym, const int *__restrict__ wwin)
+           SymLayout sym, const int *__restrict__ wwin, int Gb)
 {
     static_assert(U == 1 || U == 2, "entries per trip");
     static_assert(!(STG && U == 2), "the staged variants take one entry per trip");
@@ -203,8 +203,8 @@ k_pcg_spmv(int k, int N, int nslices, const int *__restrict__ slice_off, const i
     double cur[2];
     const bool restart_beta0 = (k == scal->first_iter);
     double prev[1] = {1.0};
-    if (restart_beta0) reduce_partials<2>(PB(partials, k & 1), cur, lds);
-    else reduce_partials2<2, 1>(PB(partials, k & 1), PB(partials, (k + 1) & 1), cur, prev, lds);
+    if (restart_beta0) reduce_partials<2>(PB(partials, k & 1), cur, lds, Gb);
+    else reduce_partials2<2, 1>(PB(partials, k & 1), PB(partials, (k + 1) & 1), cur, prev, lds, Gb, Gb);
     const double rzk = cur[0], rrk = cur[1];
     const double thr = fmax(scal->tol2 * scal->bnorm2, scal->delta2 * scal->rmax2);
     if (!isfinite(rrk) || !isfinite(rzk) || rrk <= thr) {
@@ -453,7 +453,7 @@ template <class T, class TR, bool NT, int W, int PD>
 __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(W, W)))
 k_pcg_spmv_patch(int k, PatchLayout pl, const T *__restrict__ Mm, const unsigned char *__restrict__ fixmask,
                  const T *__restrict__ z, const T *__restrict__ pold, T *__restrict__ pnew, T *__restrict__ q,
-                 SolverScalars *scal, double *partials)
+                 SolverScalars *scal, double *partials, int Gb)
 {
     using R = SymRec<TR>;
     typedef typename R::v2 v2;
@@ -504,8 +504,8 @@ k_pcg_spmv_patch(int k, PatchLayout pl, const T *__restrict__ Mm, const unsigned
     double cur[2];
     const bool restart_beta0 = (k == scal->first_iter);
     double prev[1] = {1.0};
-    if (restart_beta0) reduce_partials<2>(PB(partials, k & 1), cur, lds);
-    else reduce_partials2<2, 1>(PB(partials, k & 1), PB(partials, (k + 1) & 1), cur, prev, lds);
+    if (restart_beta0) reduce_partials<2>(PB(partials, k & 1), cur, lds, Gb);
+    else reduce_partials2<2, 1>(PB(partials, k & 1), PB(partials, (k + 1) & 1), cur, prev, lds, Gb, Gb);
     const double rzk = cur[0], rrk = cur[1];
     const double thr = fmax(scal->tol2 * scal->bnorm2, scal->delta2 * scal->rmax2);
     if (!isfinite(rrk) || !isfinite(rzk) || rrk <= thr) {
@@ -632,17 +632,228 @@ k_pcg_spmv_patch(int k, PatchLayout pl, const T *__restrict__ Mm, const unsigned
 }
 
 // ---------------------------------------------------------------------------
+// Small meshes (N <= kSplitRows): the product and the residual with one workgroup of four
+// wavefronts per slice.  On a few hundred slices the kernels above leave most of the
+// chip idle (16 slices per workgroup) and a wavefront walks its rows' 11 blocks one
+// dependent load after the other; here wavefront w takes the entries k = w, w + 4,
+// w + 8, ..., four of them at a time with every load of the four issued together and
+// before beta is known, and leaves their products in LDS, where three wavefronts (one
+// per component) add them in the order of k.  The row sums are therefore the bits of
+// the one-wavefront kernels; p.q is summed per slice.  Two slices per workgroup took
+// 13.9 and 26.9 us at 257^2 vertices.  Per product, FP32 and FP64, against one
+// wavefront per slice (us; r: arbitrary vertex order):
+//    441 vertices  6.0  6.7   9.3 15.9
+//    16,641        6.4  8.1  12.7 27.5   r  7.7  9.7  17.8 45.3
+//    66,049       12.8 22.6  15.7 32.1   r 16.8 30.9  34.3 64.8
+//    131,769      21.0 40.5  17.6 33.5   r 29.2 58.9  38.4 71.3
+// where the matrix no longer fits what the few workgroups in flight can keep coming.
+constexpr int kSplitRows = 90000;
+constexpr int kSplitBatch = 16;   // entries per row and pass: four wavefronts, four each
+
+template <class T, bool P2> struct SplitEntries {
+    T a[4][9], z[4][3], p[4][3];
+    int j[4];
+    bool ok[4];
+    __device__ __forceinline__ void columns(const int *__restrict__ cl, int k0, int len)
+    {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int k = k0 + 4 * u;
+            ok[u] = k < len;
+            j[u] = ok[u] ? cl[k * eolc::kSlice] : 0;
+        }
+    }
+    __device__ __forceinline__ void values(const T *__restrict__ A, int64_t nbs, int k0, const T *__restrict__ zv,
+                                           const T *__restrict__ pold)
+    {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (ok[u]) {
+                const T *__restrict__ ae = A + (k0 + 4 * u) * eolc::kSlice;
+#pragma unroll
+                for (int c = 0; c < 9; ++c) a[u][c] = ae[c * nbs];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    z[u][c] = zv[3 * j[u] + c];
+                    if (P2) p[u][c] = pold[3 * j[u] + c];
+                }
+            }
+    }
+};
+
+// The sums over the slice's rows: the wavefront's share of each row's blocks into
+// prod, then y (wavefront w < 3: component w of the row) += the products in order.
+// make(e, u, out): the three products of entry u of e.
+template <class T, bool P2, class Make>
+__device__ __forceinline__ void split_rows(SplitEntries<T, P2> &e, const T *__restrict__ A, int64_t nbs,
+                                           const int *__restrict__ cl, int len, int maxlen, const T *__restrict__ zv,
+                                           const T *__restrict__ pold, double *__restrict__ prod, double &y, Make make)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int kb = 0; kb < maxlen; kb += kSplitBatch) {   // uniform in the workgroup
+        if (kb > 0) {
+            e.columns(cl, kb + w, len);
+            e.values(A, nbs, kb + w, zv, pold);
+            __syncthreads();   // the sums of the pass before have read prod
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (e.ok[u]) {
+                double o[3];
+                make(e, u, o);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) prod[((4 * u + w) * 3 + c) * 64 + lane] = o[c];
+            }
+        __syncthreads();
+        if (w < 3) {
+            const int n = min(len - kb, kSplitBatch);
+            for (int k = 0; k < n; ++k) y += prod[(3 * k + w) * 64 + lane];
+        }
+    }
+}
+
+constexpr int kSplitWG = 256;
+
+template <class T, bool DIFF>
+__global__ void __launch_bounds__(kSplitWG)
+k_pcg_spmv_split(int k, int N, int nslices, const int *__restrict__ slice_off, const int *__restrict__ srow,
+                 const int *__restrict__ slen, const int *__restrict__ scol, const T *__restrict__ A,
+                 const T *__restrict__ Mm, int64_t nbs, const unsigned char *__restrict__ fixmask,
+                 const T *__restrict__ z, const T *__restrict__ pold, T *__restrict__ pnew, T *__restrict__ q,
+                 SolverScalars *scal, double *partials, int Gb)
+{
+    constexpr int W = kSplitWG;
+    __shared__ double lds[3 * (W / 64) + 3];
+    __shared__ double prod[3 * kSplitBatch * 64];
+    if (scal->done) return;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int sl = logical_wg();
+    const int g = sl * eolc::kSlice + lane;
+    const bool active = sl < nslices && g < N;
+    // the slice's rows are sorted by length: the first is the longest
+    const int maxlen = sl < nslices ? slen[sl * eolc::kSlice] - (DIFF ? 1 : 0) : 0;
+    int row = 0, len = 0, base = 0;
+    T zi[3] = {0, 0, 0}, po[3] = {0, 0, 0}, mb = 0;
+    unsigned fm = 0;
+    if (active) {
+        row = srow[g];
+        len = slen[g] - (DIFF ? 1 : 0);   // the difference form skips the diagonal (the last entry)
+        base = slice_off[sl] + lane;
+    }
+    SplitEntries<T, true> e;
+    e.columns(scol + base, w, len);
+    if (active) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            zi[c] = z[3 * row + c];
+            po[c] = pold[3 * row + c];
+        }
+        if constexpr (DIFF) mb = Mm[row];
+        fm = fixmask[row];
+    }
+    e.values(A + base, nbs, w, z, pold);
+    double cur[2];
+    const bool restart_beta0 = (k == scal->first_iter);
+    double prev[1] = {1.0};
+    if (restart_beta0) reduce_partials<2, W>(PB(partials, k & 1), cur, lds, Gb);
+    else reduce_partials2<2, 1, W>(PB(partials, k & 1), PB(partials, (k + 1) & 1), cur, prev, lds, Gb, Gb);
+    const double rzk = cur[0], rrk = cur[1];
+    const double thr = fmax(scal->tol2 * scal->bnorm2, scal->delta2 * scal->rmax2);
+    if (!isfinite(rrk) || !isfinite(rzk) || rrk <= thr) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            scal->done = 1;
+            scal->reason = (isfinite(rrk) && isfinite(rzk)) ? 1 : 4;
+            scal->rr = rrk;
+            scal->rz = rzk;
+        }
+        return;
+    }
+    const double beta = restart_beta0 ? 0.0 : rzk / prev[0];
+    const T betaT = (T)beta;
+    T ui[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) ui[c] = fma(betaT, po[c], zi[c]);
+    const T uw = w == 0 ? ui[0] : (w == 1 ? ui[1] : ui[2]);
+    double y = DIFF ? (double)(mb * uw) : 0.0;
+    split_rows<T, true>(e, A + base, nbs, scol + base, len, maxlen, z, pold, prod, y,
+                           [&](const SplitEntries<T, true> &x, int u, double (&o)[3]) {
+                               T v[3];
+#pragma unroll
+                               for (int c = 0; c < 3; ++c) v[c] = fma(betaT, x.p[u][c], x.z[u][c]);
+                               o[0] = o[1] = o[2] = 0.0;
+                               block_apply<T, DIFF>(x.a[u][0], x.a[u][1], x.a[u][2], x.a[u][3], x.a[u][4], x.a[u][5],
+                                                    x.a[u][6], x.a[u][7], x.a[u][8], v[0], v[1], v[2], ui[0], ui[1],
+                                                    ui[2], o[0], o[1], o[2]);
+                           });
+    double dot[1] = {0.0};
+    if (active && w < 3) {
+        if ((fm >> w) & 1u) y = 0;
+        const T qv = (T)y;
+        pnew[3 * row + w] = uw;
+        q[3 * row + w] = qv;
+        dot[0] = (double)uw * (double)qv;
+    }
+    write_partials<1, W>(dot, PA(partials), lds);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        scal->rr = rrk;
+        scal->rz = rzk;
+    }
+}
+
+// k_resid64 on the same split.
+__global__ void __launch_bounds__(kSplitWG)
+k_resid64_split(int N, int nslices, const int *__restrict__ slice_off, const int *__restrict__ srow,
+                const int *__restrict__ slen, const int *__restrict__ scol, const double *__restrict__ A, int64_t nbs,
+                const unsigned char *__restrict__ fixmask, const double *__restrict__ xin,
+                const double *__restrict__ b, double *__restrict__ out, double *partials)
+{
+    constexpr int W = kSplitWG;
+    __shared__ double lds[2 * (W / 64) + 2];
+    __shared__ double prod[3 * kSplitBatch * 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int sl = logical_wg();
+    const int g = sl * eolc::kSlice + lane;
+    const bool active = sl < nslices && g < N;
+    const int maxlen = sl < nslices ? slen[sl * eolc::kSlice] : 0;
+    int row = 0, len = 0, base = 0;
+    if (active) {
+        row = srow[g];
+        len = slen[g];
+        base = slice_off[sl] + lane;
+    }
+    SplitEntries<double, false> e;
+    e.columns(scol + base, w, len);
+    e.values(A + base, nbs, w, xin, nullptr);
+    double y = 0.0;
+    split_rows<double, false>(e, A + base, nbs, scol + base, len, maxlen, xin, nullptr, prod, y,
+                                 [&](const SplitEntries<double, false> &x, int u, double (&o)[3]) {
+                                     o[0] = o[1] = o[2] = 0.0;
+                                     block_apply<double, false>(x.a[u][0], x.a[u][1], x.a[u][2], x.a[u][3], x.a[u][4],
+                                                                x.a[u][5], x.a[u][6], x.a[u][7], x.a[u][8], x.z[u][0],
+                                                                x.z[u][1], x.z[u][2], 0.0, 0.0, 0.0, o[0], o[1], o[2]);
+                                 });
+    double acc[1] = {0.0};
+    if (active && w < 3) {
+        double o = (b ? b[3 * row + w] : 0.0) - y;
+        if ((fixmask[row] >> w) & 1u) o = 0;
+        out[3 * row + w] = o;
+        acc[0] = o * o;
+    }
+    write_partials<1, W>(acc, partials, lds);
+}
+
+// ---------------------------------------------------------------------------
 // The multilevel modes' update (x += alpha p, r -= alpha q, r.r) touches no 3x3
 // block, so it runs over the flat DOF arrays: workgroup lw owns DOFs
 // [lw c, lw c + c) with c = ceil(3N / G) rounded up to 4, and every thread handles 4
 // consecutive DOFs per trip with 16-byte loads (FP32) or two 16-byte loads (FP64).
 // The same arithmetic per DOF as k_pcg_update; r.r is summed per DOF range.
-template <class T, class TX>
-__global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8, 8)))
-k_pcg_update_flat(int k, int G, int n3, const T *__restrict__ pnew, const T *__restrict__ q, TX *__restrict__ x,
+template <class T, class TX, int W>
+__global__ void __launch_bounds__(W) __attribute__((amdgpu_waves_per_eu(8, 8)))
+k_pcg_update_flat(int k, int G, int Ga, int n3, const T *__restrict__ pnew, const T *__restrict__ q, TX *__restrict__ x,
                   T *__restrict__ r, SolverScalars *scal, double *partials)
 {
-    __shared__ double lds[2 * (WG / 64) + 2];
+    __shared__ double lds[2 * (W / 64) + 2];
     typedef T v4 __attribute__((ext_vector_type(4)));
     typedef TX x4 __attribute__((ext_vector_type(4)));
     if (scal->done) return;
@@ -657,7 +868,7 @@ k_pcg_update_flat(int k, int G, int n3, const T *__restrict__ pnew, const T *__r
     x4 xv0 = {};
     if (PRE && i0 + 3 < e0) xv0 = *reinterpret_cast<const x4 *>(x + i0);
     double pq[1], rz[1];
-    reduce_partials2<1, 1>(PA(partials), PB(partials, k & 1), pq, rz, lds, G);
+    reduce_partials2<1, 1, W>(PA(partials), PB(partials, k & 1), pq, rz, lds, Ga, G);
     if (!(pq[0] > 0.0)) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             scal->done = 1;
@@ -676,7 +887,7 @@ k_pcg_update_flat(int k, int G, int n3, const T *__restrict__ pnew, const T *__r
         if (lw < 0) break;   // uniform in the workgroup
         const int b = min(lw * chunk, n3), e = min(b + chunk, n3);
         double srr = 0.0;
-        for (int i = b + 4 * (int)threadIdx.x; i < e; i += 4 * WG) {
+        for (int i = b + 4 * (int)threadIdx.x; i < e; i += 4 * W) {
             if (i + 3 < e) {
                 // i is a multiple of 4: aligned 4-element vector loads and stores
                 const v4 pv = *reinterpret_cast<const v4 *>(pnew + i), qv = *reinterpret_cast<const v4 *>(q + i);
@@ -704,7 +915,7 @@ k_pcg_update_flat(int k, int G, int n3, const T *__restrict__ pnew, const T *__r
             }
         }
         double v[1] = {srr};
-        write_partials<1>(v, PB(partials, (k + 1) & 1) + eolc::kMaxPartials, lds, lw);
+        write_partials<1, W>(v, PB(partials, (k + 1) & 1) + eolc::kMaxPartials, lds, lw);
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         scal->iters = k + 1;
@@ -714,14 +925,13 @@ k_pcg_update_flat(int k, int G, int n3, const T *__restrict__ pnew, const T *__r
 }
 
 // ---------------------------------------------------------------------------
-// TX is the solution accumulator (double in FP64 mode, float in mixed mode).  ML:
-// the multilevel kernels form z and r.z afterwards (k_ml.hip); only r.r here.
-template <class T, class TX, bool ML>
-__global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8, 8)))
-k_pcg_update(int k, int N, const T *__restrict__ D, const T *__restrict__ pnew, const T *__restrict__ q,
+// TX is the solution accumulator (FP64 in both modes).
+template <class T, class TX, int W>
+__global__ void __launch_bounds__(W) __attribute__((amdgpu_waves_per_eu(8, 8)))
+k_pcg_update(int k, int Ga, int N, const T *__restrict__ D, const T *__restrict__ pnew, const T *__restrict__ q,
              TX *__restrict__ x, T *__restrict__ r, T *__restrict__ z, SolverScalars *scal, double *partials)
 {
-    __shared__ double lds[2 * (WG / 64) + 2];
+    __shared__ double lds[2 * (W / 64) + 2];
     if (scal->done) return;
     // the thread's first vertex is loaded before the partial sums are re-reduced
     // (the loads do not depend on alpha), so the two latencies overlap
@@ -737,7 +947,7 @@ k_pcg_update(int k, int N, const T *__restrict__ D, const T *__restrict__ pnew, 
         }
     }
     double pq[1], rz[1];
-    reduce_partials2<1, 1>(PA(partials), PB(partials, k & 1), pq, rz, lds);
+    reduce_partials2<1, 1, W>(PA(partials), PB(partials, k & 1), pq, rz, lds, Ga, gridDim.x);
     if (!(pq[0] > 0.0)) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             scal->done = 1;
@@ -749,7 +959,7 @@ k_pcg_update(int k, int N, const T *__restrict__ D, const T *__restrict__ pnew, 
     const double alpha = rz[0] / pq[0];
     const T alphaT = (T)alpha;
     double srz = 0.0, srr = 0.0;
-    for (int i = i0; i < re; i += WG) {
+    for (int i = i0; i < re; i += W) {
         if (i != i0) {
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
@@ -768,21 +978,14 @@ k_pcg_update(int k, int N, const T *__restrict__ D, const T *__restrict__ pnew, 
         const T r1 = fma(-alphaT, qv[1], rv[1]);
         const T r2 = fma(-alphaT, qv[2], rv[2]);
         r[3 * i] = r0; r[3 * i + 1] = r1; r[3 * i + 2] = r2;
-        if constexpr (!ML) {
-            T z0, z1, z2;
-            eolc::apply_sym3<T>(D + i, N, r0, r1, r2, z0, z1, z2);
-            z[3 * i] = z0; z[3 * i + 1] = z1; z[3 * i + 2] = z2;
-            srz += ((double)r0 * (double)z0 + (double)r1 * (double)z1) + (double)r2 * (double)z2;
-        }
+        T z0, z1, z2;
+        eolc::apply_sym3<T>(D + i, N, r0, r1, r2, z0, z1, z2);
+        z[3 * i] = z0; z[3 * i + 1] = z1; z[3 * i + 2] = z2;
+        srz += ((double)r0 * (double)z0 + (double)r1 * (double)z1) + (double)r2 * (double)z2;
         srr += ((double)r0 * (double)r0 + (double)r1 * (double)r1) + (double)r2 * (double)r2;
     }
-    if constexpr (ML) {
-        double v[1] = {srr};
-        write_partials<1>(v, PB(partials, (k + 1) & 1) + eolc::kMaxPartials, lds);
-    } else {
-        double v[2] = {srz, srr};
-        write_partials<2>(v, PB(partials, (k + 1) & 1), lds);
-    }
+    double v[2] = {srz, srr};
+    write_partials<2, W>(v, PB(partials, (k + 1) & 1), lds);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         scal->iters = k + 1;
         scal->pq = pq[0];
@@ -844,16 +1047,16 @@ __global__ void __launch_bounds__(WG) k_reduce_to(int G, const double *__restric
 
 // z = D r (r converted from FP64 to T), partials r.z, r.r -> PB[parity].  ML: r and
 // r.r only; the multilevel kernels form z and r.z.
-template <class T, bool ML>
-__global__ void __launch_bounds__(WG)
+template <class T, bool ML, int W>
+__global__ void __launch_bounds__(W)
 k_precond_init(int parity, int N, const T *__restrict__ D, const double *r64, T *r, T *__restrict__ z,
                double *partials)
 {
-    __shared__ double lds[2 * (WG / 64) + 2];
+    __shared__ double lds[2 * (W / 64) + 2];
     int rb, re;
     wg_rows(N, &rb, &re);
     double rz = 0.0, rr = 0.0;
-    for (int i = rb + threadIdx.x; i < re; i += WG) {
+    for (int i = rb + threadIdx.x; i < re; i += W) {
         const T r0 = (T)r64[3 * i], r1 = (T)r64[3 * i + 1], r2 = (T)r64[3 * i + 2];
         r[3 * i] = r0; r[3 * i + 1] = r1; r[3 * i + 2] = r2;
         const double s0 = r0, s1 = r1, s2 = r2;
@@ -870,10 +1073,10 @@ k_precond_init(int parity, int N, const T *__restrict__ D, const double *r64, T 
     }
     if constexpr (ML) {
         double v[1] = {rr};
-        write_partials<1>(v, PB(partials, parity) + eolc::kMaxPartials, lds);
+        write_partials<1, W>(v, PB(partials, parity) + eolc::kMaxPartials, lds);
     } else {
         double v[2] = {rz, rr};
-        write_partials<2>(v, PB(partials, parity), lds);
+        write_partials<2, W>(v, PB(partials, parity), lds);
     }
 }
 
@@ -1105,28 +1308,45 @@ void launch_spmv_one(eolc_ctx *c, int k, int G, const T *A, const T *Mm, const T
 {
     const eolc::Topology &t = c->topo;
     constexpr bool diff = std::is_same<T, float>::value;
+    const int Gb = eolc::vec_grid(t.N);
     if constexpr (LAY == 5) {
         using TR = T;
         const PatchLayout pl{c->pt_row, c->pt_cnt, c->pt_roff, c->pt_soff, c->pt_loff, c->pt_woff, c->pt_win,
                              c->pt_lo,  c->P32,    c->P64,     t.pt_slots, c->smask,   c->sellbase, c->scol,
                              c->A64s};
         hipLaunchKernelGGL((k_pcg_spmv_patch<T, TR, NT, W, U>), dim3(G), dim3(WG), 0, c->stream, k, pl, Mm, c->fixmask,
-                           z, pold, pnew, q, c->scal, c->partials);
+                           z, pold, pnew, q, c->scal, c->partials, Gb);
     } else {
         const SymLayout sym{c->supper, c->uoff, c->loff, c->lrec, c->S32u, c->S32a, c->S64u};
         hipLaunchKernelGGL((k_pcg_spmv<T, diff || LAY == 4, U, PF, NT, W, (diff || LAY >= 3) ? LAY : 0, STG>),
                            dim3(G), dim3(WG), 0, c->stream, k, t.N, t.nslices, c->slice_off, c->srow, c->slen, c->scol,
-                           A, Mm, t.nbs, c->fixmask, z, pold, pnew, q, c->scal, c->partials, sym, c->wwin);
+                           A, Mm, t.nbs, c->fixmask, z, pold, pnew, q, c->scal, c->partials, sym, c->wwin, Gb);
     }
+}
+
+// Workgroups of the split kernels (a multiple of 8, as logical_wg needs it).
+inline int split_grid(int nslices) { return (nslices + 7) & ~7; }
+
+// partial sums of p.q that the product of `variant` leaves
+inline int spmv_partials(const eolc::Topology &t, bool mixed, int variant)
+{
+    return eolc::spmv_runs(t, mixed, variant) == eolc::kSpmvSplit ? split_grid(t.nslices)
+                                                                  : eolc::pcg_grid(t.N);
 }
 
 template <class T>
 void launch_spmv(eolc_ctx *c, int variant, int k, int G, const T *A, const T *Mm, const T *z, const T *pold, T *pnew,
                  T *q)
 {
-    // a staged or patch variant chosen for an earlier mesh that this mesh cannot run:
-    // its twin with the same bits
-    if (!eolc::spmv_usable(c->topo, variant)) variant = eolc::spmv_fallback(variant);
+    constexpr bool mixed = std::is_same<T, float>::value;
+    variant = eolc::spmv_runs(c->topo, mixed, variant);
+    if (variant == eolc::kSpmvSplit) {
+        const eolc::Topology &t = c->topo;
+        hipLaunchKernelGGL((k_pcg_spmv_split<T, mixed>), dim3(split_grid(t.nslices)), dim3(kSplitWG), 0, c->stream, k,
+                           t.N, t.nslices, c->slice_off, c->srow, c->slen, c->scol, A, Mm, t.nbs, c->fixmask, z, pold,
+                           pnew, q, c->scal, c->partials, eolc::vec_grid(t.N));
+        return;
+    }
 #define EOLC_SPMV_CASE(id, U, PF, NT, W, LAY, STG)                                      \
     case id:                                                                       \
         launch_spmv_one<T, U, PF, NT, W, LAY, STG>(c, k, G, A, Mm, z, pold, pnew, q); \
@@ -1146,15 +1366,21 @@ void launch_iteration(eolc_ctx *c, int k, int G, const T *A, const T *Mm, const 
     const eolc::Topology &t = c->topo;
     const int pin = k & 1, pout = pin ^ 1;
     constexpr bool diff = std::is_same<T, float>::value;
-    launch_spmv<T>(c, c->spmv_variant[diff ? 0 : 1], k, G, A, Mm, z, p[pin], p[pout], q);
-    if (c->ml_on) {
-        hipLaunchKernelGGL((k_pcg_update_flat<T, TX>), dim3(eolc::pcg_grid_phys(G)), dim3(WG), 0, c->stream, k, G,
-                           3 * t.N, p[pout], q, x, r, c->scal, c->partials);
-        (void)eolc::ml_apply(c, diff, (k + 1) & 1, 1);   // launch errors surface at the chunk's hipGetLastError
-    } else {
-        hipLaunchKernelGGL((k_pcg_update<T, TX, false>), dim3(G), dim3(WG), 0, c->stream, k, t.N, D, p[pout], q, x,
-                           r, z, c->scal, c->partials);
-    }
+    const int variant = c->spmv_variant[diff ? 0 : 1];
+    launch_spmv<T>(c, variant, k, G, A, Mm, z, p[pin], p[pout], q);
+    const int Ga = spmv_partials(t, diff, variant), Gv = eolc::vec_grid(t.N);
+    auto update = [&](auto wg) {
+        constexpr int W = decltype(wg)::value;
+        if (c->ml_on)
+            hipLaunchKernelGGL((k_pcg_update_flat<T, TX, W>), dim3(W == WG ? eolc::pcg_grid_phys(Gv) : Gv), dim3(W), 0,
+                               c->stream, k, Gv, Ga, 3 * t.N, p[pout], q, x, r, c->scal, c->partials);
+        else
+            hipLaunchKernelGGL((k_pcg_update<T, TX, W>), dim3(Gv), dim3(W), 0, c->stream, k, Ga, t.N, D, p[pout], q, x,
+                               r, z, c->scal, c->partials);
+    };
+    if (eolc::vec_wg(t.N) == eolc::kVecWG) update(std::integral_constant<int, eolc::kVecWG>());
+    else update(std::integral_constant<int, WG>());
+    if (c->ml_on) (void)eolc::ml_apply(c, diff, (k + 1) & 1, 1);   // launch errors surface at the chunk's hipGetLastError
 }
 
 // z = P r for the residual r64 (FP64): mixed -> r32, z32; FP64 -> z64 (r64 in place);
@@ -1162,32 +1388,42 @@ void launch_iteration(eolc_ctx *c, int k, int G, const T *A, const T *Mm, const 
 hipError_t precondition(eolc_ctx *c, bool mixed, int parity)
 {
     const int N = c->topo.N;
-    const int G = eolc::pcg_grid(N);
-    if (mixed) {
-        if (c->ml_on)
-            hipLaunchKernelGGL((k_precond_init<float, true>), dim3(G), dim3(WG), 0, c->stream, parity, N, c->D32,
-                               c->r64, c->r32, c->z32, c->partials);
-        else
-            hipLaunchKernelGGL((k_precond_init<float, false>), dim3(G), dim3(WG), 0, c->stream, parity, N, c->D32,
-                               c->r64, c->r32, c->z32, c->partials);
-    } else {
-        if (c->ml_on)
-            hipLaunchKernelGGL((k_precond_init<double, true>), dim3(G), dim3(WG), 0, c->stream, parity, N, c->D64,
-                               c->r64, c->r64, c->z64, c->partials);
-        else
-            hipLaunchKernelGGL((k_precond_init<double, false>), dim3(G), dim3(WG), 0, c->stream, parity, N, c->D64,
-                               c->r64, c->r64, c->z64, c->partials);
-    }
+    auto go = [&](auto wg, auto ml, const auto *D, auto *r, auto *z) {
+        constexpr int W = decltype(wg)::value;
+        using T = std::remove_pointer_t<decltype(r)>;
+        hipLaunchKernelGGL((k_precond_init<T, decltype(ml)::value, W>), dim3(eolc::vec_grid(N)), dim3(W), 0, c->stream,
+                           parity, N, D, c->r64, r, z, c->partials);
+    };
+    auto by_type = [&](auto wg, auto ml) {
+        if (mixed) go(wg, ml, c->D32, c->r32, c->z32);
+        else go(wg, ml, c->D64, c->r64, c->z64);
+    };
+    auto by_ml = [&](auto wg) {
+        if (c->ml_on) by_type(wg, std::true_type());
+        else by_type(wg, std::false_type());
+    };
+    if (eolc::vec_wg(N) == eolc::kVecWG) by_ml(std::integral_constant<int, eolc::kVecWG>());
+    else by_ml(std::integral_constant<int, WG>());
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && c->ml_on) e = eolc::ml_apply(c, mixed, parity, 0);
     return e;
 }
 
-void launch_resid64(eolc_ctx *c, int G, const double *xin, const double *b, double *out)
+// out = b - A x; *dst = ||out||^2
+void launch_resid64(eolc_ctx *c, const double *xin, const double *b, double *out, double *dst)
 {
     const eolc::Topology &t = c->topo;
-    hipLaunchKernelGGL(k_resid64, dim3(G), dim3(WG), 0, c->stream, t.N, t.nslices, c->slice_off, c->srow, c->slen,
-                       c->scol, c->A64, t.nbs, c->fixmask, xin, b, out, c->partials + 5 * eolc::kMaxPartials);
+    double *part = c->partials + 5 * eolc::kMaxPartials;
+    int G = eolc::pcg_grid(t.N);
+    if (t.N <= kSplitRows) {
+        G = split_grid(t.nslices);
+        hipLaunchKernelGGL(k_resid64_split, dim3(G), dim3(kSplitWG), 0, c->stream, t.N, t.nslices, c->slice_off, c->srow,
+                           c->slen, c->scol, c->A64, t.nbs, c->fixmask, xin, b, out, part);
+    } else {
+        hipLaunchKernelGGL(k_resid64, dim3(G), dim3(WG), 0, c->stream, t.N, t.nslices, c->slice_off, c->srow, c->slen,
+                           c->scol, c->A64, t.nbs, c->fixmask, xin, b, out, part);
+    }
+    hipLaunchKernelGGL(k_reduce_to, dim3(1), dim3(WG), 0, c->stream, G, part, dst);
 }
 
 }  // namespace
@@ -1240,6 +1476,18 @@ bool spmv_usable(const Topology &t, int variant)
     return true;
 }
 
+// What runs for `variant` on this topology: its twin with the same bits where it cannot
+// run (a staged or patch variant chosen for an earlier mesh), and on small meshes the
+// split kernel for all that apply the same form (every FP32 variant but the patch ones;
+// in FP64 those of the assembled form): the same row sums, and they all stay bitwise
+// equal to each other.
+int spmv_runs(const Topology &t, bool mixed, int variant)
+{
+    if (!spmv_usable(t, variant)) variant = spmv_fallback(variant);
+    const bool diff64 = !mixed && fp64_layout(variant) != 0;
+    return t.N <= kSplitRows && !spmv_patch(variant) && !diff64 ? kSpmvSplit : variant;
+}
+
 // the staged variants' unstaged twins; the patch variants' symmetric-record twin (18:
 // the same sums in the same order, in both precisions)
 int spmv_fallback(int variant) { return spmv_patch(variant) ? 18 : spmv_unstaged(variant); }
@@ -1273,6 +1521,11 @@ int pcg_grid_phys(int G)
     const int E = G % 512;
     return (G > 512 && E > 0 && E <= 64) ? G - E : G;
 }
+
+// The vector kernels take 256 threads a workgroup while 1,024 would leave compute units
+// idle (fewer than 256 workgroups).
+int vec_wg(int N) { return pcg_grid(N) < 256 ? kVecWG : WG; }
+int vec_grid(int N) { return vec_wg(N) == WG ? pcg_grid(N) : ((N + kVecWG - 1) / kVecWG + 7) & ~7; }
 
 int pcg_grid(int N)
 {
@@ -1313,12 +1566,9 @@ hipError_t pcg_init(eolc_ctx *c, bool mixed)
 {
     const int N = c->topo.N;
     const int G = pcg_grid(N);
-    const double *pr = c->partials + 5 * kMaxPartials;
-    launch_resid64(c, G, c->vfix, c->rhs, c->b64);
-    hipLaunchKernelGGL(k_reduce_to, dim3(1), dim3(WG), 0, c->stream, G, pr, &c->scal->bnorm2);
+    launch_resid64(c, c->vfix, c->rhs, c->b64, &c->scal->bnorm2);
     hipLaunchKernelGGL(k_masked_copy, dim3(blocks_for(3 * N)), dim3(256), 0, c->stream, N, c->v, c->fixmask, c->xs64);
-    launch_resid64(c, G, c->xs64, c->b64, c->r64);
-    hipLaunchKernelGGL(k_reduce_to, dim3(1), dim3(WG), 0, c->stream, G, pr, &c->scal->rmax2);
+    launch_resid64(c, c->xs64, c->b64, c->r64, &c->scal->rmax2);
     hipError_t e = hipMemsetAsync(mixed ? (void *)c->p32[0] : (void *)c->p64[0], 0,
                                   (size_t)3 * N * (mixed ? sizeof(float) : sizeof(double)), c->stream);
     if (e != hipSuccess) return e;
@@ -1350,9 +1600,7 @@ hipError_t pcg_reliable_update(eolc_ctx *c)
     const int N = c->topo.N;
     const int G = pcg_grid(N);
     hipLaunchKernelGGL(k_accumulate, dim3(blocks_for(3 * N)), dim3(256), 0, c->stream, 3 * N, c->xs64, c->xl64);
-    launch_resid64(c, G, c->xs64, c->b64, c->r64);
-    hipLaunchKernelGGL(k_reduce_to, dim3(1), dim3(WG), 0, c->stream, G, c->partials + 5 * kMaxPartials,
-                       &c->scal->rmax2);
+    launch_resid64(c, c->xs64, c->b64, c->r64, &c->scal->rmax2);
     return hipGetLastError();
 }
 
@@ -1369,9 +1617,7 @@ hipError_t pcg_restart_from_guess(eolc_ctx *c)
     hipLaunchKernelGGL(k_masked_copy, dim3(blocks_for(3 * N)), dim3(256), 0, c->stream, N, c->v, c->fixmask, c->xs64);
     hipError_t e = hipMemsetAsync(c->xl64, 0, (size_t)3 * N * sizeof(double), c->stream);
     if (e != hipSuccess) return e;
-    launch_resid64(c, G, c->xs64, c->b64, c->r64);
-    hipLaunchKernelGGL(k_reduce_to, dim3(1), dim3(WG), 0, c->stream, G, c->partials + 5 * kMaxPartials,
-                       &c->scal->rmax2);
+    launch_resid64(c, c->xs64, c->b64, c->r64, &c->scal->rmax2);
     return hipGetLastError();
 }
 
@@ -1387,9 +1633,7 @@ hipError_t pcg_precondition(eolc_ctx *c, bool mixed) { return precondition(c, mi
 hipError_t pcg_replace_residual64(eolc_ctx *c)
 {
     const int G = pcg_grid(c->topo.N);
-    launch_resid64(c, G, c->xs64, c->b64, c->r64);
-    hipLaunchKernelGGL(k_reduce_to, dim3(1), dim3(WG), 0, c->stream, G, c->partials + 5 * kMaxPartials,
-                       &c->scal->rmax2);
+    launch_resid64(c, c->xs64, c->b64, c->r64, &c->scal->rmax2);
     return hipGetLastError();
 }
 
@@ -1426,9 +1670,7 @@ hipError_t spmv_true_residual(eolc_ctx *c, const double *v)
 {
     const int N = c->topo.N;
     const int G = pcg_grid(N);
-    launch_resid64(c, G, v, c->rhs, c->r64);
-    hipLaunchKernelGGL(k_reduce_to, dim3(1), dim3(WG), 0, c->stream, G, c->partials + 5 * kMaxPartials,
-                       &c->scal->true_rr);
+    launch_resid64(c, v, c->rhs, c->r64, &c->scal->true_rr);
     return hipGetLastError();
 }
 

@@ -56,11 +56,12 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
-// Sum over the workgroup of K values per thread; result broadcast to all threads.
-template <int K>
-__device__ __forceinline__ void block_allsum(double (&v)[K], double *lds /* K * WG/64 + K */)
+// Sum over the workgroup (W threads) of K values per thread; result broadcast to all
+// threads.
+template <int K, int W = WG>
+__device__ __forceinline__ void block_allsum(double (&v)[K], double *lds /* K * W/64 + K */)
 {
-    constexpr int NW = WG / 64;
+    constexpr int NW = W / 64;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     __syncthreads();
 #pragma unroll
@@ -85,7 +86,7 @@ __device__ __forceinline__ void block_allsum(double (&v)[K], double *lds /* K * 
 
 // Fixed-order sum of K partial arrays (stride kMaxPartials) of length G, done by
 // every workgroup; the result is identical everywhere.
-template <int K>
+template <int K, int W = WG>
 __device__ __forceinline__ void reduce_partials(const double *__restrict__ part, double (&out)[K], double *lds,
                                                 int G = -1)
 {
@@ -93,40 +94,45 @@ __device__ __forceinline__ void reduce_partials(const double *__restrict__ part,
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         double s = 0.0;
-        for (int i = threadIdx.x; i < G; i += WG) s += part[k * eolc::kMaxPartials + i];
+        for (int i = threadIdx.x; i < G; i += W) s += part[k * eolc::kMaxPartials + i];
         out[k] = s;
     }
-    block_allsum<K>(out, lds);
+    block_allsum<K, W>(out, lds);
 }
 
 // Two partial arrays in one pass (K1 sums of p1, then K2 of p2): the same per-array
 // order as two reduce_partials calls, so the same bits, with one load round and one
-// workgroup sum instead of two.  lds: (K1 + K2) * WG/64 + K1 + K2 doubles.
-template <int K1, int K2>
+// workgroup sum instead of two.  p1 holds G1 partials per sum, p2 G2 (the kernels that
+// wrote them may have run on different grids).  lds: (K1 + K2) * W/64 + K1 + K2 doubles.
+template <int K1, int K2, int W = WG>
 __device__ __forceinline__ void reduce_partials2(const double *__restrict__ p1, const double *__restrict__ p2,
-                                                 double (&o1)[K1], double (&o2)[K2], double *lds, int G = -1)
+                                                 double (&o1)[K1], double (&o2)[K2], double *lds, int G1, int G2)
 {
-    if (G < 0) G = gridDim.x;
     double v[K1 + K2];
 #pragma unroll
     for (int k = 0; k < K1 + K2; ++k) v[k] = 0.0;
-    for (int i = threadIdx.x; i < G; i += WG) {
+    for (int i = threadIdx.x; i < max(G1, G2); i += W) {
+        // both arrays' loads together (a branch around either would wait for it)
+        const int i1 = min(i, G1 - 1), i2 = min(i, G2 - 1);
+        double x[K1 + K2];
 #pragma unroll
-        for (int k = 0; k < K1; ++k) v[k] += p1[k * eolc::kMaxPartials + i];
+        for (int k = 0; k < K1; ++k) x[k] = p1[k * eolc::kMaxPartials + i1];
 #pragma unroll
-        for (int k = 0; k < K2; ++k) v[K1 + k] += p2[k * eolc::kMaxPartials + i];
+        for (int k = 0; k < K2; ++k) x[K1 + k] = p2[k * eolc::kMaxPartials + i2];
+#pragma unroll
+        for (int k = 0; k < K1 + K2; ++k) v[k] += i < (k < K1 ? G1 : G2) ? x[k] : 0.0;
     }
-    block_allsum<K1 + K2>(v, lds);
+    block_allsum<K1 + K2, W>(v, lds);
 #pragma unroll
     for (int k = 0; k < K1; ++k) o1[k] = v[k];
 #pragma unroll
     for (int k = 0; k < K2; ++k) o2[k] = v[K1 + k];
 }
 
-template <int K>
+template <int K, int W = WG>
 __device__ __forceinline__ void write_partials(double (&v)[K], double *__restrict__ part, double *lds, int lw = -1)
 {
-    block_allsum<K>(v, lds);
+    block_allsum<K, W>(v, lds);
     if (threadIdx.x == 0) {
         if (lw < 0) lw = logical_wg();
 #pragma unroll

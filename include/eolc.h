@@ -459,7 +459,9 @@ int eolc_stream_read(eolc_ctx *ctx, int64_t bytes, int reps, double *avg_ms);
  * true residual is always formed from the assembled FP64 matrix), that the patch
  * variants sum the dot product p.q per patch (other rounding of alpha; their
  * products q are the same bits, except for blocks above the stiff threshold, see
- * eolc_set_stiff_threshold).  ms (may be NULL)
+ * eolc_set_stiff_threshold).  On small meshes (up to 90,000 vertices) one kernel with a
+ * workgroup per 64 rows runs for all of 0-24 but 18 and 22 in FP64: the same row
+ * sums, p.q summed per 64 rows.  ms (may be NULL)
  * receives EOLC_SPMV_VARIANTS average times; *best (may be NULL) the choice.
  * eolc_set_spmv_variant sets the choice directly. */
 #define EOLC_SPMV_VARIANTS 29
