@@ -75,19 +75,92 @@ __device__ __forceinline__ void slice_partial(const double (&v)[K], int sl, doub
     }
 }
 
+// Products of a row's SELL entries added in order, AH entries' loads in flight: a
+// workgroup owns a whole instance, so a wavefront walks up to 17 slices one after the
+// other and every dependent load is waited for.  apply(j, a): one entry's block (9
+// values) on column j.
+template <class T, int AH, class Apply>
+__device__ __forceinline__ void row_entries(const T *__restrict__ A, int64_t nbs, const int *__restrict__ cl, int base,
+                                            int len, Apply apply)
+{
+    for (int k0 = 0; k0 < len; k0 += AH) {
+        T a[AH][9];
+        int j[AH];
+#pragma unroll
+        for (int u = 0; u < AH; ++u)
+            if (k0 + u < len) {
+                const int e = base + (k0 + u) * SL;
+                j[u] = cl[e];
+#pragma unroll
+                for (int c = 0; c < 9; ++c) a[u][c] = A[c * nbs + e];
+            }
+        apply(j, a, len - k0);
+    }
+}
+
 // FP64 row product y = (A x)_row over the SELL entries of one row.
 __device__ __forceinline__ void row_spmv64(const double *__restrict__ A, int64_t nbs, const int *__restrict__ cl,
                                            int base, int len, const double *__restrict__ x, double &y0, double &y1,
                                            double &y2)
 {
     y0 = y1 = y2 = 0.0;
-    for (int kk = 0; kk < len; ++kk) {
-        const int e = base + kk * SL;
-        const int j = cl[e];
-        const double u0 = x[3 * j], u1 = x[3 * j + 1], u2 = x[3 * j + 2];
-        y0 += fma(A[2 * nbs + e], u2, fma(A[1 * nbs + e], u1, A[0 * nbs + e] * u0));
-        y1 += fma(A[5 * nbs + e], u2, fma(A[4 * nbs + e], u1, A[3 * nbs + e] * u0));
-        y2 += fma(A[8 * nbs + e], u2, fma(A[7 * nbs + e], u1, A[6 * nbs + e] * u0));
+    constexpr int AH = 2;   // four spill at 1,024 threads
+    row_entries<double, AH>(A, nbs, cl, base, len, [&](const int (&j)[AH], const double (&a)[AH][9], int n) {
+        double u[AH][3];
+#pragma unroll
+        for (int t = 0; t < AH; ++t)
+            if (t < n)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) u[t][c] = x[3 * j[t] + c];
+#pragma unroll
+        for (int t = 0; t < AH; ++t)
+            if (t < n) {
+                y0 += fma(a[t][2], u[t][2], fma(a[t][1], u[t][1], a[t][0] * u[t][0]));
+                y1 += fma(a[t][5], u[t][2], fma(a[t][4], u[t][1], a[t][3] * u[t][0]));
+                y2 += fma(a[t][8], u[t][2], fma(a[t][7], u[t][1], a[t][6] * u[t][0]));
+            }
+    });
+}
+
+// FP32 difference form: y += S'_ij (p_j - p_i) over the entries, p by get(j, c).
+template <class Get>
+__device__ __forceinline__ void row_spmv32(const float *__restrict__ S, int64_t nbs, const int *__restrict__ cl,
+                                           int base, int len, float ui0, float ui1, float ui2, double &y0, double &y1,
+                                           double &y2, Get get)
+{
+    constexpr int AH = 4;
+    row_entries<float, AH>(S, nbs, cl, base, len, [&](const int (&j)[AH], const float (&a)[AH][9], int n) {
+        float u[AH][3];
+#pragma unroll
+        for (int t = 0; t < AH; ++t)
+            if (t < n)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) u[t][c] = get(j[t], c);
+#pragma unroll
+        for (int t = 0; t < AH; ++t)
+            if (t < n) {
+                const float d0 = u[t][0] - ui0, d1 = u[t][1] - ui1, d2 = u[t][2] - ui2;
+                y0 += (double)fmaf(a[t][2], d2, fmaf(a[t][1], d1, a[t][0] * d0));
+                y1 += (double)fmaf(a[t][5], d2, fmaf(a[t][4], d1, a[t][3] * d0));
+                y2 += (double)fmaf(a[t][8], d2, fmaf(a[t][7], d1, a[t][6] * d0));
+            }
+    });
+}
+
+// Runs load and then use on the instance's slices, two slices a trip.  The vector passes take the rows in vertex order (slice s
+// holds the vertices 64 s .. 64 s + 63), without the storage order's index load.
+template <int WGS, class Slice, class Load, class Use>
+__device__ __forceinline__ void each_slice(const eolc::BatchInst &I, Load load, Use use)
+{
+    constexpr int NW = WGS / 64;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    for (int sl = I.s0 + wave; sl < I.s1; sl += 2 * NW) {
+        Slice a, b;
+        const bool two = sl + NW < I.s1;   // uniform in the wavefront
+        load(a, sl * SL + lane);
+        if (two) load(b, (sl + NW) * SL + lane);
+        use(a, sl, sl * SL + lane);
+        if (two) use(b, sl + NW, (sl + NW) * SL + lane);
     }
 }
 
@@ -124,26 +197,31 @@ __device__ double inst_residual64(const eolc::BatchInst &I, const int *__restric
 
 // r32 = (float) r64, z = D r32; returns (r.z, r.r) over the instance.
 template <int WGS>
-__device__ void inst_precond(const eolc::BatchInst &I, const int *__restrict__ srow, int N,
-                             const float *__restrict__ D, const double *__restrict__ r64, float *__restrict__ r32,
-                             float *__restrict__ z32, double *part, int nslices, double *red, double &rz, double &rr)
+__device__ void inst_precond(const eolc::BatchInst &I, int N, const float *__restrict__ D,
+                             const double *__restrict__ r64, float *__restrict__ r32, float *__restrict__ z32,
+                             double *part, int nslices, double *red, double &rz, double &rr)
 {
-    constexpr int NW = WGS / 64;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    for (int sl = I.s0 + wave; sl < I.s1; sl += NW) {
-        const int i = srow[sl * SL + lane];
-        const float r0 = (float)r64[3 * i], r1 = (float)r64[3 * i + 1], r2 = (float)r64[3 * i + 2];
-        r32[3 * i] = r0; r32[3 * i + 1] = r1; r32[3 * i + 2] = r2;
-        const float *d = D + i;
-        const double s0 = r0, s1 = r1, s2 = r2;
-        const double e00 = d[0], e01 = d[N], e02 = d[2 * N], e11 = d[3 * N], e12 = d[4 * N], e22 = d[5 * N];
-        const float z0 = (float)fma(e02, s2, fma(e01, s1, e00 * s0));
-        const float z1 = (float)fma(e12, s2, fma(e11, s1, e01 * s0));
-        const float z2 = (float)fma(e22, s2, fma(e12, s1, e02 * s0));
-        z32[3 * i] = z0; z32[3 * i + 1] = z1; z32[3 * i + 2] = z2;
-        const double v[2] = {(s0 * (double)z0 + s1 * (double)z1) + s2 * (double)z2, (s0 * s0 + s1 * s1) + s2 * s2};
-        slice_partial<2>(v, sl, part, nslices);
-    }
+    struct In { double r[3]; float d[6]; };
+    each_slice<WGS, In>(
+        I,
+        [&](In &x, int i) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) x.r[c] = r64[3 * i + c];
+#pragma unroll
+            for (int c = 0; c < 6; ++c) x.d[c] = D[c * N + i];
+        },
+        [&](const In &x, int sl, int i) {
+            const float r0 = (float)x.r[0], r1 = (float)x.r[1], r2 = (float)x.r[2];
+            r32[3 * i] = r0; r32[3 * i + 1] = r1; r32[3 * i + 2] = r2;
+            const double s0 = r0, s1 = r1, s2 = r2;
+            const double e00 = x.d[0], e01 = x.d[1], e02 = x.d[2], e11 = x.d[3], e12 = x.d[4], e22 = x.d[5];
+            const float z0 = (float)fma(e02, s2, fma(e01, s1, e00 * s0));
+            const float z1 = (float)fma(e12, s2, fma(e11, s1, e01 * s0));
+            const float z2 = (float)fma(e22, s2, fma(e12, s1, e02 * s0));
+            z32[3 * i] = z0; z32[3 * i + 1] = z1; z32[3 * i + 2] = z2;
+            const double v[2] = {(s0 * (double)z0 + s1 * (double)z1) + s2 * (double)z2, (s0 * s0 + s1 * s1) + s2 * s2};
+            slice_partial<2>(v, sl, part, nslices);
+        });
     double s[2];
     inst_sum<2>(s, I, part, nslices, red);
     rz = s[0];
@@ -170,44 +248,61 @@ __device__ __forceinline__ void ml_inv_apply(const double *__restrict__ d, doubl
     c2 = fma(d[5], r2, fma(d[4], r1, d[2] * r0));
 }
 
+// Sum of n 3-vectors in order, eight loads in flight; get(k, c): component c of the kth.
+template <class Get> __device__ __forceinline__ void sum3(int k0, int k1, double (&t)[3], Get get)
+{
+    t[0] = t[1] = t[2] = 0.0;
+    for (int k = k0; k < k1; k += 8) {
+        double v[8][3];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int q = min(k + u, k1 - 1);
+            get(q, v[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (k + u < k1)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) t[c] += v[u][c];
+    }
+}
+
 // z = D r + sum_l Z_l D_l^-1 Z_l^T r over instance b (r32 of its rows complete);
 // returns r.z over the instance.  Sums in member / child order, FP64.
 template <int WGS>
-__device__ double inst_ml_apply(const eolc::BatchInst &I, int b, const BatchML &m, const int *__restrict__ srow,
-                                int N, const float *__restrict__ D, const float *__restrict__ r32,
-                                float *__restrict__ z32, const unsigned char *__restrict__ fixmask, double *part,
-                                int nslices, double *red)
+__device__ double inst_ml_apply(const eolc::BatchInst &I, int b, const BatchML &m, int N, const float *__restrict__ D,
+                                const float *__restrict__ r32, float *__restrict__ z32,
+                                const unsigned char *__restrict__ fixmask, double *part, int nslices, double *red)
 {
-    constexpr int NW = WGS / 64;
     constexpr int S = eolc::kMLMaxLevels + 1;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int L = m.lv.L;
     __syncthreads();   // every row's r32 is written
     {
         const int lo = m.lo[b * S + 1], hi = m.lo[(b + 1) * S + 1];
         for (int a = lo + (int)threadIdx.x; a < hi; a += WGS) {
-            double t0 = 0.0, t1 = 0.0, t2 = 0.0;
-            for (int k = m.ptr1[a]; k < m.ptr1[a + 1]; ++k) {
+            double t[3];
+            sum3(m.ptr1[a], m.ptr1[a + 1], t, [&](int k, double (&v)[3]) {
                 const int i = m.hord[k];
-                t0 += (double)r32[3 * i];
-                t1 += (double)r32[3 * i + 1];
-                t2 += (double)r32[3 * i + 2];
-            }
-            m.R[3 * a] = t0; m.R[3 * a + 1] = t1; m.R[3 * a + 2] = t2;
+#pragma unroll
+                for (int c = 0; c < 3; ++c) v[c] = (double)r32[3 * i + c];
+            });
+#pragma unroll
+            for (int c = 0; c < 3; ++c) m.R[3 * a + c] = t[c];
         }
     }
     __syncthreads();
     for (int l = 2; l <= L; ++l) {
         const int lo = m.lo[b * S + l], hi = m.lo[(b + 1) * S + l];
         for (int A = lo + (int)threadIdx.x; A < hi; A += WGS) {
-            const int c0 = m.cptr[m.lv.coff[l] + A], c1 = m.cptr[m.lv.coff[l] + A + 1];
-            double t0 = 0.0, t1 = 0.0, t2 = 0.0;
-            for (int a = c0; a < c1; ++a) {
+            double t[3];
+            sum3(m.cptr[m.lv.coff[l] + A], m.cptr[m.lv.coff[l] + A + 1], t, [&](int a, double (&v)[3]) {
                 const double *q = m.R + 3 * (int64_t)(m.lv.off[l - 1] + a);
-                t0 += q[0]; t1 += q[1]; t2 += q[2];
-            }
+#pragma unroll
+                for (int c = 0; c < 3; ++c) v[c] = q[c];
+            });
             double *o = m.R + 3 * (int64_t)(m.lv.off[l] + A);
-            o[0] = t0; o[1] = t1; o[2] = t2;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) o[c] = t[c];
         }
         __syncthreads();
     }
@@ -225,20 +320,30 @@ __device__ double inst_ml_apply(const eolc::BatchInst &I, int b, const BatchML &
         }
         __syncthreads();
     }
-    for (int sl = I.s0 + wave; sl < I.s1; sl += NW) {
-        const int i = srow[sl * SL + lane];
-        const float r0 = r32[3 * i], r1 = r32[3 * i + 1], r2 = r32[3 * i + 2];
-        float f0, f1, f2;
-        eolc::apply_sym3<float>(D + i, N, r0, r1, r2, f0, f1, f2);
-        const double *cc = m.C + 3 * (int64_t)m.agg1[i];
-        const unsigned fm = fixmask[i];
-        const float z0 = (fm & 1u) ? 0.0f : (float)((double)f0 + cc[0]);
-        const float z1 = (fm & 2u) ? 0.0f : (float)((double)f1 + cc[1]);
-        const float z2 = (fm & 4u) ? 0.0f : (float)((double)f2 + cc[2]);
-        z32[3 * i] = z0; z32[3 * i + 1] = z1; z32[3 * i + 2] = z2;
-        const double v[1] = {((double)r0 * (double)z0 + (double)r1 * (double)z1) + (double)r2 * (double)z2};
-        slice_partial<1>(v, sl, part, nslices);
-    }
+    struct In { float r[3], d[6]; double c[3]; unsigned fm; };
+    each_slice<WGS, In>(
+        I,
+        [&](In &x, int i) {
+            const double *cc = m.C + 3 * (int64_t)m.agg1[i];
+#pragma unroll
+            for (int c = 0; c < 6; ++c) x.d[c] = D[c * N + i];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) x.r[c] = r32[3 * i + c];
+            x.fm = fixmask[i];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) x.c[c] = cc[c];
+        },
+        [&](const In &x, int sl, int i) {
+            const float r0 = x.r[0], r1 = x.r[1], r2 = x.r[2];
+            float f0, f1, f2;
+            eolc::apply_sym3<float>(x.d, 1, r0, r1, r2, f0, f1, f2);
+            const float z0 = (x.fm & 1u) ? 0.0f : (float)((double)f0 + x.c[0]);
+            const float z1 = (x.fm & 2u) ? 0.0f : (float)((double)f1 + x.c[1]);
+            const float z2 = (x.fm & 4u) ? 0.0f : (float)((double)f2 + x.c[2]);
+            z32[3 * i] = z0; z32[3 * i + 1] = z1; z32[3 * i + 2] = z2;
+            const double v[1] = {((double)r0 * (double)z0 + (double)r1 * (double)z1) + (double)r2 * (double)z2};
+            slice_partial<1>(v, sl, part, nslices);
+        });
     double s[1];
     inst_sum<1>(s, I, part, nslices, red);
     return s[0];
@@ -246,13 +351,13 @@ __device__ double inst_ml_apply(const eolc::BatchInst &I, int b, const BatchML &
 
 // r32 = (float) r64 and r.r over the instance (the multilevel path forms z after).
 template <int WGS>
-__device__ double inst_convert(const eolc::BatchInst &I, const int *__restrict__ srow, const double *__restrict__ r64,
-                               float *__restrict__ r32, double *part, int nslices, double *red)
+__device__ double inst_convert(const eolc::BatchInst &I, const double *__restrict__ r64, float *__restrict__ r32,
+                               double *part, int nslices, double *red)
 {
     constexpr int NW = WGS / 64;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int sl = I.s0 + wave; sl < I.s1; sl += NW) {
-        const int i = srow[sl * SL + lane];
+        const int i = sl * SL + lane;
         const float r0 = (float)r64[3 * i], r1 = (float)r64[3 * i + 1], r2 = (float)r64[3 * i + 2];
         r32[3 * i] = r0; r32[3 * i + 1] = r1; r32[3 * i + 2] = r2;
         const double s0 = r0, s1 = r1, s2 = r2;
@@ -281,18 +386,28 @@ struct BatchArgs {
     int maxit;
     int *stats;
     double *dstats;
+    int stage;   // rows of LDS (3 floats each) the launch provides
     BatchML ml;
 };
 
 // Persistent mixed-precision PCG, one workgroup per instance.  ML: the preconditioner
-// adds the instance's multilevel coarse levels to the block-Jacobi blocks.
+// adds the instance's multilevel coarse levels to the block-Jacobi blocks.  The search
+// direction of an instance of at most `stage` rows is kept in LDS for the product, whose
+// column gathers (six dwords a block from two vectors) otherwise take more of the compute
+// unit's address rate than the block's own nine.  A 96 x 96 sheet's iteration takes 95 us
+// (190 us with one entry's loads at a time and the direction gathered from global
+// memory): 51 the product, the rest the passes over its vectors at 80 GB/s and the
+// barriers.  The next entries loaded ahead (56-60 us a product), the direction in LDS
+// alone and the levels >= 2 in LDS gained nothing.
 template <int WGS, bool ML>
 __global__ void __launch_bounds__(WGS) k_batch_pcg(BatchArgs a)
 {
     constexpr int NW = WGS / 64;
     __shared__ double red[4];
+    extern __shared__ float su[];   // 3 per row of a staged instance
     const int b = a.order[blockIdx.x];
     const eolc::BatchInst I = a.inst[b];
+    const bool staged = I.v1 - I.v0 <= a.stage;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int N = a.N, ns = a.nslices;
     const int64_t nbs = a.nbs;
@@ -315,10 +430,10 @@ __global__ void __launch_bounds__(WGS) k_batch_pcg(BatchArgs a)
                                         a.r64, a.part, ns, red);
     double rz, rr;
     if constexpr (ML) {
-        rr = inst_convert<WGS>(I, a.srow, a.r64, a.r32, a.part, ns, red);
-        rz = inst_ml_apply<WGS>(I, b, a.ml, a.srow, N, a.D32, a.r32, a.z32, a.fixmask, a.part, ns, red);
+        rr = inst_convert<WGS>(I, a.r64, a.r32, a.part, ns, red);
+        rz = inst_ml_apply<WGS>(I, b, a.ml, N, a.D32, a.r32, a.z32, a.fixmask, a.part, ns, red);
     } else {
-        inst_precond<WGS>(I, a.srow, N, a.D32, a.r64, a.r32, a.z32, a.part, ns, red, rz, rr);
+        inst_precond<WGS>(I, N, a.D32, a.r64, a.r32, a.z32, a.part, ns, red, rz, rr);
     }
     double rz_prev = 1.0;
     int k = 0, first = 0, refinements = 0, status = EOLC_ERR_MAXIT;
@@ -354,43 +469,57 @@ __global__ void __launch_bounds__(WGS) k_batch_pcg(BatchArgs a)
             }
             if (k >= a.maxit || refinements > eolc::kMaxRefinements) break;
             if constexpr (ML) {
-                rr = inst_convert<WGS>(I, a.srow, a.r64, a.r32, a.part, ns, red);
-                rz = inst_ml_apply<WGS>(I, b, a.ml, a.srow, N, a.D32, a.r32, a.z32, a.fixmask, a.part, ns, red);
+                rr = inst_convert<WGS>(I, a.r64, a.r32, a.part, ns, red);
+                rz = inst_ml_apply<WGS>(I, b, a.ml, N, a.D32, a.r32, a.z32, a.fixmask, a.part, ns, red);
             } else {
-                inst_precond<WGS>(I, a.srow, N, a.D32, a.r64, a.r32, a.z32, a.part, ns, red, rz, rr);
+                inst_precond<WGS>(I, N, a.D32, a.r64, a.r32, a.z32, a.part, ns, red, rz, rr);
             }
             continue;
         }
         if (k >= a.maxit) break;
         const double beta = (k == first) ? 0.0 : rz / rz_prev;
         const float betaT = (float)beta;
-        // p_new = z + beta p_old (own rows; neighbours formed on the fly), q = A p_new
+        // p_new = z + beta p_old of every row, then q = A p_new with p_new from LDS (from
+        // global memory when the instance is too large for it)
+        {
+            struct In { float z[3], p[3]; };
+            each_slice<WGS, In>(
+                I,
+                [&](In &x, int i) {
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        x.z[c] = a.z32[3 * i + c];
+                        x.p[c] = pold[3 * i + c];
+                    }
+                },
+                [&](const In &x, int sl, int i) {
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        const float u = fmaf(betaT, x.p[c], x.z[c]);
+                        pnew[3 * i + c] = u;
+                        if (staged) su[3 * (i - I.v0) + c] = u;
+                    }
+                });
+        }
+        __syncthreads();
         for (int sl = I.s0 + wave; sl < I.s1; sl += NW) {
             const int g = sl * SL + lane;
             const int row = a.srow[g], len = a.slen[g] - 1;   // the diagonal (last entry) is skipped
             const int base = a.slice_off[sl] + lane;
-            const float ui0 = fmaf(betaT, pold[3 * row], a.z32[3 * row]);
-            const float ui1 = fmaf(betaT, pold[3 * row + 1], a.z32[3 * row + 1]);
-            const float ui2 = fmaf(betaT, pold[3 * row + 2], a.z32[3 * row + 2]);
             const float mb = a.M32[row];
-            double y0 = (double)(mb * ui0), y1 = (double)(mb * ui1), y2 = (double)(mb * ui2);
-            for (int kk = 0; kk < len; ++kk) {
-                const int e = base + kk * SL;
-                const int j = a.scol[e];
-                const float u0 = fmaf(betaT, pold[3 * j], a.z32[3 * j]);
-                const float u1 = fmaf(betaT, pold[3 * j + 1], a.z32[3 * j + 1]);
-                const float u2 = fmaf(betaT, pold[3 * j + 2], a.z32[3 * j + 2]);
-                const float d0 = u0 - ui0, d1 = u1 - ui1, d2 = u2 - ui2;
-                const float *s = a.S32 + e;
-                y0 += (double)fmaf(s[2 * nbs], d2, fmaf(s[1 * nbs], d1, s[0 * nbs] * d0));
-                y1 += (double)fmaf(s[5 * nbs], d2, fmaf(s[4 * nbs], d1, s[3 * nbs] * d0));
-                y2 += (double)fmaf(s[8 * nbs], d2, fmaf(s[7 * nbs], d1, s[6 * nbs] * d0));
-            }
             const unsigned fm = a.fixmask[row];
+            double y0, y1, y2;
+            float ui0, ui1, ui2;
+            auto rows = [&](auto get) {
+                ui0 = get(row, 0); ui1 = get(row, 1); ui2 = get(row, 2);
+                y0 = (double)(mb * ui0); y1 = (double)(mb * ui1); y2 = (double)(mb * ui2);
+                row_spmv32(a.S32, nbs, a.scol, base, len, ui0, ui1, ui2, y0, y1, y2, get);
+            };
+            if (staged) rows([&](int j, int c) { return su[3 * (j - I.v0) + c]; });
+            else rows([&](int j, int c) { return pnew[3 * j + c]; });
             if (fm & 1) y0 = 0.0;
             if (fm & 2) y1 = 0.0;
             if (fm & 4) y2 = 0.0;
-            pnew[3 * row] = ui0; pnew[3 * row + 1] = ui1; pnew[3 * row + 2] = ui2;
             const float q0 = (float)y0, q1 = (float)y1, q2 = (float)y2;
             a.q32[3 * row] = q0; a.q32[3 * row + 1] = q1; a.q32[3 * row + 2] = q2;
             const double v[1] = {((double)ui0 * (double)q0 + (double)ui1 * (double)q1) + (double)ui2 * (double)q2};
@@ -405,32 +534,48 @@ __global__ void __launch_bounds__(WGS) k_batch_pcg(BatchArgs a)
         const double alpha = rz / pq[0];
         const float alphaT = (float)alpha;
         // x += alpha p, r -= alpha q, z = D r
-        for (int sl = I.s0 + wave; sl < I.s1; sl += NW) {
-            const int i = a.srow[sl * SL + lane];
+        {
+            struct In { float p[3], q[3], r[3], x[3], d[ML ? 1 : 6]; };
+            each_slice<WGS, In>(
+                I,
+                [&](In &x, int i) {
 #pragma unroll
-            for (int c = 0; c < 3; ++c) a.xl32[3 * i + c] = fmaf(alphaT, pnew[3 * i + c], a.xl32[3 * i + c]);
-            const float r0 = fmaf(-alphaT, a.q32[3 * i], a.r32[3 * i]);
-            const float r1 = fmaf(-alphaT, a.q32[3 * i + 1], a.r32[3 * i + 1]);
-            const float r2 = fmaf(-alphaT, a.q32[3 * i + 2], a.r32[3 * i + 2]);
-            a.r32[3 * i] = r0; a.r32[3 * i + 1] = r1; a.r32[3 * i + 2] = r2;
-            if constexpr (ML) {
-                const double v[1] = {((double)r0 * (double)r0 + (double)r1 * (double)r1) + (double)r2 * (double)r2};
-                slice_partial<1>(v, sl, a.part, ns);
-            } else {
-                float z0, z1, z2;
-                eolc::apply_sym3<float>(a.D32 + i, N, r0, r1, r2, z0, z1, z2);
-                a.z32[3 * i] = z0; a.z32[3 * i + 1] = z1; a.z32[3 * i + 2] = z2;
-                const double v[2] = {((double)r0 * (double)z0 + (double)r1 * (double)z1) + (double)r2 * (double)z2,
-                                     ((double)r0 * (double)r0 + (double)r1 * (double)r1) + (double)r2 * (double)r2};
-                slice_partial<2>(v, sl, a.part, ns);
-            }
+                    for (int c = 0; c < 3; ++c) {
+                        x.p[c] = pnew[3 * i + c];
+                        x.q[c] = a.q32[3 * i + c];
+                        x.r[c] = a.r32[3 * i + c];
+                        x.x[c] = a.xl32[3 * i + c];
+                    }
+                    if constexpr (!ML)
+#pragma unroll
+                        for (int c = 0; c < 6; ++c) x.d[c] = a.D32[c * N + i];
+                },
+                [&](const In &x, int sl, int i) {
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) a.xl32[3 * i + c] = fmaf(alphaT, x.p[c], x.x[c]);
+                    const float r0 = fmaf(-alphaT, x.q[0], x.r[0]);
+                    const float r1 = fmaf(-alphaT, x.q[1], x.r[1]);
+                    const float r2 = fmaf(-alphaT, x.q[2], x.r[2]);
+                    a.r32[3 * i] = r0; a.r32[3 * i + 1] = r1; a.r32[3 * i + 2] = r2;
+                    if constexpr (ML) {
+                        const double v[1] = {((double)r0 * (double)r0 + (double)r1 * (double)r1) + (double)r2 * (double)r2};
+                        slice_partial<1>(v, sl, a.part, ns);
+                    } else {
+                        float z0, z1, z2;
+                        eolc::apply_sym3<float>(x.d, 1, r0, r1, r2, z0, z1, z2);
+                        a.z32[3 * i] = z0; a.z32[3 * i + 1] = z1; a.z32[3 * i + 2] = z2;
+                        const double v[2] = {((double)r0 * (double)z0 + (double)r1 * (double)z1) + (double)r2 * (double)z2,
+                                             ((double)r0 * (double)r0 + (double)r1 * (double)r1) + (double)r2 * (double)r2};
+                        slice_partial<2>(v, sl, a.part, ns);
+                    }
+                });
         }
         rz_prev = rz;
         if constexpr (ML) {
             double s1[1];
             inst_sum<1>(s1, I, a.part, ns, red);
             rr = s1[0];
-            rz = inst_ml_apply<WGS>(I, b, a.ml, a.srow, N, a.D32, a.r32, a.z32, a.fixmask, a.part, ns, red);
+            rz = inst_ml_apply<WGS>(I, b, a.ml, N, a.D32, a.r32, a.z32, a.fixmask, a.part, ns, red);
         } else {
             double s2[2];
             inst_sum<2>(s2, I, a.part, ns, red);
@@ -490,13 +635,23 @@ __global__ void k_batch_fixmask(int n, const int *__restrict__ nodes, unsigned c
     if (t < n) fixmask[nodes[t]] = 7;
 }
 
+// Rows whose direction fits the LDS of a compute unit beside the kernel's own few words;
+// the launch asks for what its largest such instance needs.
+constexpr int kBatchStage = (160 * 1024 - 256) / 12;
+
 template <int WGS>
-void launch_batch(eolc_ctx *c, const BatchArgs &args, bool ml)
+hipError_t launch_batch(eolc_ctx *c, BatchArgs args, bool ml)
 {
-    if (ml)
-        hipLaunchKernelGGL((k_batch_pcg<WGS, true>), dim3(c->batch.B), dim3(WGS), 0, c->stream, args);
-    else
-        hipLaunchKernelGGL((k_batch_pcg<WGS, false>), dim3(c->batch.B), dim3(WGS), 0, c->stream, args);
+    const auto fn = ml ? k_batch_pcg<WGS, true> : k_batch_pcg<WGS, false>;
+    args.stage = 0;
+    for (const eolc::BatchInst &I : c->batch.inst)
+        if (I.v1 - I.v0 <= kBatchStage) args.stage = std::max(args.stage, I.v1 - I.v0);
+    const size_t lds = 12 * (size_t)args.stage;
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)(12 * kBatchStage));
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(fn, dim3(c->batch.B), dim3(WGS), lds, c->stream, args);
+    return hipGetLastError();
 }
 
 }  // namespace
@@ -539,11 +694,10 @@ hipError_t batch_solve_async(eolc_ctx *c, double tol, int maxit, int variant)
     const MLState &m = c->ml;
     a.ml = BatchML{m.lv, m.hord, m.ptr1, m.agg1, m.par, m.cptr, S.d_ml_lo, m.Dinv, m.R, m.C};
     switch (variant) {
-    case 0: launch_batch<256>(c, a, ml); break;
-    case 1: launch_batch<512>(c, a, ml); break;
-    default: launch_batch<1024>(c, a, ml); break;
+    case 0: return launch_batch<256>(c, a, ml);
+    case 1: return launch_batch<512>(c, a, ml);
+    default: return launch_batch<1024>(c, a, ml);
     }
-    return hipGetLastError();
 }
 
 }  // namespace eolc

@@ -187,3 +187,41 @@ def test_batch_instances_match_the_oracle():
               f"MDK {errs[1]:.1e} f {errs[2]:.1e}; v vs dense {ev:.1e} ({st[b].iters} iterations)", flush=True)
         assert max(errs) <= 1e-10
         assert ev <= 1e-6
+
+
+@pytest.mark.parametrize("sides", [(1, 2, 7), (115, 116, 40)])
+def test_instances_around_the_staged_size(sides):
+    """Instances from one slice to both sides of the LDS limit of the search direction
+    (13,632 rows: 115 x 115 quads are staged, 116 x 116 are not, in one launch): each
+    solves its own block of the downloaded system to the tolerance, and the three
+    workgroup sizes agree bit for bit."""
+    inst = [scene.Scene(s, 1e-3, 0.05, seed_x=50 + s, seed_v=90 + s) for s in sides]
+    with eolc.Context(0) as c:
+        off = c.set_batch_topology([i.X for i in inst], [i.tri for i in inst], [i.hinge for i in inst],
+                                   [i.fixed for i in inst])
+        c.set_material(0.1, 1.0, 0.3, 1e-5, 0.0, 1.0)
+        c.set_batch_material([500.0] * len(inst), [1e-5] * len(inst))
+        c.set_options(eolc.OPT_SPD_PROJECT_BENDING)
+        x, v = np.zeros(3 * off[-1]), np.zeros(3 * off[-1])
+        for b, i in enumerate(inst):
+            x[3 * off[b]:3 * off[b] + i.x0.size] = i.x0
+            v[3 * off[b]:3 * off[b] + i.v0.size] = i.v0
+        for ml in (False, True):
+            c.set_batch_multilevel(ml)
+            ref = None
+            for variant in range(eolc.BATCH_VARIANTS):
+                c.set_batch_variant(variant)
+                c.upload_state(x, v)
+                rc, st = c.batch_step(GRAV, H, tol=1e-9, maxit=20000, eager=True)
+                got = c.download_state()[1]
+                print(f"sides {sides} ml {ml} variant {variant}: iterations {[s.iters for s in st]}", flush=True)
+                assert rc == 0 and (ref is None or np.array_equal(got, ref))
+                ref = got
+            A, M = c.download_csr(eolc.MAT_MDK), c.download_csr(eolc.MAT_M)
+            rhs = M @ v + H * c.download_forces()
+            for b, i in enumerate(inst):
+                free = np.zeros(3 * off[-1], bool)
+                free[3 * off[b]:3 * off[b] + 3 * i.N] = True
+                free[(3 * (off[b] + np.asarray(i.fixed))[:, None] + np.arange(3)).reshape(-1)] = False
+                bred = rhs - A @ np.where(free, 0.0, ref)
+                assert np.linalg.norm((rhs - A @ ref)[free]) <= 1.001e-9 * np.linalg.norm(bred[free])
