@@ -458,7 +458,6 @@ hipError_t launch_update_x(eolc_ctx *c, double h);
 int pcg_grid(int N);
 int vec_wg(int N);          // workgroup size and workgroups of the PCG's vector kernels
 int vec_grid(int N);
-int pcg_grid_phys(int G);   // physical workgroups of the row kernels with a second logical one
 hipError_t pcg_setup(eolc_ctx *c, bool mixed, int precond_kind, bool ml_linear = true);
 hipError_t pcg_init(eolc_ctx *c, bool mixed);
 hipError_t pcg_chunk(eolc_ctx *c, bool mixed, int k0, int iters);
@@ -507,7 +506,17 @@ std::string ml_build(const Topology &t, std::vector<std::vector<int>> &agg_level
                      std::vector<int> &ptr1, std::vector<int> &agg1, std::vector<int> &cptr, std::vector<int> &par,
                      std::vector<unsigned char> &lam, MLLevels &lv);
 hipError_t ml_setup(eolc_ctx *c, bool linear = true);         // Galerkin diagonal blocks of every level
-hipError_t ml_apply(eolc_ctx *c, bool mixed, int parity, int check_done);   // z = D0 r + coarse, r.z partials
+// The vector update of iteration k that the restriction does first: p_new, q (of the
+// residual's type) and the solution, and the partials of p.q.
+struct MLUpdate {
+    int k, Ga;
+    const void *p, *q;
+    double *x;
+};
+// z = D0 r + coarse; r.z and r.r partials -> PB[parity].  u: with the iteration's vector
+// update, and no-op launches once the solve has stopped.
+hipError_t ml_apply(eolc_ctx *c, bool mixed, int parity, const MLUpdate *u);
+int ml_restrict_grid(const eolc_ctx *c);   // workgroups of the restriction: partials of r.r
 hipError_t ml_coarse64(eolc_ctx *c);                          // z64 = coarse corrections of r64 (no fine term)
 // velocity transfer after a remesh (k_transfer.hip); host arrays in and out
 hipError_t velocity_transfer(eolc_ctx *c, int n_old, const double *u_old, const double *v_old, int f_old,

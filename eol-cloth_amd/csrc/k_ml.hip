@@ -18,8 +18,8 @@
 // (`lam`, precomputed per SELL entry); k_ml_diagup adds children upwards.  Every
 // level's blocks are inverted in FP64.
 //
-// Per PCG iteration, after the vector update (ml_apply):
-//   k_ml_restrict : one wavefront per level-2 aggregate, vertices staged through LDS:
+// Per PCG iteration, after the product (ml_apply):
+//   k_ml_restrict : the vector update x += alpha p, r -= alpha q; one wavefront per level-2 aggregate, vertices staged through LDS:
 //                   R_1(a) = sum of r over a's members, R_2 = sum of the children's R_1,
 //                   and per level-1 aggregate a, C(a) = D_1^-1 R_1(a) + D_2^-1 R_2(parent)
 //   k_ml_coarse   : one workgroup (levels >= 3 only): R_l for l >= 3, then
@@ -41,6 +41,7 @@
 // from which the coarse kernel gets every level >= 3 by the exact change of
 // centroid and radius; the prolongation evaluates the level-3 field at each vertex.
 // The batched solve keeps the translations on every level.
+#include <algorithm>
 #include <type_traits>
 
 #include "eolc_internal.h"
@@ -326,14 +327,27 @@ __device__ __forceinline__ void wave_sync()
 }
 
 // Restriction of r to levels 1 and 2: one wavefront per level-2 aggregate.  Its
-// vertices are a contiguous range of hord; the lanes stage 64 of them at a time in
-// LDS (one vertex per lane), then each lane sums the members of one level-1 child
-// that fall in the chunk, in member order.  R_2 is the wavefront sum of the
-// children's R_1 (fixed shuffle tree).  With a single level, a wavefront takes 64
-// level-1 aggregates.
+// vertices are a contiguous range of hord; the lanes stage up to kStageRows of them in
+// LDS, four per lane with the loads of all four together, then each lane sums the
+// members of one level-1 child that fall in the stage, in member order.  R_2 is the
+// wavefront sum of the children's R_1 (fixed shuffle tree).  With a single level, a
+// wavefront takes 64 level-1 aggregates.
 // two wavefronts per workgroup: 13.9 us per restriction at 1024^2, against 14.8 (1),
 // 14.2 (4) and 14.4 (8) in the same kernel trace
 constexpr int kRestrictWG = 128;
+constexpr int kStageRows = 256;
+
+// The PCG's vector update x += alpha p, r -= alpha q, done by the restriction as it
+// reads r (UPD): the residual is written once and read once, and a launch is saved.
+// The members of an aggregate are a compact patch of the sheet, so their scattered
+// 12- and 24-byte pieces share most cache lines.
+template <class T> struct VecUpdate {
+    const T *p, *q;
+    double *x;
+    T *r;
+    T alphaT;
+    double alpha;
+};
 
 __device__ __forceinline__ void lift9(const double *__restrict__ q, double al, double bu, double bv, double *sm)
 {
@@ -358,18 +372,17 @@ __device__ __forceinline__ void lower9(const double *__restrict__ P, double al, 
 // or of the 64 level-1 aggregates from w * 64 (one level).  Writes R_1 of its
 // children, R_2(w) and C of its children; returns R_2(w) in every lane and, with
 // feat2 (the members' level-2 coordinate features in hord order), the first moments
-// sum phi_1 r and sum phi_2 r in lane 0.  Without the moments (LIN false) the
-// inverse blocks load before the member loop, hiding their latency; with them they
-// load after it, which keeps the loop's registers at six waves per SIMD.
-template <class T, bool LIN>
+// sum phi_1 r and sum phi_2 r in lane 0.  srr += r.r of the lane's members.
+template <class T, bool LIN, bool UPD>
 __device__ __forceinline__ void restrict_wave(const MLLevels &lv, int w, const int *__restrict__ hord,
                                               const int *__restrict__ ptr1, const int *__restrict__ cptr,
-                                              const int *__restrict__ kptr2, const T *__restrict__ r,
+                                              const int *__restrict__ kptr2, const VecUpdate<T> &up,
                                               double *__restrict__ R, const double *__restrict__ Dinv,
                                               double *__restrict__ C, const double *__restrict__ feat2,
                                               double *__restrict__ buf, double &s0, double &s1, double &s2,
-                                              double (&mom)[6], const SolverScalars *scal, int check_done)
+                                              double (&mom)[6], double &srr)
 {
+    constexpr int NC = kStageRows / 64;
     const int lane = threadIdx.x % 64;
     const bool two = lv.L >= 2;
     int a0, a1, ka = 0, kz = 0;
@@ -382,21 +395,6 @@ __device__ __forceinline__ void restrict_wave(const MLLevels &lv, int w, const i
         a0 = w * 64;
         a1 = min(a0 + 64, lv.n[1]);
     }
-    // the stop flag is read together with the ranges (one latency round; a stopped
-    // launch only reads these words)
-    if (check_done && scal->done) return;
-    // inverse blocks of the level-2 aggregate and of this lane's first child: they do
-    // not depend on r, so they load with the member indices
-    double dw[6] = {0, 0, 0, 0, 0, 0}, da[6] = {0, 0, 0, 0, 0, 0};
-    auto load_inv = [&]() {
-        const int64_t gw = lv.off[2] + w;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) dw[k] = Dinv[6 * gw + k];
-        if (a0 + lane < a1)
-#pragma unroll
-            for (int k = 0; k < 6; ++k) da[k] = Dinv[6 * (int64_t)(a0 + lane) + k];
-    };
-    if (two && !LIN) load_inv();
     s0 = s1 = s2 = 0.0;
     double f0 = 0.0, f1 = 0.0, f2 = 0.0;   // R_1 of this lane's first child
     double mu0 = 0.0, mu1 = 0.0, mu2 = 0.0, mv0 = 0.0, mv1 = 0.0, mv2 = 0.0;
@@ -408,29 +406,60 @@ __device__ __forceinline__ void restrict_wave(const MLLevels &lv, int w, const i
         const int m0 = mine ? ptr1[a] : 0, m1 = mine ? ptr1[a + 1] : 0;
         const int k1 = (two && g1 == a1) ? kz : ptr1[g1];
         double t0 = 0.0, t1 = 0.0, t2 = 0.0;
-        for (int kb = k0; kb < k1; kb += 64) {
-            const int k = kb + lane;
-            if (k < k1) {
-                double u = 0.0, v = 0.0;   // features first: they do not wait for hord
-                if (LIN) {
-                    u = feat2[2 * (int64_t)k];
-                    v = feat2[2 * (int64_t)k + 1];
-                }
-                const int i = hord[k];
-                // the compiler otherwise issues the feature load after the gather of r
-                // below, a third dependent memory round per 64 members
-                if (LIN) asm volatile("" ::: "memory");
-                const double q0 = (double)r[3 * i], q1 = (double)r[3 * i + 1], q2 = (double)r[3 * i + 2];
-                buf[3 * lane] = q0;
-                buf[3 * lane + 1] = q1;
-                buf[3 * lane + 2] = q2;
-                if (LIN) {
-                    mu0 = fma(u, q0, mu0); mu1 = fma(u, q1, mu1); mu2 = fma(u, q2, mu2);
-                    mv0 = fma(v, q0, mv0); mv1 = fma(v, q1, mv1); mv2 = fma(v, q2, mv2);
+        for (int kb = k0; kb < k1; kb += kStageRows) {
+            int i[NC];
+            double u[NC], v[NC];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const int k = kb + 64 * c + lane;
+                if (k < k1) {
+                    i[c] = hord[k];
+                    if (LIN) {
+                        u[c] = feat2[2 * (int64_t)k];
+                        v[c] = feat2[2 * (int64_t)k + 1];
+                    }
                 }
             }
+            // (the compiler otherwise issues the features' loads after the gathers below)
+            if (LIN) asm volatile("" ::: "memory");
+            T pv[NC][3], qv[NC][3], rv[NC][3];
+            double xv[NC][3];
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                if (kb + 64 * c + lane < k1)
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) {
+                        const int64_t j = 3 * (int64_t)i[c] + d;
+                        rv[c][d] = up.r[j];
+                        if (UPD) {
+                            qv[c][d] = up.q[j];
+                            pv[c][d] = up.p[j];
+                            xv[c][d] = up.x[j];
+                        }
+                    }
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                if (kb + 64 * c + lane < k1) {
+                    double q[3];
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) {
+                        if (UPD) {
+                            const int64_t j = 3 * (int64_t)i[c] + d;
+                            rv[c][d] = fma(-up.alphaT, qv[c][d], rv[c][d]);
+                            up.r[j] = rv[c][d];
+                            up.x[j] = fma(up.alpha, (double)pv[c][d], xv[c][d]);
+                        }
+                        q[d] = (double)rv[c][d];
+                        srr += q[d] * q[d];
+                        buf[3 * (64 * c + lane) + d] = q[d];
+                    }
+                    if (LIN) {
+                        mu0 = fma(u[c], q[0], mu0); mu1 = fma(u[c], q[1], mu1); mu2 = fma(u[c], q[2], mu2);
+                        mv0 = fma(v[c], q[0], mv0); mv1 = fma(v[c], q[1], mv1); mv2 = fma(v[c], q[2], mv2);
+                    }
+                }
             wave_sync();
-            const int e0 = max(m0, kb), e1 = min(m1, kb + 64);
+            const int e0 = max(m0, kb), e1 = min(m1, kb + kStageRows);
             for (int m = e0; m < e1; ++m) {
                 t0 += buf[3 * (m - kb)];
                 t1 += buf[3 * (m - kb) + 1];
@@ -446,7 +475,16 @@ __device__ __forceinline__ void restrict_wave(const MLLevels &lv, int w, const i
         k0 = k1;   // the next group starts where this one ends
     }
     if (!two) return;
-    if (LIN) load_inv();
+    // inverse blocks of the level-2 aggregate and of this lane's first child
+    double dw[6], da[6] = {0, 0, 0, 0, 0, 0};
+    {
+        const int64_t gw = lv.off[2] + w;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) dw[k] = Dinv[6 * gw + k];
+        if (a0 + lane < a1)
+#pragma unroll
+            for (int k = 0; k < 6; ++k) da[k] = Dinv[6 * (int64_t)(a0 + lane) + k];
+    }
     // wave_sum leaves the total in lane 0; every lane needs it below
     s0 = __shfl(wave_sum(s0), 0, 64);
     s1 = __shfl(wave_sum(s1), 0, 64);
@@ -478,21 +516,64 @@ __device__ __forceinline__ void restrict_wave(const MLLevels &lv, int w, const i
     }
 }
 
-// Translations only: one wavefront per level-2 aggregate (or per 64 level-1 ones).
-template <class T>
-__global__ void __launch_bounds__(kRestrictWG) k_ml_restrict(MLLevels lv, const int *__restrict__ hord,
-                                                             const int *__restrict__ ptr1, const int *__restrict__ cptr,
-                                                             const int *__restrict__ kptr2,
-                                                             const T *__restrict__ r, double *__restrict__ R,
-                                                             const double *__restrict__ Dinv, double *__restrict__ C,
-                                                             const SolverScalars *scal, int check_done)
+// What the two restriction kernels share.  In an iteration (UPD) alpha = r.z / p.q from
+// the partials of the product (Ga) and of the prolongation (Gz), and the stop on
+// p.q <= 0.  Every workgroup leaves its r.r in PB[parity].
+struct RestrictArgs {
+    MLLevels lv;
+    const int *hord, *ptr1, *cptr, *kptr2;
+    double *R, *C;
+    const double *Dinv, *feat2, *geo;
+    double *R9p;
+    SolverScalars *scal;
+    double *partials;
+    int k, Ga, Gz;        // iteration and partial counts (UPD)
+    int parity;
+};
+
+// alpha of the iteration; false: the solve stops here (the flag is set by workgroup 0).
+template <class T, int W>
+__device__ __forceinline__ bool restrict_alpha(const RestrictArgs &g, VecUpdate<T> &up, double *lds)
 {
-    __shared__ double stage[kRestrictWG / 64][3 * 64];
-    const int w = (blockIdx.x * blockDim.x + threadIdx.x) / 64;   // uniform in the wavefront
-    if (lv.L >= 2 ? w >= lv.n[2] : w * 64 >= lv.n[1]) return;
-    double s0, s1, s2, mom[6];
-    restrict_wave<T, false>(lv, w, hord, ptr1, cptr, kptr2, r, R, Dinv, C, nullptr, stage[threadIdx.x / 64], s0, s1, s2,
-                     mom, scal, check_done);
+    double v[2];
+    reduce_partials<2, W>({PA(g.partials), PB(g.partials, g.k & 1)}, {g.Ga, g.Gz}, v, lds);
+    const double pq = v[0], rz = v[1];
+    SolverScalars *scal = g.scal;
+    if (!(pq > 0.0)) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            scal->done = 1;
+            scal->reason = isfinite(pq) ? 2 : 4;
+            scal->pq = pq;
+        }
+        return false;
+    }
+    up.alpha = rz / pq;
+    up.alphaT = (T)up.alpha;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        scal->iters = g.k + 1;
+        scal->pq = pq;
+        scal->alpha = up.alpha;
+    }
+    return true;
+}
+
+// Translations only: one wavefront per level-2 aggregate (or per 64 level-1 ones), on at
+// most kRestrictGrid workgroups (every workgroup of the next product sums their r.r).
+constexpr int kRestrictGrid = 4096;
+template <class T, bool UPD>
+__global__ void __launch_bounds__(kRestrictWG) k_ml_restrict(RestrictArgs g, VecUpdate<T> up)
+{
+    constexpr int NW = kRestrictWG / 64;
+    __shared__ double stage[NW][3 * kStageRows];
+    __shared__ double lds[2 * NW + 2];
+    if (UPD && g.scal->done) return;
+    if (UPD && !restrict_alpha<T, kRestrictWG>(g, up, lds)) return;
+    double s0, s1, s2, mom[6], srr[1] = {0.0};
+    const int waves = g.lv.L >= 2 ? g.lv.n[2] : (g.lv.n[1] + 63) / 64;
+    for (int w = logical_wg() * NW + (int)threadIdx.x / 64; w < waves; w += gridDim.x * NW)   // uniform
+        restrict_wave<T, false, UPD>(g.lv, w, g.hord, g.ptr1, g.cptr, g.kptr2, up, g.R, g.Dinv, g.C, nullptr,
+                                     stage[threadIdx.x / 64], s0, s1, s2, mom, srr[0]);
+    write_partials<1, kRestrictWG>(srr, PB(g.partials, g.parity) + eolc::kMaxPartials, lds);
 }
 
 // Linear coarse fields: kRestrict3Parts workgroups per level-3 aggregate U, whose
@@ -501,44 +582,46 @@ __global__ void __launch_bounds__(kRestrictWG) k_ml_restrict(MLLevels lv, const 
 // first moments are re-expressed on U's basis, (R_2, alpha M_1 + beta_u R_2, alpha
 // M_2 + beta_v R_2) with alpha = s_w / s_U and beta = (c_w - c_U) / s_U, summed per
 // wavefront in child order and over the workgroup's wavefronts in order: one partial
-// R9 per workgroup, which the coarse kernel adds in order.  At 1024^2 the kernel takes
-// 26 us against 14 us for the translations' restriction.  It ran at 31 us with the
-// inverse blocks loaded before the member loop (101 VGPRs, four waves per SIMD) and
-// at 28 us with the feature load issued after the gather of r; 512-thread workgroups
-// (32 wavefronts per level-3 aggregate) took 36 us, and loading the next 64 members'
-// indices and features during the gather gained nothing.
+// R9 per workgroup, which the coarse kernel adds in order.  With the vector update, FP32
+// (us; the update and the restriction apart before): 131 x 97 quads 9.0 (4.4 + 8.3),
+// 512^2 19.3 (9.3 + 16.5), 1024^2 48.4 (22.3 + 25.9), a launch less each.  There it is
+// bound by the scattered pieces (122 MB in all, less than half of the card's rate): 54 us
+// without the workgroups in XCD order, the same with 64 to 256 members staged at once,
+// which is worth 1 us at 131 x 97 and 5 in the translations' kernel on a renumbered mesh.
 constexpr int kRestrict3WG = 256;
 using eolc::kRestrict3Parts;
-template <class T>
-__global__ void __launch_bounds__(kRestrict3WG) k_ml_restrict3(MLLevels lv, const int *__restrict__ hord,
-                                                               const int *__restrict__ ptr1,
-                                                               const int *__restrict__ cptr,
-                                                               const int *__restrict__ kptr2, const T *__restrict__ r,
-                                                               double *__restrict__ R, const double *__restrict__ Dinv,
-                                                               double *__restrict__ C,
-                                                               const double *__restrict__ feat2,
-                                                               const double *__restrict__ geo, double *__restrict__ R9p,
-                                                               const SolverScalars *scal, int check_done)
+template <class T, bool UPD>
+__global__ void __launch_bounds__(kRestrict3WG) k_ml_restrict3(RestrictArgs g, VecUpdate<T> up)
 {
     constexpr int NW = kRestrict3WG / 64;
-    __shared__ double stage[NW][3 * 64];
+    __shared__ double stage[NW][3 * kStageRows];
     __shared__ double red[NW][9];
-    const int U = blockIdx.x / kRestrict3Parts, part = blockIdx.x % kRestrict3Parts;
+    __shared__ double lds[2 * NW + 2];
+    const MLLevels &lv = g.lv;
+    // consecutive aggregates on one XCD: neighbouring patches share cache lines of the
+    // vectors (the grid is padded to a multiple of 8; a workgroup without one only
+    // leaves its empty r.r)
+    const int lw = logical_wg();
+    const int U = min(lw / kRestrict3Parts, lv.n[3] - 1), part = lw % kRestrict3Parts;
+    const bool own = lw < lv.n[3] * kRestrict3Parts;
     const int lane = threadIdx.x % 64, wid = threadIdx.x / 64;
-    const int c0 = cptr[lv.coff[3] + U], c1 = cptr[lv.coff[3] + U + 1];
+    const int c0 = g.cptr[lv.coff[3] + U], c1 = own ? g.cptr[lv.coff[3] + U + 1] : 0;
     const int64_t gU = lv.off[3] + U;
-    const double cu = geo[4 * gU], cv = geo[4 * gU + 1], is = geo[4 * gU + 3];
-    if (check_done && scal->done) return;
+    const double cu = g.geo[4 * gU], cv = g.geo[4 * gU + 1], is = g.geo[4 * gU + 3];
+    if (UPD && g.scal->done) return;
+    if (UPD && !restrict_alpha<T, kRestrict3WG>(g, up, lds)) return;
     // lane 0 keeps the wavefront's running sum in LDS
     if (lane == 0)
 #pragma unroll
         for (int q = 0; q < 9; ++q) red[wid][q] = 0.0;
+    double srr[1] = {0.0};
     for (int w = c0 + part * NW + wid; w < c1; w += NW * kRestrict3Parts) {
         double s0, s1, s2, mom[6];
-        restrict_wave<T, true>(lv, w, hord, ptr1, cptr, kptr2, r, R, Dinv, C, feat2, stage[wid], s0, s1, s2, mom, scal, 0);
+        restrict_wave<T, true, UPD>(lv, w, g.hord, g.ptr1, g.cptr, g.kptr2, up, g.R, g.Dinv, g.C, g.feat2, stage[wid],
+                                    s0, s1, s2, mom, srr[0]);
         if (lane == 0) {
             const int64_t gw = lv.off[2] + w;
-            const double al = geo[4 * gw + 2] * is, bu = (geo[4 * gw] - cu) * is, bv = (geo[4 * gw + 1] - cv) * is;
+            const double al = g.geo[4 * gw + 2] * is, bu = (g.geo[4 * gw] - cu) * is, bv = (g.geo[4 * gw + 1] - cv) * is;
             double t[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
             const double q[9] = {s0, s1, s2, mom[0], mom[1], mom[2], mom[3], mom[4], mom[5]};
             lift9(q, al, bu, bv, t);
@@ -547,12 +630,13 @@ __global__ void __launch_bounds__(kRestrict3WG) k_ml_restrict3(MLLevels lv, cons
         }
     }
     __syncthreads();
-    if (threadIdx.x < 9) {
+    if (own && threadIdx.x < 9) {
         double v = 0.0;
 #pragma unroll
         for (int k = 0; k < NW; ++k) v += red[k][threadIdx.x];
-        R9p[9 * (int64_t)blockIdx.x + threadIdx.x] = v;
+        g.R9p[9 * (int64_t)lw + threadIdx.x] = v;
     }
+    write_partials<1, kRestrict3WG>(srr, PB(g.partials, g.parity) + eolc::kMaxPartials, lds, lw);
 }
 
 // Levels >= 3 in one workgroup: R_l from the children (l = 3..L), then from the top
@@ -917,37 +1001,40 @@ hipError_t ml_setup(eolc_ctx *c, bool linear)
     return hipGetLastError();
 }
 
-// The restriction, the coarse levels and the prolongation's coarse term, with the
-// linear fields when the last ml_setup formed them.
-static void ml_coarse_chain(eolc_ctx *c, bool mixed, int check_done)
+static bool ml_linear_on(const eolc_ctx *c) { return c->ml.lin_on && c->ml.lv.L >= kMLLinFrom; }
+
+int ml_restrict_grid(const eolc_ctx *c)
+{
+    const MLLevels &lv = c->ml.lv;
+    if (ml_linear_on(c)) return (lv.n[3] * kRestrict3Parts + 7) & ~7;   // (a multiple of 8, as logical_wg needs)
+    const int waves = lv.L >= 2 ? lv.n[2] : (lv.n[1] + 63) / 64;
+    return std::min((blocks_for((int64_t)64 * waves, kRestrictWG) + 7) & ~7, kRestrictGrid);
+}
+
+// The restriction (with the vector update when there is one) and the coarse levels, with
+// the linear fields when the last ml_setup formed them.
+template <class T>
+static void ml_coarse_chain(eolc_ctx *c, T *r, int parity, const MLUpdate *u)
 {
     const MLState &m = c->ml;
     const MLLevels &lv = m.lv;
-    const bool lin = m.lin_on && lv.L >= kMLLinFrom;
-    if (lin) {
-        if (mixed)
-            hipLaunchKernelGGL(k_ml_restrict3<float>, dim3(lv.n[3] * kRestrict3Parts), dim3(kRestrict3WG), 0,
-                               c->stream, lv, m.hord, m.ptr1, m.cptr, m.kptr2, c->r32, m.R, m.Dinv, m.C, m.feat2,
-                               m.geo, m.R9p, c->scal, check_done);
-        else
-            hipLaunchKernelGGL(k_ml_restrict3<double>, dim3(lv.n[3] * kRestrict3Parts), dim3(kRestrict3WG), 0,
-                               c->stream, lv, m.hord, m.ptr1, m.cptr, m.kptr2, c->r64, m.R, m.Dinv, m.C, m.feat2,
-                               m.geo, m.R9p, c->scal, check_done);
+    RestrictArgs g{lv,    m.hord, m.ptr1, m.cptr, m.kptr2, m.R, m.C,     m.Dinv, m.feat2,
+                   m.geo, m.R9p,  c->scal, c->partials, u ? u->k : 0, u ? u->Ga : 0, vec_grid(c->topo.N), parity};
+    VecUpdate<T> up{u ? static_cast<const T *>(u->p) : nullptr, u ? static_cast<const T *>(u->q) : nullptr,
+                    u ? u->x : nullptr, r, (T)0, 0.0};
+    const dim3 grid(ml_restrict_grid(c));
+    if (ml_linear_on(c)) {
+        if (u) hipLaunchKernelGGL((k_ml_restrict3<T, true>), grid, dim3(kRestrict3WG), 0, c->stream, g, up);
+        else hipLaunchKernelGGL((k_ml_restrict3<T, false>), grid, dim3(kRestrict3WG), 0, c->stream, g, up);
         hipLaunchKernelGGL(k_ml_coarse9, dim3(1), dim3(kCoarse9WG), 0, c->stream, lv, m.cptr, m.par, m.geo, m.D9,
-                           m.R9p, m.C9, c->scal, check_done);
+                           m.R9p, m.C9, c->scal, u != nullptr);
         return;
     }
-    const int waves = lv.L >= 2 ? lv.n[2] : (lv.n[1] + 63) / 64;
-    const int rblocks = blocks_for((int64_t)64 * waves, kRestrictWG);
-    if (mixed)
-        hipLaunchKernelGGL(k_ml_restrict<float>, dim3(rblocks), dim3(kRestrictWG), 0, c->stream, lv, m.hord, m.ptr1,
-                           m.cptr, m.kptr2, c->r32, m.R, m.Dinv, m.C, c->scal, check_done);
-    else
-        hipLaunchKernelGGL(k_ml_restrict<double>, dim3(rblocks), dim3(kRestrictWG), 0, c->stream, lv, m.hord, m.ptr1,
-                           m.cptr, m.kptr2, c->r64, m.R, m.Dinv, m.C, c->scal, check_done);
+    if (u) hipLaunchKernelGGL((k_ml_restrict<T, true>), grid, dim3(kRestrictWG), 0, c->stream, g, up);
+    else hipLaunchKernelGGL((k_ml_restrict<T, false>), grid, dim3(kRestrictWG), 0, c->stream, g, up);
     if (lv.L >= 3)
         hipLaunchKernelGGL(k_ml_coarse, dim3(1), dim3(kCoarseWG), 0, c->stream, lv, m.cptr, m.par, m.Dinv, m.R, m.C,
-                           c->scal, check_done);
+                           c->scal, u != nullptr);
 }
 
 // The prolongation on the vector kernels' grid (vec_wg, vec_grid).
@@ -957,7 +1044,7 @@ static void launch_prolong(eolc_ctx *c, int parity, const T *D, const T *r, T *z
     const MLState &m = c->ml;
     const MLLevels &lv = m.lv;
     const int N = c->topo.N;
-    const double *c9 = (m.lin_on && lv.L >= kMLLinFrom) ? m.C9 : nullptr;
+    const double *c9 = ml_linear_on(c) ? m.C9 : nullptr;
     auto go = [&](auto w) {
         constexpr int W = decltype(w)::value;
         hipLaunchKernelGGL((k_ml_prolong<T, FINE, W>), dim3(vec_grid(N)), dim3(W), 0, c->stream, parity, N, lv, m.agg1,
@@ -967,11 +1054,15 @@ static void launch_prolong(eolc_ctx *c, int parity, const T *D, const T *r, T *z
     else go(std::integral_constant<int, WG>());
 }
 
-hipError_t ml_apply(eolc_ctx *c, bool mixed, int parity, int check_done)
+hipError_t ml_apply(eolc_ctx *c, bool mixed, int parity, const MLUpdate *u)
 {
-    ml_coarse_chain(c, mixed, check_done);
-    if (mixed) launch_prolong<float, true>(c, parity, c->D32, c->r32, c->z32, check_done);
-    else launch_prolong<double, true>(c, parity, c->D64, c->r64, c->z64, check_done);
+    if (mixed) {
+        ml_coarse_chain<float>(c, c->r32, parity, u);
+        launch_prolong<float, true>(c, parity, c->D32, c->r32, c->z32, u != nullptr);
+    } else {
+        ml_coarse_chain<double>(c, c->r64, parity, u);
+        launch_prolong<double, true>(c, parity, c->D64, c->r64, c->z64, u != nullptr);
+    }
     return hipGetLastError();
 }
 
@@ -979,7 +1070,7 @@ hipError_t ml_apply(eolc_ctx *c, bool mixed, int parity, int check_done)
 hipError_t ml_coarse64(eolc_ctx *c)
 {
     if (c->ml.lv.L <= 0) return hipMemsetAsync(c->z64, 0, sizeof(double) * 3 * (size_t)c->topo.N, c->stream);
-    ml_coarse_chain(c, false, 0);
+    ml_coarse_chain<double>(c, c->r64, 0, nullptr);
     launch_prolong<double, false>(c, 0, c->D64, c->r64, c->z64, 0);
     return hipGetLastError();
 }

@@ -10,8 +10,8 @@
 //                     q = A p_new; partial p_new.q -> PA.
 //   k_pcg_update<k> : pq <- sum of PA; alpha = rz_k / pq; x += alpha p_new,
 //                     r -= alpha q, z = D^-1 r; partials r.z, r.r -> PB[(k+1)&1].
-// With the multilevel preconditioner the update forms x, r and r.r only, and the
-// restriction, coarse-level and prolongation kernels of k_ml.hip form z and r.z.
+// With the multilevel preconditioner the restriction kernel of k_ml.hip does the update
+// (x, r and r.r), and the coarse-level and prolongation kernels form z and r.z.
 // There is no grid-wide fence inside a kernel: every workgroup re-reduces the
 // previous kernel's per-workgroup partials itself, in one fixed order, so all
 // workgroups reach bitwise-identical scalars and identical stop decisions.  The
@@ -42,6 +42,16 @@ using eolc::SolverScalars;
 #pragma clang fp contract(off)
 
 namespace {
+
+// ---------------------------------------------------------------------------
+// r.z and r.r of iterate k and r.z of the one before (meaningless, and not used, in an
+// iteration that starts with beta = 0).
+template <int W>
+__device__ __forceinline__ void reduce_rz(double *partials, int k, int Gz, int Gr, double (&sums)[3], double *lds)
+{
+    const double *b = PB(partials, k & 1);
+    reduce_partials<3, W>({b, b + eolc::kMaxPartials, PB(partials, (k + 1) & 1)}, {Gz, Gr, Gz}, sums, lds);
+}
 
 // ---------------------------------------------------------------------------
 // DIFF = false (FP64 path): q = A p with the assembled blocks of MDK.
@@ -158,7 +168,7 @@ k_pcg_spmv(int k, int N, int nslices, const int *__restrict__ slice_off, const i
            const int *__restrict__ slen, const int *__restrict__ scol, const T *__restrict__ A,
            const T *__restrict__ Mm, int64_t nbs, const unsigned char *__restrict__ fixmask, const T *__restrict__ z,
            const T *__restrict__ pold, T *__restrict__ pnew, T *__restrict__ q, SolverScalars *scal, double *partials,
-           SymLayout sym, const int *__restrict__ wwin, int Gb)
+           SymLayout sym, const int *__restrict__ wwin, int Gz, int Gr)
 {
     static_assert(U == 1 || U == 2, "entries per trip");
     static_assert(!(STG && U == 2), "the staged variants take one entry per trip");
@@ -200,12 +210,10 @@ k_pcg_spmv(int k, int N, int nslices, const int *__restrict__ slice_off, const i
             sz[t] = f < nf ? zw[f] : (T)0;
         }
     }
-    double cur[2];
     const bool restart_beta0 = (k == scal->first_iter);
-    double prev[1] = {1.0};
-    if (restart_beta0) reduce_partials<2>(PB(partials, k & 1), cur, lds, Gb);
-    else reduce_partials2<2, 1>(PB(partials, k & 1), PB(partials, (k + 1) & 1), cur, prev, lds, Gb, Gb);
-    const double rzk = cur[0], rrk = cur[1];
+    double sums[3];   // r.z and r.r of this iterate, r.z of the one before
+    reduce_rz<WG>(partials, k, Gz, Gr, sums, lds);
+    const double rzk = sums[0], rrk = sums[1];
     const double thr = fmax(scal->tol2 * scal->bnorm2, scal->delta2 * scal->rmax2);
     if (!isfinite(rrk) || !isfinite(rzk) || rrk <= thr) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -216,7 +224,7 @@ k_pcg_spmv(int k, int N, int nslices, const int *__restrict__ slice_off, const i
         }
         return;
     }
-    const double beta = restart_beta0 ? 0.0 : rzk / prev[0];
+    const double beta = restart_beta0 ? 0.0 : rzk / sums[2];
     const T betaT = (T)beta;   // p_new = z + beta p is formed in T, identically everywhere
     if constexpr (STG) {
 #pragma unroll
@@ -453,7 +461,7 @@ template <class T, class TR, bool NT, int W, int PD>
 __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(W, W)))
 k_pcg_spmv_patch(int k, PatchLayout pl, const T *__restrict__ Mm, const unsigned char *__restrict__ fixmask,
                  const T *__restrict__ z, const T *__restrict__ pold, T *__restrict__ pnew, T *__restrict__ q,
-                 SolverScalars *scal, double *partials, int Gb)
+                 SolverScalars *scal, double *partials, int Gz, int Gr)
 {
     using R = SymRec<TR>;
     typedef typename R::v2 v2;
@@ -501,12 +509,10 @@ k_pcg_spmv_patch(int k, PatchLayout pl, const T *__restrict__ Mm, const unsigned
             sz[t] = z[3 * v + c];
         }
     }
-    double cur[2];
     const bool restart_beta0 = (k == scal->first_iter);
-    double prev[1] = {1.0};
-    if (restart_beta0) reduce_partials<2>(PB(partials, k & 1), cur, lds, Gb);
-    else reduce_partials2<2, 1>(PB(partials, k & 1), PB(partials, (k + 1) & 1), cur, prev, lds, Gb, Gb);
-    const double rzk = cur[0], rrk = cur[1];
+    double sums[3];   // r.z and r.r of this iterate, r.z of the one before
+    reduce_rz<WG>(partials, k, Gz, Gr, sums, lds);
+    const double rzk = sums[0], rrk = sums[1];
     const double thr = fmax(scal->tol2 * scal->bnorm2, scal->delta2 * scal->rmax2);
     if (!isfinite(rrk) || !isfinite(rzk) || rrk <= thr) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -517,7 +523,7 @@ k_pcg_spmv_patch(int k, PatchLayout pl, const T *__restrict__ Mm, const unsigned
         }
         return;
     }
-    const double beta = restart_beta0 ? 0.0 : rzk / prev[0];
+    const double beta = restart_beta0 ? 0.0 : rzk / sums[2];
     const T betaT = (T)beta;   // p_new = z + beta p is formed in T, identically everywhere
 #pragma unroll
     for (int t = 0; t < kPer; ++t) {
@@ -720,7 +726,7 @@ k_pcg_spmv_split(int k, int N, int nslices, const int *__restrict__ slice_off, c
                  const int *__restrict__ slen, const int *__restrict__ scol, const T *__restrict__ A,
                  const T *__restrict__ Mm, int64_t nbs, const unsigned char *__restrict__ fixmask,
                  const T *__restrict__ z, const T *__restrict__ pold, T *__restrict__ pnew, T *__restrict__ q,
-                 SolverScalars *scal, double *partials, int Gb)
+                 SolverScalars *scal, double *partials, int Gz, int Gr)
 {
     constexpr int W = kSplitWG;
     __shared__ double lds[3 * (W / 64) + 3];
@@ -752,12 +758,10 @@ k_pcg_spmv_split(int k, int N, int nslices, const int *__restrict__ slice_off, c
         fm = fixmask[row];
     }
     e.values(A + base, nbs, w, z, pold);
-    double cur[2];
     const bool restart_beta0 = (k == scal->first_iter);
-    double prev[1] = {1.0};
-    if (restart_beta0) reduce_partials<2, W>(PB(partials, k & 1), cur, lds, Gb);
-    else reduce_partials2<2, 1, W>(PB(partials, k & 1), PB(partials, (k + 1) & 1), cur, prev, lds, Gb, Gb);
-    const double rzk = cur[0], rrk = cur[1];
+    double sums[3];   // r.z and r.r of this iterate, r.z of the one before
+    reduce_rz<W>(partials, k, Gz, Gr, sums, lds);
+    const double rzk = sums[0], rrk = sums[1];
     const double thr = fmax(scal->tol2 * scal->bnorm2, scal->delta2 * scal->rmax2);
     if (!isfinite(rrk) || !isfinite(rzk) || rrk <= thr) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -768,7 +772,7 @@ k_pcg_spmv_split(int k, int N, int nslices, const int *__restrict__ slice_off, c
         }
         return;
     }
-    const double beta = restart_beta0 ? 0.0 : rzk / prev[0];
+    const double beta = restart_beta0 ? 0.0 : rzk / sums[2];
     const T betaT = (T)beta;
     T ui[3];
 #pragma unroll
@@ -843,88 +847,6 @@ k_resid64_split(int N, int nslices, const int *__restrict__ slice_off, const int
 }
 
 // ---------------------------------------------------------------------------
-// The multilevel modes' update (x += alpha p, r -= alpha q, r.r) touches no 3x3
-// block, so it runs over the flat DOF arrays: workgroup lw owns DOFs
-// [lw c, lw c + c) with c = ceil(3N / G) rounded up to 4, and every thread handles 4
-// consecutive DOFs per trip with 16-byte loads (FP32) or two 16-byte loads (FP64).
-// The same arithmetic per DOF as k_pcg_update; r.r is summed per DOF range.
-template <class T, class TX, int W>
-__global__ void __launch_bounds__(W) __attribute__((amdgpu_waves_per_eu(8, 8)))
-k_pcg_update_flat(int k, int G, int Ga, int n3, const T *__restrict__ pnew, const T *__restrict__ q, TX *__restrict__ x,
-                  T *__restrict__ r, SolverScalars *scal, double *partials)
-{
-    __shared__ double lds[2 * (W / 64) + 2];
-    typedef T v4 __attribute__((ext_vector_type(4)));
-    typedef TX x4 __attribute__((ext_vector_type(4)));
-    if (scal->done) return;
-    const int chunk = (((n3 + G - 1) / G) + 3) & ~3;
-    const int lw0 = logical_wg(), lwx = extra_logical_wg(G);
-    // mixed precision: the first trip's FP64 accumulator (half the bytes read) loads
-    // before the partial sums are re-reduced (it does not depend on alpha), so the two
-    // latencies overlap.  The other vectors too, or the FP64 mode's, would spill at
-    // eight waves per SIMD.
-    constexpr bool PRE = sizeof(T) == 4;
-    const int b0 = min(lw0 * chunk, n3), e0 = min(b0 + chunk, n3), i0 = b0 + 4 * (int)threadIdx.x;
-    x4 xv0 = {};
-    if (PRE && i0 + 3 < e0) xv0 = *reinterpret_cast<const x4 *>(x + i0);
-    double pq[1], rz[1];
-    reduce_partials2<1, 1, W>(PA(partials), PB(partials, k & 1), pq, rz, lds, Ga, G);
-    if (!(pq[0] > 0.0)) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            scal->done = 1;
-            scal->reason = isfinite(pq[0]) ? 2 : 4;
-            scal->pq = pq[0];
-        }
-        return;
-    }
-    const double alpha = rz[0] / pq[0];
-    const T alphaT = (T)alpha;
-    // the G logical ranges may run on fewer workgroups: the first ones then take a
-    // second range
-#pragma unroll 1
-    for (int pass = 0; pass < 2; ++pass) {
-        const int lw = pass == 0 ? lw0 : lwx;
-        if (lw < 0) break;   // uniform in the workgroup
-        const int b = min(lw * chunk, n3), e = min(b + chunk, n3);
-        double srr = 0.0;
-        for (int i = b + 4 * (int)threadIdx.x; i < e; i += 4 * W) {
-            if (i + 3 < e) {
-                // i is a multiple of 4: aligned 4-element vector loads and stores
-                const v4 pv = *reinterpret_cast<const v4 *>(pnew + i), qv = *reinterpret_cast<const v4 *>(q + i);
-                const v4 rv = *reinterpret_cast<const v4 *>(r + i);
-                const x4 xv = (PRE && pass == 0 && i == i0) ? xv0 : *reinterpret_cast<const x4 *>(x + i);
-                x4 xo;
-                v4 ro;
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    if constexpr (std::is_same<TX, T>::value) xo[u] = fma(alphaT, pv[u], xv[u]);
-                    else xo[u] = fma((TX)alpha, (TX)pv[u], xv[u]);
-                    ro[u] = fma(-alphaT, qv[u], rv[u]);
-                    srr += (double)ro[u] * (double)ro[u];
-                }
-                *reinterpret_cast<x4 *>(x + i) = xo;
-                *reinterpret_cast<v4 *>(r + i) = ro;
-            } else {
-                for (int u = i; u < e; ++u) {
-                    if constexpr (std::is_same<TX, T>::value) x[u] = fma(alphaT, pnew[u], x[u]);
-                    else x[u] = fma((TX)alpha, (TX)pnew[u], x[u]);
-                    const T rn = fma(-alphaT, q[u], r[u]);
-                    r[u] = rn;
-                    srr += (double)rn * (double)rn;
-                }
-            }
-        }
-        double v[1] = {srr};
-        write_partials<1, W>(v, PB(partials, (k + 1) & 1) + eolc::kMaxPartials, lds, lw);
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        scal->iters = k + 1;
-        scal->pq = pq[0];
-        scal->alpha = alpha;
-    }
-}
-
-// ---------------------------------------------------------------------------
 // TX is the solution accumulator (FP64 in both modes).
 template <class T, class TX, int W>
 __global__ void __launch_bounds__(W) __attribute__((amdgpu_waves_per_eu(8, 8)))
@@ -946,17 +868,19 @@ k_pcg_update(int k, int Ga, int N, const T *__restrict__ D, const T *__restrict_
             pv[c] = pnew[3 * i0 + c]; qv[c] = q[3 * i0 + c]; rv[c] = r[3 * i0 + c]; xv[c] = x[3 * i0 + c];
         }
     }
-    double pq[1], rz[1];
-    reduce_partials2<1, 1, W>(PA(partials), PB(partials, k & 1), pq, rz, lds, Ga, gridDim.x);
-    if (!(pq[0] > 0.0)) {
+    double sums[2];
+    const int Gv = gridDim.x;
+    reduce_partials<2, W>({PA(partials), PB(partials, k & 1)}, {Ga, Gv}, sums, lds);
+    const double pq = sums[0], rz = sums[1];
+    if (!(pq > 0.0)) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             scal->done = 1;
-            scal->reason = isfinite(pq[0]) ? 2 : 4;
-            scal->pq = pq[0];
+            scal->reason = isfinite(pq) ? 2 : 4;
+            scal->pq = pq;
         }
         return;
     }
-    const double alpha = rz[0] / pq[0];
+    const double alpha = rz / pq;
     const T alphaT = (T)alpha;
     double srz = 0.0, srr = 0.0;
     for (int i = i0; i < re; i += W) {
@@ -988,7 +912,7 @@ k_pcg_update(int k, int Ga, int N, const T *__restrict__ D, const T *__restrict_
     write_partials<2, W>(v, PB(partials, (k + 1) & 1), lds);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         scal->iters = k + 1;
-        scal->pq = pq[0];
+        scal->pq = pq;
         scal->alpha = alpha;
     }
 }
@@ -1045,8 +969,8 @@ __global__ void __launch_bounds__(WG) k_reduce_to(int G, const double *__restric
     if (threadIdx.x == 0) *dst = s[0];
 }
 
-// z = D r (r converted from FP64 to T), partials r.z, r.r -> PB[parity].  ML: r and
-// r.r only; the multilevel kernels form z and r.z.
+// z = D r (r converted from FP64 to T), partials r.z, r.r -> PB[parity].  ML: r only; the
+// multilevel kernels form the rest.
 template <class T, bool ML, int W>
 __global__ void __launch_bounds__(W)
 k_precond_init(int parity, int N, const T *__restrict__ D, const double *r64, T *r, T *__restrict__ z,
@@ -1071,10 +995,7 @@ k_precond_init(int parity, int N, const T *__restrict__ D, const double *r64, T 
         }
         rr += (s0 * s0 + s1 * s1) + s2 * s2;
     }
-    if constexpr (ML) {
-        double v[1] = {rr};
-        write_partials<1, W>(v, PB(partials, parity) + eolc::kMaxPartials, lds);
-    } else {
+    if constexpr (!ML) {
         double v[2] = {rz, rr};
         write_partials<2, W>(v, PB(partials, parity), lds);
     }
@@ -1303,24 +1224,27 @@ constexpr int lay_bit(int lay)
     case id:                                           \
         return LAY == 4 ? eolc::kLaySym64 : LAY == 5 ? eolc::kLayPatch64 : 0;
 
+// partials of r.r: the restriction's with the multilevel levels, else the update's
+inline int rr_partials(const eolc_ctx *c) { return c->ml_on ? eolc::ml_restrict_grid(c) : eolc::vec_grid(c->topo.N); }
+
 template <class T, int U, bool PF, bool NT, int W, int LAY, bool STG>
 void launch_spmv_one(eolc_ctx *c, int k, int G, const T *A, const T *Mm, const T *z, const T *pold, T *pnew, T *q)
 {
     const eolc::Topology &t = c->topo;
     constexpr bool diff = std::is_same<T, float>::value;
-    const int Gb = eolc::vec_grid(t.N);
+    const int Gz = eolc::vec_grid(t.N), Gr = rr_partials(c);
     if constexpr (LAY == 5) {
         using TR = T;
         const PatchLayout pl{c->pt_row, c->pt_cnt, c->pt_roff, c->pt_soff, c->pt_loff, c->pt_woff, c->pt_win,
                              c->pt_lo,  c->P32,    c->P64,     t.pt_slots, c->smask,   c->sellbase, c->scol,
                              c->A64s};
         hipLaunchKernelGGL((k_pcg_spmv_patch<T, TR, NT, W, U>), dim3(G), dim3(WG), 0, c->stream, k, pl, Mm, c->fixmask,
-                           z, pold, pnew, q, c->scal, c->partials, Gb);
+                           z, pold, pnew, q, c->scal, c->partials, Gz, Gr);
     } else {
         const SymLayout sym{c->supper, c->uoff, c->loff, c->lrec, c->S32u, c->S32a, c->S64u};
         hipLaunchKernelGGL((k_pcg_spmv<T, diff || LAY == 4, U, PF, NT, W, (diff || LAY >= 3) ? LAY : 0, STG>),
                            dim3(G), dim3(WG), 0, c->stream, k, t.N, t.nslices, c->slice_off, c->srow, c->slen, c->scol,
-                           A, Mm, t.nbs, c->fixmask, z, pold, pnew, q, c->scal, c->partials, sym, c->wwin, Gb);
+                           A, Mm, t.nbs, c->fixmask, z, pold, pnew, q, c->scal, c->partials, sym, c->wwin, Gz, Gr);
     }
 }
 
@@ -1344,7 +1268,7 @@ void launch_spmv(eolc_ctx *c, int variant, int k, int G, const T *A, const T *Mm
         const eolc::Topology &t = c->topo;
         hipLaunchKernelGGL((k_pcg_spmv_split<T, mixed>), dim3(split_grid(t.nslices)), dim3(kSplitWG), 0, c->stream, k,
                            t.N, t.nslices, c->slice_off, c->srow, c->slen, c->scol, A, Mm, t.nbs, c->fixmask, z, pold,
-                           pnew, q, c->scal, c->partials, eolc::vec_grid(t.N));
+                           pnew, q, c->scal, c->partials, eolc::vec_grid(t.N), rr_partials(c));
         return;
     }
 #define EOLC_SPMV_CASE(id, U, PF, NT, W, LAY, STG)                                      \
@@ -1368,19 +1292,19 @@ void launch_iteration(eolc_ctx *c, int k, int G, const T *A, const T *Mm, const 
     constexpr bool diff = std::is_same<T, float>::value;
     const int variant = c->spmv_variant[diff ? 0 : 1];
     launch_spmv<T>(c, variant, k, G, A, Mm, z, p[pin], p[pout], q);
-    const int Ga = spmv_partials(t, diff, variant), Gv = eolc::vec_grid(t.N);
+    const int Ga = spmv_partials(t, diff, variant);
+    if (c->ml_on) {   // launch errors surface at the chunk's hipGetLastError
+        const eolc::MLUpdate u{k, Ga, p[pout], q, x};
+        (void)eolc::ml_apply(c, diff, (k + 1) & 1, &u);
+        return;
+    }
     auto update = [&](auto wg) {
         constexpr int W = decltype(wg)::value;
-        if (c->ml_on)
-            hipLaunchKernelGGL((k_pcg_update_flat<T, TX, W>), dim3(W == WG ? eolc::pcg_grid_phys(Gv) : Gv), dim3(W), 0,
-                               c->stream, k, Gv, Ga, 3 * t.N, p[pout], q, x, r, c->scal, c->partials);
-        else
-            hipLaunchKernelGGL((k_pcg_update<T, TX, W>), dim3(Gv), dim3(W), 0, c->stream, k, Ga, t.N, D, p[pout], q, x,
-                               r, z, c->scal, c->partials);
+        hipLaunchKernelGGL((k_pcg_update<T, TX, W>), dim3(eolc::vec_grid(t.N)), dim3(W), 0, c->stream, k, Ga, t.N, D,
+                           p[pout], q, x, r, z, c->scal, c->partials);
     };
     if (eolc::vec_wg(t.N) == eolc::kVecWG) update(std::integral_constant<int, eolc::kVecWG>());
     else update(std::integral_constant<int, WG>());
-    if (c->ml_on) (void)eolc::ml_apply(c, diff, (k + 1) & 1, 1);   // launch errors surface at the chunk's hipGetLastError
 }
 
 // z = P r for the residual r64 (FP64): mixed -> r32, z32; FP64 -> z64 (r64 in place);
@@ -1405,7 +1329,7 @@ hipError_t precondition(eolc_ctx *c, bool mixed, int parity)
     if (eolc::vec_wg(N) == eolc::kVecWG) by_ml(std::integral_constant<int, eolc::kVecWG>());
     else by_ml(std::integral_constant<int, WG>());
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess && c->ml_on) e = eolc::ml_apply(c, mixed, parity, 0);
+    if (e == hipSuccess && c->ml_on) e = eolc::ml_apply(c, mixed, parity, nullptr);
     return e;
 }
 
@@ -1509,17 +1433,6 @@ int fp64_layout(int variant)
     default:
         return 0;
     }
-}
-
-// Physical workgroups of the row kernels that can take a second logical workgroup
-// (the patch SpMV, the multilevel update and prolongation): when G exceeds a
-// multiple of 512 (two resident 1,024-thread workgroups on each of the 256 CUs; four
-// rounds of one for the FP64 patch SpMV) by at most 64, the excess rides on the first
-// workgroups, which start first, instead of running as a nearly empty last round.
-int pcg_grid_phys(int G)
-{
-    const int E = G % 512;
-    return (G > 512 && E > 0 && E <= 64) ? G - E : G;
 }
 
 // The vector kernels take 256 threads a workgroup while 1,024 would leave compute units

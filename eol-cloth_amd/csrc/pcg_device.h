@@ -28,24 +28,6 @@ __device__ __forceinline__ void wg_rows(int N, int *begin, int *end)
     *end = e < N ? e : N;
 }
 
-// A row kernel may run on fewer workgroups than the G logical ones (pcg_grid): the
-// first G - gridDim.x workgroups (the first dispatched, one per XCD in turn) then
-// also do logical workgroup gridDim.x + blockIdx.x.  Returns that index or -1.
-__device__ __forceinline__ int extra_logical_wg(int G)
-{
-    const int x = (int)gridDim.x + (int)blockIdx.x;
-    return x < G ? x : -1;
-}
-
-// rows of logical workgroup lw of G
-__device__ __forceinline__ void wg_rows_at(int N, int G, int lw, int *begin, int *end)
-{
-    int per = (N + G - 1) / G;
-    int b = lw * per, e = b + per;
-    *begin = b < N ? b : N;
-    *end = e < N ? e : N;
-}
-
 // slice owned by this wavefront (16 per workgroup)
 __device__ __forceinline__ int wave_slice() { return logical_wg() * (WG / 64) + (threadIdx.x >> 6); }
 
@@ -84,49 +66,28 @@ __device__ __forceinline__ void block_allsum(double (&v)[K], double *lds /* K * 
     for (int k = 0; k < K; ++k) v[k] = lds[K * NW + k];
 }
 
-// Fixed-order sum of K partial arrays (stride kMaxPartials) of length G, done by
-// every workgroup; the result is identical everywhere.
+// Fixed-order sums of K partial arrays part[k] of G[k] entries each (the kernels that
+// wrote them may have run on different grids), done by every workgroup in one load round
+// and one workgroup sum; the result is identical everywhere.  lds: K * W/64 + K doubles.
 template <int K, int W = WG>
-__device__ __forceinline__ void reduce_partials(const double *__restrict__ part, double (&out)[K], double *lds,
-                                                int G = -1)
+__device__ __forceinline__ void reduce_partials(const double *const (&part)[K], const int (&G)[K], double (&out)[K],
+                                                double *lds)
 {
-    if (G < 0) G = gridDim.x;
+    int most = 0;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        double s = 0.0;
-        for (int i = threadIdx.x; i < G; i += W) s += part[k * eolc::kMaxPartials + i];
-        out[k] = s;
+        out[k] = 0.0;
+        most = max(most, G[k]);
+    }
+    for (int i = threadIdx.x; i < most; i += W) {
+        // the arrays' loads together (a branch around one would wait for it)
+        double x[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) x[k] = part[k][min(i, G[k] - 1)];
+#pragma unroll
+        for (int k = 0; k < K; ++k) out[k] += i < G[k] ? x[k] : 0.0;
     }
     block_allsum<K, W>(out, lds);
-}
-
-// Two partial arrays in one pass (K1 sums of p1, then K2 of p2): the same per-array
-// order as two reduce_partials calls, so the same bits, with one load round and one
-// workgroup sum instead of two.  p1 holds G1 partials per sum, p2 G2 (the kernels that
-// wrote them may have run on different grids).  lds: (K1 + K2) * W/64 + K1 + K2 doubles.
-template <int K1, int K2, int W = WG>
-__device__ __forceinline__ void reduce_partials2(const double *__restrict__ p1, const double *__restrict__ p2,
-                                                 double (&o1)[K1], double (&o2)[K2], double *lds, int G1, int G2)
-{
-    double v[K1 + K2];
-#pragma unroll
-    for (int k = 0; k < K1 + K2; ++k) v[k] = 0.0;
-    for (int i = threadIdx.x; i < max(G1, G2); i += W) {
-        // both arrays' loads together (a branch around either would wait for it)
-        const int i1 = min(i, G1 - 1), i2 = min(i, G2 - 1);
-        double x[K1 + K2];
-#pragma unroll
-        for (int k = 0; k < K1; ++k) x[k] = p1[k * eolc::kMaxPartials + i1];
-#pragma unroll
-        for (int k = 0; k < K2; ++k) x[K1 + k] = p2[k * eolc::kMaxPartials + i2];
-#pragma unroll
-        for (int k = 0; k < K1 + K2; ++k) v[k] += i < (k < K1 ? G1 : G2) ? x[k] : 0.0;
-    }
-    block_allsum<K1 + K2, W>(v, lds);
-#pragma unroll
-    for (int k = 0; k < K1; ++k) o1[k] = v[k];
-#pragma unroll
-    for (int k = 0; k < K2; ++k) o2[k] = v[K1 + k];
 }
 
 template <int K, int W = WG>
@@ -146,7 +107,7 @@ __device__ __forceinline__ void load3(const T *__restrict__ a, int i, double &x,
     x = (double)a[3 * i]; y = (double)a[3 * i + 1]; z = (double)a[3 * i + 2];
 }
 
-// Partials layout (doubles, stride kMaxPartials): PA at slot 0, PB[parity] (r.z, r.r)
+// Partials layout (doubles, stride kMaxPartials): PA (p.q) at slot 0, PB[parity] (r.z, r.r)
 // at slots 1 + 2 parity and 2 + 2 parity, residual-norm partials at slot 5.
 __device__ __forceinline__ double *PA(double *p) { return p; }
 __device__ __forceinline__ double *PB(double *p, int parity) { return p + (1 + 2 * parity) * eolc::kMaxPartials; }
