@@ -309,12 +309,13 @@ SPMV_VARIANTS = [(1, False, False, 8, 0, False), (1, True, False, 8, 0, False), 
                  (1, False, False, 4, 5, False), (2, False, False, 4, 5, False)]
 
 
-def spmv_kernel_name(fp32, variant):
+def spmv_kernel_name(fp32, variant, N):
     u, pf, nt, w, lay, stg = SPMV_VARIANTS[variant]
     b = lambda x: "true" if x else "false"
-    if lay == 5:
+    if lay == 5:   # patches of 256 or 512 rows; eight waves per SIMD with FP32 records one ahead
         t = "float" if fp32 else "double"
-        return f"k_pcg_spmv_patch<{t}, {t}, {b(nt)}, {w}, {u}>"
+        w = (6 if u == 2 and w == 8 else w) if fp32 else 4
+        return f"k_pcg_spmv_patch<{t}, {t}, {b(nt)}, {w}, {u}, {256 if N <= 524288 else 512}>"
     t = "float, true" if fp32 else ("double, true" if lay == 4 else "double, false")
     return f"k_pcg_spmv<{t}, {u}, {b(pf)}, {b(nt)}, {w}, {lay if (fp32 or lay >= 3) else 0}, {b(stg)}>"
 
@@ -625,7 +626,7 @@ def main():
             own = (10 * s) * (nb - sc.N) // 2 + 8 * (nb - sc.N) // 2 + 8 * sc.N + (4 * s * 3 + s + 1) * sc.N
         else:
             own = full
-        kname = spmv_kernel_name(fp32, variant)
+        kname = spmv_kernel_name(fp32, variant, sc.N)
         return {"bound": "hbm", "achieved": full / (ms * 1e-3) / 1e9, "peak": PEAK_HBM / 1e9, "unit": "GB/s",
                 "frac": full / (ms * 1e-3) / PEAK_HBM, "traffic": measured_traffic(kname, args.n),
                 "kernel": kname, "variant": variant, "algorithmic_bytes": full, "avg_launch_ms": ms,

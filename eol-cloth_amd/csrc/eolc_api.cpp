@@ -509,19 +509,19 @@ std::string build_topology(Topology &t, int N, int F, const int *tri, int H, con
 }
 
 // Patch layout of SpMV layout 5 (Topology::pt_*).  The vertices are cut into
-// G = pcg_grid(N) patches by recursive coordinate bisection of the material
+// G = patch_grid(N, PR) patches by recursive coordinate bisection of the material
 // coordinates X: a range of `parts` patches is split at the proportional rank along
 // its wider axis (ties by vertex index), so every patch holds floor or ceil of N / G
-// vertices (at most kPcgWG) and is compact in the material plane, which keeps most
+// vertices (at most PR) and is compact in the material plane, which keeps most
 // stencil pairs inside one patch.  Any mesh gets a valid layout: locality only
 // decides how many pairs are cross blocks.  Inside a patch the rows are ordered by
 // decreasing upper count (vertex index within equal counts).  Returns "" or why the
 // layout does not apply (the patch variants then run their symmetric-record twin).
-std::string build_patch_layout(Topology &t, const double *X)
+std::string build_patch_layout(Topology &t, const double *X, int PR)
 {
-    const int N = t.N, C = eolc::kSlice, S = eolc::kPcgWG / C;
-    const int G = eolc::pcg_grid(N);
-    if ((int64_t)G * eolc::kPcgWG < N) return "more vertices than PCG workgroup rows";
+    const int N = t.N, C = eolc::kSlice, S = PR / C;
+    const int G = eolc::patch_grid(N, PR), pool = eolc::kPatchPool, most = eolc::patch_win(PR);
+    t.pt_rows = PR;
     std::vector<int> ord(N);
     for (int i = 0; i < N; ++i) ord[i] = i;
     std::vector<int> poff(G + 1, 0);
@@ -555,7 +555,7 @@ std::string build_patch_layout(Topology &t, const double *X)
     }
     std::vector<int> patch(N, -1);
     for (int p = 0; p < G; ++p) {
-        if (poff[p + 1] - poff[p] > eolc::kPcgWG) return "a patch holds more than one workgroup's rows";
+        if (poff[p + 1] - poff[p] > PR) return "a patch holds more than one workgroup's rows";
         for (int k = poff[p]; k < poff[p + 1]; ++k) patch[ord[k]] = p;
     }
     // per-row counts: upper blocks, cross lower blocks, lower blocks
@@ -575,8 +575,8 @@ std::string build_patch_layout(Topology &t, const double *X)
     for (int i = 0; i < N; ++i)
         if (nup[i] + nlo[i] > 64) return "a row has more than 64 off-diagonal blocks";
     // storage positions: within a patch, decreasing upper count, then vertex index
-    t.pt_row.assign((size_t)G * eolc::kPcgWG, -1);
-    t.pt_cnt.assign((size_t)G * eolc::kPcgWG, 0);
+    t.pt_row.assign((size_t)G * PR, -1);
+    t.pt_cnt.assign((size_t)G * PR, 0);
     std::vector<int> pos(N, -1);
     host_parallel(G, 8, [&](int64_t p0, int64_t p1) {
         std::vector<int> v;
@@ -584,7 +584,7 @@ std::string build_patch_layout(Topology &t, const double *X)
             v.assign(ord.begin() + poff[p], ord.begin() + poff[p + 1]);
             std::sort(v.begin(), v.end(), [&](int i, int j) { return nup[i] > nup[j] || (nup[i] == nup[j] && i < j); });
             for (int k = 0; k < (int)v.size(); ++k) {
-                const int g = p * eolc::kPcgWG + k;
+                const int g = p * PR + k;
                 t.pt_row[g] = v[k];
                 t.pt_cnt[g] = nup[v[k]] | (nlo[v[k]] << 16);
                 pos[v[k]] = g;
@@ -623,7 +623,7 @@ std::string build_patch_layout(Topology &t, const double *X)
         for (int p = (int)p0; p < (int)p1; ++p) {
             std::vector<int> &h = halo[p];
             for (int k = 0; k < poff[p + 1] - poff[p]; ++k) {
-                const int i = t.pt_row[(size_t)p * eolc::kPcgWG + k];
+                const int i = t.pt_row[(size_t)p * PR + k];
                 for (int b = t.rowptr[i]; b < t.rowptr[i + 1]; ++b)
                     if (patch[t.col[b]] != p) h.push_back(t.col[b]);
             }
@@ -638,21 +638,21 @@ std::string build_patch_layout(Topology &t, const double *X)
         wmax = std::max(wmax, w);
         t.pt_woff[p + 1] = t.pt_woff[p] + w;
     }
-    if (wmax > eolc::kPatchWin)
+    if (wmax > most)
         return "a patch window holds " + std::to_string(wmax) + " vertices (limit " +
-               std::to_string(eolc::kPatchWin) + ")";
-    if (slots_max + wmax > eolc::kPatchPool)
+               std::to_string(most) + ")";
+    if (slots_max + wmax > pool)
         return "a patch needs " + std::to_string(slots_max) + " LDS slots and " + std::to_string(wmax) +
-               " window vertices (limit " + std::to_string(eolc::kPatchPool) + " together)";
+               " window vertices (limit " + std::to_string(pool) + " together)";
     t.pt_win.assign(std::max(t.pt_woff[G], 1), 0);
     for (int p = 0; p < G; ++p) {
         const int n = poff[p + 1] - poff[p];
-        for (int k = 0; k < n; ++k) t.pt_win[t.pt_woff[p] + k] = t.pt_row[(size_t)p * eolc::kPcgWG + k];
+        for (int k = 0; k < n; ++k) t.pt_win[t.pt_woff[p] + k] = t.pt_row[(size_t)p * PR + k];
         std::copy(halo[p].begin(), halo[p].end(), t.pt_win.begin() + t.pt_woff[p] + n);
     }
     t.pt_wmax = wmax;
     auto local = [&](int p, int j) {   // window index of vertex j in patch p's window
-        if (patch[j] == p) return pos[j] - p * eolc::kPcgWG;
+        if (patch[j] == p) return pos[j] - p * PR;
         return poff[p + 1] - poff[p] + (int)(std::lower_bound(halo[p].begin(), halo[p].end(), j) - halo[p].begin());
     };
     t.pt_slots = slots_max;
@@ -1103,7 +1103,10 @@ static int set_topology_impl(eolc_ctx *c, int N, const double *X, int F, const i
     Topology t;
     std::string msg = build_topology(t, N, F, tri, H, hinge, seg);
     if (!msg.empty()) return fail(c, EOLC_ERR_INVALID, "set_topology: " + msg);
-    t.pt_why = build_patch_layout(t, X);
+    for (int rows = t.N <= eolc::kPatchSmallN ? 256 : 512; rows <= eolc::kPcgWG; rows *= 2) {
+        t.pt_why = build_patch_layout(t, X, rows);
+        if (t.pt_why.empty()) break;
+    }
     t.pt_ok = t.pt_why.empty();
     if (!t.pt_ok) {   // the patch variants fall back to their symmetric-record twin
         t.pt_row.clear(); t.pt_cnt.clear(); t.pt_roff.clear(); t.pt_soff.clear(); t.pt_loff.clear();

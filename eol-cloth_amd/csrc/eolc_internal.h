@@ -80,16 +80,17 @@ struct Topology {
     // wmax = the widest range (the LDS-staged SpMV variants need wmax <= kStageVerts)
     std::vector<int> wwin;
     int wmax = 0;
-    // Patch layout (SpMV layout 5): the vertices are cut into pcg_grid(N) compact
-    // patches of at most kPcgWG vertices (recursive coordinate bisection of the
-    // material coordinates), one per PCG workgroup, each stored as 16 slices of 64
-    // rows at positions 1024 lw + 64 slice + lane.  A row's records are its upper
+    // Patch layout (SpMV layout 5): the vertices are cut into patch_grid(N, pt_rows)
+    // compact patches of at most pt_rows vertices (recursive coordinate bisection of the
+    // material coordinates), one per workgroup, each stored as slices of 64
+    // rows at positions pt_rows lw + 64 slice + lane.  A row's records are its upper
     // blocks (column > row) in increasing column order, then its lower blocks whose
     // column lies in another patch (cross blocks); a lower block inside the patch is
     // not stored again: its owner (the upper row) leaves the transposed product in
     // LDS for it, and the row's lower list names that LDS slot (or kPatchCross: take
     // the row's next cross record).
     bool pt_ok = false;
+    int pt_rows = 0;                     // rows per patch (kPatchRows or kPcgWG)
     std::string pt_why;                  // why the layout does not apply to this mesh
     std::vector<int> pt_row;             // per storage position: row or -1
     std::vector<int> pt_cnt;             // per storage position: upper records | lower entries << 16
@@ -107,13 +108,21 @@ struct Topology {
     int pt_wmax = 0;                     // largest window
 };
 
-// Patch layout limits.  A workgroup's LDS pool holds 3 values per transposed-product
-// slot and per window vertex: kPatchPool entries (81,000 B in FP32, two workgroups
-// per CU; 162,000 B in FP64, one).  A window holds at most kPatchWin vertices (staged
-// through registers before beta is known).  kPatchCross marks a cross lower entry.
+// Patch layout limits for patches of `rows` vertices.  A workgroup's LDS holds 3 values
+// per transposed-product slot and per window vertex: at most kPatchPool entries (162,000 B
+// in FP64); the launch asks for what the mesh needs.  A window holds at most 2 rows
+// vertices (staged through registers before beta is known).  kPatchCross marks a cross
+// lower entry.
+// Rows per patch: 256 on meshes of at most kPatchSmallN vertices, 512 above, and the
+// next larger (up to kPcgWG) where a mesh does not fit.  Smaller patches put more
+// workgroups in different phases on a compute unit (the window's loads, the record
+// stream, the LDS sums) and shorten the last round of workgroups, but cut more blocks.
+// Product with 256, 512, 768 and 1,024 rows (us): FP32 263,169 vertices 22.5 23.4 24.1
+// 26.2 (arbitrary order 34.7 37.0 38.8 44.8), 1,050,625 vertices 89.4 82.3 95.1 85.6; FP64
+// 36.7 37.7 38.6 44.7 (58.4 71.3 58.5 65.5) and 161 151 163 166.
+constexpr int kPatchSmallN = 524288;
 constexpr int kPatchPool = 6750;
-constexpr int kPatchWin = 2048;
-constexpr int kPatchSlots = kPatchPool;   // slot indices stay below this
+constexpr int patch_win(int rows) { return 2 * rows; }
 constexpr unsigned short kPatchCross = 0xffff;
 
 // Preconditioner blocks are symmetric by construction (block-Jacobi inverse by the
@@ -456,6 +465,7 @@ hipError_t launch_rhs(eolc_ctx *c, double h);
 hipError_t launch_update_x(eolc_ctx *c, double h);
 
 int pcg_grid(int N);
+int patch_grid(int N, int rows);   // patches of at most `rows` vertices (a multiple of 8)
 int vec_wg(int N);          // workgroup size and workgroups of the PCG's vector kernels
 int vec_grid(int N);
 hipError_t pcg_setup(eolc_ctx *c, bool mixed, int precond_kind, bool ml_linear = true);

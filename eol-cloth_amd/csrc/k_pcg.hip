@@ -407,7 +407,7 @@ k_pcg_spmv(int k, int N, int nslices, const int *__restrict__ slice_off, const i
 
 // ---------------------------------------------------------------------------
 // Patch layout (LAY 5; difference form in either precision).  Workgroup lw owns the
-// rows of patch lw, a compact set of at most 1024 vertices (Topology::pt_*), and
+// rows of patch lw, a compact set of at most PR vertices (Topology::pt_*), and
 // stages p_new = z + beta p_old of the patch's window (its rows, then the vertices of
 // other patches they reference) in LDS; records name their column by window index,
 // so no product gathers from global memory.
@@ -426,7 +426,7 @@ k_pcg_spmv(int k, int N, int nslices, const int *__restrict__ slice_off, const i
 // The workgroup partial of p.q sums the patch's rows instead of 1,024 consecutive
 // rows, so p.q, and with it alpha, can differ in the last bits.
 //
-// LDS pool (kPatchPool entries of 3 values): transposed products, component c of
+// LDS pool (patch_pool entries of 3 values): transposed products, component c of
 // slot s at c S + s (S = slots of the largest patch), then the window, vertex w at
 // 3 S + 3 w.
 struct PatchLayout {
@@ -457,16 +457,17 @@ constexpr int kPatchLo = 8;   // lower entries per row loaded before phase 1 (th
 // collapsed element, up to 1e10 times the others) adds errors of 6e-8 of its size
 // in every direction, also in its own null directions where the rest of the
 // matrix is soft, and no FP32 iteration then converges.
-template <class T, class TR, bool NT, int W, int PD>
-__global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(W, W)))
+template <class T, class TR, bool NT, int W, int PD, int PR>
+__global__ void __launch_bounds__(PR) __attribute__((amdgpu_waves_per_eu(W, W)))
 k_pcg_spmv_patch(int k, PatchLayout pl, const T *__restrict__ Mm, const unsigned char *__restrict__ fixmask,
                  const T *__restrict__ z, const T *__restrict__ pold, T *__restrict__ pnew, T *__restrict__ q,
                  SolverScalars *scal, double *partials, int Gz, int Gr)
 {
     using R = SymRec<TR>;
     typedef typename R::v2 v2;
-    __shared__ double lds[3 * (WG / 64) + 3];
-    __shared__ T pool[3 * eolc::kPatchPool];
+    __shared__ double lds[3 * (PR / 64) + 3];
+    extern __shared__ __align__(16) unsigned char patch_lds[];   // 3 (slots + largest window) values
+    T *const pool = reinterpret_cast<T *>(patch_lds);
     if (scal->done) return;
     const int S = pl.S;
     T *const su = pool + 3 * S;   // window values
@@ -475,7 +476,7 @@ k_pcg_spmv_patch(int k, PatchLayout pl, const T *__restrict__ Mm, const unsigned
     // p_old and z of the window.
     const int lw = logical_wg();
     const int lane = threadIdx.x & 63;
-    const int sl = lw * (WG / 64) + (threadIdx.x >> 6);
+    const int sl = lw * (PR / 64) + (threadIdx.x >> 6);
     const int g = sl * eolc::kSlice + lane;
     const int row = pl.row[g];
     const bool active = row >= 0;
@@ -496,11 +497,11 @@ k_pcg_spmv_patch(int k, PatchLayout pl, const T *__restrict__ Mm, const unsigned
     const TR *__restrict__ rb = patch_records<TR>(pl) + (size_t)10 * (pl.roff[sl] + lane);
     const int s0 = pl.soff[sl] + lane;
     const int w0 = pl.woff[lw], nf = 3 * (pl.woff[lw + 1] - w0);
-    constexpr int kPer = (3 * eolc::kPatchWin + WG - 1) / WG;
+    constexpr int kPer = (3 * eolc::patch_win(PR) + PR - 1) / PR;
     T spo[kPer], sz[kPer];
 #pragma unroll
     for (int t = 0; t < kPer; ++t) {
-        const int f = t * WG + (int)threadIdx.x;
+        const int f = t * PR + (int)threadIdx.x;
         spo[t] = 0;
         sz[t] = 0;
         if (f < nf) {
@@ -511,7 +512,7 @@ k_pcg_spmv_patch(int k, PatchLayout pl, const T *__restrict__ Mm, const unsigned
     }
     const bool restart_beta0 = (k == scal->first_iter);
     double sums[3];   // r.z and r.r of this iterate, r.z of the one before
-    reduce_rz<WG>(partials, k, Gz, Gr, sums, lds);
+    reduce_rz<PR>(partials, k, Gz, Gr, sums, lds);
     const double rzk = sums[0], rrk = sums[1];
     const double thr = fmax(scal->tol2 * scal->bnorm2, scal->delta2 * scal->rmax2);
     if (!isfinite(rrk) || !isfinite(rzk) || rrk <= thr) {
@@ -527,7 +528,7 @@ k_pcg_spmv_patch(int k, PatchLayout pl, const T *__restrict__ Mm, const unsigned
     const T betaT = (T)beta;   // p_new = z + beta p is formed in T, identically everywhere
 #pragma unroll
     for (int t = 0; t < kPer; ++t) {
-        const int f = t * WG + (int)threadIdx.x;
+        const int f = t * PR + (int)threadIdx.x;
         if (f < nf) su[f] = fma(betaT, spo[t], sz[t]);
     }
     __syncthreads();
@@ -630,7 +631,7 @@ k_pcg_spmv_patch(int k, PatchLayout pl, const T *__restrict__ Mm, const unsigned
         dot = ((double)ui0 * (double)q0 + (double)ui1 * (double)q1) + (double)ui2 * (double)q2;
     }
     double v[1] = {dot};
-    write_partials<1>(v, PA(partials), lds);
+    write_partials<1, PR>(v, PA(partials), lds);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         scal->rr = rrk;
         scal->rz = rzk;
@@ -1179,7 +1180,7 @@ __global__ void k_fill(int n, double v, double *__restrict__ out)
 // records in either precision.  The staged variants (19-24) need every workgroup's
 // vertex window within kStageVerts; their LDS (65 KB FP32, 131 KB FP64) allows two
 // workgroups per CU in FP32 and one in FP64.  Layout 5 (25-28) is the patch layout
-// in either precision (k_pcg_spmv_patch; 81 KB of LDS in FP32, 162 KB in FP64).
+// in either precision (k_pcg_spmv_patch, its LDS what the mesh's patches need).
 #define EOLC_SPMV_VARIANT_LIST(X)      \
     X(0, 1, false, false, 8, 0, false) \
     X(1, 1, true, false, 8, 0, false) \
@@ -1235,11 +1236,19 @@ void launch_spmv_one(eolc_ctx *c, int k, int G, const T *A, const T *Mm, const T
     const int Gz = eolc::vec_grid(t.N), Gr = rr_partials(c);
     if constexpr (LAY == 5) {
         using TR = T;
+        // eight waves per SIMD spill in FP64 and with records two ahead
+        constexpr int WP = std::is_same<T, double>::value ? 4 : (U == 2 && W == 8) ? 6 : W;
         const PatchLayout pl{c->pt_row, c->pt_cnt, c->pt_roff, c->pt_soff, c->pt_loff, c->pt_woff, c->pt_win,
                              c->pt_lo,  c->P32,    c->P64,     t.pt_slots, c->smask,   c->sellbase, c->scol,
                              c->A64s};
-        hipLaunchKernelGGL((k_pcg_spmv_patch<T, TR, NT, W, U>), dim3(G), dim3(WG), 0, c->stream, k, pl, Mm, c->fixmask,
-                           z, pold, pnew, q, c->scal, c->partials, Gz, Gr);
+        auto go = [&](auto pr) {
+            constexpr int PR = decltype(pr)::value;
+            hipLaunchKernelGGL((k_pcg_spmv_patch<T, TR, NT, WP, U, PR>), dim3(eolc::patch_grid(t.N, PR)), dim3(PR),
+                               3 * sizeof(T) * (size_t)(t.pt_slots + t.pt_wmax), c->stream, k, pl, Mm, c->fixmask, z, pold, pnew, q, c->scal, c->partials, Gz, Gr);
+        };
+        if (t.pt_rows == 256) go(std::integral_constant<int, 256>());
+        else if (t.pt_rows == 512) go(std::integral_constant<int, 512>());
+        else go(std::integral_constant<int, WG>());
     } else {
         const SymLayout sym{c->supper, c->uoff, c->loff, c->lrec, c->S32u, c->S32a, c->S64u};
         hipLaunchKernelGGL((k_pcg_spmv<T, diff || LAY == 4, U, PF, NT, W, (diff || LAY >= 3) ? LAY : 0, STG>),
@@ -1254,8 +1263,9 @@ inline int split_grid(int nslices) { return (nslices + 7) & ~7; }
 // partial sums of p.q that the product of `variant` leaves
 inline int spmv_partials(const eolc::Topology &t, bool mixed, int variant)
 {
-    return eolc::spmv_runs(t, mixed, variant) == eolc::kSpmvSplit ? split_grid(t.nslices)
-                                                                  : eolc::pcg_grid(t.N);
+    variant = eolc::spmv_runs(t, mixed, variant);
+    if (eolc::spmv_patch(variant)) return eolc::patch_grid(t.N, t.pt_rows);
+    return variant == eolc::kSpmvSplit ? split_grid(t.nslices) : eolc::pcg_grid(t.N);
 }
 
 template <class T>
@@ -1439,6 +1449,8 @@ int fp64_layout(int variant)
 // idle (fewer than 256 workgroups).
 int vec_wg(int N) { return pcg_grid(N) < 256 ? kVecWG : WG; }
 int vec_grid(int N) { return vec_wg(N) == WG ? pcg_grid(N) : ((N + kVecWG - 1) / kVecWG + 7) & ~7; }
+
+int patch_grid(int N, int rows) { return ((N + rows - 1) / rows + 7) & ~7; }
 
 int pcg_grid(int N)
 {

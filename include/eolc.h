@@ -452,7 +452,7 @@ int eolc_stream_read(eolc_ctx *ctx, int64_t bytes, int reps, double *avg_ms);
  * two vertices share a patch is read once, its transposed product passed to the
  * other row through LDS; they apply when every patch needs at most 6,750 LDS entries
  * (the same reporting and refusal otherwise).  26 and 28 load each row's records
- * two ahead instead of one (8 and 4 waves per SIMD).  All variants give bitwise-identical
+ * two ahead instead of one (6 and 4 waves per SIMD).  All variants give bitwise-identical
  * results within a precision, except that variants 18, 22 and 25-28 read the
  * symmetric or patch records in FP64 too and there apply the operator in the
  * difference form of the FP32 product (the same matrix, rounded differently; the

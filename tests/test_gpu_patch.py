@@ -181,3 +181,31 @@ def test_patch_kernels_with_a_second_logical_workgroup(ctx):
         assert rel_err(out[(name, 25)], out[(name, 0)]) <= 1e-4
     ctx.set_spmv_variant(32, 0)
     ctx.set_spmv_variant(64, 0)
+
+
+@pytest.mark.parametrize("n,wmin,wmax", [(480, 1, 512), (900, 513, 1024), (1800, 1025, 2048)])
+def test_patch_rows_follow_the_window(ctx, n, wmin, wmax):
+    """Triangles between random points of the plane reference nearly every vertex from
+    every patch: windows of up to 512 vertices run patches of 256 rows, up to 1,024 those
+    of 512 rows, up to 2,048 those of 1,024.  All agree with the SELL kernels."""
+    rng = np.random.default_rng(n)
+    X = rng.uniform(size=(n, 2))
+    t = rng.permutation(np.tile(np.arange(n), 5))
+    t = t[: 3 * (len(t) // 3)].reshape(-1, 3)
+    t = t[(t[:, 0] != t[:, 1]) & (t[:, 0] != t[:, 2]) & (t[:, 1] != t[:, 2])]
+    d1, d2 = X[t[:, 1]] - X[t[:, 0]], X[t[:, 2]] - X[t[:, 0]]
+    area = d1[:, 0] * d2[:, 1] - d1[:, 1] * d2[:, 0]
+    t = np.where(area[:, None] > 0, t, t[:, [0, 2, 1]])[np.abs(area) > 1e-3].astype(np.int32)
+    x = np.concatenate([X, np.zeros((n, 1))], axis=1).reshape(-1) + scene.gaussian(3, 3 * n, 1e-3)
+    v = scene.gaussian(4, 3 * n, 0.05)
+    mesh = (X, t, np.zeros((0, 4), dtype=np.int32), x, v, np.array([0], dtype=np.int32))
+    ctx.set_topology(*mesh[:3])
+    info = ctx.spmv_layout_info()
+    print(f"{n} vertices, {len(t)} faces: {info}", flush=True)
+    assert info["applies"] == 1 and wmin <= info["window_max"] <= wmax
+    for prec in (32, 64):
+        ref, _ = solve(ctx, mesh, prec, 0)
+        for var in (25, 28):
+            out, st = solve(ctx, mesh, prec, var)
+            assert rel_err(out, ref) <= 1e-6
+        ctx.set_spmv_variant(prec, 0)
