@@ -256,19 +256,118 @@ k_hinge_eval(int H, int F, const int *__restrict__ hinge, const double *__restri
 }
 
 // ---------------------------------------------------------------------------
-// SPD-projected variant.  Q = orthonormal basis (12x9) of the complement of the
-// translations: contrasts c1 = (1,-1,0,0)/sqrt2, c2 = (1,1,-2,0)/sqrt6,
-// c3 = (1,1,1,-3)/sqrt12 (each times I3).  K9 = Q^T K Q is diagonalised with
-// cyclic Jacobi (rotation order (0,1), (0,2), ..., (7,8); at most 30 sweeps, until
-// the off-diagonal mass falls below 1e-30 of the Frobenius mass), negative
-// eigenvalues are zeroed and K+ = Q V L+ V^T Q^T.
-// K9 is kept as its 45 upper entries and V as 81 values in registers; every index is
-// a compile-time constant (all loops over matrix entries are unrolled), so nothing
-// goes through LDS (one wave per SIMD, no LDS occupancy limit, no scratch).
+// SPD-projected variant.  The Hessian annihilates the translations and, as the angle
+// depends on neither, the stretch along the hinge edge: x_i -> x_i + (x_i . e) e keeps
+// both normals and every foot and height that the gradient is made of, so K d = 0 for d_i =
+// ((x_i - mean) . e) e.  K8 = Q^T K Q with Q (12x8) an orthonormal basis of the rest:
+// contrasts of the vertices (three rows of 4, T cw, the third along the vertices'
+// coordinates on e) times an orthonormal frame R with e first, without (third contrast,
+// e).  K8 is diagonalised with cyclic Jacobi (at most 30 sweeps, until the off-diagonal
+// mass falls below 1e-30 of the Frobenius mass), negative eigenvalues are zeroed and
+// K+ = Q V L+ V^T Q^T.
+// K8 is kept as its 36 upper entries and V as 64 values in registers; every index is a
+// compile-time constant (all loops over matrix entries are unrolled), so nothing goes
+// through LDS and nothing to scratch, at one wave per SIMD.  The chain of square
+// roots behind a rotation's angle is therefore what the time goes into: a sweep runs in
+// seven rounds of four rotations on disjoint pairs (Brent and Luk's tournament order),
+// whose angles are independent.  3.14 M hinges: 6.2 ms row by row with IEEE divisions and
+// roots on the 9 x 9 complement of the translations alone, 4.3 ms in rounds, 3.3 ms on
+// 8 x 8; the assembled matrix is off a 64-bit eigensolver's by 3e-16 to 3e-15 of its
+// norm (5e-16 to 3e-15 before).
 namespace proj {
 constexpr double r2 = 0.70710678118654752440, r6 = 0.40824829046386301637, r12 = 0.28867513459481288225;
+// contrasts (1,-1,0,0)/sqrt2, (1,1,-2,0)/sqrt6, (1,1,1,-3)/sqrt12
 constexpr double cw[3][4] = {{r2, -r2, 0, 0}, {r6, r6, -2 * r6, 0}, {r12, r12, r12, -3 * r12}};
-constexpr int ix(int P, int Q) { return P <= Q ? P * 9 - P * (P - 1) / 2 + (Q - P) : Q * 9 - Q * (Q - 1) / 2 + (P - Q); }
+constexpr int ix(int P, int Q) { return P <= Q ? P * 8 - P * (P - 1) / 2 + (Q - P) : Q * 8 - Q * (Q - 1) / 2 + (P - Q); }
+// K8 index of (contrast c, axis a): e first; (2, e) is left out (negative)
+constexpr int dof(int c, int a) { return c < 2 ? 3 * c + a : (a == 0 ? -1 : 5 + a); }
+// pair i of a round: (round, 7) and (round + i, round - i) mod 7
+constexpr int one(int round, int i) { return (round + i) % 7; }
+constexpr int two(int round, int i) { return i == 0 ? 7 : (round + 7 - i) % 7; }
+constexpr int lo(int round, int i) { return one(round, i) < two(round, i) ? one(round, i) : two(round, i); }
+constexpr int hi(int round, int i) { return one(round, i) < two(round, i) ? two(round, i) : one(round, i); }
+
+// 1 / sqrt(x) without division: the hardware's estimate and Newton steps, the last with the
+// residual 1 - x r^2 formed from the exact product x r (within an ulp: an error here
+// scales the eigenvectors, twenty times a sweep).
+__device__ __forceinline__ double rsqrt_n(double x)
+{
+    double r = __builtin_amdgcn_rsq(x);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) r = r * fma(-0.5 * x * r, r, 1.5);
+    const double y = x * r, dy = fma(x, r, -y);
+    return fma(0.5 * r, fma(-dy, r, fma(-y, r, 1.0)), r);
+}
+
+// The Jacobi rotation that zeroes apr, of at most 45 degrees: cos 2t = |d| / h and
+// sin 2t = 2 apr sign(d) / h with d = arr - app, h^2 = d^2 + (2 apr)^2; the identity where h
+// is zero or leaves the range.
+__device__ __forceinline__ void rotation(double app, double apr, double arr, double &c, double &sn)
+{
+    const double d = arr - app, t = 2.0 * apr, h2 = fma(d, d, t * t);
+    const double rh = rsqrt_n(h2);
+    const double c2 = fma(0.5 * fabs(d), rh, 0.5), rc = rsqrt_n(c2);
+    const bool ok = h2 > 1e-300 && h2 < 1e300;
+    c = ok ? c2 * rc : 1.0;
+    sn = ok ? 0.5 * copysign(1.0, d) * t * rh * rc : 0.0;
+}
+
+// Two unit vectors orthogonal to the unit vector n and to each other (Duff et al. 2017).
+__device__ __forceinline__ void complete(V3 n, V3 &b1, V3 &b2)
+{
+    const double sg = copysign(1.0, n.z), a = -1.0 / (sg + n.z), b = n.x * n.y * a;
+    b1 = V3{1.0 + sg * n.x * n.x * a, sg * b, -sg * n.x};
+    b2 = V3{b, sg + n.y * n.y * a, -n.y};
+}
+
+// Q of one hinge: the frame (rows e, b1, b2) and the contrasts T cw.
+struct Basis {
+    V3 R[3];
+    double cq[3][4];
+};
+__device__ __forceinline__ void basis(const double *__restrict__ x, const int *q, Basis &B)
+{
+    const V3 x0 = ld3(x + 3 * q[0]);
+    const V3 u = ld3(x + 3 * q[1]) - x0, v = ld3(x + 3 * q[2]) - x0, w = ld3(x + 3 * q[3]) - x0;
+    B.R[0] = (1.0 / sqrt(dot(u, u))) * u;
+    complete(B.R[0], B.R[1], B.R[2]);
+    const double s[4] = {0.0, dot(u, B.R[0]), dot(v, B.R[0]), dot(w, B.R[0])};   // coordinates on e
+    double eta[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) eta[c] = cw[c][1] * s[1] + cw[c][2] * s[2] + cw[c][3] * s[3];
+    const double in = 1.0 / sqrt(eta[0] * eta[0] + eta[1] * eta[1] + eta[2] * eta[2]);
+    V3 T[3];
+    T[2] = V3{in * eta[0], in * eta[1], in * eta[2]};
+    complete(T[2], T[0], T[1]);
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) B.cq[c][i] = T[c].x * cw[0][i] + T[c].y * cw[1][i] + T[c].z * cw[2][i];
+}
+
+// R M R^T (FORWARD) or R^T M R of a row-major 3x3
+template <bool FORWARD> __device__ __forceinline__ void turn(const V3 (&R)[3], const double (&M)[9], double (&out)[9])
+{
+    double t[9];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            double acc = 0.0;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) acc += (FORWARD ? comp(R[i], k) : comp(R[k], i)) * M[3 * k + j];
+            t[3 * i + j] = acc;
+        }
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            double acc = 0.0;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) acc += t[3 * i + k] * (FORWARD ? comp(R[j], k) : comp(R[k], j));
+            out[3 * i + j] = acc;
+        }
+}
 }  // namespace proj
 
 __global__ void __launch_bounds__(64)
@@ -276,115 +375,128 @@ k_hinge_eval_projr(int H, int F, const int *__restrict__ hinge, const double *__
                    const double *__restrict__ X, double beta_all, const double *__restrict__ beta_hinge, double s,
                    double *__restrict__ stageK, double *__restrict__ stageF)
 {
-    using proj::cw;
+    using proj::dof;
     using proj::ix;
     const int h = blockIdx.x * blockDim.x + threadIdx.x;
     if (h >= H) return;
-    int q[4] = {hinge[4 * h], hinge[4 * h + 1], hinge[4 * h + 2], hinge[4 * h + 3]};
-    HingeGeom G;
-    hinge_geom(x, X, q, beta_hinge ? beta_hinge[h] : beta_all, G);
+    double A[36];
+#pragma unroll
+    for (int e = 0; e < 36; ++e) A[e] = 0.0;
     {
+        int q[4] = {hinge[4 * h], hinge[4 * h + 1], hinge[4 * h + 2], hinge[4 * h + 3]};
+        HingeGeom G;
+        hinge_geom(x, X, q, beta_hinge ? beta_hinge[h] : beta_all, G);
         double *sf = stageF + (size_t)9 * F + (size_t)12 * h;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             V3 gj = cross(G.g[0], G.a[0][j]) + cross(G.g[1], G.a[1][j]);
             sf[3 * j] = G.w * gj.x; sf[3 * j + 1] = G.w * gj.y; sf[3 * j + 2] = G.w * gj.z;
         }
+        proj::Basis B;
+        proj::basis(x, q, B);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = i; j < 4; ++j) {
+                double raw[9], blk[9];
+                hinge_hess_block(G, i, j, raw);
+                if (i == j) { raw[3] = raw[1]; raw[6] = raw[2]; raw[7] = raw[5]; }
+                proj::turn<true>(B.R, raw, blk);
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+#pragma unroll
+                    for (int dd = 0; dd < 3; ++dd) {
+                        const double wgt = -G.w * (B.cq[c][i] * B.cq[dd][j]);
+                        const double wgt2 = (i != j) ? -G.w * (B.cq[c][j] * B.cq[dd][i]) : 0.0;
+#pragma unroll
+                        for (int a = 0; a < 3; ++a)
+#pragma unroll
+                            for (int b = 0; b < 3; ++b) {
+                                const int P = dof(c, a), Qc = dof(dd, b);
+                                if (P < 0 || Qc < 0 || P > Qc) continue;   // upper triangle
+                                double val = wgt * blk[3 * a + b];
+                                if (i != j) val += wgt2 * blk[3 * b + a];
+                                A[ix(P, Qc)] += val;
+                            }
+                    }
+            }
     }
-    double A[45];
+    double V[64];
 #pragma unroll
-    for (int e = 0; e < 45; ++e) A[e] = 0.0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = i; j < 4; ++j) {
-            double blk[9];
-            hinge_hess_block(G, i, j, blk);
-            if (i == j) { blk[3] = blk[1]; blk[6] = blk[2]; blk[7] = blk[5]; }
-#pragma unroll
-            for (int c = 0; c < 3; ++c)
-#pragma unroll
-                for (int dd = 0; dd < 3; ++dd) {
-                    const double wgt = cw[c][i] * cw[dd][j];
-                    const double wgt2 = (i != j) ? cw[c][j] * cw[dd][i] : 0.0;
-                    if (wgt == 0.0 && wgt2 == 0.0) continue;
-#pragma unroll
-                    for (int a = 0; a < 3; ++a)
-#pragma unroll
-                        for (int b = 0; b < 3; ++b) {
-                            const int P = 3 * c + a, Qc = 3 * dd + b;
-                            if (P > Qc) continue;   // upper triangle (the matrix is symmetric)
-                            const double val = wgt * blk[3 * a + b] + wgt2 * blk[3 * b + a];
-                            A[ix(P, Qc)] += -G.w * val;
-                        }
-                }
-        }
-    double V[81];
-#pragma unroll
-    for (int e = 0; e < 81; ++e) V[e] = (e % 10 == 0) ? 1.0 : 0.0;
+    for (int e = 0; e < 64; ++e) V[e] = (e % 9 == 0) ? 1.0 : 0.0;
     double fro = 0.0;
 #pragma unroll
-    for (int P = 0; P < 9; ++P)
+    for (int P = 0; P < 8; ++P)
 #pragma unroll
-        for (int Qc = 0; Qc < 9; ++Qc) fro += A[ix(P, Qc)] * A[ix(P, Qc)];
+        for (int Qc = 0; Qc < 8; ++Qc) fro += A[ix(P, Qc)] * A[ix(P, Qc)];
     for (int sweep = 0; sweep < 30; ++sweep) {
         double off = 0.0;
 #pragma unroll
-        for (int p = 0; p < 9; ++p)
-#pragma unroll
-            for (int r = p + 1; r < 9; ++r) off += A[ix(p, r)] * A[ix(p, r)];
-        if (!(off > 1e-30 * fro)) break;
-#pragma unroll
         for (int p = 0; p < 8; ++p)
 #pragma unroll
-            for (int r = p + 1; r < 9; ++r) {
-                const double apr = A[ix(p, r)];
-                if (apr != 0.0) {
-                    const double app = A[ix(p, p)], arr = A[ix(r, r)];
-                    const double theta = (arr - app) / (2.0 * apr);
-                    const double tt = (theta >= 0.0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
-                    const double c = 1.0 / sqrt(tt * tt + 1.0), sn = tt * c;
-                    // columns p, r then rows p, r of the symmetric matrix
+            for (int r = p + 1; r < 8; ++r) off += A[ix(p, r)] * A[ix(p, r)];
+        if (!(off > 1e-30 * fro)) break;
 #pragma unroll
-                    for (int k = 0; k < 9; ++k) {
-                        if (k == p || k == r) continue;
-                        const double akp = A[ix(k, p)], akr = A[ix(k, r)];
-                        A[ix(k, p)] = c * akp - sn * akr;
-                        A[ix(k, r)] = sn * akp + c * akr;
-                    }
-                    // the 2x2 block {p, r}: column step, then row step
-                    const double cpp = c * app - sn * apr, cpr = sn * app + c * apr;
-                    const double crp = c * apr - sn * arr, crr = sn * apr + c * arr;
-                    A[ix(p, p)] = c * cpp - sn * crp;
-                    A[ix(p, r)] = c * cpr - sn * crr;
-                    A[ix(r, r)] = sn * cpr + c * crr;
+        for (int round = 0; round < 7; ++round) {
+            double c[4], sn[4];
 #pragma unroll
-                    for (int k = 0; k < 9; ++k) {
-                        const double vkp = V[k * 9 + p], vkr = V[k * 9 + r];
-                        V[k * 9 + p] = c * vkp - sn * vkr;
-                        V[k * 9 + r] = sn * vkp + c * vkr;
-                    }
+            for (int i = 0; i < 4; ++i) {
+                const int p = proj::lo(round, i), r = proj::hi(round, i);
+                proj::rotation(A[ix(p, p)], A[ix(p, r)], A[ix(r, r)], c[i], sn[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int p = proj::lo(round, i), r = proj::hi(round, i);
+                const double app = A[ix(p, p)], apr = A[ix(p, r)], arr = A[ix(r, r)];
+                // columns p, r then rows p, r of the symmetric matrix
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    if (k == p || k == r) continue;
+                    const double akp = A[ix(k, p)], akr = A[ix(k, r)];
+                    A[ix(k, p)] = c[i] * akp - sn[i] * akr;
+                    A[ix(k, r)] = sn[i] * akp + c[i] * akr;
+                }
+                // the 2x2 block {p, r}: column step, then row step
+                const double cpp = c[i] * app - sn[i] * apr, cpr = sn[i] * app + c[i] * apr;
+                const double crp = c[i] * apr - sn[i] * arr, crr = sn[i] * apr + c[i] * arr;
+                A[ix(p, p)] = c[i] * cpp - sn[i] * crp;
+                A[ix(p, r)] = c[i] * cpr - sn[i] * crr;
+                A[ix(r, r)] = sn[i] * cpr + c[i] * crr;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const double vkp = V[k * 8 + p], vkr = V[k * 8 + r];
+                    V[k * 8 + p] = c[i] * vkp - sn[i] * vkr;
+                    V[k * 8 + r] = sn[i] * vkp + c[i] * vkr;
                 }
             }
+        }
     }
-    double lam[9];
+    double lam[8];
 #pragma unroll
-    for (int k = 0; k < 9; ++k) lam[k] = fmax(A[ix(k, k)], 0.0);
-    // K9+ = V diag(lam) V^T (upper triangle, into A)
+    for (int k = 0; k < 8; ++k) lam[k] = fmax(A[ix(k, k)], 0.0);
+    // K8+ = V diag(lam) V^T (upper triangle, into A)
 #pragma unroll
-    for (int a = 0; a < 9; ++a)
+    for (int a = 0; a < 8; ++a)
 #pragma unroll
-        for (int b = a; b < 9; ++b) {
+        for (int b = a; b < 8; ++b) {
             double acc = 0.0;
 #pragma unroll
-            for (int k = 0; k < 9; ++k) acc += V[a * 9 + k] * lam[k] * V[b * 9 + k];
+            for (int k = 0; k < 8; ++k) acc += V[a * 8 + k] * lam[k] * V[b * 8 + k];
             A[ix(a, b)] = acc;
         }
+    // Q again, from an index the compiler does not connect with the first: kept over the
+    // sweeps it would cost 21 of the registers
+    int h2 = h;
+    asm volatile("" : "+v"(h2));
+    int q[4] = {hinge[4 * h2], hinge[4 * h2 + 1], hinge[4 * h2 + 2], hinge[4 * h2 + 3]};
+    proj::Basis B;
+    proj::basis(x, q, B);
     const int pv[10] = {0, 1, 2, 3, 0, 0, 0, 1, 1, 2}, pw[10] = {0, 1, 2, 3, 1, 2, 3, 2, 3, 3};
     double *sk = stageK + (size_t)54 * F + (size_t)90 * h;
 #pragma unroll
     for (int p = 0; p < 10; ++p) {
         const int i = pv[p], j = pw[p];
+        double M[9], out[9];
 #pragma unroll
         for (int a = 0; a < 3; ++a)
 #pragma unroll
@@ -393,9 +505,15 @@ k_hinge_eval_projr(int H, int F, const int *__restrict__ hinge, const double *__
 #pragma unroll
                 for (int c = 0; c < 3; ++c)
 #pragma unroll
-                    for (int dd = 0; dd < 3; ++dd) acc += cw[c][i] * cw[dd][j] * A[ix(3 * c + a, 3 * dd + b)];
-                sk[9 * p + 3 * a + b] = s * acc;
+                    for (int dd = 0; dd < 3; ++dd)
+                        if (dof(c, a) >= 0 && dof(dd, b) >= 0)
+                            acc += B.cq[c][i] * B.cq[dd][j] * A[ix(dof(c, a), dof(dd, b))];
+                M[3 * a + b] = acc;
             }
+        proj::turn<false>(B.R, M, out);
+        if (i == j) { out[3] = out[1]; out[6] = out[2]; out[7] = out[5]; }   // exactly symmetric
+#pragma unroll
+        for (int c = 0; c < 9; ++c) sk[9 * p + c] = s * out[c];
     }
 }
 

@@ -115,3 +115,46 @@ def test_spd_projection_matches_eigh(ctx):
           f"max|diff - ref| / max|h^2 K| = {np.abs(diff - ref).max() / kmax:.2e}", flush=True)
     assert nneg > 0
     assert np.abs(diff - ref).max() <= 1e-10 * kmax
+
+
+@pytest.mark.parametrize("fold", [0.0, 0.5, 3.0, "needle"])
+@pytest.mark.parametrize("edge", [(1, 0, 0), (0, 0, 1), (0, 0, -1), (1e-9, 0, -1), (1, 2, -3)])
+def test_spd_projection_of_one_hinge(ctx, edge, fold):
+    """One hinge with its edge along the axes where the projection's frame changes sign,
+    flat (rank-deficient), folded, nearly closed, and with an apex a thousandth of the
+    edge from it: the assembled MDK minus the faces' part is h^2 times the hinge Hessian
+    with its negative eigenvalues at zero (numpy's eigh on the oracle's Hessian)."""
+    X = np.array([[0.0, 0.0], [0.1, 0.0], [0.04, 0.08], [0.07, -0.09]])
+    tri = np.array([[0, 1, 2], [0, 3, 1]], dtype=np.int32)
+    hinge = scene.hinges(4, tri)
+    e = np.asarray(edge, dtype=np.float64) / np.linalg.norm(edge)
+    a = np.linalg.qr(np.stack([e, [0.3, 0.9, 0.1], [0.2, -0.4, 0.7]], 1))[0]
+    a[:, 0] = e
+    a[:, 2] = np.cross(e, a[:, 1])
+    th = 0.0 if fold == "needle" else fold
+    loc = np.array([[0, 0, 0], [0.1, 0, 0], [0.04, 0.08, 0],
+                    [0.07, -0.09 * np.cos(th), 0.09 * np.sin(th)]])
+    if fold == "needle":
+        loc[2] = [0.04, 1e-4, 2e-5]
+        loc[3] = [0.07, -0.05, 0.06]
+    x = (loc @ a.T + [0.3, -0.2, 0.5]).reshape(-1)
+    beta, mats = 1e-2, []
+    for b in (0.0, beta):
+        ctx.set_topology(X, tri, hinge)
+        ctx.set_material(0.1, 500.0, 0.3, b, 0.0, 1.0)
+        ctx.set_options(eolc.OPT_SPD_PROJECT_BENDING)
+        ctx.upload_state(x, 0 * x)
+        ctx.forces_fill(GRAV, H)
+        mats.append(ctx.download_csr(eolc.MAT_MDK).toarray())
+    ctx.set_options(0)
+    q, p = hinge[0], x.reshape(-1, 3)
+    _, _, K = O.bending(*[p[i] for i in q], *[X[i] for i in q], beta)
+    w, V = np.linalg.eigh(0.5 * (K + K.T))
+    dofs = (3 * np.asarray(q)[:, None] + np.arange(3)).reshape(-1)
+    ref = np.zeros((12, 12))
+    ref[np.ix_(dofs, dofs)] = H * H * (V * np.maximum(w, 0.0)) @ V.T
+    # the faces' part is subtracted: its rounding counts too
+    bar = 1e-10 * H * H * np.abs(K).max() + 1e-14 * np.abs(mats[0]).max()
+    print(f"edge {edge} fold {fold}: eigenvalues {w.min():.2e} .. {w.max():.2e}, off {np.abs(mats[1] - mats[0] - ref).max() / bar:.2e} bars",
+          flush=True)
+    assert np.abs(mats[1] - mats[0] - ref).max() <= bar
