@@ -226,3 +226,37 @@ def test_multilevel_edge_cases(ctx, case):
     for v in out[1:]:
         assert rel_err(v, out[0]) <= 1e-6
         assert np.array_equal(v[fd], out[0][fd])
+
+
+@pytest.mark.parametrize("small", [40, 70])
+def test_linear_fields_of_many_sheets(ctx, small):
+    """A sheet with four levels beside 40 or 70 that end earlier, so that level 3 holds
+    fewer and more than 64 aggregates and the level above more than 512 / 9: P r with
+    linear fields on the levels >= 3 against the oracle."""
+    print(f"linear fields, one large and {small} small sheets", flush=True)
+    parts = [scene.Scene(90 if k == 0 else 6, sigma_x=1e-3, sigma_v=0.05, seed_x=7 + k, seed_v=90 + k)
+             for k in range(small + 1)]
+    off = np.concatenate([[0], np.cumsum([p.N for p in parts])])
+    N = int(off[-1])
+    X = np.vstack([p.X + [2.0 * k, 0.0] for k, p in enumerate(parts)])
+    tri, hinge = (np.vstack([getattr(p, a) + o for p, o in zip(parts, off)]) for a in ("tri", "hinge"))
+    x0 = np.concatenate([p.x0 + np.tile([2.0 * k, 0.0, 0.0], p.N) for k, p in enumerate(parts)])
+    v0 = np.concatenate([p.v0 for p in parts])
+    fd = learned.fixed_dofs(np.concatenate([p.fixed + o for p, o in zip(parts, off)]))
+    ctx.set_topology(X, tri, hinge)
+    ctx.set_material(0.1, 500.0, 0.3, 1e-5, 0.0, 1.0)
+    ctx.set_options(eolc.OPT_SPD_PROJECT_BENDING)
+    ctx.upload_state(x0, v0)
+    ctx.forces_fill(GRAV, H)
+    counts = ctx.ml_info()
+    print(f"  aggregates per level {counts}", flush=True)
+    assert len(counts) >= 5 and (counts[3] > 64) == (small > 64) and counts[4] >= small
+    A = ctx.download_csr(eolc.MAT_MDK).tocsr()
+    maps = [ctx.ml_aggregates(l) for l in range(1, len(counts))]
+    r = np.random.default_rng(3).normal(size=3 * N)
+    ctx.set_ml_linear(2)
+    z = ctx.precond_apply(r, fd, mode=eolc.SOLVE_FP64_BJ | MLF)
+    ctx.set_ml_linear(1)
+    zref = ML.apply(A, N, maps, r, fd, X=X)
+    print(f"  P r rel err {rel_err(z, zref):.2e}", flush=True)
+    assert rel_err(z, zref) <= 1e-12 and np.all(z[fd] == 0.0)
