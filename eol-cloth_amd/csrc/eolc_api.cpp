@@ -761,13 +761,12 @@ int learned_buffers(eolc_ctx *c)
     EOLC_HIP(dalloc(c, &L.o, N * eolc::kLpOut));
     EOLC_HIP(dalloc(c, &L.dO, N * eolc::kLpOut));
     EOLC_HIP(dalloc(c, &L.dinp, N * 2 * eolc::kLpHidden));
-    const size_t nblk = (N + 255) / 256;
     int Gw = 0, rows = 0;
     eolc::learned_wgrad_shape(t.N, &Gw, &rows);
-    L.gpart_n = std::max(nblk * (eolc::kLpHidden * eolc::kLpOut + eolc::kLpOut),
+    L.gpart_n = std::max((size_t)eolc::learned_out_groups(t.N) * (eolc::kLpHidden * eolc::kLpOut + eolc::kLpOut),
                          (size_t)Gw * eolc::kLpLayerSize);
     EOLC_HIP(dalloc(c, &L.gpart, L.gpart_n));
-    EOLC_HIP(dalloc(c, &L.dpart, nblk));
+    EOLC_HIP(dalloc(c, &L.dpart, (size_t)eolc::learned_dot_groups(t.N)));
     EOLC_HIP(dalloc(c, &L.scal, 8));
     EOLC_HIP(hipMemset(L.scal, 0, 8 * sizeof(double)));
     for (double **p : {&L.e, &L.r, &L.z, &L.Az}) EOLC_HIP(dalloc(c, p, 3 * N));

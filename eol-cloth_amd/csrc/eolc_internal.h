@@ -273,10 +273,10 @@ struct MLState {
     int *gcp = nullptr;           // n_3 + ... + n_L + 1: chunk range of each aggregate of levels >= 3
     int nchunks = 0;
     double *gpart = nullptr;      // 45 per chunk
-    double *D9 = nullptr;         // 54 per aggregate of levels >= 3: factors of the Galerkin block
+    double *D9 = nullptr;         // 54 x (aggregates of levels >= 3): factors of the Galerkin blocks
     double *feat2 = nullptr;      // 2 per hord position: (phi_1, phi_2) of the vertex on its level-2 aggregate
     double *feat3 = nullptr;      // 2 per vertex: (phi_1, phi_2) on its level-3 aggregate
-    double *R9p = nullptr;        // 9 per restriction workgroup (4 per level-3 aggregate): partial level-3 sums
+    double *R9p = nullptr;        // 9 x (restriction workgroups, 4 per level-3 aggregate): partial level-3 sums
     double *C9 = nullptr;         // 9 per aggregate of levels >= 3: accumulated coarse field
     std::vector<int> counts;      // host copy of n[0..L]
     std::vector<std::vector<int>> maps;   // host: level-l aggregate of every vertex (l = 1..L)
@@ -504,6 +504,8 @@ hipError_t time_spmv(eolc_ctx *c, bool mixed, int variant, int reps, float *ms);
 hipError_t stream_copy(eolc_ctx *c, size_t bytes, int reps, float *ms, int read_only);
 // learned preconditioner (k_learned.hip); buffers allocated by the API layer
 void learned_wgrad_shape(int N, int *G, int *rows);   // weight-gradient workgroups, rows per workgroup
+int learned_out_groups(int N);   // partial rows of the output layer's gradient
+int learned_dot_groups(int N);   // partial sums of the products with A
 hipError_t learned_quantize(eolc_ctx *c);
 hipError_t learned_forward(eolc_ctx *c);
 hipError_t learned_precond(eolc_ctx *c);               // forward + P -> D32 (fixmask set)

@@ -28,11 +28,13 @@
 //
 // Matrix-unit operand layout of the 16x16x16 bf16 instruction (wave64): lane l
 // supplies A[l%16][4(l/16)+t] and B[4(l/16)+t][l%16] (t = 0..3) and receives
-// D[4(l/16)+t][l%16].
+// D[4(l/16)+t][l%16]; of the 16x16x32 one A[l%16][8(l/16)+t] and B[8(l/16)+t][l%16]
+// (t = 0..7), the results as before.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "eolc_internal.h"
 
@@ -40,6 +42,7 @@ namespace {
 
 typedef short short4v __attribute__((ext_vector_type(4)));
 typedef float float4v __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int HID = eolc::kLpHidden;   // 64
 constexpr int NF = eolc::kLpFeat;      // 16
@@ -208,26 +211,31 @@ __global__ void __launch_bounds__(RT) k_lp_reduce(int n, const double *__restric
     if (threadIdx.x == 0) *out = t;
 }
 
-// Pass 2 (SELL storage order g): the 16 features of vertex srow[g] and the
-// normalised weights of its off-diagonal entries (same storage positions as A).
-__global__ void __launch_bounds__(RT)
+// Pass 2: the 16 features of every vertex and the normalised weights of its off-diagonal
+// entries (same storage positions as A).  One workgroup per slice of 64 rows, whose four
+// wavefronts take every fourth entry of each row: an entry costs a chain of dependent
+// loads, and with one thread to a row a 128 x 128 mesh fills one wavefront per CU
+// (16,641 vertices: 33 us before, 15 now).
+constexpr int FW = 4;   // wavefronts per slice
+__global__ void __launch_bounds__(64 * FW)
 k_lp_features(int N, const int *__restrict__ srow, const int *__restrict__ slice_off, const int *__restrict__ slen,
               const int *__restrict__ scol, const int *__restrict__ diagpos, const double *__restrict__ A,
               int64_t nbs, const double *__restrict__ Mval, const unsigned char *__restrict__ fixmask,
               const double *__restrict__ logt_sum, unsigned short *__restrict__ X, float *__restrict__ w)
 {
-    const int g = blockIdx.x * RT + threadIdx.x;
-    if (g >= N) return;
-    const int i = srow[g];
-    const int64_t base = slice_off[g / SL] + (g % SL);
-    const int len = slen[g];
-    const unsigned fi = fixmask[i];
-    double D[9];
-    masked_block(A, nbs, diagpos[i], fi, fi, true, D);
-    const double t = (D[0] + D[4] + D[8]) / 3.0;
+    static_assert(SL == 64, "one wavefront spans a slice");
+    __shared__ double ps[FW][64];
+    __shared__ int pd[FW][64];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int g = blockIdx.x * SL + lane;
+    const bool row = g < N;
+    const int i = row ? srow[g] : 0;
+    const int64_t base = slice_off[blockIdx.x] + lane;
+    const int len = row ? slen[g] : 0;
+    const unsigned fi = row ? fixmask[i] : 0u;
     double ssum = 0.0;
     int deg = 0;
-    for (int k = 0; k < len; ++k) {
+    for (int k = wid; k < len; k += FW) {
         const int64_t e = base + (int64_t)k * SL;
         const int j = scol[e];
         if (j == i) continue;
@@ -236,7 +244,17 @@ k_lp_features(int N, const int *__restrict__ srow, const int *__restrict__ slice
         ssum += fro(b);
         ++deg;
     }
-    for (int k = 0; k < len; ++k) {
+    ps[wid][lane] = ssum;
+    pd[wid][lane] = deg;
+    __syncthreads();
+    ssum = 0.0;
+    deg = 0;
+#pragma unroll
+    for (int q = 0; q < FW; ++q) {
+        ssum += ps[q][lane];
+        deg += pd[q][lane];
+    }
+    for (int k = wid; k < len; k += FW) {
         const int64_t e = base + (int64_t)k * SL;
         const int j = scol[e];
         float wv = 0.0f;
@@ -247,6 +265,10 @@ k_lp_features(int N, const int *__restrict__ srow, const int *__restrict__ slice
         }
         w[e] = wv;
     }
+    if (!row || wid != 0) return;
+    double D[9];
+    masked_block(A, nbs, diagpos[i], fi, fi, true, D);
+    const double t = (D[0] + D[4] + D[8]) / 3.0;
     double F[NF];
     F[0] = D[0] / t; F[1] = D[1] / t; F[2] = D[2] / t; F[3] = D[4] / t; F[4] = D[5] / t; F[5] = D[8] / t;
     F[6] = log(t) - *logt_sum / N;
@@ -274,60 +296,78 @@ k_lp_transpose_w(int64_t nbs, const int *__restrict__ tpos, const float *__restr
 // Dense layer on the matrix units.  Y[N][NOUT] = [A1 | A2] W (+ bias), where the
 // input rows are A1[N][K1] | A2[N][K2] (bf16) and W (K x NOUT) is given transposed,
 // Wt[NOUT][K] (bf16).  RELU_BF16: ReLU, bf16 output; otherwise FP32 output.
-// Each wave keeps its B fragments (the whole of W) in registers and walks 16-row
-// tiles with a grid stride.
+// Each wave keeps its fragments of W (the whole of it) in registers and walks 16-row
+// tiles with a grid stride.  The product is formed transposed (W^T times the rows), so a
+// lane ends with four consecutive outputs of one row: one store per 16 outputs.  With a
+// wave or two per SIMD and a tile or two per wave it is bound by the latency of its loads
+// and the number of its requests: 32-deep products where K allows, 16 bytes a load, every
+// fragment of a tile in flight before the first product.  16,641 vertices, 128 to 64:
+// 12.2 us before, 7.5 now; 64 to 128 in FP32 13.3 and 9.3.
 template <int K1, int K2, int NOUT, bool RELU_BF16>
 __global__ void __launch_bounds__(256)
 k_lp_dense(int N, const unsigned short *__restrict__ A1, const unsigned short *__restrict__ A2,
            const unsigned short *__restrict__ Wt, const float *__restrict__ bias, void *__restrict__ Y)
 {
-    constexpr int K = K1 + K2, KB = K / 16, NB = NOUT / 16;
+    constexpr int K = K1 + K2, NB = NOUT / 16;
+    constexpr int KS = (K1 % 32 == 0 && K2 % 32 == 0) ? 32 : 16, KB = K / KS;   // depth of a product
     static_assert(K1 % 16 == 0 && K2 % 16 == 0 && NOUT % 16 == 0, "tile sizes");
+    typedef std::conditional_t<KS == 32, bf16x8, short4v> Frag;
     const int lane = threadIdx.x & 63, q = lane >> 4, c16 = lane & 15;
-    short4v bf[KB][NB];
+    Frag wf[KB][NB];
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            const uint2 v = *reinterpret_cast<const uint2 *>(Wt + (size_t)(nb * 16 + c16) * K + kb * 16 + 4 * q);
-            bf[kb][nb] = short4v{(short)(v.x & 0xFFFFu), (short)(v.x >> 16), (short)(v.y & 0xFFFFu), (short)(v.y >> 16)};
-        }
-    float bv[NB];
+        for (int nb = 0; nb < NB; ++nb)
+            wf[kb][nb] = *reinterpret_cast<const Frag *>(Wt + (size_t)(nb * 16 + c16) * K + kb * KS + (KS / 4) * q);
+    float4v bv[NB];
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) bv[nb] = bias ? bias[nb * 16 + c16] : 0.0f;
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) bv[nb][t] = bias ? bias[nb * 16 + 4 * q + t] : 0.0f;
     const int nwaves = gridDim.x * 4;
     for (int tile = blockIdx.x * 4 + (threadIdx.x >> 6); tile * 16 < N; tile += nwaves) {
-        const int row0 = tile * 16, ar = row0 + c16;
+        // rows past the end read the last one and are not stored
+        const int row = tile * 16 + c16, ar = min(row, N - 1);
+        Frag a[KB];
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+            a[kb] = *reinterpret_cast<const Frag *>((kb * KS < K1) ? A1 + (size_t)K1 * ar + kb * KS + (KS / 4) * q
+                                                                   : A2 + (size_t)K2 * ar + (kb * KS - K1) + (KS / 4) * q);
         float4v acc[NB];
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) acc[nb] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-            uint2 v = make_uint2(0u, 0u);
-            if (ar < N) {
-                const unsigned short *src = (kb * 16 < K1) ? A1 + (size_t)K1 * ar + kb * 16 + 4 * q
-                                                           : A2 + (size_t)K2 * ar + (kb * 16 - K1) + 4 * q;
-                v = *reinterpret_cast<const uint2 *>(src);
-            }
-            const short4v a = short4v{(short)(v.x & 0xFFFFu), (short)(v.x >> 16), (short)(v.y & 0xFFFFu), (short)(v.y >> 16)};
+        for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bf[kb][nb], acc[nb], 0, 0, 0);
+            for (int nb = 0; nb < NB; ++nb) {
+                if constexpr (KS == 32)
+                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[kb][nb], a[kb], acc[nb], 0, 0, 0);
+                else
+                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wf[kb][nb], a[kb], acc[nb], 0, 0, 0);
+            }
+        if (row >= N) continue;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            const float4v y = acc[nb] + bv[nb];
+            const size_t o = (size_t)NOUT * row + nb * 16 + 4 * q;
+            if constexpr (RELU_BF16) {
+                unsigned short b[4];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) b[t] = f2bf(y[t] > 0.f ? y[t] : 0.f);
+                *reinterpret_cast<uint2 *>(static_cast<unsigned short *>(Y) + o) =
+                    make_uint2((unsigned)b[0] | ((unsigned)b[1] << 16), (unsigned)b[2] | ((unsigned)b[3] << 16));
+            } else {
+                *reinterpret_cast<float4v *>(static_cast<float *>(Y) + o) = y;
+            }
         }
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int r = row0 + 4 * q + t, col = nb * 16 + c16;
-                if (r >= N) continue;
-                const float y = acc[nb][t] + bv[nb];
-                if constexpr (RELU_BF16) static_cast<unsigned short *>(Y)[(size_t)NOUT * r + col] = f2bf(y > 0.f ? y : 0.f);
-                else static_cast<float *>(Y)[(size_t)NOUT * r + col] = y;
-            }
     }
 }
 
 // Aggregation a[i] = sum_e w[e] h[col_e] over row i's entries (bf16 in and out,
-// FP32 sums in entry order).  8 threads per row, 8 channels each.
+// FP32 sums in entry order).  8 threads per row, 8 channels each, the weights, columns and
+// rows of AE entries in flight: a gather waits on its column, and the rows are short
+// (16,641 vertices: 11.3 us one entry at a time, 6.5 now).
+constexpr int AE = 4;
 __global__ void __launch_bounds__(RT)
 k_lp_aggregate(int N, const int *__restrict__ srow, const int *__restrict__ slice_off, const int *__restrict__ slen,
                const int *__restrict__ scol, const float *__restrict__ w, const unsigned short *__restrict__ h,
@@ -342,16 +382,27 @@ k_lp_aggregate(int N, const int *__restrict__ srow, const int *__restrict__ slic
     float acc[8];
 #pragma unroll
     for (int c = 0; c < 8; ++c) acc[c] = 0.0f;
-    for (int k = 0; k < len; ++k) {
-        const int64_t e = base + (int64_t)k * SL;
-        const float wv = w[e];
-        if (wv == 0.0f) continue;
-        const uint4 v = *reinterpret_cast<const uint4 *>(h + (size_t)HID * scol[e] + cg);
-        const unsigned vv[4] = {v.x, v.y, v.z, v.w};
+    for (int k = 0; k < len; k += AE) {
+        float wv[AE];
+        int j[AE];
+        uint4 v[AE];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            acc[2 * c] += wv * bf2f((unsigned short)(vv[c] & 0xFFFFu));
-            acc[2 * c + 1] += wv * bf2f((unsigned short)(vv[c] >> 16));
+        for (int u = 0; u < AE; ++u) {
+            const int64_t e = base + (int64_t)min(k + u, len - 1) * SL;
+            wv[u] = k + u < len ? w[e] : 0.0f;
+            j[u] = scol[e];
+        }
+#pragma unroll
+        for (int u = 0; u < AE; ++u) v[u] = *reinterpret_cast<const uint4 *>(h + (size_t)HID * j[u] + cg);
+#pragma unroll
+        for (int u = 0; u < AE; ++u) {
+            if (wv[u] == 0.0f) continue;
+            const unsigned vv[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                acc[2 * c] += wv[u] * bf2f((unsigned short)(vv[c] & 0xFFFFu));
+                acc[2 * c + 1] += wv[u] * bf2f((unsigned short)(vv[c] >> 16));
+            }
         }
     }
     unsigned pk[4];
@@ -449,29 +500,37 @@ k_lp_add_coarse(int N, const double *__restrict__ zc, const double *__restrict__
     if (threadIdx.x == 0) part[blockIdx.x] = t;
 }
 
-// y = A_red x (FP64; fixed rows give 0) in SELL order, partial sums of y.u.
-__global__ void __launch_bounds__(RT)
+// y = A_red x (FP64; fixed rows give 0), partial sums of y.u.  One workgroup per slice,
+// its wavefronts on every fourth entry of each row (as in k_lp_features), a row's four
+// sums added in order.  16,641 vertices: 10.6 us with a thread per row, 6.0 now.
+__global__ void __launch_bounds__(64 * FW)
 k_lp_spmv_dot(int N, const int *__restrict__ srow, const int *__restrict__ slice_off, const int *__restrict__ slen,
               const int *__restrict__ scol, const double *__restrict__ A, int64_t nbs,
               const unsigned char *__restrict__ fixmask, const double *__restrict__ x, double *__restrict__ y,
               const double *__restrict__ u, double *__restrict__ part)
 {
-    __shared__ double s[RT];
-    const int g = blockIdx.x * RT + threadIdx.x;
+    __shared__ double s[FW][3][64];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int g = blockIdx.x * SL + lane;
+    const int64_t base = slice_off[blockIdx.x] + lane;
+    const int len = g < N ? slen[g] : 0;
+    double y0 = 0.0, y1 = 0.0, y2 = 0.0;
+    for (int k = wid; k < len; k += FW) {
+        const int64_t e = base + (int64_t)k * SL;
+        const int j = scol[e];
+        const double u0 = x[3 * j], u1 = x[3 * j + 1], u2 = x[3 * j + 2];
+        y0 += A[0 * nbs + e] * u0 + A[1 * nbs + e] * u1 + A[2 * nbs + e] * u2;
+        y1 += A[3 * nbs + e] * u0 + A[4 * nbs + e] * u1 + A[5 * nbs + e] * u2;
+        y2 += A[6 * nbs + e] * u0 + A[7 * nbs + e] * u1 + A[8 * nbs + e] * u2;
+    }
+    s[wid][0][lane] = y0; s[wid][1][lane] = y1; s[wid][2][lane] = y2;
+    __syncthreads();
+    if (wid != 0) return;
     double acc = 0.0;
     if (g < N) {
+#pragma unroll
+        for (int q = 1; q < FW; ++q) { y0 += s[q][0][lane]; y1 += s[q][1][lane]; y2 += s[q][2][lane]; }
         const int i = srow[g];
-        const int64_t base = slice_off[g / SL] + (g % SL);
-        const int len = slen[g];
-        double y0 = 0.0, y1 = 0.0, y2 = 0.0;
-        for (int k = 0; k < len; ++k) {
-            const int64_t e = base + (int64_t)k * SL;
-            const int j = scol[e];
-            const double u0 = x[3 * j], u1 = x[3 * j + 1], u2 = x[3 * j + 2];
-            y0 += A[0 * nbs + e] * u0 + A[1 * nbs + e] * u1 + A[2 * nbs + e] * u2;
-            y1 += A[3 * nbs + e] * u0 + A[4 * nbs + e] * u1 + A[5 * nbs + e] * u2;
-            y2 += A[6 * nbs + e] * u0 + A[7 * nbs + e] * u1 + A[8 * nbs + e] * u2;
-        }
         const unsigned fm = fixmask[i];
         if (fm & 1) y0 = 0.0;
         if (fm & 2) y1 = 0.0;
@@ -479,8 +538,9 @@ k_lp_spmv_dot(int N, const int *__restrict__ srow, const int *__restrict__ slice
         y[3 * i] = y0; y[3 * i + 1] = y1; y[3 * i + 2] = y2;
         acc = (y0 * u[3 * i] + y1 * u[3 * i + 1]) + y2 * u[3 * i + 2];
     }
-    const double t = block_sum(acc, s);
-    if (threadIdx.x == 0) part[blockIdx.x] = t;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
+    if (lane == 0) part[blockIdx.x] = acc;
 }
 
 __global__ void k_lp_loss(double *scal)
@@ -562,114 +622,181 @@ k_lp_dO(int N, const int *__restrict__ diagpos, const double *__restrict__ A, in
 }
 
 // Output layer backward: dpre = bf16((dO W_out^T) * (h3 > 0)); per-workgroup
-// partials of dW_out = h3^T dO (64 x 6) and db_out (6), stride 390.
+// partials of dW_out = h3^T dO (64 x 6) and db_out (6), stride 390.  64 rows to a
+// workgroup, staged in LDS: four threads a row for dpre, 16 channels each; for the
+// partials a wavefront takes the 64 channels of a quarter of the rows (dO read as
+// broadcasts), and the quarters are added in order.  16,641 vertices: 24 us with 256 rows to a
+// workgroup and a thread per gradient entry, 6.4 now.
+constexpr int OR = 64;
 __global__ void __launch_bounds__(RT)
 k_lp_out_bwd(int N, const unsigned short *__restrict__ h, const unsigned short *__restrict__ Wq,
              const float *__restrict__ dO, unsigned short *__restrict__ dpre, float *__restrict__ part)
 {
     constexpr int NG = HID * NO + NO;   // 390
     constexpr int HP = HID + 2;         // padded LDS row
+    constexpr int NW = RT / 64, CT = HID / (RT / OR);   // wavefronts; channels of a thread
+    static_assert(HID == 64 && HP % 2 == 0 && CT % 8 == 0, "a wavefront spans the channels");
     __shared__ float sW[HID * NO];
-    __shared__ float sd[RT * NO];
-    __shared__ unsigned short sh[RT * HP];
-    for (int k = threadIdx.x; k < HID * NO; k += RT) sW[k] = bf2f(Wq[k]);
-    const int r0 = blockIdx.x * RT;
-    for (int k = threadIdx.x; k < RT * NO; k += RT) {
-        const int r = r0 + k / NO;
-        sd[k] = r < N ? dO[(size_t)NO * r + (k % NO)] : 0.0f;
+    __shared__ float sd[OR * NO];
+    __shared__ unsigned sh2[OR * HP / 2];
+    __shared__ float sg[NW][NG];
+    const unsigned short *sh = reinterpret_cast<const unsigned short *>(sh2);
+    const int r0 = blockIdx.x * OR;
+#pragma unroll
+    for (int k0 = 0; k0 < OR * HID / 8; k0 += RT) {
+        const int k = k0 + threadIdx.x, rr = k / (HID / 8), r = r0 + rr;
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (r < N) v = *reinterpret_cast<const uint4 *>(h + (size_t)HID * r + 8 * (k % (HID / 8)));
+        unsigned *o = sh2 + rr * (HP / 2) + 4 * (k % (HID / 8));
+        o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
     }
-    for (int k = threadIdx.x; k < RT * HID; k += RT) {
-        const int rr = k / HID, r = r0 + rr;
-        sh[rr * HP + (k % HID)] = r < N ? h[(size_t)HID * r + (k % HID)] : (unsigned short)0;
+    for (int k = threadIdx.x; k < HID * NO; k += RT) sW[k] = bf2f(Wq[k]);
+    for (int k = threadIdx.x; k < OR * NO; k += RT) sd[k] = r0 + k / NO < N ? dO[(size_t)NO * r0 + k] : 0.0f;
+    __syncthreads();
+    {
+        const int rr = threadIdx.x / (RT / OR), cb = CT * (threadIdx.x % (RT / OR)), i = r0 + rr;
+        if (i < N) {
+            float d[NO];
+#pragma unroll
+            for (int k = 0; k < NO; ++k) d[k] = sd[NO * rr + k];
+#pragma unroll 1   // (short code: each workgroup fetches it once)
+            for (int c8 = cb; c8 < cb + CT; c8 += 8) {
+                unsigned pk[4];
+#pragma unroll
+                for (int u = 0; u < 8; u += 2) {
+                    float v[2];
+#pragma unroll
+                    for (int w2 = 0; w2 < 2; ++w2) {
+                        const int c = c8 + u + w2;
+                        float acc = 0.f;
+#pragma unroll
+                        for (int k = 0; k < NO; ++k) acc += d[k] * sW[c * NO + k];
+                        v[w2] = bf2f(sh[rr * HP + c]) > 0.f ? acc : 0.f;
+                    }
+                    pk[u >> 1] = (unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16);
+                }
+                *reinterpret_cast<uint4 *>(dpre + (size_t)HID * i + c8) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+            }
+        }
+    }
+    {
+        const int c = threadIdx.x & 63, wid = threadIdx.x >> 6;
+        float aw[NO], ab[NO];
+#pragma unroll
+        for (int k = 0; k < NO; ++k) aw[k] = ab[k] = 0.f;
+#pragma unroll 2
+        for (int rr = wid * (OR / NW); rr < (wid + 1) * (OR / NW); ++rr) {
+            const float hv = bf2f(sh[rr * HP + c]);
+#pragma unroll
+            for (int k = 0; k < NO; ++k) {
+                const float dv = sd[rr * NO + k];
+                aw[k] += hv * dv;
+                ab[k] += dv;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NO; ++k) {
+            sg[wid][c * NO + k] = aw[k];
+            if (c == 0) sg[wid][HID * NO + k] = ab[k];
+        }
     }
     __syncthreads();
-    const int i = r0 + threadIdx.x;
-    if (i < N) {
-        const float *d = sd + NO * threadIdx.x;
-        const unsigned short *hr = sh + threadIdx.x * HP;
-        unsigned short *dst = dpre + (size_t)HID * i;
-        for (int c8 = 0; c8 < HID / 8; ++c8) {
-            unsigned pk[4];
-#pragma unroll
-            for (int u = 0; u < 8; u += 2) {
-                float v[2];
-#pragma unroll
-                for (int w2 = 0; w2 < 2; ++w2) {
-                    const int c = 8 * c8 + u + w2;
-                    float acc = 0.f;
-#pragma unroll
-                    for (int k = 0; k < NO; ++k) acc += d[k] * sW[c * NO + k];
-                    v[w2] = bf2f(hr[c]) > 0.f ? acc : 0.f;
-                }
-                pk[u >> 1] = (unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16);
-            }
-            *reinterpret_cast<uint4 *>(dst + 8 * c8) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-        }
-    }
     for (int g = threadIdx.x; g < NG; g += RT) {
-        float acc = 0.f;
-        if (g < HID * NO) {
-            const int c = g / NO, k = g % NO;
-            for (int rr = 0; rr < RT; ++rr) acc += bf2f(sh[rr * HP + c]) * sd[rr * NO + k];
-        } else {
-            const int k = g - HID * NO;
-            for (int rr = 0; rr < RT; ++rr) acc += sd[rr * NO + k];
-        }
-        part[(size_t)blockIdx.x * NG + g] = acc;
+        float v = sg[0][g];
+#pragma unroll
+        for (int q = 1; q < NW; ++q) v += sg[q][g];
+        part[(size_t)blockIdx.x * NG + g] = v;
     }
 }
 
 // Weight gradient on the matrix units: per workgroup, over its row range,
 //   part[K][NOUT] = [A1 | A2]^T dY   and   part[K * NOUT + n] = sum of dY[:, n],
-// bf16 inputs staged transposed through LDS (64-row tiles), FP32 sums.
+// bf16 inputs staged transposed through LDS (64-row tiles), FP32 sums.  Bound by the
+// latency of its few tiles, so a tile is read in 16-byte pieces, all in flight at once; a
+// thread holds two rows of eight columns, written to LDS as pairs of rows (neighbouring
+// lanes, neighbouring pairs: no conflicts).  The code is kept short (not unrolled over the
+// tile's rows): each workgroup runs it once or twice, and fetching it counts.
+// The column sums are one more product, with ones.  16,641 vertices: 31 us with 2-byte
+// pieces, 22 with the next tile's loads under the products (28 KB of code), 9 now.
 template <int K1, int K2, int NOUT>
 __global__ void __launch_bounds__(256)
 k_lp_wgrad(int N, int rows_per_wg, const unsigned short *__restrict__ A1, const unsigned short *__restrict__ A2,
            const unsigned short *__restrict__ dY, float *__restrict__ part)
 {
     constexpr int K = K1 + K2;
-    constexpr int TR = 64, TP = TR + 4;   // rows per tile, padded LDS row
-    __shared__ unsigned short sA[K * TP];
-    __shared__ unsigned short sD[NOUT * TP];
+    constexpr int TR = 64, TP = TR + 8;   // rows per tile; padded LDS row, a multiple of 16 bytes
+    constexpr int CA = K / 8, CD = NOUT / 8;               // 8-column pieces of a row
+    constexpr int NA = (TR / 2) * CA, ND = (TR / 2) * CD;   // (row pair, piece) items of a tile
+    constexpr int IA = (NA + 255) / 256, ID = (ND + 255) / 256;
+    static_assert((K1 % 64 == 0 && K2 % 64 == 0) || (K2 == 0 && K1 <= 64 && K1 % 8 == 0), "64 columns of one operand to an item");
+    static_assert(NOUT % 64 == 0 && NOUT / 16 == 4, "four column blocks, one per wavefront");
+    __shared__ __align__(16) unsigned short sA[K * TP];
+    __shared__ __align__(16) unsigned short sD[NOUT * TP];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, q = lane >> 4, c16 = lane & 15;
     constexpr int NBLK = (K / 16) * (NOUT / 16);
     constexpr int PER = (NBLK + 3) / 4;
-    float4v acc[PER];
+    float4v acc[PER], bacc = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int p = 0; p < PER; ++p) acc[p] = float4v{0.f, 0.f, 0.f, 0.f};
-    float bacc = 0.0f;
     const int r_begin = blockIdx.x * rows_per_wg;
     const int r_end = min(N, r_begin + rows_per_wg);
+    // item it = u * 256 + threadIdx.x: row pair it % 32, piece it / 32.  Rows past the end
+    // read the last one and count as zero.
+    const int pr = 2 * ((int)threadIdx.x % (TR / 2)), pc = 8 * ((int)threadIdx.x / (TR / 2));
+    const bool on_a = IA > 1 || (int)threadIdx.x < NA;
+    const int kc = on_a ? pc : 0;
+    // the eight columns of a row pair, transposed: column c's pair in one 32-bit store
+    auto put = [&](unsigned short *s, int it, const uint4 (&v)[2]) {
+        const unsigned a[4] = {v[0].x, v[0].y, v[0].z, v[0].w}, b[4] = {v[1].x, v[1].y, v[1].z, v[1].w};
+        unsigned *o = reinterpret_cast<unsigned *>(s) + (8 * (it / (TR / 2)) * TP) / 2 + it % (TR / 2);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            o[(2 * c) * (TP / 2)] = (a[c] & 0xFFFFu) | (b[c] << 16);
+            o[(2 * c + 1) * (TP / 2)] = (a[c] >> 16) | (b[c] & 0xFFFF0000u);
+        }
+    };
     for (int r0 = r_begin; r0 < r_end; r0 += TR) {
-        __syncthreads();
-        for (int idx = threadIdx.x; idx < TR * K; idx += 256) {
-            const int rr = idx / K, kk = idx % K, r = r0 + rr;
-            unsigned short v = 0;
-            if (r < r_end) v = (kk < K1) ? A1[(size_t)K1 * r + kk] : A2[(size_t)K2 * r + (kk - K1)];
-            sA[kk * TP + rr] = v;
-        }
-        for (int idx = threadIdx.x; idx < TR * NOUT; idx += 256) {
-            const int rr = idx / NOUT, n = idx % NOUT, r = r0 + rr;
-            sD[n * TP + rr] = r < r_end ? dY[(size_t)NOUT * r + n] : (unsigned short)0;
-        }
-        __syncthreads();
-        if (threadIdx.x < NOUT) {
-            for (int rr = 0; rr < TR; ++rr) bacc += bf2f(sD[threadIdx.x * TP + rr]);
-        }
+        uint4 va[IA][2], vd[ID][2];
 #pragma unroll
-        for (int p = 0; p < PER; ++p) {
-            const int blk = wave * PER + p;
-            if (blk < NBLK) {
-                const int mb = blk / (NOUT / 16), nb = blk % (NOUT / 16);
+        for (int w = 0; w < 2; ++w) {
+            const int r = r0 + pr + w, rc = min(r, r_end - 1);
 #pragma unroll
-                for (int rb = 0; rb < TR; rb += 16) {
-                    const unsigned short *pa = sA + (mb * 16 + c16) * TP + rb + 4 * q;
-                    const unsigned short *pb = sD + (nb * 16 + c16) * TP + rb + 4 * q;
-                    const short4v a = short4v{(short)pa[0], (short)pa[1], (short)pa[2], (short)pa[3]};
-                    const short4v bb = short4v{(short)pb[0], (short)pb[1], (short)pb[2], (short)pb[3]};
-                    acc[p] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bb, acc[p], 0, 0, 0);
-                }
+            for (int u = 0; u < IA; ++u) {
+                // (64 columns of a wide operand to u: a uniform choice of the operand)
+                const unsigned short *a = (64 * u < K1) ? A1 + (size_t)K1 * rc + 64 * u : A2 + (size_t)K2 * rc + (64 * u - K1);
+                va[u][w] = *reinterpret_cast<const uint4 *>(a + kc);
             }
+#pragma unroll
+            for (int u = 0; u < ID; ++u)
+                vd[u][w] = *reinterpret_cast<const uint4 *>(dY + (size_t)NOUT * rc + 64 * u + pc);
+            if (r >= r_end) {
+#pragma unroll
+                for (int u = 0; u < IA; ++u) va[u][w] = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+                for (int u = 0; u < ID; ++u) vd[u][w] = make_uint4(0u, 0u, 0u, 0u);
+            }
+        }
+        __syncthreads();
+        if (on_a)
+#pragma unroll
+            for (int u = 0; u < IA; ++u) put(sA, u * 256 + threadIdx.x, va[u]);
+#pragma unroll
+        for (int u = 0; u < ID; ++u) put(sD, u * 256 + threadIdx.x, vd[u]);
+        __syncthreads();
+#pragma unroll 1
+        for (int rb = 0; rb < TR; rb += 16) {
+            auto frag = [&](const unsigned short *s, int blk) {
+                return *reinterpret_cast<const short4v *>(s + (blk * 16 + c16) * TP + rb + 4 * q);
+            };
+#pragma unroll
+            for (int p = 0; p < PER; ++p) {
+                const int blk = wave * PER + p;
+                if (blk < NBLK)
+                    acc[p] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(frag(sA, blk / (NOUT / 16)),
+                                                                       frag(sD, blk % (NOUT / 16)), acc[p], 0, 0, 0);
+            }
+            const short one = (short)0x3F80;   // bf16 1
+            bacc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(short4v{one, one, one, one}, frag(sD, wave), bacc, 0, 0, 0);
         }
     }
     float *out = part + (size_t)blockIdx.x * (K * NOUT + NOUT);
@@ -682,7 +809,7 @@ k_lp_wgrad(int N, int rows_per_wg, const unsigned short *__restrict__ A1, const 
             for (int t = 0; t < 4; ++t) out[(size_t)(mb * 16 + 4 * q + t) * NOUT + nb * 16 + c16] = acc[p][t];
         }
     }
-    if (threadIdx.x < NOUT) out[K * NOUT + threadIdx.x] = bacc;
+    if (q == 0) out[K * NOUT + wave * 16 + c16] = bacc[0];   // every row of the product is the sum
 }
 
 // Transposed aggregation for the backward of a message-passing layer:
@@ -703,13 +830,28 @@ k_lp_agg_bwd(int N, const int *__restrict__ srow, const int *__restrict__ slice_
     const float *own = dinp + (size_t)2 * HID * i + cg;
 #pragma unroll
     for (int c = 0; c < 8; ++c) acc[c] = own[c];
-    for (int k = 0; k < len; ++k) {
-        const int64_t e = base + (int64_t)k * SL;
-        const float wv = wT[e];
-        if (wv == 0.0f) continue;
-        const float *src = dinp + (size_t)2 * HID * scol[e] + HID + cg;
+    for (int k = 0; k < len; k += AE) {
+        float wv[AE];
+        int j[AE];
+        float4v v[AE][2];
 #pragma unroll
-        for (int c = 0; c < 8; ++c) acc[c] += wv * src[c];
+        for (int u = 0; u < AE; ++u) {
+            const int64_t e = base + (int64_t)min(k + u, len - 1) * SL;
+            wv[u] = k + u < len ? wT[e] : 0.0f;
+            j[u] = scol[e];
+        }
+#pragma unroll
+        for (int u = 0; u < AE; ++u) {
+            const float4v *src = reinterpret_cast<const float4v *>(dinp + (size_t)2 * HID * j[u] + HID + cg);
+            v[u][0] = src[0];
+            v[u][1] = src[1];
+        }
+#pragma unroll
+        for (int u = 0; u < AE; ++u) {
+            if (wv[u] == 0.0f) continue;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) acc[c] += wv[u] * v[u][c / 4][c % 4];
+        }
     }
     const uint4 hv = *reinterpret_cast<const uint4 *>(h + (size_t)HID * i + cg);
     const unsigned hh[4] = {hv.x, hv.y, hv.z, hv.w};
@@ -723,15 +865,25 @@ k_lp_agg_bwd(int N, const int *__restrict__ srow, const int *__restrict__ slice_
     *reinterpret_cast<uint4 *>(dpre + (size_t)HID * i + cg) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
 }
 
-// out[k] = sum over G partial rows (stride L) of part[g * L + k], in row order.
-__global__ void __launch_bounds__(RT)
+// out[k] = sum over G partial rows (stride L) of part[g * L + k]: 32 columns (one cache
+// line) per workgroup, every 32nd row to a thread, the 32 sums added in order.  Few
+// columns and many rows: a thread per column waited for one load per row
+// (8,256 columns of 131 rows: 32 us before, 4 now).
+constexpr int PC = 32, PG = 32;
+__global__ void __launch_bounds__(PC * PG)
 k_lp_sum_partials(int G, int L, const float *__restrict__ part, float *__restrict__ out)
 {
-    const int k = blockIdx.x * RT + threadIdx.x;
-    if (k >= L) return;
-    float s = 0.0f;
-    for (int g = 0; g < G; ++g) s += part[(size_t)g * L + k];
-    out[k] = s;
+    __shared__ float s[PG][PC + 1];
+    const int c = threadIdx.x % PC, w = threadIdx.x / PC, k = blockIdx.x * PC + c;
+    float v = 0.0f;
+    if (k < L)
+#pragma unroll 4
+        for (int g = w; g < G; g += PG) v += part[(size_t)g * L + k];
+    s[w][c] = v;
+    __syncthreads();
+    if (w != 0 || k >= L) return;
+    for (int q = 1; q < PG; ++q) v += s[q][c];
+    out[k] = v;
 }
 
 // Adam (Kingma & Ba 2015) with bias correction.
@@ -786,6 +938,9 @@ void learned_wgrad_shape(int N, int *G, int *rows)
     *G = (N + per - 1) / per;
 }
 
+int learned_out_groups(int N) { return blocks_for(N, OR); }
+int learned_dot_groups(int N) { return blocks_for(N, SL); }
+
 hipError_t learned_quantize(eolc_ctx *c)
 {
     hipLaunchKernelGGL(k_lp_quantize, dim3(blocks_for(kLqSize)), dim3(RT), 0, c->stream, c->lp.theta, c->lp.wq);
@@ -807,7 +962,7 @@ hipError_t learned_forward(eolc_ctx *c)
     const int nblk = blocks_for(N);
     hipLaunchKernelGGL(k_lp_logt, dim3(nblk), dim3(RT), 0, c->stream, N, c->diagpos, c->A64, t.nbs, c->fixmask, L.dpart);
     hipLaunchKernelGGL(k_lp_reduce, dim3(1), dim3(RT), 0, c->stream, nblk, L.dpart, L.scal + 0);
-    hipLaunchKernelGGL(k_lp_features, dim3(nblk), dim3(RT), 0, c->stream, N, c->srow, c->slice_off, c->slen, c->scol,
+    hipLaunchKernelGGL(k_lp_features, dim3(blocks_for(N, SL)), dim3(64 * FW), 0, c->stream, N, c->srow, c->slice_off, c->slen, c->scol,
                        c->diagpos, c->A64, t.nbs, c->Mval, c->fixmask, L.scal + 0, L.X, L.w);
     hipLaunchKernelGGL(k_lp_transpose_w, dim3(blocks_for(t.nbs)), dim3(RT), 0, c->stream, t.nbs, L.tpos, L.w, L.wT);
     const int dg = dense_grid(N);
@@ -841,13 +996,13 @@ hipError_t learned_loss_grad(eolc_ctx *c)
     LearnedState &L = c->lp;
     const Topology &t = c->topo;
     const int N = t.N;
-    const int nblk = blocks_for(N);
+    const int nblk = blocks_for(N), ndot = learned_dot_groups(N);
     hipError_t err = learned_forward(c);
     if (err != hipSuccess) return err;
     // r = A e (r.e), z = P r (z.r), Az (z.Az), loss
-    hipLaunchKernelGGL(k_lp_spmv_dot, dim3(nblk), dim3(RT), 0, c->stream, N, c->srow, c->slice_off, c->slen, c->scol,
+    hipLaunchKernelGGL(k_lp_spmv_dot, dim3(ndot), dim3(64 * FW), 0, c->stream, N, c->srow, c->slice_off, c->slen, c->scol,
                        c->A64, t.nbs, c->fixmask, L.e, L.r, L.e, L.dpart);
-    hipLaunchKernelGGL(k_lp_reduce, dim3(1), dim3(RT), 0, c->stream, nblk, L.dpart, L.scal + 1);
+    hipLaunchKernelGGL(k_lp_reduce, dim3(1), dim3(RT), 0, c->stream, ndot, L.dpart, L.scal + 1);
     hipLaunchKernelGGL(k_lp_precond, dim3(nblk), dim3(RT), 0, c->stream, N, c->diagpos, c->A64, t.nbs, c->fixmask, L.o,
                        (float *)nullptr, L.r, L.z, L.dpart);
     if (c->ml_on) {
@@ -860,17 +1015,18 @@ hipError_t learned_loss_grad(eolc_ctx *c)
         hipLaunchKernelGGL(k_lp_add_coarse, dim3(nblk), dim3(RT), 0, c->stream, N, c->z64, L.r, L.z, L.dpart);
     }
     hipLaunchKernelGGL(k_lp_reduce, dim3(1), dim3(RT), 0, c->stream, nblk, L.dpart, L.scal + 2);
-    hipLaunchKernelGGL(k_lp_spmv_dot, dim3(nblk), dim3(RT), 0, c->stream, N, c->srow, c->slice_off, c->slen, c->scol,
+    hipLaunchKernelGGL(k_lp_spmv_dot, dim3(ndot), dim3(64 * FW), 0, c->stream, N, c->srow, c->slice_off, c->slen, c->scol,
                        c->A64, t.nbs, c->fixmask, L.z, L.Az, L.z, L.dpart);
-    hipLaunchKernelGGL(k_lp_reduce, dim3(1), dim3(RT), 0, c->stream, nblk, L.dpart, L.scal + 3);
+    hipLaunchKernelGGL(k_lp_reduce, dim3(1), dim3(RT), 0, c->stream, ndot, L.dpart, L.scal + 3);
     hipLaunchKernelGGL(k_lp_loss, dim3(1), dim3(1), 0, c->stream, L.scal);
     // backward
     hipLaunchKernelGGL(k_lp_dO, dim3(nblk), dim3(RT), 0, c->stream, N, c->diagpos, c->A64, t.nbs, c->fixmask, L.o, L.r,
                        L.Az, L.scal, L.dO);
     constexpr int NGO = HID * NO + NO;
-    hipLaunchKernelGGL(k_lp_out_bwd, dim3(nblk), dim3(RT), 0, c->stream, N, L.h[kLpLayers], L.wq + kLqOut, L.dO,
+    const int nout = learned_out_groups(N);
+    hipLaunchKernelGGL(k_lp_out_bwd, dim3(nout), dim3(RT), 0, c->stream, N, L.h[kLpLayers], L.wq + kLqOut, L.dO,
                        L.dpre[0], L.gpart);
-    hipLaunchKernelGGL(k_lp_sum_partials, dim3(blocks_for(NGO)), dim3(RT), 0, c->stream, nblk, NGO, L.gpart,
+    hipLaunchKernelGGL(k_lp_sum_partials, dim3(blocks_for(NGO, PC)), dim3(PC * PG), 0, c->stream, nout, NGO, L.gpart,
                        L.grad + kLpOffOut);
     int Gw, rows;
     learned_wgrad_shape(N, &Gw, &rows);
@@ -880,7 +1036,7 @@ hipError_t learned_loss_grad(eolc_ctx *c)
     for (int l = kLpLayers - 1; l >= 0; --l) {
         hipLaunchKernelGGL((k_lp_wgrad<HID, HID, HID>), dim3(Gw), dim3(256), 0, c->stream, N, rows, L.h[l], L.a[l],
                            L.dpre[cur], L.gpart);
-        hipLaunchKernelGGL(k_lp_sum_partials, dim3(blocks_for(NGL)), dim3(RT), 0, c->stream, Gw, NGL, L.gpart,
+        hipLaunchKernelGGL(k_lp_sum_partials, dim3(blocks_for(NGL, PC)), dim3(PC * PG), 0, c->stream, Gw, NGL, L.gpart,
                            L.grad + kLpOffLayer0 + l * kLpLayerSize);
         // dinp = dpre W_l^T: W_l [128][64] is the transposed operand of this product
         hipLaunchKernelGGL((k_lp_dense<HID, 0, 2 * HID, false>), dim3(dg), dim3(256), 0, c->stream, N, L.dpre[cur],
@@ -893,7 +1049,7 @@ hipError_t learned_loss_grad(eolc_ctx *c)
     constexpr int NGI = NF * HID + HID;
     hipLaunchKernelGGL((k_lp_wgrad<NF, 0, HID>), dim3(Gw), dim3(256), 0, c->stream, N, rows, L.X,
                        (const unsigned short *)nullptr, L.dpre[cur], L.gpart);
-    hipLaunchKernelGGL(k_lp_sum_partials, dim3(blocks_for(NGI)), dim3(RT), 0, c->stream, Gw, NGI, L.gpart,
+    hipLaunchKernelGGL(k_lp_sum_partials, dim3(blocks_for(NGI, PC)), dim3(PC * PG), 0, c->stream, Gw, NGI, L.gpart,
                        L.grad + kLpOffIn);
     return hipGetLastError();
 }

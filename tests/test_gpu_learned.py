@@ -125,6 +125,26 @@ def test_loss_and_gradient_match_oracle(ctx):
         assert rel < 2e-3, name   # measured 2e-5 .. 2e-4
 
 
+@pytest.mark.parametrize("n", [2, 8, 33])
+def test_gradient_at_partial_tiles(ctx, n):
+    """9, 81 and 1,156 vertices: less than a 16-row tile, a 64-row tile and some, many
+    workgroups with a last one of 4 rows.  Tolerance as at 20 x 20: both sides round the
+    activations to bfloat16 (2^-9), a part of which the sums over vertices cancel."""
+    sc = scene.Scene(n, sigma_x=1e-3, sigma_v=0.05)
+    print(f"learned: gradient at {sc.N} vertices", flush=True)
+    setup(ctx, sc)
+    Ar, mass, fixmask, fd = reduced_system(ctx, sc)
+    th = random_theta(5)
+    ctx.learned_set_weights(th)
+    e = np.random.default_rng(9).normal(size=3 * sc.N)
+    e[fd] = 0.0
+    loss, g = ctx.learned_loss_grad(e, fd)
+    lo, go, _ = MO.loss_and_grad(th.astype(np.float64), Ar, mass, sc.N, fixmask, Ar @ e, e, quant=True)
+    rel = np.linalg.norm(g - go) / np.linalg.norm(go)
+    print(f"  loss gpu {loss:.9f} oracle {lo:.9f}, gradient rel err {rel:.2e}", flush=True)
+    assert abs(loss - lo) <= 1e-4 * abs(lo) and rel < 2e-3
+
+
 def test_training_lowers_loss_and_is_deterministic(ctx):
     sc = scene.Scene(24, sigma_x=1e-3, sigma_v=0.05)
     print("learned: 40 Adam steps on one 24x24 system, twice", flush=True)
