@@ -778,7 +778,7 @@ int learned_buffers(eolc_ctx *c)
 // Geometry and set-up chunks of the linear coarse fields (levels >= kMLLinFrom): the
 // centroid, RMS radius and inverse radius of every aggregate in the material
 // coordinates, and per aggregate of those levels its hord range cut into chunks of
-// at most kGal9Rows positions.  A hierarchy whose aggregates are not contiguous in
+// at most gal9_rows(N) positions.  A hierarchy whose aggregates are not contiguous in
 // hord keeps the translations alone (lin_ok false).
 hipError_t ml_prepare_linear(eolc_ctx *c, const std::vector<int> &hord)
 {
@@ -832,17 +832,18 @@ hipError_t ml_prepare_linear(eolc_ctx *c, const std::vector<int> &hord)
             k1[h] = k + 1;
         }
     }
+    const int rows = eolc::gal9_rows(N);
     std::vector<int> chunk, gcp(n_hi + 1, 0);
     if (contiguous) {
         for (int l = l0; l <= L; ++l)
             for (int A = 0; A < lv.n[l]; ++A) {
                 const int h = lv.off[l] - lv.off[l0] + A;
                 gcp[h] = (int)chunk.size() / 4;
-                for (int k = k0[h]; k < k1[h]; k += eolc::kGal9Rows) {
+                for (int k = k0[h]; k < k1[h]; k += rows) {
                     chunk.push_back(l);
                     chunk.push_back(lv.off[l] + A);
                     chunk.push_back(k);
-                    chunk.push_back(std::min(k + eolc::kGal9Rows, k1[h]));
+                    chunk.push_back(std::min(k + rows, k1[h]));
                 }
             }
         gcp[n_hi] = (int)chunk.size() / 4;

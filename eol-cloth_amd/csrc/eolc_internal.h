@@ -230,7 +230,14 @@ struct BatchState {
 // starts at aggregate `off[l]`.
 constexpr int kMLMaxLevels = 8;
 constexpr int kMLLinFrom = 3;     // first level with linear coarse fields
-constexpr int kGal9Rows = 2048;   // hord positions per set-up chunk of a 9 x 9 Galerkin block
+// hord positions per set-up chunk of a 9 x 9 Galerkin block: a workgroup's 256 threads take
+// a row each while that gives a level up to two chunks per CU, several rows on larger
+// meshes (up to 2,048, so that an aggregate's chunk sums stay few)
+inline int gal9_rows(int N)
+{
+    const int r = 256 * ((N + 256 * 512 - 1) / (256 * 512));
+    return r < 2048 ? r : 2048;
+}
 constexpr int kRestrict3Parts = 4;   // restriction workgroups per level-3 aggregate (linear fields)
 constexpr int kCoarse9WG = 512;      // the linear fields' coarse kernel: at most this many aggregates on levels >= 3
 struct MLLevels {
@@ -262,7 +269,7 @@ struct MLState {
     // keeps the translations): per aggregate of every level its centroid in the
     // material coordinates, RMS radius s and 1/s; the Galerkin blocks on the basis
     // phi = (1, (X - c) / s) of each component (9 x 9, upper triangle packed, 45
-    // values) are summed per chunk of at most kGal9Rows hord positions of one
+    // values) are summed per chunk of at most gal9_rows(N) hord positions of one
     // aggregate, then per aggregate, and factored (ml_setup).
     bool lin_built = false;       // the data below built for this hierarchy (on first use)
     std::vector<int> hord_h;      // host copy of hord

@@ -94,9 +94,25 @@ __device__ __forceinline__ void apply_inv(const double *__restrict__ d, double r
     c2 = fma(d[5], r2, fma(d[4], r1, d[2] * r0));
 }
 
-// One thread per level-1 aggregate: V_1[m](a) = sum over a's member rows of the
-// blocks (fixed DOFs masked) whose first common level is <= m + 1, m = 0..L-1;
-// D_1^-1 from V_1[0].
+// The block of entry e with its fixed rows and columns zeroed (loads first: none waits on
+// the masks).
+__device__ __forceinline__ void masked9(const double *__restrict__ A, int64_t nbs, int64_t e, unsigned fi, unsigned fj,
+                                        double (&b)[9])
+{
+#pragma unroll
+    for (int c = 0; c < 9; ++c) b[c] = A[(int64_t)c * nbs + e];
+#pragma unroll
+    for (int c = 0; c < 9; ++c)
+        if (((fi >> (c / 3)) | (fj >> (c % 3))) & 1u) b[c] = 0.0;
+}
+
+// V_1[m](a) = sum over level-1 aggregate a's member rows of the blocks (fixed DOFs masked)
+// whose first common level is <= m + 1, m = 0..L-1; D_1^-1 from V_1[0].  An entry is a
+// chain of dependent loads and an aggregate has about 12 rows of 13: kDiagLanes lanes to
+// an aggregate, a row each, their sums added in a fixed tree.  With a thread to an
+// aggregate 131 x 97 quads ran on four workgroups: 241 us,
+// 30 now; 64 meshes of 32^2 to 96^2 quads 395 and 132; 512^2 quads 385 and 130.
+constexpr int kDiagLanes = 16;
 __global__ void __launch_bounds__(256) k_ml_diag1(MLLevels lv, const int *__restrict__ hord,
                                                   const int *__restrict__ ptr1, const int *__restrict__ gpos,
                                                   const int *__restrict__ slice_off, const int *__restrict__ slen,
@@ -105,15 +121,17 @@ __global__ void __launch_bounds__(256) k_ml_diag1(MLLevels lv, const int *__rest
                                                   const unsigned char *__restrict__ fixmask, double *__restrict__ V,
                                                   double *__restrict__ Dinv)
 {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+    const int a = (int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kDiagLanes);
+    const int sub = threadIdx.x % kDiagLanes;
     const int n1 = lv.n[1], L = lv.L;
-    if (a >= n1) return;
+    if (a >= n1) return;   // all lanes of an aggregate together
     double acc[kML][9];
 #pragma unroll
     for (int m = 0; m < kML; ++m)
 #pragma unroll
         for (int c = 0; c < 9; ++c) acc[m][c] = 0.0;
-    for (int k = ptr1[a]; k < ptr1[a + 1]; ++k) {
+    const int k1 = ptr1[a + 1];
+    for (int k = ptr1[a] + sub; k < k1; k += kDiagLanes) {
         const int i = hord[k];
         const int g = gpos[i];
         const int len = slen[g];
@@ -123,13 +141,8 @@ __global__ void __launch_bounds__(256) k_ml_diag1(MLLevels lv, const int *__rest
             const int e = base + kk * eolc::kSlice;
             const int lm = lam[e];
             if (lm > L) continue;
-            const unsigned fj = fixmask[scol[e]];
             double b[9];
-#pragma unroll
-            for (int c = 0; c < 9; ++c) {
-                const int r = c / 3, s = c % 3;
-                b[c] = (((fi >> r) | (fj >> s)) & 1u) ? 0.0 : A[(int64_t)c * nbs + e];
-            }
+            masked9(A, nbs, e, fi, fixmask[scol[e]], b);
 #pragma unroll
             for (int m = 0; m < kML; ++m)
                 if (m < L && lm <= m + 1)
@@ -141,30 +154,43 @@ __global__ void __launch_bounds__(256) k_ml_diag1(MLLevels lv, const int *__rest
     for (int m = 0; m < kML; ++m)
         if (m < L)
 #pragma unroll
-            for (int c = 0; c < 9; ++c) V[(int64_t)(m * 9 + c) * n1 + a] = acc[m][c];
-    inv_spd3(acc[0], Dinv + 6 * (int64_t)a);
+            for (int c = 0; c < 9; ++c) {
+                double v = acc[m][c];
+#pragma unroll
+                for (int o = kDiagLanes / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kDiagLanes);
+                acc[m][c] = v;
+                if (sub == (9 * m + c) % kDiagLanes) V[(int64_t)(m * 9 + c) * n1 + a] = v;
+            }
+    if (sub == 0) inv_spd3(acc[0], Dinv + 6 * (int64_t)a);
 }
 
-// One thread per level-l aggregate (l >= 2): V_l[m] = sum of the children's V_{l-1}[m]
-// for m >= l - 1; D_l^-1 from V_l[l - 1].
-__global__ void __launch_bounds__(256) k_ml_diagup(int l, MLLevels lv, const int *__restrict__ cptr,
-                                                   double *__restrict__ V, double *__restrict__ Dinv)
+// One wavefront per level-l aggregate (l >= 2), a lane per sum: V_l[m] = sum of the
+// children's V_{l-1}[m] for m >= l - 1; D_l^-1 from V_l[l - 1].  (One thread per aggregate
+// ran a few of them at a time through every sum: 82 us for
+// the three levels of 131 x 97 quads, 14 now.)
+__global__ void __launch_bounds__(64) k_ml_diagup(int l, MLLevels lv, const int *__restrict__ cptr,
+                                                  double *__restrict__ V, double *__restrict__ Dinv)
 {
-    const int A = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ double d[9];
+    const int A = blockIdx.x;
     const int L = lv.L, nl = lv.n[l], nc = lv.n[l - 1];
-    if (A >= nl) return;
     const double *__restrict__ Vc = V + (int64_t)9 * L * lv.off[l - 1];
     double *__restrict__ Vl = V + (int64_t)9 * L * lv.off[l];
     const int c0 = cptr[lv.coff[l] + A], c1 = cptr[lv.coff[l] + A + 1];
-    double d[9];
-    for (int m = l - 1; m < L; ++m)
-        for (int c = 0; c < 9; ++c) {
-            double s = 0.0;
-            for (int a = c0; a < c1; ++a) s += Vc[(int64_t)(m * 9 + c) * nc + a];
-            Vl[(int64_t)(m * 9 + c) * nl + A] = s;
-            if (m == l - 1) d[c] = s;
-        }
-    inv_spd3(d, Dinv + 6 * (int64_t)(lv.off[l] + A));
+    for (int t = 9 * (l - 1) + (int)threadIdx.x; t < 9 * L; t += 64) {
+        double s = 0.0;
+#pragma unroll 4
+        for (int a = c0; a < c1; ++a) s += Vc[(int64_t)t * nc + a];
+        Vl[(int64_t)t * nl + A] = s;
+        if (t < 9 * l) d[t - 9 * (l - 1)] = s;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double v[9];
+#pragma unroll
+        for (int c = 0; c < 9; ++c) v[c] = d[c];
+        inv_spd3(v, Dinv + 6 * (int64_t)(lv.off[l] + A));
+    }
 }
 
 // Upper triangle of a symmetric 9 x 9 block, row by row: 45 entries.
@@ -246,6 +272,7 @@ __device__ __forceinline__ void apply9(const double *__restrict__ F, const doubl
 // sum over the chunk's rows i and their entries (i, j) inside g (first common level
 // <= l) of phi(i) phi(j)^T (x) A_ij, fixed DOFs masked, in the aggregate's basis;
 // the upper triangle (45 sums) in a fixed order per thread, then over the workgroup.
+// 131 x 97 quads: 177 us in chunks of 2,048 rows, 37 in chunks of 256.
 constexpr int kGalWG = 256;
 __global__ void __launch_bounds__(kGalWG) k_ml_gal9_part(const int *__restrict__ gchunk, const int *__restrict__ hord,
                                                          const int *__restrict__ gpos,
@@ -278,11 +305,7 @@ __global__ void __launch_bounds__(kGalWG) k_ml_gal9_part(const int *__restrict__
             const unsigned fj = fixmask[j];
             const double pj[3] = {1.0, (X[2 * (int64_t)j] - cu) * is, (X[2 * (int64_t)j + 1] - cv) * is};
             double b[9];
-#pragma unroll
-            for (int c = 0; c < 9; ++c) {
-                const int r = c / 3, t = c % 3;
-                b[c] = (((fi >> r) | (fj >> t)) & 1u) ? 0.0 : A[(int64_t)c * nbs + e];
-            }
+            masked9(A, nbs, e, fi, fj, b);
 #pragma unroll
             for (int p = 0; p < 9; ++p)
 #pragma unroll
@@ -304,18 +327,22 @@ __global__ void __launch_bounds__(kGalWG) k_ml_gal9_part(const int *__restrict__
     }
 }
 
-// One thread per aggregate of levels >= 3: its chunks' sums in order, then the
-// block's factors.
+// One wavefront per aggregate of levels >= 3: its chunks' sums in order, a lane per
+// value, then the block's factors.
 __global__ void __launch_bounds__(64) k_ml_gal9_fin(int n_hi, const int *__restrict__ gcp,
                                                     const double *__restrict__ gpart, double *__restrict__ D9)
 {
-    const int h = blockIdx.x * 64 + threadIdx.x;
-    if (h >= n_hi) return;
-    double G[45];
-    for (int p = 0; p < 45; ++p) G[p] = 0.0;
-    for (int ch = gcp[h]; ch < gcp[h + 1]; ++ch)
-        for (int p = 0; p < 45; ++p) G[p] += gpart[45 * (int64_t)ch + p];
-    fact9_psd(G, D9 + h, n_hi);
+    __shared__ double sG[45];
+    const int h = blockIdx.x, p = threadIdx.x;
+    if (p < 45) {
+        const int c1 = gcp[h + 1];
+        double v = 0.0;
+#pragma unroll 8
+        for (int ch = gcp[h]; ch < c1; ++ch) v += gpart[45 * (int64_t)ch + p];
+        sG[p] = v;
+    }
+    __syncthreads();
+    if (p == 0) fact9_psd(sG, D9 + h, n_hi);
 }
 
 // Ordering of LDS traffic between the lanes of one wavefront (no workgroup barrier:
@@ -1003,16 +1030,16 @@ hipError_t ml_setup(eolc_ctx *c, bool linear)
     m.lin_on = false;
     if (lv.L <= 0) return hipSuccess;
     const Topology &t = c->topo;
-    hipLaunchKernelGGL(k_ml_diag1, dim3(blocks_for(lv.n[1])), dim3(256), 0, c->stream, lv, m.hord, m.ptr1, m.gpos,
+    hipLaunchKernelGGL(k_ml_diag1, dim3(blocks_for((int64_t)lv.n[1] * kDiagLanes)), dim3(256), 0, c->stream, lv, m.hord, m.ptr1, m.gpos,
                        c->slice_off, c->slen, c->scol, m.lam, c->A64, t.nbs, c->fixmask, m.V, m.Dinv);
     for (int l = 2; l <= lv.L; ++l)
-        hipLaunchKernelGGL(k_ml_diagup, dim3(blocks_for(lv.n[l])), dim3(256), 0, c->stream, l, lv, m.cptr, m.V,
+        hipLaunchKernelGGL(k_ml_diagup, dim3(lv.n[l]), dim3(64), 0, c->stream, l, lv, m.cptr, m.V,
                            m.Dinv);
     if (linear && m.lin_ok) {
         const int n_hi = lv.off[lv.L + 1] - lv.off[kMLLinFrom];
         hipLaunchKernelGGL(k_ml_gal9_part, dim3(m.nchunks), dim3(kGalWG), 0, c->stream, m.gchunk, m.hord, m.gpos,
                            c->slice_off, c->slen, c->scol, m.lam, c->A64, t.nbs, c->fixmask, c->X, m.geo, m.gpart);
-        hipLaunchKernelGGL(k_ml_gal9_fin, dim3(blocks_for(n_hi, 64)), dim3(64), 0, c->stream, n_hi, m.gcp, m.gpart,
+        hipLaunchKernelGGL(k_ml_gal9_fin, dim3(n_hi), dim3(64), 0, c->stream, n_hi, m.gcp, m.gpart,
                            m.D9);
         m.lin_on = true;
     }
