@@ -125,60 +125,6 @@ void make_box(BoxGeom &B, const double *whd, const double *E1 /* column-major 4x
     }
 }
 
-// Device memory of one collide call.  Heap mode (base == nullptr): every buffer is
-// a hipMalloc, freed when the call ends or at release().  Arena mode: buffers are
-// carved in order, 256-byte aligned, from a fixed region (the scratch array of
-// eolc_collide_noalloc); release() rewinds to a mark, and no allocation is made.
-// Reuse after a rewind is safe because every kernel runs on the context's one
-// stream and every host read of a released buffer has been synchronised.
-struct Workspace {
-    char *base = nullptr;
-    size_t cap = 0, used = 0, peak = 0;
-    bool exhausted = false;
-    std::vector<void *> owned;
-    Workspace() = default;
-    Workspace(const Workspace &) = delete;
-    Workspace &operator=(const Workspace &) = delete;
-    ~Workspace()
-    {
-        for (void *p : owned) (void)hipFree(p);
-    }
-    template <class T> hipError_t get(T **p, size_t n)
-    {
-        const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
-        if (!base) {
-            void *q = nullptr;
-            const hipError_t e = hipMalloc(&q, bytes);
-            if (e == hipSuccess) {
-                owned.push_back(q);
-                *p = static_cast<T *>(q);
-            }
-            return e;
-        }
-        const size_t off = (used + 255) & ~(size_t)255;
-        if (off > cap || bytes > cap - off) {
-            exhausted = true;
-            return hipErrorOutOfMemory;
-        }
-        *p = reinterpret_cast<T *>(base + off);
-        used = off + bytes;
-        peak = std::max(peak, used);
-        return hipSuccess;
-    }
-    size_t mark() const { return base ? used : owned.size(); }
-    void release(size_t m)
-    {
-        if (base) {
-            used = m;
-            return;
-        }
-        while (owned.size() > m) {
-            (void)hipFree(owned.back());
-            owned.pop_back();
-        }
-    }
-};
-
 }  // namespace
 
 namespace eolc {
@@ -273,7 +219,7 @@ struct CdStatus {
 };
 
 // The queries against the uniform grid over the cloth faces.
-int query_grid(eolc_ctx *c, Workspace &ws, double thr, int Q, const double *qpts, const double *qnrm, const double *xj,
+int query_grid(eolc_ctx *c, eolc::Workspace &ws, double thr, int Q, const double *qpts, const double *qnrm, const double *xj,
                const double *fn, const double *aabb, eolc_collision *qrec)
 {
     const int F = c->topo.F;
@@ -300,7 +246,7 @@ int query_grid(eolc_ctx *c, Workspace &ws, double thr, int Q, const double *qpts
     const unsigned tbl = grid_table_size(F);
     g.mask = tbl - 1;
     g.cond_max = kGridCondMax;
-    const size_t m = ws.mark();
+    const eolc::Workspace::Mark m = ws.mark();
     unsigned *bcnt = nullptr, *bstart = nullptr, *cursor = nullptr, *total = nullptr, *nalways = nullptr, *sums = nullptr;
     int *always = nullptr, *entries = nullptr;
     EOLC_HIP(ws.get(&bcnt, tbl));
@@ -320,11 +266,11 @@ int query_grid(eolc_ctx *c, Workspace &ws, double thr, int Q, const double *qpts
     EOLC_HIP(ws.get(&entries, nentries));
     EOLC_HIP(eolc::cd_grid_build(c, g, xj, bcnt, bstart, cursor, entries, nalways, always, sums, total, true));
     EOLC_HIP(eolc::cd_query(c, g, Q, qpts, qnrm, thr, aabb, xj, fn, bstart, bcnt, entries, nalways, always, qrec));
-    if (ws.base) ws.release(m);   // (the kernels of this stream are done with it before the next ones start)
+    if (ws.arena) ws.release(m);   // (the kernels of this stream are done with it before the next ones start)
     return EOLC_OK;
 }
 
-int collide_impl(eolc_ctx *c, Workspace &ws, double thr, int P, const double *pts, const double *nrm, int B,
+int collide_impl(eolc_ctx *c, eolc::Workspace &ws, double thr, int P, const double *pts, const double *nrm, int B,
                  const double *whd, const double *Eb, int eol_points, int box_npts, int box_nedges,
                  std::vector<eolc_collision> &out)
 {
@@ -423,7 +369,7 @@ int collide_impl(eolc_ctx *c, Workspace &ws, double thr, int P, const double *pt
         EOLC_HIP(hipMemcpyAsync(&ne, offs + N, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
         EOLC_HIP(hipStreamSynchronize(c->stream));
         if (ne) {
-            const size_t m = ws.mark();
+            const eolc::Workspace::Mark m = ws.mark();
             eolc_collision *o = nullptr;
             EOLC_HIP(ws.get(&o, ne));
             out.resize(ne);
@@ -458,10 +404,10 @@ int collide_impl(eolc_ctx *c, Workspace &ws, double thr, int P, const double *pt
         // the group's records, box after box, vertices before edges: in one piece, or box by
         // box where a fixed workspace has no room for all
         recs.resize(st.first[2 * nb]);
-        const size_t m = ws.mark();
+        const eolc::Workspace::Mark m = ws.mark();
         eolc_collision *o = nullptr;
         const bool whole = recs.empty() || ws.get(&o, recs.size()) == hipSuccess;
-        if (!whole && !ws.base) EOLC_HIP(hipErrorOutOfMemory);
+        if (!whole && !ws.arena) EOLC_HIP(hipErrorOutOfMemory);
         if (!whole) ws.exhausted = false;
         for (int b = 0; b < nb; b += whole ? nb : 1) {
             const int b1 = whole ? nb : b + 1;
@@ -497,7 +443,7 @@ int collide_impl(eolc_ctx *c, Workspace &ws, double thr, int P, const double *pt
             } else {
                 std::vector<int> amb((size_t)E);
                 int *eamb = nullptr;
-                const size_t ma = ws.mark();
+                const eolc::Workspace::Mark ma = ws.mark();
                 EOLC_HIP(ws.get(&eamb, (size_t)E));
                 EOLC_HIP(eolc::cd_ambiguous(c, thr, dbox + b, xj, eamb));
                 EOLC_HIP(hipMemcpyAsync(amb.data(), eamb, sizeof(int) * (size_t)E, hipMemcpyDeviceToHost, c->stream));
@@ -580,7 +526,7 @@ try {
     }
     EOLC_HIP(hipSetDevice(c->device));
     std::vector<eolc_collision> recs;
-    Workspace ws;   // heap mode: device buffers allocated for this call
+    eolc::Workspace ws(c->kept);   // the context's block, and device buffers allocated for this call
     int rc = collide_impl(c, ws, threshold, P, pts, nrm, B, whd, E, eol_points, box_npts, box_nedges, recs);
     if (rc) return rc;
     *count = (int)recs.size();
@@ -625,9 +571,7 @@ try {
     void *base = nullptr;
     EOLC_HIP(eolc::collide_scratch(c->device, &base));
     std::lock_guard<std::mutex> lk(*eolc::collide_scratch_lock(c->device));
-    Workspace ws;
-    ws.base = static_cast<char *>(base);
-    ws.cap = eolc::kCollideScratchBytes;
+    eolc::Workspace ws(static_cast<char *>(base), eolc::kCollideScratchBytes);
     std::vector<eolc_collision> recs;
     int rc = collide_impl(c, ws, threshold, P, pts, nrm, B, whd, E, eol_points, box_npts, box_nedges, recs);
     if (ws.exhausted) {

@@ -123,6 +123,7 @@ void free_topology_buffers(eolc_ctx *c)
     c->bj_iters_hint = c->bj_iters_hint_ml = 0;
     c->fp64_sticky = 0;
     c->alloc_bytes = 0;
+    c->kept.give_back();
 }
 
 void free_learned_weights(eolc_ctx *c)

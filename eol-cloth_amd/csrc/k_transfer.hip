@@ -293,9 +293,10 @@ struct Events {
 };
 
 template <class T> struct DevBuf {
+    eolc::Workspace &ws;
     T *p = nullptr;
-    hipError_t alloc(size_t n) { return hipMalloc((void **)&p, std::max<size_t>(n, 1) * sizeof(T)); }
-    ~DevBuf() { if (p) (void)hipFree(p); }
+    explicit DevBuf(eolc::Workspace &w) : ws(w) {}
+    hipError_t alloc(size_t n) { return ws.get(&p, n); }
 };
 
 }  // namespace
@@ -324,8 +325,10 @@ hipError_t velocity_transfer(eolc_ctx *c, int n_old, const double *u_old, const 
     g.nx = std::max(1, (int)std::ceil(w / s)) + 1;
     g.ny = std::max(1, (int)std::ceil(h / s)) + 1;
     const int ncell = g.nx * g.ny;
-    DevBuf<double> du_old, dv_old, du_new, dv_new, dbary;
-    DevBuf<int> dtri, vcnt, vstart, vslot, vlist, fcnt, fstart, fslot, flist, totals, dsrc, dface, dmiss;
+    Workspace ws(c->kept);
+    DevBuf<double> du_old(ws), dv_old(ws), du_new(ws), dv_new(ws), dbary(ws);
+    DevBuf<int> dtri(ws), vcnt(ws), vstart(ws), vslot(ws), vlist(ws), fcnt(ws), fstart(ws), fslot(ws), flist(ws),
+        totals(ws), dsrc(ws), dface(ws), dmiss(ws);
     hipError_t e;
 #define TRY(x) do { if ((e = (x)) != hipSuccess) return e; } while (0)
     TRY(du_old.alloc(2 * (size_t)n_old)); TRY(dv_old.alloc(3 * (size_t)n_old));
@@ -339,8 +342,8 @@ hipError_t velocity_transfer(eolc_ctx *c, int n_old, const double *u_old, const 
     TRY(hipMemcpyAsync(dv_old.p, v_old, 3 * (size_t)n_old * sizeof(double), hipMemcpyHostToDevice, st));
     TRY(hipMemcpyAsync(du_new.p, u_new, 2 * (size_t)n_new * sizeof(double), hipMemcpyHostToDevice, st));
     TRY(hipMemcpyAsync(dtri.p, tri_old, 3 * (size_t)f_old * sizeof(int), hipMemcpyHostToDevice, st));
-    DevBuf<double> dx_old, dV;
-    DevBuf<int> deidx;
+    DevBuf<double> dx_old(ws), dV(ws);
+    DevBuf<int> deidx(ws);
     if (eol_old) {
         TRY(dx_old.alloc(3 * (size_t)n_old)); TRY(deidx.alloc(n_old)); TRY(dV.alloc(2 * (size_t)n_eol));
         TRY(hipMemcpyAsync(dx_old.p, x_old, 3 * (size_t)n_old * sizeof(double), hipMemcpyHostToDevice, st));

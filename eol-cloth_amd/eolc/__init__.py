@@ -416,15 +416,17 @@ class Context:
         Es = _d(Es)
         P, B = pts.size // 3, whd.size // 3
         while True:
-            buf = (CollisionRec * cap)()
+            # (not zeroed, and only the records that the call wrote are copied)
+            raw = np.empty(max(cap, 1) * C.sizeof(CollisionRec), dtype=np.uint8)
             cnt = C.c_int(0)
             rc = fn(self._h, float(threshold), P, _ptr(pts), _ptr(nrm), B, _ptr(whd),
                     _ptr(Es), int(bool(eol_points)), int(box_npts), int(box_nedges),
-                    buf, cap, C.byref(cnt))
+                    raw.ctypes.data_as(C.POINTER(CollisionRec)), cap, C.byref(cnt))
             if rc == ERR_OVERFLOW and cnt.value > cap:
                 cap = cnt.value
                 continue
             self._check(rc)
+            buf = (CollisionRec * cnt.value).from_buffer_copy(raw)
             return [buf[i] for i in range(cnt.value)]
 
     def set_mixed_stall(self, first_cycle=10000, min_cycle=1000, sticky=8):

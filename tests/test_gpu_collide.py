@@ -238,3 +238,35 @@ def test_sweep_list_overflow_takes_the_grid(ctx):
     print(f"{len(g)} records", flush=True)
     assert len(g) == len(o) == P
     assert all(rec_tuple(a) == rec_tuple(b) for a, b in zip(g, o))
+
+
+@pytest.mark.parametrize("order", [(0, 6, 1, 6, 0, 2), (6, 6, 6)])
+def test_calls_that_share_the_kept_block(ctx, order):
+    """Queries of different sizes after one another on one topology (the context's block
+    grows, then holds less than it could), a velocity transfer between them: every call's
+    records are those of a context that makes this call alone."""
+    sc, pts, nrm, whd, E = thin_box_scene(24, 1e-3)
+    x, thr = sc.x0, 5e-3
+
+    def on(c):
+        c.set_topology(sc.X, sc.tri, sc.hinge)
+        c.upload_state(x, np.zeros_like(x))
+        return c
+
+    def call(c, nb):
+        return [rec_tuple(r) for r in c.collide(thr, pts, nrm, whd[:nb], E[:nb])]
+
+    want = {}
+    for nb in set(order):
+        with eolc.Context(0) as c:
+            want[nb] = call(on(c), nb)
+    assert len(want[max(order)]) > 0
+    on(ctx)
+    new = np.random.default_rng(4).uniform(0.05, 0.95, (500, 2)) * sc.X.max(axis=0)
+    moved = None
+    for k, nb in enumerate(order):
+        print(f"kept block: call {k}, {nb} boxes", flush=True)
+        assert call(ctx, nb) == want[nb]
+        got = ctx.velocity_transfer(sc.X, sc.v0, sc.tri, new)[1]
+        assert moved is None or np.array_equal(got, moved)
+        moved = got
