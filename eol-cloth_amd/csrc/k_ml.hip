@@ -673,6 +673,96 @@ __global__ void __launch_bounds__(kRestrict3WG) k_ml_restrict3(RestrictArgs g, V
 // in LDS and only C_3 is written out.  Larger hierarchies loop over global memory.
 constexpr int kCoarseWG = 1024;
 constexpr int kCoarseLds = 1024;
+
+// The levels >= 3, at most one aggregate to a thread of the workgroup: C_l of aggregate
+// off[3] + j in Cl[3 j ..], visible to all; false: the solve has stopped.
+__device__ __forceinline__ bool coarse_levels(const MLLevels &lv, const int *__restrict__ cptr,
+                                              const int *__restrict__ par, const double *__restrict__ Dinv,
+                                              const double *__restrict__ R, const SolverScalars *scal, int check_done,
+                                              double *__restrict__ Rl, double *__restrict__ Cl)
+{
+    // one aggregate per thread: its inverse block, parent and child range are
+    // loaded up front (with level 3's children sums), then every phase runs in LDS
+    const int L = lv.L, base = lv.off[3], M = lv.off[L + 1] - base;
+    const int j = threadIdx.x;
+    int l = 0, pa = 0, c0 = 0, c1 = 0, offm1 = 0, offp1 = 0;
+    double d[6] = {0, 0, 0, 0, 0, 0};
+    if (j < M) {
+        // the level and its neighbours' offsets from constant indices into the
+        // arguments (scalar loads; a variable index costs a vector load per use)
+        l = 3;
+        int offl = lv.off[3], coffl = lv.coff[3];
+        offm1 = lv.off[2];
+        offp1 = lv.off[4];
+#pragma unroll
+        for (int k = 4; k <= eolc::kMLMaxLevels; ++k)
+            if (k <= L && j >= lv.off[k] - base) {   // offsets increase with the level
+                l = k;
+                offl = lv.off[k];
+                coffl = lv.coff[k];
+                offm1 = lv.off[k - 1];
+                offp1 = lv.off[k + 1];
+            }
+        const int a = j - (offl - base);
+        const int64_t g = base + j;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) d[k] = Dinv[6 * g + k];
+        if (l < L) pa = par[g];
+        c0 = cptr[coffl + a];
+        c1 = cptr[coffl + a + 1];
+    }
+    // the stop flag is read with the first loads (uniform: every thread leaves
+    // before the first barrier, or none does)
+    if (check_done && scal->done) return false;
+    if (j < M) {
+        if (l == 3) {
+            const double *src = R + 3 * (int64_t)lv.off[2];
+            double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+            for (int b = c0; b < c1; b += 8) {   // children in order, 8 loads in flight
+                double v[8][3];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const bool ok = b + u < c1;
+                    const double *q = src + 3 * (ok ? b + u : c0);
+                    v[u][0] = ok ? q[0] : 0.0;
+                    v[u][1] = ok ? q[1] : 0.0;
+                    v[u][2] = ok ? q[2] : 0.0;
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    s0 += v[u][0]; s1 += v[u][1]; s2 += v[u][2];
+                }
+            }
+            Rl[3 * j] = s0; Rl[3 * j + 1] = s1; Rl[3 * j + 2] = s2;
+        }
+    }
+    __syncthreads();
+    for (int lev = 4; lev <= L; ++lev) {
+        if (j < M && l == lev) {
+            const int cb = offm1 - base;   // level lev - 1
+            double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+            for (int b = c0; b < c1; ++b) {
+                s0 += Rl[3 * (cb + b)]; s1 += Rl[3 * (cb + b) + 1]; s2 += Rl[3 * (cb + b) + 2];
+            }
+            Rl[3 * j] = s0; Rl[3 * j + 1] = s1; Rl[3 * j + 2] = s2;
+        }
+        __syncthreads();
+    }
+    for (int lev = L; lev >= 3; --lev) {
+        if (j < M && l == lev) {
+            double e0, e1, e2;
+            apply_inv(d, Rl[3 * j], Rl[3 * j + 1], Rl[3 * j + 2], e0, e1, e2);
+            if (lev < L) {
+                const int up = offp1 - base + pa;   // the parent on level lev + 1
+                e0 += Cl[3 * up]; e1 += Cl[3 * up + 1]; e2 += Cl[3 * up + 2];
+            }
+            Cl[3 * j] = e0; Cl[3 * j + 1] = e1; Cl[3 * j + 2] = e2;
+        }
+        __syncthreads();
+    }
+    return true;
+}
+
 __global__ void __launch_bounds__(kCoarseWG) k_ml_coarse(MLLevels lv, const int *__restrict__ cptr,
                                                          const int *__restrict__ par, const double *__restrict__ Dinv,
                                                          double *__restrict__ R, double *__restrict__ C,
@@ -683,89 +773,9 @@ __global__ void __launch_bounds__(kCoarseWG) k_ml_coarse(MLLevels lv, const int 
     const int base = lv.off[3];
     const int M = lv.off[L + 1] - base;   // aggregates of levels >= 3
     if (M <= kCoarseWG) {
-        // one aggregate per thread: its inverse block, parent and child range are
-        // loaded up front (with level 3's children sums), then every phase runs in LDS
-        double *Rl = lds, *Cl = lds + 3 * kCoarseLds;
-        const int j = threadIdx.x;
-        int l = 0, pa = 0, c0 = 0, c1 = 0, offm1 = 0, offp1 = 0;
-        double d[6] = {0, 0, 0, 0, 0, 0};
-        if (j < M) {
-            // the level and its neighbours' offsets from constant indices into the
-            // arguments (scalar loads; a variable index costs a vector load per use)
-            l = 3;
-            int offl = lv.off[3], coffl = lv.coff[3];
-            offm1 = lv.off[2];
-            offp1 = lv.off[4];
-#pragma unroll
-            for (int k = 4; k <= eolc::kMLMaxLevels; ++k)
-                if (k <= L && j >= lv.off[k] - base) {   // offsets increase with the level
-                    l = k;
-                    offl = lv.off[k];
-                    coffl = lv.coff[k];
-                    offm1 = lv.off[k - 1];
-                    offp1 = lv.off[k + 1];
-                }
-            const int a = j - (offl - base);
-            const int64_t g = base + j;
-#pragma unroll
-            for (int k = 0; k < 6; ++k) d[k] = Dinv[6 * g + k];
-            if (l < L) pa = par[g];
-            c0 = cptr[coffl + a];
-            c1 = cptr[coffl + a + 1];
-        }
-        // the stop flag is read with the first loads (uniform: every thread leaves
-        // before the first barrier, or none does)
-        if (check_done && scal->done) return;
-        if (j < M) {
-            if (l == 3) {
-                const double *src = R + 3 * (int64_t)lv.off[2];
-                double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-                for (int b = c0; b < c1; b += 8) {   // children in order, 8 loads in flight
-                    double v[8][3];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) {
-                        const bool ok = b + u < c1;
-                        const double *q = src + 3 * (ok ? b + u : c0);
-                        v[u][0] = ok ? q[0] : 0.0;
-                        v[u][1] = ok ? q[1] : 0.0;
-                        v[u][2] = ok ? q[2] : 0.0;
-                    }
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) {
-                        s0 += v[u][0]; s1 += v[u][1]; s2 += v[u][2];
-                    }
-                }
-                Rl[3 * j] = s0; Rl[3 * j + 1] = s1; Rl[3 * j + 2] = s2;
-            }
-        }
-        __syncthreads();
-        for (int lev = 4; lev <= L; ++lev) {
-            if (j < M && l == lev) {
-                const int cb = offm1 - base;   // level lev - 1
-                double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-                for (int b = c0; b < c1; ++b) {
-                    s0 += Rl[3 * (cb + b)]; s1 += Rl[3 * (cb + b) + 1]; s2 += Rl[3 * (cb + b) + 2];
-                }
-                Rl[3 * j] = s0; Rl[3 * j + 1] = s1; Rl[3 * j + 2] = s2;
-            }
-            __syncthreads();
-        }
-        for (int lev = L; lev >= 3; --lev) {
-            if (j < M && l == lev) {
-                double e0, e1, e2;
-                apply_inv(d, Rl[3 * j], Rl[3 * j + 1], Rl[3 * j + 2], e0, e1, e2);
-                if (lev < L) {
-                    const int up = offp1 - base + pa;   // the parent on level lev + 1
-                    e0 += Cl[3 * up]; e1 += Cl[3 * up + 1]; e2 += Cl[3 * up + 2];
-                }
-                Cl[3 * j] = e0; Cl[3 * j + 1] = e1; Cl[3 * j + 2] = e2;
-            }
-            __syncthreads();
-        }
-        if (j < M && l == 3) {
-            double *o = C + 3 * ((int64_t)base + j);
-            o[0] = Cl[3 * j]; o[1] = Cl[3 * j + 1]; o[2] = Cl[3 * j + 2];
-        }
+        double *Cl = lds + 3 * kCoarseLds;
+        if (!coarse_levels(lv, cptr, par, Dinv, R, scal, check_done, lds, Cl)) return;
+        for (int t = threadIdx.x; t < 3 * lv.n[3]; t += kCoarseWG) C[3 * (int64_t)base + t] = Cl[t];
         return;
     }
     if (check_done && scal->done) return;
@@ -838,19 +848,22 @@ __global__ void __launch_bounds__(kCoarseWG) k_ml_coarse(MLLevels lv, const int 
 // by one and a level's factors applied after the other, 11.2 now with one workgroup, 9.0
 // with six; 512^2 8.4 and 5.4; a dozen aggregates 3.8 either way.
 using eolc::kCoarse9WG;
-__global__ void __launch_bounds__(kCoarse9WG) k_ml_coarse9(MLLevels lv, const int *__restrict__ cptr,
-                                                           const int *__restrict__ par, const double *__restrict__ geo,
-                                                           const double *__restrict__ D9, const double *__restrict__ R9p,
-                                                           double *__restrict__ C9, const SolverScalars *scal,
-                                                           int check_done)
+
+// One aggregate of the levels >= 3 to a thread (W threads, at least as many): the fields
+// of the level-3 aggregates [own0, own1), and of every one above, in sC[9 h ..], visible
+// to all; false: the solve has stopped.  LDS: sT and sC 9 values an aggregate, sg 4, sc 2.
+template <int W>
+__device__ __forceinline__ bool coarse9_levels(const MLLevels &lv, const int *__restrict__ cptr,
+                                               const int *__restrict__ par, const double *__restrict__ geo,
+                                               const double *__restrict__ D9, const double *__restrict__ R9p,
+                                               const SolverScalars *scal, int check_done, int own0, int own1,
+                                               double *__restrict__ sT, double *__restrict__ sC,
+                                               double *__restrict__ sg, int *__restrict__ sc)
 {
-    __shared__ double sT[9 * kCoarse9WG], sC[9 * kCoarse9WG], sg[4 * kCoarse9WG];
-    __shared__ int sc[2 * kCoarse9WG];
     const int L = lv.L, base = lv.off[3];
     const int M = lv.off[L + 1] - base, n3 = lv.n[3];
     const int h = threadIdx.x;   // this thread's aggregate (levels >= 3 concatenated)
-    // this workgroup's 64 of level 3, and every aggregate above
-    const bool mine = h >= n3 || h / 64 == (int)blockIdx.x;
+    const bool mine = h >= n3 || (h >= own0 && h < own1);
     // Every load is issued before the first wait, without branches between them (clamped
     // indexes).  The level and the offsets of its neighbour levels come from the uniform
     // offsets with constant indices (scalar loads; a variable index reads the argument
@@ -888,7 +901,7 @@ __global__ void __launch_bounds__(kCoarse9WG) k_ml_coarse9(MLLevels lv, const in
     // the children and the parent as threads
     const int c0 = offm1 - base + ca, c1 = offm1 - base + cz;
     const int hp = l < L ? offp1 - base + pp : 0;
-    if (check_done && scal->done) return;
+    if (check_done && scal->done) return false;
     if (h < M) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) sg[4 * h + k] = g4[k];
@@ -923,7 +936,7 @@ __global__ void __launch_bounds__(kCoarse9WG) k_ml_coarse9(MLLevels lv, const in
         }
         __syncthreads();
         const int p0 = lv.off[lev] - base;
-        for (int t = h; t < 9 * lv.n[lev]; t += kCoarse9WG) {
+        for (int t = h; t < 9 * lv.n[lev]; t += W) {
             const int p = p0 + t / 9, q = t % 9, e = sc[2 * p + 1];
             double v = 0.0;
 #pragma unroll 4
@@ -945,8 +958,21 @@ __global__ void __launch_bounds__(kCoarse9WG) k_ml_coarse9(MLLevels lv, const in
         }
         __syncthreads();
     }
-    const int t0 = 9 * 64 * blockIdx.x, t1 = min(t0 + 9 * 64, 9 * n3);
-    for (int t = t0 + (int)threadIdx.x; t < t1; t += kCoarse9WG) C9[t] = sC[t];
+    return true;
+}
+
+__global__ void __launch_bounds__(kCoarse9WG) k_ml_coarse9(MLLevels lv, const int *__restrict__ cptr,
+                                                           const int *__restrict__ par, const double *__restrict__ geo,
+                                                           const double *__restrict__ D9, const double *__restrict__ R9p,
+                                                           double *__restrict__ C9, const SolverScalars *scal,
+                                                           int check_done)
+{
+    __shared__ double sT[9 * kCoarse9WG], sC[9 * kCoarse9WG], sg[4 * kCoarse9WG];
+    __shared__ int sc[2 * kCoarse9WG];
+    // this workgroup's 64 of level 3
+    const int own0 = 64 * blockIdx.x, own1 = min(own0 + 64, lv.n[3]);
+    if (!coarse9_levels<kCoarse9WG>(lv, cptr, par, geo, D9, R9p, scal, check_done, own0, own1, sT, sC, sg, sc)) return;
+    for (int t = 9 * own0 + (int)threadIdx.x; t < 9 * own1; t += kCoarse9WG) C9[t] = sC[t];
 }
 
 // z = D0 r + coarse correction (zero on fixed DOFs); r.z partials -> PB[parity] slot 0.
@@ -1017,6 +1043,71 @@ k_ml_prolong(int parity, int N, MLLevels lv, const int *__restrict__ agg1, const
     write_partials<1, W>(v, PB(partials, parity), lds);
 }
 
+// The prolongation of a small mesh, a vertex to a thread, with the levels >= 3 formed by
+// every workgroup for itself: the same operations as the coarse kernels, so the same z, a
+// launch less and most of its latency hidden.  131 x 97 quads, mixed: 3.8 us and 4.0 in two
+// kernels, 4.9 in one.
+constexpr int kFusedCoarse = 64, kFusedLinear = 40;
+template <class T, bool LIN>
+__global__ void __launch_bounds__(eolc::kVecWG)
+k_ml_prolong_coarse(int parity, int N, MLLevels lv, const int *__restrict__ agg1, const int *__restrict__ anc3,
+                    const int *__restrict__ cptr, const int *__restrict__ par, const double *__restrict__ geo,
+                    const double *__restrict__ D9, const double *__restrict__ R9p, const double *__restrict__ Dinv,
+                    const double *__restrict__ R, const double *__restrict__ C, const T *__restrict__ D,
+                    const T *__restrict__ r, T *__restrict__ z, const unsigned char *__restrict__ fixmask,
+                    const SolverScalars *scal, double *partials, int check_done, const double *__restrict__ feat3)
+{
+    constexpr int W = eolc::kVecWG, K = kFusedCoarse;
+    __shared__ double lds[2 * (W / 64) + 2];
+    __shared__ double sT[9 * K], sC[9 * K], sg[4 * K];
+    __shared__ int sc[2 * K];
+    int rb, re;
+    wg_rows(N, &rb, &re);
+    const int i = rb + (int)threadIdx.x;
+    const bool on = i < re;
+    // the vertex's own values are on their way while the levels are formed
+    int a = 0, u = 0;
+    double gu = 0.0, gv = 0.0;
+    T rv[3] = {0, 0, 0}, f[3] = {0, 0, 0};
+    unsigned fm = 0;
+    if (on) {
+        a = agg1[i];
+        u = anc3[i];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) rv[c] = r[3 * i + c];
+        fm = fixmask[i];
+        if (LIN) {
+            gu = feat3[2 * (int64_t)i];
+            gv = feat3[2 * (int64_t)i + 1];
+        }
+    }
+    double c[3] = {0, 0, 0};
+    if (on) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) c[k] = C[3 * a + k];
+        eolc::apply_sym3<T>(D + i, N, rv[0], rv[1], rv[2], f[0], f[1], f[2]);
+    }
+    if (LIN) {
+        if (!coarse9_levels<W>(lv, cptr, par, geo, D9, R9p, scal, check_done, 0, lv.n[3], sT, sC, sg, sc)) return;
+    } else {
+        if (!coarse_levels(lv, cptr, par, Dinv, R, scal, check_done, sT, sC)) return;
+    }
+    double v[1] = {0.0};
+    if (on) {
+        const double *P = sC + (LIN ? 9 : 3) * (u - lv.off[3]);
+        T zv[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            if (LIN) c[k] += fma(gv, P[6 + k], fma(gu, P[3 + k], P[k]));
+            else c[k] += P[k];
+            zv[k] = ((fm >> k) & 1u) ? (T)0 : (T)((double)f[k] + c[k]);
+            z[3 * i + k] = zv[k];
+        }
+        v[0] = ((double)rv[0] * (double)zv[0] + (double)rv[1] * (double)zv[1]) + (double)rv[2] * (double)zv[2];
+    }
+    write_partials<1, W>(v, PB(partials, parity), lds);
+}
+
 inline int blocks_for(int64_t n, int t = 256) { return (int)((n + t - 1) / t); }
 
 }  // namespace
@@ -1056,10 +1147,22 @@ int ml_restrict_grid(const eolc_ctx *c)
     return std::min((blocks_for((int64_t)64 * waves, kRestrictWG) + 7) & ~7, kRestrictGrid);
 }
 
+// The prolongation forms the levels >= 3 where a vertex kernel has 256 threads a workgroup
+// and these levels hold few aggregates: every workgroup reads all their factors.  Steps of
+// n^2 quads, two kernels and one (ms): linear fields 48: 3.83 3.51, 131: 6.11 5.52, 200: 8.53
+// 7.93, 300 (37 aggregates): 16.1 15.5, 380 (57): 27.5 29.0; translations, whose factors are a
+// ninth, 131: 6.00 5.55, 300: 22.4 21.8, 380: 40.0 39.1.
+static bool ml_fused(const eolc_ctx *c)
+{
+    const MLLevels &lv = c->ml.lv;
+    return lv.L >= 3 && lv.off[lv.L + 1] - lv.off[3] <= (ml_linear_on(c) ? kFusedLinear : kFusedCoarse) && vec_wg(c->topo.N) == kVecWG;
+}
+
 // The restriction (with the vector update when there is one) and the coarse levels, with
-// the linear fields when the last ml_setup formed them.
+// the linear fields when the last ml_setup formed them; fused: without the coarse levels,
+// which the prolongation forms.
 template <class T>
-static void ml_coarse_chain(eolc_ctx *c, T *r, int parity, const MLUpdate *u)
+static void ml_coarse_chain(eolc_ctx *c, T *r, int parity, const MLUpdate *u, bool fused = false)
 {
     const MLState &m = c->ml;
     const MLLevels &lv = m.lv;
@@ -1071,13 +1174,14 @@ static void ml_coarse_chain(eolc_ctx *c, T *r, int parity, const MLUpdate *u)
     if (ml_linear_on(c)) {
         if (u) hipLaunchKernelGGL((k_ml_restrict3<T, true>), grid, dim3(kRestrict3WG), 0, c->stream, g, up);
         else hipLaunchKernelGGL((k_ml_restrict3<T, false>), grid, dim3(kRestrict3WG), 0, c->stream, g, up);
-        hipLaunchKernelGGL(k_ml_coarse9, dim3(blocks_for(lv.n[3], 64)), dim3(kCoarse9WG), 0, c->stream, lv, m.cptr, m.par, m.geo, m.D9,
+        if (!fused)
+            hipLaunchKernelGGL(k_ml_coarse9, dim3(blocks_for(lv.n[3], 64)), dim3(kCoarse9WG), 0, c->stream, lv, m.cptr, m.par, m.geo, m.D9,
                            m.R9p, m.C9, c->scal, u != nullptr);
         return;
     }
     if (u) hipLaunchKernelGGL((k_ml_restrict<T, true>), grid, dim3(kRestrictWG), 0, c->stream, g, up);
     else hipLaunchKernelGGL((k_ml_restrict<T, false>), grid, dim3(kRestrictWG), 0, c->stream, g, up);
-    if (lv.L >= 3)
+    if (lv.L >= 3 && !fused)
         hipLaunchKernelGGL(k_ml_coarse, dim3(1), dim3(kCoarseWG), 0, c->stream, lv, m.cptr, m.par, m.Dinv, m.R, m.C,
                            c->scal, u != nullptr);
 }
@@ -1099,15 +1203,31 @@ static void launch_prolong(eolc_ctx *c, int parity, const T *D, const T *r, T *z
     else go(std::integral_constant<int, WG>());
 }
 
+template <class T>
+static void launch_prolong_coarse(eolc_ctx *c, int parity, const T *D, const T *r, T *z, int check_done)
+{
+    const MLState &m = c->ml;
+    const int N = c->topo.N;
+    auto go = [&](auto lin) {
+        hipLaunchKernelGGL((k_ml_prolong_coarse<T, decltype(lin)::value>), dim3(vec_grid(N)), dim3(kVecWG), 0, c->stream,
+                           parity, N, m.lv, m.agg1, m.anc3, m.cptr, m.par, m.geo, m.D9, m.R9p, m.Dinv, m.R, m.C, D, r, z,
+                           c->fixmask, c->scal, c->partials, check_done, m.feat3);
+    };
+    if (ml_linear_on(c)) go(std::true_type());
+    else go(std::false_type());
+}
+
 hipError_t ml_apply(eolc_ctx *c, bool mixed, int parity, const MLUpdate *u)
 {
-    if (mixed) {
-        ml_coarse_chain<float>(c, c->r32, parity, u);
-        launch_prolong<float, true>(c, parity, c->D32, c->r32, c->z32, u != nullptr);
-    } else {
-        ml_coarse_chain<double>(c, c->r64, parity, u);
-        launch_prolong<double, true>(c, parity, c->D64, c->r64, c->z64, u != nullptr);
-    }
+    const bool fused = ml_fused(c);
+    auto apply = [&](const auto *D, auto *r, auto *z) {
+        using T = std::remove_pointer_t<decltype(r)>;
+        ml_coarse_chain<T>(c, r, parity, u, fused);
+        if (fused) launch_prolong_coarse<T>(c, parity, D, r, z, u != nullptr);
+        else launch_prolong<T, true>(c, parity, D, r, z, u != nullptr);
+    };
+    if (mixed) apply(c->D32, c->r32, c->z32);
+    else apply(c->D64, c->r64, c->z64);
     return hipGetLastError();
 }
 

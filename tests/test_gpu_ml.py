@@ -228,12 +228,13 @@ def test_multilevel_edge_cases(ctx, case):
         assert np.array_equal(v[fd], out[0][fd])
 
 
-@pytest.mark.parametrize("small", [40, 70])
-def test_linear_fields_of_many_sheets(ctx, small):
-    """A sheet with four levels beside 40 or 70 that end earlier, so that level 3 holds
-    fewer and more than 64 aggregates and the level above more than 512 / 9: P r with
-    linear fields on the levels >= 3 against the oracle."""
-    print(f"linear fields, one large and {small} small sheets", flush=True)
+@pytest.mark.parametrize("small", [15, 20, 28, 31, 40, 70])
+def test_coarse_levels_of_many_sheets(ctx, small):
+    """A sheet with four levels beside some that end earlier: P r with linear fields on the
+    levels >= 3 and with translations against the oracle.  These levels hold 35 to 145
+    aggregates (the prolongation forms up to 40 and 64 of them itself), level 3 fewer and
+    more than 64, the level above more than 512 / 9."""
+    print(f"coarse levels, one large and {small} small sheets", flush=True)
     parts = [scene.Scene(90 if k == 0 else 6, sigma_x=1e-3, sigma_v=0.05, seed_x=7 + k, seed_v=90 + k)
              for k in range(small + 1)]
     off = np.concatenate([[0], np.cumsum([p.N for p in parts])])
@@ -250,13 +251,14 @@ def test_linear_fields_of_many_sheets(ctx, small):
     ctx.forces_fill(GRAV, H)
     counts = ctx.ml_info()
     print(f"  aggregates per level {counts}", flush=True)
-    assert len(counts) >= 5 and (counts[3] > 64) == (small > 64) and counts[4] >= small
+    assert len(counts) == 5 and counts[3:] == [small + 4, small + 1]
     A = ctx.download_csr(eolc.MAT_MDK).tocsr()
     maps = [ctx.ml_aggregates(l) for l in range(1, len(counts))]
     r = np.random.default_rng(3).normal(size=3 * N)
-    ctx.set_ml_linear(2)
-    z = ctx.precond_apply(r, fd, mode=eolc.SOLVE_FP64_BJ | MLF)
-    ctx.set_ml_linear(1)
-    zref = ML.apply(A, N, maps, r, fd, X=X)
-    print(f"  P r rel err {rel_err(z, zref):.2e}", flush=True)
-    assert rel_err(z, zref) <= 1e-12 and np.all(z[fd] == 0.0)
+    for linear in (True, False):
+        ctx.set_ml_linear(2 if linear else 1)
+        z = ctx.precond_apply(r, fd, mode=eolc.SOLVE_FP64_BJ | MLF)
+        ctx.set_ml_linear(1)
+        zref = ML.apply(A, N, maps, r, fd, X=X if linear else None)
+        print(f"  linear {linear}: P r rel err {rel_err(z, zref):.2e}", flush=True)
+        assert rel_err(z, zref) <= 1e-12 and np.all(z[fd] == 0.0)
