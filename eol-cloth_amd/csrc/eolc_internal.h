@@ -623,7 +623,7 @@ std::string ml_build(const Topology &t, std::vector<std::vector<int>> &agg_level
                      std::vector<int> &ptr1, std::vector<int> &agg1, std::vector<int> &cptr, std::vector<int> &par,
                      std::vector<unsigned char> &lam, MLLevels &lv);
 hipError_t ml_setup(eolc_ctx *c, bool linear = true);         // Galerkin diagonal blocks of every level
-// The vector update of iteration k that the restriction does first: p_new, q (of the
+// The vector update of iteration k, r in the restriction and x in the prolongation: p_new, q (of the
 // residual's type) and the solution, and the partials of p.q.
 struct MLUpdate {
     int k, Ga;

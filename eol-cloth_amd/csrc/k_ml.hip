@@ -365,16 +365,18 @@ __device__ __forceinline__ void wave_sync()
 constexpr int kRestrictWG = 128;
 constexpr int kStageRows = 256;
 
-// The PCG's vector update x += alpha p, r -= alpha q, done by the restriction as it
-// reads r (UPD): the residual is written once and read once, and a launch is saved.
-// The members of an aggregate are a compact patch of the sheet, so their scattered
-// 12- and 24-byte pieces share most cache lines.
+// The PCG's residual update r -= alpha q, done by the restriction as it reads r (UPD): the
+// residual is written once and read once, and a launch is saved.  The members of an
+// aggregate are a compact patch of the sheet, so their scattered pieces share most cache
+// lines; still they cost more than a pass in row order does, and far more on a renumbered
+// mesh, so x += alpha p is left to the prolongation, which goes over the rows in order
+// (restriction + prolongation, us, before and now: 22,000 remeshed
+// vertices in FP64 24.6 + 6.7 and 18.1 + 7.0, 1024^2 mixed 50.5 + 19.0 and 38.3 + 29.6, 512^2
+// 20.0 + 6.9 and 16.9 + 10.0; a renumbered 700^2 step 158 and 129 ms).
 template <class T> struct VecUpdate {
-    const T *p, *q;
-    double *x;
+    const T *q;
     T *r;
-    T alphaT;
-    double alpha;
+    T alpha;
 };
 
 __device__ __forceinline__ void lift9(const double *__restrict__ q, double al, double bu, double bv, double *sm)
@@ -450,8 +452,7 @@ __device__ __forceinline__ void restrict_wave(const MLLevels &lv, int w, const i
             }
             // (the compiler otherwise issues the features' loads after the gathers below)
             if (LIN) asm volatile("" ::: "memory");
-            T pv[NC][3], qv[NC][3], rv[NC][3];
-            double xv[NC][3];
+            T qv[NC][3], rv[NC][3];
 #pragma unroll
             for (int c = 0; c < NC; ++c)
                 if (kb + 64 * c + lane < k1)
@@ -459,11 +460,7 @@ __device__ __forceinline__ void restrict_wave(const MLLevels &lv, int w, const i
                     for (int d = 0; d < 3; ++d) {
                         const int64_t j = 3 * (int64_t)i[c] + d;
                         rv[c][d] = up.r[j];
-                        if (UPD) {
-                            qv[c][d] = up.q[j];
-                            pv[c][d] = up.p[j];
-                            xv[c][d] = up.x[j];
-                        }
+                        if (UPD) qv[c][d] = up.q[j];
                     }
 #pragma unroll
             for (int c = 0; c < NC; ++c)
@@ -473,9 +470,8 @@ __device__ __forceinline__ void restrict_wave(const MLLevels &lv, int w, const i
                     for (int d = 0; d < 3; ++d) {
                         if (UPD) {
                             const int64_t j = 3 * (int64_t)i[c] + d;
-                            rv[c][d] = fma(-up.alphaT, qv[c][d], rv[c][d]);
+                            rv[c][d] = fma(-up.alpha, qv[c][d], rv[c][d]);
                             up.r[j] = rv[c][d];
-                            up.x[j] = fma(up.alpha, (double)pv[c][d], xv[c][d]);
                         }
                         q[d] = (double)rv[c][d];
                         srr += q[d] * q[d];
@@ -545,8 +541,8 @@ __device__ __forceinline__ void restrict_wave(const MLLevels &lv, int w, const i
 }
 
 // What the two restriction kernels share.  In an iteration (UPD) alpha = r.z / p.q from
-// the partials of the product (Ga) and of the prolongation (Gz), and the stop on
-// p.q <= 0.  Every workgroup leaves its r.r in PB[parity].
+// the partials of the product (Ga) and of the prolongation (Gz), left in the scalars for
+// the prolongation, and the stop on p.q <= 0.  Every workgroup leaves its r.r in PB[parity].
 struct RestrictArgs {
     MLLevels lv;
     const int *hord, *ptr1, *cptr, *kptr2;
@@ -575,12 +571,12 @@ __device__ __forceinline__ bool restrict_alpha(const RestrictArgs &g, VecUpdate<
         }
         return false;
     }
-    up.alpha = rz / pq;
-    up.alphaT = (T)up.alpha;
+    const double alpha = rz / pq;
+    up.alpha = (T)alpha;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         scal->iters = g.k + 1;
         scal->pq = pq;
-        scal->alpha = up.alpha;
+        scal->alpha = alpha;
     }
     return true;
 }
@@ -610,12 +606,12 @@ __global__ void __launch_bounds__(kRestrictWG) k_ml_restrict(RestrictArgs g, Vec
 // first moments are re-expressed on U's basis, (R_2, alpha M_1 + beta_u R_2, alpha
 // M_2 + beta_v R_2) with alpha = s_w / s_U and beta = (c_w - c_U) / s_U, summed per
 // wavefront in child order and over the workgroup's wavefronts in order: one partial
-// R9 per workgroup, which the coarse kernel adds in order.  With the vector update, FP32
-// (us; the update and the restriction apart before): 131 x 97 quads 9.0 (4.4 + 8.3),
-// 512^2 19.3 (9.3 + 16.5), 1024^2 48.4 (22.3 + 25.9), a launch less each.  There it is
-// bound by the scattered pieces (122 MB in all, less than half of the card's rate): 54 us
-// without the workgroups in XCD order, the same with 64 to 256 members staged at once,
-// which is worth 1 us at 131 x 97 and 5 in the translations' kernel on a renumbered mesh.
+// R9 per workgroup, which the coarse kernel adds in order.  With the residual update, FP32
+// (us): 131 x 97 quads 8.7, 512^2 16.9, 1024^2 38.3.  There it is bound by the scattered
+// pieces and its chain of dependent rounds (59 MB of vectors): slower without the
+// workgroups in XCD order, the same with 128 or 256 members staged at once and with four
+// wavefronts per SIMD instead of three; with eight parts to an aggregate it takes 15.0 at
+// 512^2 but 47.7 at 1024^2, and the coarse kernel twice as long.
 constexpr int kRestrict3WG = 256;
 using eolc::kRestrict3Parts;
 template <class T, bool UPD>
@@ -978,6 +974,7 @@ __global__ void __launch_bounds__(kCoarse9WG) k_ml_coarse9(MLLevels lv, const in
 // z = D0 r + coarse correction (zero on fixed DOFs); r.z partials -> PB[parity] slot 0.
 // Levels 1 and 2 are applied here, per vertex, from the restricted sums; levels >= 3
 // arrive accumulated in C_3.
+// In an iteration (x given) x += alpha p too, with the restriction's alpha.
 // FINE = false: the coarse corrections alone (z_i = C(a_i) + C_3), for the learned
 // blocks' training loss, whose fine term is the network's.
 template <class T, bool FINE, int W>
@@ -986,7 +983,8 @@ k_ml_prolong(int parity, int N, MLLevels lv, const int *__restrict__ agg1, const
              const double *__restrict__ Dinv, const double *__restrict__ R, const double *__restrict__ C,
              const T *__restrict__ D, const T *__restrict__ r, T *__restrict__ z,
              const unsigned char *__restrict__ fixmask, const SolverScalars *scal, double *partials, int check_done,
-             const double *__restrict__ feat3, const double *__restrict__ C9)
+             const double *__restrict__ feat3, const double *__restrict__ C9, const T *__restrict__ p,
+             double *__restrict__ x)
 {
     __shared__ double lds[2 * (W / 64) + 2];
     int rb, re;
@@ -1000,6 +998,7 @@ k_ml_prolong(int parity, int N, MLLevels lv, const int *__restrict__ agg1, const
         if (lv.L >= 3) u = anc3[i0];
     }
     if (check_done && scal->done) return;
+    const double alpha = x ? scal->alpha : 0.0;
     double srz = 0.0;
     for (int i = i0; i < re; i += W) {
         if (i != i0) {
@@ -1026,6 +1025,9 @@ k_ml_prolong(int parity, int N, MLLevels lv, const int *__restrict__ agg1, const
             apply_inv(Dinv + 6 * (int64_t)a, R[3 * a], R[3 * a + 1], R[3 * a + 2], c0, c1, c2);
         }
         const T r0 = r[3 * i], r1 = r[3 * i + 1], r2 = r[3 * i + 2];
+        if (x)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) x[3 * (int64_t)i + c] = fma(alpha, (double)p[3 * (int64_t)i + c], x[3 * (int64_t)i + c]);
         double g0 = 0.0, g1 = 0.0, g2 = 0.0;
         if constexpr (FINE) {
             T f0, f1, f2;
@@ -1055,7 +1057,8 @@ k_ml_prolong_coarse(int parity, int N, MLLevels lv, const int *__restrict__ agg1
                     const double *__restrict__ D9, const double *__restrict__ R9p, const double *__restrict__ Dinv,
                     const double *__restrict__ R, const double *__restrict__ C, const T *__restrict__ D,
                     const T *__restrict__ r, T *__restrict__ z, const unsigned char *__restrict__ fixmask,
-                    const SolverScalars *scal, double *partials, int check_done, const double *__restrict__ feat3)
+                    const SolverScalars *scal, double *partials, int check_done, const double *__restrict__ feat3,
+                    const T *__restrict__ p, double *__restrict__ x)
 {
     constexpr int W = eolc::kVecWG, K = kFusedCoarse;
     __shared__ double lds[2 * (W / 64) + 2];
@@ -1068,9 +1071,16 @@ k_ml_prolong_coarse(int parity, int N, MLLevels lv, const int *__restrict__ agg1
     // the vertex's own values are on their way while the levels are formed
     int a = 0, u = 0;
     double gu = 0.0, gv = 0.0;
-    T rv[3] = {0, 0, 0}, f[3] = {0, 0, 0};
+    T rv[3] = {0, 0, 0}, f[3] = {0, 0, 0}, pv[3];
+    double xv[3];
     unsigned fm = 0;
     if (on) {
+        if (x)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                pv[c] = p[3 * i + c];
+                xv[c] = x[3 * i + c];
+            }
         a = agg1[i];
         u = anc3[i];
 #pragma unroll
@@ -1094,6 +1104,11 @@ k_ml_prolong_coarse(int parity, int N, MLLevels lv, const int *__restrict__ agg1
     }
     double v[1] = {0.0};
     if (on) {
+        if (x) {
+            const double alpha = scal->alpha;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) x[3 * i + k] = fma(alpha, (double)pv[k], xv[k]);
+        }
         const double *P = sC + (LIN ? 9 : 3) * (u - lv.off[3]);
         T zv[3];
 #pragma unroll
@@ -1168,8 +1183,7 @@ static void ml_coarse_chain(eolc_ctx *c, T *r, int parity, const MLUpdate *u, bo
     const MLLevels &lv = m.lv;
     RestrictArgs g{lv,    m.hord, m.ptr1, m.cptr, m.kptr2, m.R, m.C,     m.Dinv, m.feat2,
                    m.geo, m.R9p,  c->scal, c->partials, u ? u->k : 0, u ? u->Ga : 0, vec_grid(c->topo.N), parity};
-    VecUpdate<T> up{u ? static_cast<const T *>(u->p) : nullptr, u ? static_cast<const T *>(u->q) : nullptr,
-                    u ? u->x : nullptr, r, (T)0, 0.0};
+    VecUpdate<T> up{u ? static_cast<const T *>(u->q) : nullptr, r, (T)0};
     const dim3 grid(ml_restrict_grid(c));
     if (ml_linear_on(c)) {
         if (u) hipLaunchKernelGGL((k_ml_restrict3<T, true>), grid, dim3(kRestrict3WG), 0, c->stream, g, up);
@@ -1188,7 +1202,7 @@ static void ml_coarse_chain(eolc_ctx *c, T *r, int parity, const MLUpdate *u, bo
 
 // The prolongation on the vector kernels' grid (vec_wg, vec_grid).
 template <class T, bool FINE>
-static void launch_prolong(eolc_ctx *c, int parity, const T *D, const T *r, T *z, int check_done)
+static void launch_prolong(eolc_ctx *c, int parity, const T *D, const T *r, T *z, const MLUpdate *u)
 {
     const MLState &m = c->ml;
     const MLLevels &lv = m.lv;
@@ -1197,21 +1211,23 @@ static void launch_prolong(eolc_ctx *c, int parity, const T *D, const T *r, T *z
     auto go = [&](auto w) {
         constexpr int W = decltype(w)::value;
         hipLaunchKernelGGL((k_ml_prolong<T, FINE, W>), dim3(vec_grid(N)), dim3(W), 0, c->stream, parity, N, lv, m.agg1,
-                           m.anc3, m.Dinv, m.R, m.C, D, r, z, c->fixmask, c->scal, c->partials, check_done, m.feat3, c9);
+                           m.anc3, m.Dinv, m.R, m.C, D, r, z, c->fixmask, c->scal, c->partials, u != nullptr, m.feat3, c9,
+                           u ? static_cast<const T *>(u->p) : nullptr, u ? u->x : nullptr);
     };
     if (vec_wg(N) == kVecWG) go(std::integral_constant<int, kVecWG>());
     else go(std::integral_constant<int, WG>());
 }
 
 template <class T>
-static void launch_prolong_coarse(eolc_ctx *c, int parity, const T *D, const T *r, T *z, int check_done)
+static void launch_prolong_coarse(eolc_ctx *c, int parity, const T *D, const T *r, T *z, const MLUpdate *u)
 {
     const MLState &m = c->ml;
     const int N = c->topo.N;
     auto go = [&](auto lin) {
         hipLaunchKernelGGL((k_ml_prolong_coarse<T, decltype(lin)::value>), dim3(vec_grid(N)), dim3(kVecWG), 0, c->stream,
                            parity, N, m.lv, m.agg1, m.anc3, m.cptr, m.par, m.geo, m.D9, m.R9p, m.Dinv, m.R, m.C, D, r, z,
-                           c->fixmask, c->scal, c->partials, check_done, m.feat3);
+                           c->fixmask, c->scal, c->partials, u != nullptr, m.feat3,
+                           u ? static_cast<const T *>(u->p) : nullptr, u ? u->x : nullptr);
     };
     if (ml_linear_on(c)) go(std::true_type());
     else go(std::false_type());
@@ -1223,8 +1239,8 @@ hipError_t ml_apply(eolc_ctx *c, bool mixed, int parity, const MLUpdate *u)
     auto apply = [&](const auto *D, auto *r, auto *z) {
         using T = std::remove_pointer_t<decltype(r)>;
         ml_coarse_chain<T>(c, r, parity, u, fused);
-        if (fused) launch_prolong_coarse<T>(c, parity, D, r, z, u != nullptr);
-        else launch_prolong<T, true>(c, parity, D, r, z, u != nullptr);
+        if (fused) launch_prolong_coarse<T>(c, parity, D, r, z, u);
+        else launch_prolong<T, true>(c, parity, D, r, z, u);
     };
     if (mixed) apply(c->D32, c->r32, c->z32);
     else apply(c->D64, c->r64, c->z64);
@@ -1236,7 +1252,7 @@ hipError_t ml_coarse64(eolc_ctx *c)
 {
     if (c->ml.lv.L <= 0) return hipMemsetAsync(c->z64, 0, sizeof(double) * 3 * (size_t)c->topo.N, c->stream);
     ml_coarse_chain<double>(c, c->r64, 0, nullptr);
-    launch_prolong<double, false>(c, 0, c->D64, c->r64, c->z64, 0);
+    launch_prolong<double, false>(c, 0, c->D64, c->r64, c->z64, nullptr);
     return hipGetLastError();
 }
 

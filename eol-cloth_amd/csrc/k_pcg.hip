@@ -1446,8 +1446,10 @@ int fp64_layout(int variant)
 }
 
 // The vector kernels take 256 threads a workgroup while 1,024 would leave compute units
-// idle (fewer than 256 workgroups).
-int vec_wg(int N) { return pcg_grid(N) < 256 ? kVecWG : WG; }
+// idle, or give a second workgroup to only a few of the 256: mixed multilevel steps of
+// n^2 quads with 256 and 1,024 threads, ms: 512 (264 workgroups of 1,024) 42.3 and 43.8, 570
+// (320) 46.4 and 45.3, 640 (400) 60.0 and 58.1.
+int vec_wg(int N) { return pcg_grid(N) <= 288 ? kVecWG : WG; }
 int vec_grid(int N) { return vec_wg(N) == WG ? pcg_grid(N) : ((N + kVecWG - 1) / kVecWG + 7) & ~7; }
 
 int patch_grid(int N, int rows) { return ((N + rows - 1) / rows + 7) & ~7; }
