@@ -1099,12 +1099,12 @@ static int set_topology_impl(eolc_ctx *c, int N, const double *X, int F, const i
             return fail(c, EOLC_ERR_DEGENERATE,
                         "set_topology: face " + std::to_string(f) + " has non-positive material area (must be CCW)");
     }
-    if (eolc::pcg_grid(N) > eolc::kMaxPartials)
+    if (eolc::most_partials(N) > eolc::kMaxPartials)
         return fail(c, EOLC_ERR_INVALID, "set_topology: mesh too large for the PCG reduction buffers");
     Topology t;
     std::string msg = build_topology(t, N, F, tri, H, hinge, seg);
     if (!msg.empty()) return fail(c, EOLC_ERR_INVALID, "set_topology: " + msg);
-    for (int rows = t.N <= eolc::kPatchSmallN ? 256 : 512; rows <= eolc::kPcgWG; rows *= 2) {
+    for (int rows = eolc::patch_rows(t.N); rows <= eolc::kPcgWG; rows *= 2) {
         t.pt_why = build_patch_layout(t, X, rows);
         if (t.pt_why.empty()) break;
     }

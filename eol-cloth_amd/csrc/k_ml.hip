@@ -1154,6 +1154,7 @@ hipError_t ml_setup(eolc_ctx *c, bool linear)
 
 static bool ml_linear_on(const eolc_ctx *c) { return c->ml.lin_on && c->ml.lv.L >= kMLLinFrom; }
 
+static_assert(kRestrictGrid <= kMaxPartials && kCoarse9WG * kRestrict3Parts + 7 <= kMaxPartials, "partials of r.r");
 int ml_restrict_grid(const eolc_ctx *c)
 {
     const MLLevels &lv = c->ml.lv;

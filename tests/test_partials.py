@@ -1,0 +1,33 @@
+"""CPU: the kernels of the solve leave one partial sum per workgroup in arrays of 16,384;
+on no mesh that set_topology accepts may a grid be larger (the sums of the workgroups
+beyond would land in the next array while other workgroups read it)."""
+import ctypes as C
+
+import pytest
+
+import eolc
+
+MOST = 16384   # stride of one array of partial sums
+LAST = 16384 * 1024   # the largest mesh
+
+
+def rule(name, *args):
+    return C.CDLL(eolc.LIB_PATH)[f"_ZN4eolc{len(name)}{name}E" + "i" * len(args)](*args)
+
+
+@pytest.mark.parametrize("n,rows", [(1, 256), (524288, 256), (524289, 512), (8388608, 512), (8388609, 1024),
+                                    (12000000, 1024), (LAST, 1024)])
+def test_patches_fit_the_partial_sums(n, rows):
+    assert rule("patch_rows", n) == rows
+    assert rule("patch_grid", n, rows) <= MOST
+
+
+def test_every_grid_fits_the_partial_sums():
+    sizes = {LAST + 1, LAST + 1024}
+    for edge in (64, 256, 90000, 288 * 1024, 524288, 8388608, LAST):
+        sizes |= {max(1, edge + d) for d in (-1024, -64, -1, 0, 1, 64, 1024)}
+    sizes |= set(range(1, LAST, 65537))
+    for n in sorted(sizes):
+        most = rule("most_partials", n)
+        assert most >= max(rule("pcg_grid", n), rule("vec_grid", n), rule("patch_grid", n, rule("patch_rows", n)))
+        assert (most <= MOST) == (n <= LAST), n   # set_topology refuses by this
