@@ -115,15 +115,19 @@ struct Topology {
 // in FP64); the launch asks for what the mesh needs.  A window holds at most 2 rows
 // vertices (staged through registers before beta is known).  kPatchCross marks a cross
 // lower entry.
-// Rows per patch: 256 on meshes of at most kPatchSmallN vertices, 512 above, and the
-// next larger (up to kPcgWG) where a mesh does not fit, or where the patches, each of
-// which leaves a partial sum of p.q, would be more than kMaxPartials (patch_rows).  Smaller patches put more
-// workgroups in different phases on a compute unit (the window's loads, the record
-// stream, the LDS sums) and shorten the last round of workgroups, but cut more blocks.
-// Product with 256, 512, 768 and 1,024 rows (us): FP32 263,169 vertices 22.5 23.4 24.1
-// 26.2 (arbitrary order 34.7 37.0 38.8 44.8), 1,050,625 vertices 89.4 82.3 95.1 85.6; FP64
-// 36.7 37.7 38.6 44.7 (58.4 71.3 58.5 65.5) and 161 151 163 166.
-constexpr int kPatchSmallN = 524288;
+// Rows per patch: 256 on meshes of at most kPatchSmallN vertices, 512 up to kPatchMidN,
+// kPcgWG above, and the next larger (up to kPcgWG) where a mesh does not fit.  Smaller
+// patches put more workgroups in different phases on a compute unit (the window's loads,
+// the record stream, the LDS sums) and shorten the last round of workgroups, but cut more
+// blocks, which counts where the records come from HBM.  Product alone with 256, 512, 768
+// and 1,024 rows (us): FP32 263,169 vertices 22.5 23.4 24.1 26.2 (arbitrary order 34.7 37.0
+// 38.8 44.8), 1,050,625 vertices 89.4 82.3 95.1 85.6; FP64 36.7 37.7 38.6 44.7 (58.4 71.3
+// 58.5 65.5) and 161 151 163 166.  512 and 1,024 rows, us per multilevel iteration of n^2
+// quads: mixed 724 108.7 112.4, 860 142.6 142.1, 1024 199.1 199.0, 1100 224.9 220.6, 1200
+// 238.6 226.6, 1600 427.7 409.4, 2048 695.1 662.7; FP64 724 134.0 145.4, 1024 255.7 264.8,
+// 1200 335.8 334.8, 1600 593.8 579.8.  (A patch also leaves one partial sum of p.q: 512 rows
+// would be more than kMaxPartials from 8,388,609 vertices on.)
+constexpr int kPatchSmallN = 524288, kPatchMidN = 1310720;
 constexpr int kPatchPool = 6750;
 constexpr int patch_win(int rows) { return 2 * rows; }
 constexpr unsigned short kPatchCross = 0xffff;

@@ -1454,15 +1454,8 @@ int vec_grid(int N) { return vec_wg(N) == WG ? pcg_grid(N) : ((N + kVecWG - 1) /
 
 int patch_grid(int N, int rows) { return ((N + rows - 1) / rows + 7) & ~7; }
 
-// Rows of the smallest patches tried on an N-vertex mesh: kPatchSmallN's rule, and
-// twice as many (up to kPcgWG) while the patches would outnumber the partial sums of a
-// reduction (512 rows: above 8,388,608 vertices).
-int patch_rows(int N)
-{
-    int rows = N <= kPatchSmallN ? 256 : 512;
-    while (rows < kPcgWG && patch_grid(N, rows) > kMaxPartials) rows *= 2;
-    return rows;
-}
+// Rows of the smallest patches tried on an N-vertex mesh (why: kPatchSmallN).
+int patch_rows(int N) { return N <= kPatchSmallN ? 256 : N <= kPatchMidN ? 512 : kPcgWG; }
 
 // The most partial sums that a kernel of the solve leaves on an N-vertex mesh (the
 // restriction's count is bounded by itself, ml_restrict_grid).

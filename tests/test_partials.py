@@ -15,16 +15,17 @@ def rule(name, *args):
     return C.CDLL(eolc.LIB_PATH)[f"_ZN4eolc{len(name)}{name}E" + "i" * len(args)](*args)
 
 
-@pytest.mark.parametrize("n,rows", [(1, 256), (524288, 256), (524289, 512), (8388608, 512), (8388609, 1024),
-                                    (12000000, 1024), (LAST, 1024)])
+@pytest.mark.parametrize("n,rows", [(1, 256), (524288, 256), (524289, 512), (1310720, 512), (1310721, 1024),
+                                    (8388608, 1024), (8388609, 1024), (LAST, 1024)])
 def test_patches_fit_the_partial_sums(n, rows):
+    """The row count on both sides of its lines, and the patches that it gives."""
     assert rule("patch_rows", n) == rows
     assert rule("patch_grid", n, rows) <= MOST
 
 
 def test_every_grid_fits_the_partial_sums():
     sizes = {LAST + 1, LAST + 1024}
-    for edge in (64, 256, 90000, 288 * 1024, 524288, 8388608, LAST):
+    for edge in (64, 256, 90000, 288 * 1024, 524288, 1310720, 8388608, LAST):
         sizes |= {max(1, edge + d) for d in (-1024, -64, -1, 0, 1, 64, 1024)}
     sizes |= set(range(1, LAST, 65537))
     for n in sorted(sizes):
