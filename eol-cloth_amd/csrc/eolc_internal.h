@@ -92,7 +92,7 @@ struct Topology {
     // LDS for it, and the row's lower list names that LDS slot (or kPatchCross: take
     // the row's next cross record).
     bool pt_ok = false;
-    int pt_rows = 0;                     // rows per patch (patch_rows or the next larger, up to kPcgWG)
+    int pt_rows = 0;                     // rows per patch (the first choice of patch_rows that fits)
     std::string pt_why;                  // why the layout does not apply to this mesh
     std::vector<int> pt_row;             // per storage position: row or -1
     std::vector<int> pt_cnt;             // per storage position: upper records | lower entries << 16
@@ -116,7 +116,9 @@ struct Topology {
 // vertices (staged through registers before beta is known).  kPatchCross marks a cross
 // lower entry.
 // Rows per patch: 256 on meshes of at most kPatchSmallN vertices, 512 up to kPatchMidN,
-// kPcgWG above, and the next larger (up to kPcgWG) where a mesh does not fit.  Smaller
+// kPcgWG above.  Where a mesh does not fit, the next larger up to kPcgWG (a window holds
+// twice as many vertices), and 512 after kPcgWG (a mesh in arbitrary vertex order needs
+// more LDS slots per row).  Smaller
 // patches put more workgroups in different phases on a compute unit (the window's loads,
 // the record stream, the LDS sums) and shorten the last round of workgroups, but cut more
 // blocks, which counts where the records come from HBM.  Product alone with 256, 512, 768
@@ -576,7 +578,7 @@ hipError_t launch_update_x(eolc_ctx *c, double h);
 
 int pcg_grid(int N);
 int patch_grid(int N, int rows);   // patches of at most `rows` vertices (a multiple of 8)
-int patch_rows(int N);      // rows of the smallest patches tried
+int patch_rows(int N, int choice);   // rows per patch to try, in turn; 0: none left
 int most_partials(int N);   // at most kMaxPartials on every mesh that set_topology accepts
 int vec_wg(int N);          // workgroup size and workgroups of the PCG's vector kernels
 int vec_grid(int N);

@@ -1454,15 +1454,24 @@ int vec_grid(int N) { return vec_wg(N) == WG ? pcg_grid(N) : ((N + kVecWG - 1) /
 
 int patch_grid(int N, int rows) { return ((N + rows - 1) / rows + 7) & ~7; }
 
-// Rows of the smallest patches tried on an N-vertex mesh (why: kPatchSmallN).
-int patch_rows(int N) { return N <= kPatchSmallN ? 256 : N <= kPatchMidN ? 512 : kPcgWG; }
+// Rows of the patches of an N-vertex mesh, the first, second, ... choice (why: kPatchSmallN);
+// 0: no choice is left whose patches fit the partial sums.
+int patch_rows(int N, int choice)
+{
+    int rows = 0;
+    if (N > kPatchMidN) rows = choice == 0 ? kPcgWG : choice == 1 ? 512 : 0;
+    else if (choice < 3) rows = (N <= kPatchSmallN ? 256 : 512) << choice;
+    return rows > 0 && rows <= kPcgWG && patch_grid(N, rows) <= kMaxPartials ? rows : 0;
+}
 
 // The most partial sums that a kernel of the solve leaves on an N-vertex mesh (the
 // restriction's count is bounded by itself, ml_restrict_grid).
 int most_partials(int N)
 {
-    const int split = N <= kSplitRows ? split_grid((N + kSlice - 1) / kSlice) : 0;
-    return std::max({pcg_grid(N), vec_grid(N), patch_grid(N, patch_rows(N)), split});
+    int most = std::max(pcg_grid(N), vec_grid(N));
+    if (N <= kSplitRows) most = std::max(most, split_grid((N + kSlice - 1) / kSlice));
+    for (int choice = 0, rows; (rows = patch_rows(N, choice)); ++choice) most = std::max(most, patch_grid(N, rows));
+    return most;
 }
 
 int pcg_grid(int N)

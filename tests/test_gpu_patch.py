@@ -209,3 +209,31 @@ def test_patch_rows_follow_the_window(ctx, n, wmin, wmax):
             out, st = solve(ctx, mesh, prec, var)
             assert rel_err(out, ref) <= 1e-6
         ctx.set_spmv_variant(prec, 0)
+
+
+def test_large_mesh_in_arbitrary_order(ctx):
+    """1,311,025 vertices in arbitrary order need more LDS slots than patches of 1,024 rows
+    have room for: 512 rows apply, and the product gives the SELL kernels' answer."""
+    sc = scene.Scene(1144, sigma_x=1e-3, sigma_v=0.05)
+    rng = np.random.default_rng(11)
+    new = rng.permutation(sc.N)
+    X, x, v = np.empty_like(sc.X), np.empty((sc.N, 3)), np.empty((sc.N, 3))
+    X[new], x[new], v[new] = sc.X, sc.x0.reshape(-1, 3), sc.v0.reshape(-1, 3)
+    tri, fixed = new[sc.tri].astype(np.int32), new[sc.fixed].astype(np.int32)
+    mesh = (X, tri, scene.hinges(sc.N, tri), x.reshape(-1), v.reshape(-1), fixed)
+    ctx.set_topology(*mesh[:3])
+    info = ctx.spmv_layout_info()
+    print(f"{sc.N} vertices in arbitrary order: {info}", flush=True)
+    assert info["applies"] == 1 and 512 < info["window_max"] <= 1024
+    out = []
+    for var in (0, 25):
+        ctx.set_spmv_variant(32, var)
+        ctx.set_material(0.1, 500.0, 0.3, 1e-5, 0.0, 1.0)
+        ctx.set_options(eolc.OPT_SPD_PROJECT_BENDING)
+        ctx.upload_state(*mesh[3:5])
+        rc, st = ctx.step(GRAV, H, fixed, tol=1e-6, maxit=20000, mode=eolc.SOLVE_MIXED_BJ | eolc.SOLVE_MULTILEVEL)
+        print(f"  variant {var}: {st.iters} iterations, true residual {st.true_relres:.2e}", flush=True)
+        assert rc == 0 and st.true_relres <= 1e-6
+        out.append(ctx.download_state()[1])
+    ctx.set_spmv_variant(32, 0)
+    assert rel_err(out[1], out[0]) <= 1e-3

@@ -15,12 +15,13 @@ def rule(name, *args):
     return C.CDLL(eolc.LIB_PATH)[f"_ZN4eolc{len(name)}{name}E" + "i" * len(args)](*args)
 
 
-@pytest.mark.parametrize("n,rows", [(1, 256), (524288, 256), (524289, 512), (1310720, 512), (1310721, 1024),
-                                    (8388608, 1024), (8388609, 1024), (LAST, 1024)])
+@pytest.mark.parametrize("n,rows", [(1, [256, 512, 1024]), (524288, [256, 512, 1024]), (524289, [512, 1024]),
+                                    (1310720, [512, 1024]), (1310721, [1024, 512]), (8388608, [1024, 512]),
+                                    (8388609, [1024]), (LAST, [1024])])
 def test_patches_fit_the_partial_sums(n, rows):
-    """The row count on both sides of its lines, and the patches that it gives."""
-    assert rule("patch_rows", n) == rows
-    assert rule("patch_grid", n, rows) <= MOST
+    """The row counts tried on both sides of their lines, and the patches that they give."""
+    assert [rule("patch_rows", n, k) for k in range(4)] == rows + [0] * (4 - len(rows))
+    assert all(rule("patch_grid", n, r) <= MOST for r in rows)
 
 
 def test_every_grid_fits_the_partial_sums():
@@ -30,5 +31,7 @@ def test_every_grid_fits_the_partial_sums():
     sizes |= set(range(1, LAST, 65537))
     for n in sorted(sizes):
         most = rule("most_partials", n)
-        assert most >= max(rule("pcg_grid", n), rule("vec_grid", n), rule("patch_grid", n, rule("patch_rows", n)))
+        grids = [rule("pcg_grid", n), rule("vec_grid", n)]
+        grids += [rule("patch_grid", n, r) for r in (rule("patch_rows", n, k) for k in range(4)) if r]
+        assert most >= max(grids)
         assert (most <= MOST) == (n <= LAST), n   # set_topology refuses by this
