@@ -19,7 +19,9 @@
 // level's blocks are inverted in FP64.
 //
 // Per PCG iteration, after the product (ml_apply):
-//   k_ml_restrict : the vector update x += alpha p, r -= alpha q; one wavefront per level-2 aggregate, vertices staged through LDS:
+//   k_ml_update   : on large meshes the vector update x += alpha p, r -= alpha q (on others
+//                   the restriction updates r, the prolongation x)
+//   k_ml_restrict : one wavefront per level-2 aggregate, vertices staged through LDS:
 //                   R_1(a) = sum of r over a's members, R_2 = sum of the children's R_1,
 //                   and per level-1 aggregate a, C(a) = D_1^-1 R_1(a) + D_2^-1 R_2(parent)
 //   k_ml_coarse   : one workgroup (levels >= 3 only): R_l for l >= 3, then
@@ -551,13 +553,14 @@ struct RestrictArgs {
     double *R9p;
     SolverScalars *scal;
     double *partials;
-    int k, Ga, Gz;        // iteration and partial counts (UPD)
+    int k, Ga, Gz;        // iteration and partial counts (the vector update)
     int parity;
+    bool check;           // no-op once the solve has stopped
 };
 
 // alpha of the iteration; false: the solve stops here (the flag is set by workgroup 0).
 template <class T, int W>
-__device__ __forceinline__ bool restrict_alpha(const RestrictArgs &g, VecUpdate<T> &up, double *lds)
+__device__ __forceinline__ bool restrict_alpha(const RestrictArgs &g, VecUpdate<T> &up, double &alpha, double *lds)
 {
     double v[2];
     reduce_partials<2, W>({PA(g.partials), PB(g.partials, g.k & 1)}, {g.Ga, g.Gz}, v, lds);
@@ -571,7 +574,7 @@ __device__ __forceinline__ bool restrict_alpha(const RestrictArgs &g, VecUpdate<
         }
         return false;
     }
-    const double alpha = rz / pq;
+    alpha = rz / pq;
     up.alpha = (T)alpha;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         scal->iters = g.k + 1;
@@ -579,6 +582,49 @@ __device__ __forceinline__ bool restrict_alpha(const RestrictArgs &g, VecUpdate<
         scal->alpha = alpha;
     }
     return true;
+}
+
+// The vector update of a large mesh on its own (ml_update_apart), x += alpha p and r -=
+// alpha q over the flat arrays: four consecutive values a thread, 16 bytes a load (two for
+// FP64), bound by the bytes.
+template <class T>
+__global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8, 8)))
+k_ml_update(RestrictArgs g, VecUpdate<T> up, int n3, const T *__restrict__ p, double *__restrict__ x)
+{
+    typedef T v4 __attribute__((ext_vector_type(4)));
+    typedef double x4 __attribute__((ext_vector_type(4)));
+    __shared__ double lds[2 * (WG / 64) + 2];
+    if (g.scal->done) return;
+    const int G = gridDim.x, chunk = (((n3 + G - 1) / G) + 3) & ~3;
+    const int b = min(logical_wg() * chunk, n3), e = min(b + chunk, n3), i0 = b + 4 * (int)threadIdx.x;
+    // mixed precision: the first trip's x (half the bytes read) loads before the partial
+    // sums are reduced; more would spill at eight waves per SIMD
+    constexpr bool PRE = sizeof(T) == 4;
+    x4 xv0 = {};
+    if (PRE && i0 + 3 < e) xv0 = *reinterpret_cast<const x4 *>(x + i0);
+    double alpha;
+    if (!restrict_alpha<T, WG>(g, up, alpha, lds)) return;
+    for (int i = i0; i < e; i += 4 * WG) {
+        if (i + 3 < e) {   // i is a multiple of 4: aligned vectors
+            const v4 pv = *reinterpret_cast<const v4 *>(p + i), qv = *reinterpret_cast<const v4 *>(up.q + i);
+            const v4 rv = *reinterpret_cast<const v4 *>(up.r + i);
+            const x4 xv = (PRE && i == i0) ? xv0 : *reinterpret_cast<const x4 *>(x + i);
+            x4 xo;
+            v4 ro;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                xo[c] = fma(alpha, (double)pv[c], xv[c]);
+                ro[c] = fma(-up.alpha, qv[c], rv[c]);
+            }
+            *reinterpret_cast<x4 *>(x + i) = xo;
+            *reinterpret_cast<v4 *>(up.r + i) = ro;
+        } else {
+            for (int c = i; c < e; ++c) {
+                x[c] = fma(alpha, (double)p[c], x[c]);
+                up.r[c] = fma(-up.alpha, up.q[c], up.r[c]);
+            }
+        }
+    }
 }
 
 // Translations only: one wavefront per level-2 aggregate (or per 64 level-1 ones), on at
@@ -590,8 +636,9 @@ __global__ void __launch_bounds__(kRestrictWG) k_ml_restrict(RestrictArgs g, Vec
     constexpr int NW = kRestrictWG / 64;
     __shared__ double stage[NW][3 * kStageRows];
     __shared__ double lds[2 * NW + 2];
-    if (UPD && g.scal->done) return;
-    if (UPD && !restrict_alpha<T, kRestrictWG>(g, up, lds)) return;
+    if (g.check && g.scal->done) return;
+    double alpha;
+    if (UPD && !restrict_alpha<T, kRestrictWG>(g, up, alpha, lds)) return;
     double s0, s1, s2, mom[6], srr[1] = {0.0};
     const int waves = g.lv.L >= 2 ? g.lv.n[2] : (g.lv.n[1] + 63) / 64;
     for (int w = logical_wg() * NW + (int)threadIdx.x / 64; w < waves; w += gridDim.x * NW)   // uniform
@@ -632,8 +679,9 @@ __global__ void __launch_bounds__(kRestrict3WG) k_ml_restrict3(RestrictArgs g, V
     const int c0 = g.cptr[lv.coff[3] + U], c1 = own ? g.cptr[lv.coff[3] + U + 1] : 0;
     const int64_t gU = lv.off[3] + U;
     const double cu = g.geo[4 * gU], cv = g.geo[4 * gU + 1], is = g.geo[4 * gU + 3];
-    if (UPD && g.scal->done) return;
-    if (UPD && !restrict_alpha<T, kRestrict3WG>(g, up, lds)) return;
+    if (g.check && g.scal->done) return;
+    double alpha;
+    if (UPD && !restrict_alpha<T, kRestrict3WG>(g, up, alpha, lds)) return;
     // lane 0 keeps the wavefront's running sum in LDS
     if (lane == 0)
 #pragma unroll
@@ -1174,7 +1222,15 @@ static bool ml_fused(const eolc_ctx *c)
     return lv.L >= 3 && lv.off[lv.L + 1] - lv.off[3] <= (ml_linear_on(c) ? kFusedLinear : kFusedCoarse) && vec_wg(c->topo.N) == kVecWG;
 }
 
-// The restriction (with the vector update when there is one) and the coarse levels, with
+// On large meshes the vectors come from HBM whole, and the restriction's scattered pieces of
+// q and r cost more than a pass of their own.  With the update in the restriction and the
+// prolongation, and apart, us per multilevel iteration of n^2 quads: mixed 724 108.7 116.0,
+// 1024 199.1 202.6, 1200 226.6 227.8, 1300 274.3 269.2, 1600 409.4 408.0, 2048 662.7 657.4;
+// FP64 512 68.1 72.0, 1024 255.7 253.5, 1200 334.8 335.0, 1600 579.8 566.7.
+constexpr int kApartN = 1572864;
+static bool ml_update_apart(const eolc_ctx *c) { return c->topo.N > kApartN; }
+
+// The restriction (with or after the vector update when there is one) and the coarse levels, with
 // the linear fields when the last ml_setup formed them; fused: without the coarse levels,
 // which the prolongation forms.
 template <class T>
@@ -1183,18 +1239,23 @@ static void ml_coarse_chain(eolc_ctx *c, T *r, int parity, const MLUpdate *u, bo
     const MLState &m = c->ml;
     const MLLevels &lv = m.lv;
     RestrictArgs g{lv,    m.hord, m.ptr1, m.cptr, m.kptr2, m.R, m.C,     m.Dinv, m.feat2,
-                   m.geo, m.R9p,  c->scal, c->partials, u ? u->k : 0, u ? u->Ga : 0, vec_grid(c->topo.N), parity};
+                   m.geo, m.R9p,  c->scal, c->partials, u ? u->k : 0, u ? u->Ga : 0, vec_grid(c->topo.N), parity,
+                   u != nullptr};
     VecUpdate<T> up{u ? static_cast<const T *>(u->q) : nullptr, r, (T)0};
+    const bool apart = u && ml_update_apart(c), with = u && !apart;
+    if (apart)
+        hipLaunchKernelGGL((k_ml_update<T>), dim3(pcg_grid(c->topo.N)), dim3(WG), 0, c->stream, g, up, 3 * c->topo.N,
+                           static_cast<const T *>(u->p), u->x);
     const dim3 grid(ml_restrict_grid(c));
     if (ml_linear_on(c)) {
-        if (u) hipLaunchKernelGGL((k_ml_restrict3<T, true>), grid, dim3(kRestrict3WG), 0, c->stream, g, up);
+        if (with) hipLaunchKernelGGL((k_ml_restrict3<T, true>), grid, dim3(kRestrict3WG), 0, c->stream, g, up);
         else hipLaunchKernelGGL((k_ml_restrict3<T, false>), grid, dim3(kRestrict3WG), 0, c->stream, g, up);
         if (!fused)
             hipLaunchKernelGGL(k_ml_coarse9, dim3(blocks_for(lv.n[3], 64)), dim3(kCoarse9WG), 0, c->stream, lv, m.cptr, m.par, m.geo, m.D9,
                            m.R9p, m.C9, c->scal, u != nullptr);
         return;
     }
-    if (u) hipLaunchKernelGGL((k_ml_restrict<T, true>), grid, dim3(kRestrictWG), 0, c->stream, g, up);
+    if (with) hipLaunchKernelGGL((k_ml_restrict<T, true>), grid, dim3(kRestrictWG), 0, c->stream, g, up);
     else hipLaunchKernelGGL((k_ml_restrict<T, false>), grid, dim3(kRestrictWG), 0, c->stream, g, up);
     if (lv.L >= 3 && !fused)
         hipLaunchKernelGGL(k_ml_coarse, dim3(1), dim3(kCoarseWG), 0, c->stream, lv, m.cptr, m.par, m.Dinv, m.R, m.C,
@@ -1209,11 +1270,12 @@ static void launch_prolong(eolc_ctx *c, int parity, const T *D, const T *r, T *z
     const MLLevels &lv = m.lv;
     const int N = c->topo.N;
     const double *c9 = ml_linear_on(c) ? m.C9 : nullptr;
+    const bool with = u && !ml_update_apart(c);   // x += alpha p here
     auto go = [&](auto w) {
         constexpr int W = decltype(w)::value;
         hipLaunchKernelGGL((k_ml_prolong<T, FINE, W>), dim3(vec_grid(N)), dim3(W), 0, c->stream, parity, N, lv, m.agg1,
                            m.anc3, m.Dinv, m.R, m.C, D, r, z, c->fixmask, c->scal, c->partials, u != nullptr, m.feat3, c9,
-                           u ? static_cast<const T *>(u->p) : nullptr, u ? u->x : nullptr);
+                           with ? static_cast<const T *>(u->p) : nullptr, with ? u->x : nullptr);
     };
     if (vec_wg(N) == kVecWG) go(std::integral_constant<int, kVecWG>());
     else go(std::integral_constant<int, WG>());

@@ -262,3 +262,24 @@ def test_coarse_levels_of_many_sheets(ctx, small):
         zref = ML.apply(A, N, maps, r, fd, X=X if linear else None)
         print(f"  linear {linear}: P r rel err {rel_err(z, zref):.2e}", flush=True)
         assert rel_err(z, zref) <= 1e-12 and np.all(z[fd] == 0.0)
+
+
+@pytest.mark.parametrize("n", [1253, 1256])
+def test_both_sides_of_the_separate_vector_update(ctx, n):
+    """1,572,516 vertices are among the last whose restriction and prolongation do the
+    vector update, 1,580,049 have a kernel of its own (its last three values a remainder):
+    the answers meet the tolerance by the FP64 true residual, and mixed and FP64
+    iterations agree to what two residuals of 1e-8 leave."""
+    sc = scene.Scene(n, sigma_x=1e-3, sigma_v=0.05)
+    print(f"separate vector update: {sc.N} vertices", flush=True)
+    ctx.set_topology(sc.X, sc.tri, sc.hinge)
+    ctx.set_material(0.1, 500.0, 0.3, 1e-5, 0.0, 1.0)
+    ctx.set_options(eolc.OPT_SPD_PROJECT_BENDING)
+    out = []
+    for mode in (eolc.SOLVE_MIXED_BJ, eolc.SOLVE_FP64_BJ):
+        ctx.upload_state(sc.x0, sc.v0)
+        rc, st = ctx.step(GRAV, H, sc.fixed, tol=1e-8, maxit=20000, mode=mode | MLF)
+        print(f"  mode {mode}: {st.iters} iterations, true residual {st.true_relres:.2e}", flush=True)
+        assert rc == 0 and st.true_relres <= 1e-8
+        out.append(ctx.download_state()[1])
+    assert rel_err(out[1], out[0]) <= 1e-4
