@@ -193,9 +193,10 @@ unsigned grid_table_size(int F)
     return tbl;
 }
 
-// A bound of the device bytes of a collide call before the data-dependent buffers (the
-// grid's entry list and the record outputs), alignment included; what
-// eolc_collide_noalloc refuses a query by.
+// A bound of the device bytes of a spare collide call (one box at a time, every query on
+// the grid) before the data-dependent buffers (the grid's entry list and the record
+// outputs), alignment included; what eolc_collide_noalloc refuses a query by.  It counts a
+// record per vertex, which leaves room for the vertices' and edges' records of a box.
 size_t collide_fixed_bytes(const eolc_ctx *c, int P, int B)
 {
     const size_t N = (size_t)c->topo.N, F = (size_t)c->topo.F, E = (size_t)c->n_cedges;
@@ -270,21 +271,22 @@ int query_grid(eolc_ctx *c, eolc::Workspace &ws, double thr, int Q, const double
     return EOLC_OK;
 }
 
-int collide_impl(eolc_ctx *c, eolc::Workspace &ws, double thr, int P, const double *pts, const double *nrm, int B,
-                 const double *whd, const double *Eb, int eol_points, int box_npts, int box_nedges,
+// spare: with the least device memory, the same records (collide_fixed_bytes).
+int collide_impl(eolc_ctx *c, eolc::Workspace &ws, bool spare, double thr, int P, const double *pts, const double *nrm,
+                 int B, const double *whd, const double *Eb, int eol_points, int box_npts, int box_nedges,
                  std::vector<eolc_collision> &out)
 {
     const int N = c->topo.N, F = c->topo.F, E = c->n_cedges;
     const size_t NE = (size_t)N + E;
     // boxes per launch: their counts are numbered with 31 bits
-    const int group = std::max(1, (int)std::min<size_t>(eolc::kCdBoxes, INT_MAX / NE));
-    const int Q = P + 8 * B, nbg = std::min(B, group);
+    const int group = std::max(1, (int)std::min<size_t>(spare ? 1 : eolc::kCdBoxes, INT_MAX / NE));
+    const int Q = P + 8 * B, nbg = std::min(B, group), nbd = spare ? nbg : B;   // boxes per launch, on the device
     // ---- queries and boxes in one upload: points and corners, their normals, the boxes
     std::vector<BoxGeom> boxes((size_t)B);
     for (int b = 0; b < B; ++b) make_box(boxes[b], whd + 3 * b, Eb + 16 * b);
     const size_t nbox = sizeof(BoxGeom) / sizeof(double);
     static_assert(sizeof(BoxGeom) % sizeof(double) == 0, "boxes are packed behind the queries");
-    std::vector<double> hin(6 * (size_t)Q + nbox * (size_t)B);
+    std::vector<double> hin(6 * (size_t)Q + nbox * (size_t)nbd);
     double *hq = hin.data(), *hn = hq + 3 * (size_t)Q;
     for (int i = 0; i < 3 * P; ++i) { hq[i] = pts[i]; hn[i] = nrm[i]; }
     for (int b = 0; b < B; ++b)
@@ -293,7 +295,7 @@ int collide_impl(eolc_ctx *c, eolc::Workspace &ws, double thr, int P, const doub
                 hq[3 * (P + 8 * b + i1) + k] = boxes[b].v[i1][k];
                 hn[3 * (P + 8 * b + i1) + k] = boxes[b].vn[i1][k];
             }
-    if (B) std::memcpy(hn + 3 * (size_t)Q, boxes.data(), sizeof(BoxGeom) * B);
+    if (nbd) std::memcpy(hn + 3 * (size_t)Q, boxes.data(), sizeof(BoxGeom) * nbd);
     double *xj = nullptr, *fn = nullptr, *aabb_part = nullptr, *aabb = nullptr, *din = nullptr;
     char *dst = nullptr, *cand = nullptr;
     unsigned *cnt = nullptr, *offs = nullptr, *sums = nullptr, *pairs = nullptr;
@@ -313,13 +315,14 @@ int collide_impl(eolc_ctx *c, eolc::Workspace &ws, double thr, int P, const doub
     eolc_collision *qrec = reinterpret_cast<eolc_collision *>(dst + sizeof(CdStatus));
     static_assert(sizeof(CdStatus) % 8 == 0, "records follow the status");
     const double *qpts = din, *qnrm = din + 3 * (size_t)Q;
-    const BoxGeom *dbox = reinterpret_cast<const BoxGeom *>(din + 6 * (size_t)Q);
+    BoxGeom *const dboxes = reinterpret_cast<BoxGeom *>(din + 6 * (size_t)Q);
     if (!hin.empty())
         EOLC_HIP(hipMemcpyAsync(din, hin.data(), hin.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
     EOLC_HIP(hipMemsetAsync(dst, 0, sizeof(CdStatus), c->stream));
     EOLC_HIP(eolc::cd_prep(c, thr, xj, fn, aabb_part, aabb));
     // ---- point / corner queries against the faces
-    const bool sweep = Q > 0 && Q <= kCdSweepQueries;
+    const bool sweep = !spare && Q > 0 && Q <= kCdSweepQueries;
+    const eolc::Workspace::Mark before_cand = ws.mark();
     if (sweep) {
         EOLC_HIP(ws.get(&cand, 16 * (size_t)eolc::kCdCandidates));
         EOLC_HIP(eolc::cd_sweep(c, Q, qpts, qnrm, thr, aabb, xj, fn, &dstat->ncand, cand, qrec));
@@ -335,8 +338,8 @@ int collide_impl(eolc_ctx *c, eolc::Workspace &ws, double thr, int P, const doub
         return r;
     };
     // counts, offsets and read-back of one group of boxes
-    auto count_boxes = [&](int g0, int nb) -> int {
-        EOLC_HIP(eolc::cd_boxes(c, 0, nb, thr, dbox + g0, xj, fn, cnt, nullptr, &dstat->npairs, pairs, dstat->nambig,
+    auto count_boxes = [&](const BoxGeom *dbox, int nb) -> int {
+        EOLC_HIP(eolc::cd_boxes(c, 0, nb, thr, dbox, xj, fn, cnt, nullptr, &dstat->npairs, pairs, dstat->nambig,
                                 &dstat->err, nullptr));
         EOLC_HIP(eolc::cd_scan(c, (unsigned)(NE * nb), cnt, offs, sums, offs + NE * nb));
         EOLC_HIP(eolc::cd_first(c, nb, offs, dstat->first));
@@ -349,8 +352,9 @@ int collide_impl(eolc_ctx *c, eolc::Workspace &ws, double thr, int P, const doub
     };
     int rc = EOLC_OK;
     const bool eol_pass = eol_points && P > 0;
-    if (!eol_pass && nbg && (rc = count_boxes(0, nbg))) return rc;   // (the EOL pass uses the counts first)
+    if (!eol_pass && nbg && (rc = count_boxes(dboxes, nbg))) return rc;   // (the EOL pass uses the counts first)
     if ((rc = read_status(nst))) return rc;
+    if (ws.arena) ws.release(before_cand);   // (the list has been read)
     if (sweep && status().ncand > eolc::kCdCandidates) {
         if ((rc = query_grid(c, ws, thr, Q, qpts, qnrm, xj, fn, aabb, qrec))) return rc;
         if ((rc = read_status(nst))) return rc;
@@ -391,9 +395,12 @@ int collide_impl(eolc_ctx *c, eolc::Workspace &ws, double thr, int P, const doub
     std::vector<eolc_collision> recs, clst;
     for (int g0 = 0; g0 < B; g0 += group) {
         const int nb = std::min(B - g0, group);
+        const BoxGeom *dbox = spare ? dboxes : dboxes + g0;   // the group's boxes
         if (g0 > 0 || eol_pass) {
+            if (spare && g0 > 0)
+                EOLC_HIP(hipMemcpyAsync(dboxes, &boxes[g0], sizeof(BoxGeom) * nb, hipMemcpyHostToDevice, c->stream));
             EOLC_HIP(hipMemsetAsync(&dstat->npairs, 0, sizeof(unsigned) * (1 + eolc::kCdBoxes), c->stream));
-            if ((rc = count_boxes(g0, nb)) || (rc = read_status(sizeof(CdStatus)))) return rc;
+            if ((rc = count_boxes(dbox, nb)) || (rc = read_status(sizeof(CdStatus)))) return rc;
         }
         const CdStatus st = status();
         if (st.err) {
@@ -414,7 +421,7 @@ int collide_impl(eolc_ctx *c, eolc::Workspace &ws, double thr, int P, const doub
             const size_t r0 = st.first[2 * b], n = st.first[2 * b1] - r0;
             if (!n) continue;
             if (!whole) EOLC_HIP(ws.get(&o, n));
-            EOLC_HIP(eolc::cd_boxes(c, b, b1, thr, dbox + g0, xj, fn, cnt, offs, &dstat->npairs, pairs, nullptr,
+            EOLC_HIP(eolc::cd_boxes(c, b, b1, thr, dbox, xj, fn, cnt, offs, &dstat->npairs, pairs, nullptr,
                                     &dstat->err, o));
             EOLC_HIP(hipMemcpyAsync(recs.data() + r0, o, sizeof(eolc_collision) * n, hipMemcpyDeviceToHost, c->stream));
             EOLC_HIP(hipStreamSynchronize(c->stream));
@@ -445,7 +452,7 @@ int collide_impl(eolc_ctx *c, eolc::Workspace &ws, double thr, int P, const doub
                 int *eamb = nullptr;
                 const eolc::Workspace::Mark ma = ws.mark();
                 EOLC_HIP(ws.get(&eamb, (size_t)E));
-                EOLC_HIP(eolc::cd_ambiguous(c, thr, dbox + b, xj, eamb));
+                EOLC_HIP(eolc::cd_ambiguous(c, thr, dbox + bg, xj, eamb));
                 EOLC_HIP(hipMemcpyAsync(amb.data(), eamb, sizeof(int) * (size_t)E, hipMemcpyDeviceToHost, c->stream));
                 if (hx.empty()) {
                     hx.resize(3 * (size_t)N);
@@ -527,7 +534,7 @@ try {
     EOLC_HIP(hipSetDevice(c->device));
     std::vector<eolc_collision> recs;
     eolc::Workspace ws(c->kept);   // the context's block, and device buffers allocated for this call
-    int rc = collide_impl(c, ws, threshold, P, pts, nrm, B, whd, E, eol_points, box_npts, box_nedges, recs);
+    int rc = collide_impl(c, ws, false, threshold, P, pts, nrm, B, whd, E, eol_points, box_npts, box_nedges, recs);
     if (rc) return rc;
     *count = (int)recs.size();
     if ((int)recs.size() > cap || (!out && !recs.empty())) {
@@ -573,9 +580,21 @@ try {
     std::lock_guard<std::mutex> lk(*eolc::collide_scratch_lock(c->device));
     eolc::Workspace ws(static_cast<char *>(base), eolc::kCollideScratchBytes);
     std::vector<eolc_collision> recs;
-    int rc = collide_impl(c, ws, threshold, P, pts, nrm, B, whd, E, eol_points, box_npts, box_nedges, recs);
-    if (ws.exhausted) {
+    int rc = EOLC_OK;
+    for (const bool spare : {false, true}) {   // what does not fit is tried again with less
+        const std::string last = c->err;
+        const auto decisions = c->cd_host_decisions;
+        rc = collide_impl(c, ws, spare, threshold, P, pts, nrm, B, whd, E, eol_points, box_npts, box_nedges, recs);
+        if (!ws.exhausted) break;
         (void)hipStreamSynchronize(c->stream);
+        if (spare) break;
+        ws.release({0, 0});
+        ws.exhausted = false;
+        recs.clear();
+        c->err = last;
+        c->cd_host_decisions = decisions;
+    }
+    if (ws.exhausted) {
         c->err = "collide_noalloc: the query's grid or record buffers need more device memory than the " +
                  std::to_string(eolc::kCollideScratchBytes >> 20) + " MiB scratch; use eolc_collide";
         return EOLC_ERR_INVALID;

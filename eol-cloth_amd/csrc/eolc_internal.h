@@ -653,10 +653,10 @@ hipError_t velocity_transfer(eolc_ctx *c, int n_old, const double *u_old, const 
 hipError_t batch_set_fixmask(eolc_ctx *c, const int *d_nodes, int n);
 hipError_t batch_solve_async(eolc_ctx *c, double tol, int maxit, int variant);
 void build_collision_edges(eolc_ctx *c, int F, const int *tri);
-// Proximity queries: boxes per launch of the box kernels (two words per box, vertex and
-// edge and one per box and edge: for 8 boxes less than eolc_collide_noalloc's bound
-// counts per vertex and edge), and the candidates the face sweep keeps (16 bytes each;
-// a query that finds more takes the grid).
+// Proximity queries: boxes per launch of the box kernels (counts, offsets and the list of
+// pairs: 8 bytes per box and vertex, 12 per box and edge), and the candidates the face sweep
+// keeps (16 bytes each; a query that finds more takes the grid).  Where eolc_collide_noalloc
+// has no room for that, it runs one box at a time on the grid.
 constexpr int kCdBoxes = 8;
 constexpr unsigned kCdCandidates = 65536;
 // scratch of eolc_collide_noalloc (k_collide.hip): the device address of this GPU's

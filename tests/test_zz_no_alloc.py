@@ -2,8 +2,8 @@
 per-GPU scratch array) against eolc_collide on the same inputs, through the C ABI:
 record sets equal bit for bit, on two calls in a row with the second smaller (a
 smaller cloth, fewer obstacles, CD instead of CD2), with an allocating call between
-them; and a mesh whose query cannot fit the scratch is refused with a message
-before any device work."""
+them; a query that fills the scratch all but whole; and a mesh whose query cannot fit the
+scratch is refused with a message before any device work."""
 import numpy as np
 import pytest
 
@@ -40,6 +40,21 @@ def test_noalloc_matches_collide_twice_second_smaller():
             same_records(again, ref)
             calls.append(len(ref))
         assert calls[1] < calls[0]
+
+
+def test_noalloc_near_the_end_of_the_scratch():
+    """491,401 vertices, 2,100 points and 8 boxes: counts for all boxes at once beside the
+    points' grid are more than the 256 MiB, one box at a time fits."""
+    sc = scene.Scene(700, sigma_x=1e-3)
+    pts, nrm, whd, E = scene.obstacles(seed=77, P=2100, B=8)
+    with eolc.Context(0) as c:
+        c.set_topology(sc.X, sc.tri, sc.hinge)
+        c.upload_state(sc.x0, sc.v0)
+        ref = c.collide(1e-3, pts, nrm, whd, E)
+        got = c.collide(1e-3, pts, nrm, whd, E, noalloc=True)
+        print(f"noalloc near the end of the scratch: {len(ref)} records", flush=True)
+        assert len(ref) > 2100
+        same_records(got, ref)
 
 
 def test_noalloc_refuses_a_mesh_beyond_the_scratch():
