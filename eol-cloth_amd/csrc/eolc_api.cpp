@@ -123,7 +123,6 @@ void free_topology_buffers(eolc_ctx *c)
     c->bj_iters_hint = c->bj_iters_hint_ml = 0;
     c->fp64_sticky = 0;
     c->alloc_bytes = 0;
-    c->kept.give_back();
 }
 
 void free_learned_weights(eolc_ctx *c)
@@ -1063,6 +1062,7 @@ void eolc_destroy(eolc_ctx *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     free_topology_buffers(c);
     free_learned_weights(c);
+    c->kept.give_back();
     dfree(c->scal); dfree(c->partials); dfree(c->counter);
     if (c->hscal) (void)hipHostFree(c->hscal);
     if (c->stream) (void)hipStreamDestroy(c->stream);

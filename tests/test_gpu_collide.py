@@ -6,6 +6,7 @@ distances, normals, positions and weights compared by bit pattern), in the
 reference's order."""
 import numpy as np
 import pytest
+import torch
 
 import eolc
 import oracle as O
@@ -270,3 +271,29 @@ def test_calls_that_share_the_kept_block(ctx, order):
         got = ctx.velocity_transfer(sc.X, sc.v0, sc.tri, new)[1]
         assert moved is None or np.array_equal(got, moved)
         moved = got
+
+
+def test_kept_block_after_a_call_beyond_its_limit():
+    """A query that needs more than the 256 MB a context keeps (1,000,000 points, 316 bytes
+    each) leaves the block to the smaller queries after it: their memory (200,000 points)
+    is held from the second one on, also over a new topology, and given back with the
+    context."""
+    sc, pts, nrm, _, _ = thin_box_scene(24, 1e-3)
+    rng = np.random.default_rng(6)
+    many = np.concatenate([rng.uniform(0.0, 1.0, (1_000_000, 2)), np.full((1_000_000, 1), 5.0)], axis=1)
+    up = np.tile([0.0, 0.0, 1.0], (len(many), 1))
+    free = lambda: torch.cuda.mem_get_info(0)[0]
+    with eolc.Context(0) as c:
+        for k in range(2):
+            c.set_topology(sc.X, sc.tri, sc.hinge)
+            c.upload_state(sc.x0, np.zeros_like(sc.x0))
+            if k == 0:
+                start = free()
+                for n in (1_000_000, 200_000, 200_000):
+                    print(f"kept block: {n} points, {(start - free()) >> 20} MB held before", flush=True)
+                    assert c.collide(1e-3, many[:n], up[:n]) == []
+            held = start - free()
+            print(f"kept block: {held >> 20} MB held", flush=True)
+            assert 50 << 20 <= held <= 256 << 20
+    print(f"kept block: {(start - free()) >> 20} MB held after the context", flush=True)
+    assert start - free() <= 8 << 20
