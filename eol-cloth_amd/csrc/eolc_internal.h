@@ -334,7 +334,7 @@ struct LearnedState {
     float *dinp = nullptr;               // N x 128
     float *gpart = nullptr;              // weight-gradient partials
     size_t gpart_n = 0;
-    double *dpart = nullptr;             // FP64 per-workgroup partial sums (ceil(N / 256))
+    double *dpart = nullptr;             // FP64 per-workgroup partial sums (ceil(N / 64), learned_dot_groups)
     double *scal = nullptr;              // 8: sum log t, r.e, z.r, z.Az, loss
     double *e = nullptr, *r = nullptr, *z = nullptr, *Az = nullptr;   // 3N training vectors
 };

@@ -713,10 +713,9 @@ __global__ void __launch_bounds__(kRestrict3WG) k_ml_restrict3(RestrictArgs g, V
 
 // Levels >= 3 in one workgroup: R_l from the children (l = 3..L), then from the top
 // down C_l = D_l^-1 R_l + C_{l+1}(parent) (l = L..3).  These levels hold a few hundred
-// aggregates for a million vertices: then each thread owns one, their R and C live
-// in LDS and only C_3 is written out.  Larger hierarchies loop over global memory.
+// aggregates for a million vertices: up to kCoarseWG, each thread owns one, their R and C
+// live in LDS and only C_3 is written out.  Larger hierarchies loop over global memory.
 constexpr int kCoarseWG = 1024;
-constexpr int kCoarseLds = 1024;
 
 // The levels >= 3, at most one aggregate to a thread of the workgroup: C_l of aggregate
 // off[3] + j in Cl[3 j ..], visible to all; false: the solve has stopped.
@@ -812,20 +811,18 @@ __global__ void __launch_bounds__(kCoarseWG) k_ml_coarse(MLLevels lv, const int 
                                                          double *__restrict__ R, double *__restrict__ C,
                                                          const SolverScalars *scal, int check_done)
 {
-    __shared__ double lds[6 * kCoarseLds];
+    __shared__ double lds[6 * kCoarseWG];
     const int L = lv.L;
     const int base = lv.off[3];
     const int M = lv.off[L + 1] - base;   // aggregates of levels >= 3
     if (M <= kCoarseWG) {
-        double *Cl = lds + 3 * kCoarseLds;
+        double *Cl = lds + 3 * kCoarseWG;
         if (!coarse_levels(lv, cptr, par, Dinv, R, scal, check_done, lds, Cl)) return;
         for (int t = threadIdx.x; t < 3 * lv.n[3]; t += kCoarseWG) C[3 * (int64_t)base + t] = Cl[t];
         return;
     }
     if (check_done && scal->done) return;
-    const bool in_lds = M <= kCoarseLds;
-    double *Rb = in_lds ? lds : R + 3 * (int64_t)base;   // level l at off[l] - off[3]
-    double *Cb = in_lds ? lds + 3 * kCoarseLds : C + 3 * (int64_t)base;
+    double *Rb = R + 3 * (int64_t)base, *Cb = C + 3 * (int64_t)base;   // level l at off[l] - off[3]
     for (int l = 3; l <= L; ++l) {
         for (int A = threadIdx.x; A < lv.n[l]; A += kCoarseWG) {
             const int c0 = cptr[lv.coff[l] + A], c1 = cptr[lv.coff[l] + A + 1];
@@ -868,8 +865,6 @@ __global__ void __launch_bounds__(kCoarseWG) k_ml_coarse(MLLevels lv, const int 
         }
         __syncthreads();
     }
-    if (in_lds)
-        for (int t = threadIdx.x; t < 3 * lv.n[3]; t += kCoarseWG) C[3 * (int64_t)base + t] = Cb[t];
 }
 
 // Levels >= 3 with linear fields, in one workgroup, from the level-3 sums R9_3 of

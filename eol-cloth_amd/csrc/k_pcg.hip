@@ -1521,7 +1521,6 @@ hipError_t set_fixed(eolc_ctx *c, int n, const int *d_dofs, const double *d_vals
 hipError_t pcg_init(eolc_ctx *c, bool mixed)
 {
     const int N = c->topo.N;
-    const int G = pcg_grid(N);
     launch_resid64(c, c->vfix, c->rhs, c->b64, &c->scal->bnorm2);
     hipLaunchKernelGGL(k_masked_copy, dim3(blocks_for(3 * N)), dim3(256), 0, c->stream, N, c->v, c->fixmask, c->xs64);
     launch_resid64(c, c->xs64, c->b64, c->r64, &c->scal->rmax2);
@@ -1554,7 +1553,6 @@ hipError_t pcg_chunk(eolc_ctx *c, bool mixed, int k0, int iters)
 hipError_t pcg_reliable_update(eolc_ctx *c)
 {
     const int N = c->topo.N;
-    const int G = pcg_grid(N);
     hipLaunchKernelGGL(k_accumulate, dim3(blocks_for(3 * N)), dim3(256), 0, c->stream, 3 * N, c->xs64, c->xl64);
     launch_resid64(c, c->xs64, c->b64, c->r64, &c->scal->rmax2);
     return hipGetLastError();
@@ -1569,7 +1567,6 @@ hipError_t pcg_reliable_update(eolc_ctx *c)
 hipError_t pcg_restart_from_guess(eolc_ctx *c)
 {
     const int N = c->topo.N;
-    const int G = pcg_grid(N);
     hipLaunchKernelGGL(k_masked_copy, dim3(blocks_for(3 * N)), dim3(256), 0, c->stream, N, c->v, c->fixmask, c->xs64);
     hipError_t e = hipMemsetAsync(c->xl64, 0, (size_t)3 * N * sizeof(double), c->stream);
     if (e != hipSuccess) return e;
@@ -1588,7 +1585,6 @@ hipError_t pcg_precondition(eolc_ctx *c, bool mixed) { return precondition(c, mi
 // the mixed mode's reliable updates); ||r||^2 -> scal->rmax2.
 hipError_t pcg_replace_residual64(eolc_ctx *c)
 {
-    const int G = pcg_grid(c->topo.N);
     launch_resid64(c, c->xs64, c->b64, c->r64, &c->scal->rmax2);
     return hipGetLastError();
 }
@@ -1624,8 +1620,6 @@ hipError_t scal_set(eolc_ctx *c, double tol2, double delta2, int reset)
 // ||rhs - A v||^2 over free DOFs (v = a solution incl. fixed values) -> scal->true_rr
 hipError_t spmv_true_residual(eolc_ctx *c, const double *v)
 {
-    const int N = c->topo.N;
-    const int G = pcg_grid(N);
     launch_resid64(c, v, c->rhs, c->r64, &c->scal->true_rr);
     return hipGetLastError();
 }
