@@ -155,12 +155,11 @@ def test_patch_layout_refused_falls_back(ctx):
     assert rel_err(out[32], out[64]) <= 1e-6
 
 
-def test_patch_kernels_with_a_second_logical_workgroup(ctx):
-    """At 730x730 the row kernels have 528 logical workgroups: 512 run, and the first
-    16 also take logical workgroups 512-527 (a second patch of the SpMV, a second
-    row range of the update and the prolongation).  The mixed multilevel step with
-    the patch SpMV must meet the FP64 true residual (formed by the SELL kernel, so a
-    wrong row in the second pass would show) and agree with the SELL variant."""
+def test_patches_of_512_rows_against_the_sell_kernels(ctx):
+    """730 x 730 quads, 534,361 vertices: patches of 512 rows (1,044 and a padded grid of
+    1,048) and vector kernels of 1,024 threads (528 workgroups).  The multilevel step with
+    the patch product must meet the FP64 true residual (formed by the SELL kernel) and agree
+    with the SELL product's."""
     n = 730
     sc = scene.Scene(n, sigma_x=1e-3, sigma_v=0.05)
     ctx.set_topology(sc.X, sc.tri, sc.hinge)
