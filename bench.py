@@ -309,13 +309,19 @@ SPMV_VARIANTS = [(1, False, False, 8, 0, False), (1, True, False, 8, 0, False), 
                  (1, False, False, 4, 5, False), (2, False, False, 4, 5, False)]
 
 
-def spmv_kernel_name(fp32, variant, N):
+def spmv_kernel_name(fp32, variant, N, positions):
+    """The kernel that runs for the variant on a mesh of N vertices (positions: of the
+    patch layout's storage, which tell the rows of a patch)."""
     u, pf, nt, w, lay, stg = SPMV_VARIANTS[variant]
     b = lambda x: "true" if x else "false"
-    if lay == 5:   # patches of 256 or 512 rows; eight waves per SIMD with FP32 records one ahead
+    if lay == 5:   # eight waves per SIMD with FP32 records one ahead
         t = "float" if fp32 else "double"
         w = (6 if u == 2 and w == 8 else w) if fp32 else 4
-        return f"k_pcg_spmv_patch<{t}, {t}, {b(nt)}, {w}, {u}, {256 if N <= 524288 else 512}>"
+        rows = (256, 512, 1024) if N <= 524288 else (512, 1024) if N <= 1310720 else (1024, 512)
+        pr = next((r for r in rows if r * (-(-N // r) + 7 & ~7) == positions), rows[0])
+        return f"k_pcg_spmv_patch<{t}, {t}, {b(nt)}, {w}, {u}, {pr}>"
+    if N <= 90000 and (fp32 or lay != 4):   # one workgroup per slice of rows
+        return "k_pcg_spmv_split<float, true>" if fp32 else "k_pcg_spmv_split<double, false>"
     t = "float, true" if fp32 else ("double, true" if lay == 4 else "double, false")
     return f"k_pcg_spmv<{t}, {u}, {b(pf)}, {b(nt)}, {w}, {lay if (fp32 or lay >= 3) else 0}, {b(stg)}>"
 
@@ -626,7 +632,7 @@ def main():
             own = (10 * s) * (nb - sc.N) // 2 + 8 * (nb - sc.N) // 2 + 8 * sc.N + (4 * s * 3 + s + 1) * sc.N
         else:
             own = full
-        kname = spmv_kernel_name(fp32, variant, sc.N)
+        kname = spmv_kernel_name(fp32, variant, sc.N, layout["positions"])
         return {"bound": "hbm", "achieved": full / (ms * 1e-3) / 1e9, "peak": PEAK_HBM / 1e9, "unit": "GB/s",
                 "frac": full / (ms * 1e-3) / PEAK_HBM, "traffic": measured_traffic(kname, args.n),
                 "kernel": kname, "variant": variant, "algorithmic_bytes": full, "avg_launch_ms": ms,
