@@ -116,20 +116,25 @@ struct Topology {
 // vertices (staged through registers before beta is known).  kPatchCross marks a cross
 // lower entry.
 // Rows per patch: 256 on meshes of at most kPatchSmallN vertices, 512 up to kPatchMidN,
-// kPcgWG above.  Where a mesh does not fit, the next larger up to kPcgWG (a window holds
-// twice as many vertices), and 512 after kPcgWG (a mesh in arbitrary vertex order needs
-// more LDS slots per row).  Smaller
-// patches put more workgroups in different phases on a compute unit (the window's loads,
-// the record stream, the LDS sums) and shorten the last round of workgroups, but cut more
-// blocks, which counts where the records come from HBM.  Product alone with 256, 512, 768
-// and 1,024 rows (us): FP32 263,169 vertices 22.5 23.4 24.1 26.2 (arbitrary order 34.7 37.0
-// 38.8 44.8), 1,050,625 vertices 89.4 82.3 95.1 85.6; FP64 36.7 37.7 38.6 44.7 (58.4 71.3
-// 58.5 65.5) and 161 151 163 166.  512 and 1,024 rows, us per multilevel iteration of n^2
-// quads: mixed 724 108.7 112.4, 860 142.6 142.1, 1024 199.1 199.0, 1100 224.9 220.6, 1200
-// 238.6 226.6, 1600 427.7 409.4, 2048 695.1 662.7; FP64 724 134.0 145.4, 1024 255.7 264.8,
-// 1200 335.8 334.8, 1600 593.8 579.8.  (A patch also leaves one partial sum of p.q: 512 rows
-// would be more than kMaxPartials from 8,388,609 vertices on.)
-constexpr int kPatchSmallN = 524288, kPatchMidN = 1310720;
+// kPcgWG above, and also from kPatchRoundN to 524,288 vertices, where the patches of 1,024
+// rows all but fill one round of two workgroups per compute unit.  Where a mesh does not
+// fit, the next larger up to kPcgWG (a window holds twice as many vertices), and 512 after
+// kPcgWG (a mesh in arbitrary vertex order needs more LDS slots per row).  Smaller patches
+// put more workgroups in different phases on a compute unit (the window's loads, the record
+// stream, the LDS sums) and shorten the last round of workgroups, but cut more blocks,
+// which counts where the records come from HBM.  Product alone with 256, 512, 768 and 1,024
+// rows (us): FP32 263,169 vertices 22.5 23.4 24.1 26.2 (arbitrary order 34.7 37.0 38.8 44.8),
+// 1,050,625 vertices 89.4 82.3 95.1 85.6; FP64 36.7 37.7 38.6 44.7 (58.4 71.3 58.5 65.5) and
+// 161 151 163 166.  256, 512 and 1,024 rows, us per multilevel iteration of n^2 quads: mixed
+// 400 54.1 57.0 55.5, 512 64.7 66.4 67.8, 540 65.0 64.4 66.3, 600 78.1 74.9 77.3, 640 87.2
+// 87.3 81.7, 680 92.4 83.4 81.3, 720 112.3 104.8 96.9, 760 123.7 119.7 122.0, 900 166.1 160.6
+// 162.6; FP64 400 46.0 46.9 47.6, 512 68.2 67.5 74.6, 540 70.8 70.5 77.1, 600 88.0 84.3 89.9,
+// 640 108.9 99.0 98.6, 720 134.2 118.5 117.5, 760 146.8 138.3 150.0, 900 224.8 200.2 209.0; 512
+// and 1,024 rows: mixed 1024 199.1 199.0, 1100 224.9 220.6, 1200 238.6 226.6, 1600 427.7 409.4,
+// 2048 695.1 662.7; FP64 1024 255.7 264.8, 1200 335.8 334.8, 1600 593.8 579.8.  (A patch also
+// leaves one partial sum of p.q: 512 rows would be more than kMaxPartials from 8,388,609
+// vertices on.)
+constexpr int kPatchSmallN = 294912, kPatchRoundN = 393216, kPatchMidN = 1310720;
 constexpr int kPatchPool = 6750;
 constexpr int patch_win(int rows) { return 2 * rows; }
 constexpr unsigned short kPatchCross = 0xffff;

@@ -1468,7 +1468,7 @@ int patch_grid(int N, int rows) { return ((N + rows - 1) / rows + 7) & ~7; }
 int patch_rows(int N, int choice)
 {
     int rows = 0;
-    if (N > kPatchMidN) rows = choice == 0 ? kPcgWG : choice == 1 ? 512 : 0;
+    if (N > kPatchMidN || (N > kPatchRoundN && N <= 512 * kPcgWG)) rows = choice == 0 ? kPcgWG : choice == 1 ? 512 : 0;
     else if (choice < 3) rows = (N <= kPatchSmallN ? 256 : 512) << choice;
     return rows > 0 && rows <= kPcgWG && patch_grid(N, rows) <= kMaxPartials ? rows : 0;
 }

@@ -15,9 +15,10 @@ def rule(name, *args):
     return C.CDLL(eolc.LIB_PATH)[f"_ZN4eolc{len(name)}{name}E" + "i" * len(args)](*args)
 
 
-@pytest.mark.parametrize("n,rows", [(1, [256, 512, 1024]), (524288, [256, 512, 1024]), (524289, [512, 1024]),
-                                    (1310720, [512, 1024]), (1310721, [1024, 512]), (8388608, [1024, 512]),
-                                    (8388609, [1024]), (LAST, [1024])])
+@pytest.mark.parametrize("n,rows", [(1, [256, 512, 1024]), (294912, [256, 512, 1024]), (294913, [512, 1024]),
+                                    (393216, [512, 1024]), (393217, [1024, 512]), (524288, [1024, 512]),
+                                    (524289, [512, 1024]), (1310720, [512, 1024]), (1310721, [1024, 512]),
+                                    (8388608, [1024, 512]), (8388609, [1024]), (LAST, [1024])])
 def test_patches_fit_the_partial_sums(n, rows):
     """The row counts tried on both sides of their lines, and the patches that they give."""
     assert [rule("patch_rows", n, k) for k in range(4)] == rows + [0] * (4 - len(rows))
@@ -26,7 +27,7 @@ def test_patches_fit_the_partial_sums(n, rows):
 
 def test_every_grid_fits_the_partial_sums():
     sizes = {LAST + 1, LAST + 1024}
-    for edge in (64, 256, 90000, 288 * 1024, 524288, 1310720, 8388608, LAST):
+    for edge in (64, 256, 90000, 288 * 1024, 393216, 524288, 1310720, 8388608, LAST):
         sizes |= {max(1, edge + d) for d in (-1024, -64, -1, 0, 1, 64, 1024)}
     sizes |= set(range(1, LAST, 65537))
     for n in sorted(sizes):
