@@ -118,8 +118,8 @@ struct Topology {
 // Rows per patch: 256 on meshes of at most kPatchSmallN vertices, 512 up to kPatchMidN,
 // kPcgWG above, and also from kPatchRoundN to 524,288 vertices, where the patches of 1,024
 // rows all but fill one round of two workgroups per compute unit.  Where a mesh does not
-// fit, the next larger up to kPcgWG (a window holds twice as many vertices), and 512 after
-// kPcgWG (a mesh in arbitrary vertex order needs more LDS slots per row).  Smaller patches
+// fit, the other sizes: larger ones (a window holds twice as many vertices), then smaller ones
+// (a mesh in arbitrary vertex order needs more LDS slots per row).  Smaller patches
 // put more workgroups in different phases on a compute unit (the window's loads, the record
 // stream, the LDS sums) and shorten the last round of workgroups, but cut more blocks,
 // which counts where the records come from HBM.  Product alone with 256, 512, 768 and 1,024

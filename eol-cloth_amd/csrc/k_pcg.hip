@@ -1467,10 +1467,11 @@ int patch_grid(int N, int rows) { return ((N + rows - 1) / rows + 7) & ~7; }
 // 0: no choice is left whose patches fit the partial sums.
 int patch_rows(int N, int choice)
 {
-    int rows = 0;
-    if (N > kPatchMidN || (N > kPatchRoundN && N <= 512 * kPcgWG)) rows = choice == 0 ? kPcgWG : choice == 1 ? 512 : 0;
-    else if (choice < 3) rows = (N <= kPatchSmallN ? 256 : 512) << choice;
-    return rows > 0 && rows <= kPcgWG && patch_grid(N, rows) <= kMaxPartials ? rows : 0;
+    constexpr int order[3][3] = {{256, 512, kPcgWG}, {512, kPcgWG, 256}, {kPcgWG, 512, 256}};
+    const bool most = N > kPatchMidN || (N > kPatchRoundN && N <= 512 * kPcgWG);
+    if (choice > 2) return 0;
+    const int rows = order[most ? 2 : N > kPatchSmallN][choice];
+    return patch_grid(N, rows) <= kMaxPartials ? rows : 0;
 }
 
 // The most partial sums that a kernel of the solve leaves on an N-vertex mesh (the

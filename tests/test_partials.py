@@ -15,10 +15,13 @@ def rule(name, *args):
     return C.CDLL(eolc.LIB_PATH)[f"_ZN4eolc{len(name)}{name}E" + "i" * len(args)](*args)
 
 
-@pytest.mark.parametrize("n,rows", [(1, [256, 512, 1024]), (294912, [256, 512, 1024]), (294913, [512, 1024]),
-                                    (393216, [512, 1024]), (393217, [1024, 512]), (524288, [1024, 512]),
-                                    (524289, [512, 1024]), (1310720, [512, 1024]), (1310721, [1024, 512]),
-                                    (8388608, [1024, 512]), (8388609, [1024]), (LAST, [1024])])
+UP, MID, DOWN = [256, 512, 1024], [512, 1024, 256], [1024, 512, 256]
+
+
+@pytest.mark.parametrize("n,rows", [(1, UP), (294912, UP), (294913, MID), (393216, MID), (393217, DOWN),
+                                    (524288, DOWN), (524289, MID), (1310720, MID), (1310721, DOWN),
+                                    (4194304, DOWN), (4194305, DOWN[:2]), (8388608, DOWN[:2]),
+                                    (8388609, DOWN[:1]), (LAST, DOWN[:1])])
 def test_patches_fit_the_partial_sums(n, rows):
     """The row counts tried on both sides of their lines, and the patches that they give."""
     assert [rule("patch_rows", n, k) for k in range(4)] == rows + [0] * (4 - len(rows))
