@@ -318,7 +318,7 @@ def spmv_kernel_name(fp32, variant, N, positions):
         t = "float" if fp32 else "double"
         w = (6 if u == 2 and w == 8 else w) if fp32 else 4
         rows = ((256, 512, 1024) if N <= 294912 else
-                (1024, 512) if N > 1310720 or 393216 < N <= 524288 else (512, 1024))
+                (1024, 512, 256) if N > 1310720 or 393216 < N <= 524288 else (512, 1024, 256))
         pr = next((r for r in rows if r * (-(-N // r) + 7 & ~7) == positions), rows[0])
         return f"k_pcg_spmv_patch<{t}, {t}, {b(nt)}, {w}, {u}, {pr}>"
     if N <= 90000 and (fp32 or lay != 4):   # one workgroup per slice of rows

@@ -6,7 +6,6 @@ distances, normals, positions and weights compared by bit pattern), in the
 reference's order."""
 import numpy as np
 import pytest
-import torch
 
 import eolc
 import oracle as O
@@ -278,6 +277,8 @@ def test_kept_block_after_a_call_beyond_its_limit():
     each) leaves the block to the smaller queries after it: their memory (200,000 points)
     is held from the second one on, also over a new topology, and given back with the
     context."""
+    import torch
+
     sc, pts, nrm, _, _ = thin_box_scene(24, 1e-3)
     rng = np.random.default_rng(6)
     many = np.concatenate([rng.uniform(0.0, 1.0, (1_000_000, 2)), np.full((1_000_000, 1), 5.0)], axis=1)
