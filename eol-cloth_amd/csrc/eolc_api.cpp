@@ -1104,7 +1104,8 @@ static int set_topology_impl(eolc_ctx *c, int N, const double *X, int F, const i
     Topology t;
     std::string msg = build_topology(t, N, F, tri, H, hinge, seg);
     if (!msg.empty()) return fail(c, EOLC_ERR_INVALID, "set_topology: " + msg);
-    for (int choice = 0, rows; (rows = eolc::patch_rows(N, choice)); ++choice) {
+    const bool local = t.wmax <= N / 8;   // no workgroup's rows reach over an eighth of the vertices
+    for (int choice = 0, rows; (rows = eolc::patch_rows(N, local, choice)); ++choice) {
         t.pt_why = build_patch_layout(t, X, rows);
         if (t.pt_why.empty()) break;
     }

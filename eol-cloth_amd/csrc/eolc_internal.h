@@ -117,9 +117,10 @@ struct Topology {
 // lower entry.
 // Rows per patch: 256 on meshes of at most kPatchSmallN vertices, 512 up to kPatchMidN,
 // kPcgWG above, and also from kPatchRoundN to 524,288 vertices, where the patches of 1,024
-// rows all but fill one round of two workgroups per compute unit.  Where a mesh does not
-// fit, the other sizes: larger ones (a window holds twice as many vertices), then smaller ones
-// (a mesh in arbitrary vertex order needs more LDS slots per row).  Smaller patches
+// rows all but fill one round of two workgroups per compute unit (512 on a mesh in arbitrary
+// vertex order, which needs more LDS slots per row).  Where a mesh does not
+// fit, the other sizes: larger ones (a window holds twice as many vertices), then smaller
+// ones.  Smaller patches
 // put more workgroups in different phases on a compute unit (the window's loads, the record
 // stream, the LDS sums) and shorten the last round of workgroups, but cut more blocks,
 // which counts where the records come from HBM.  Product alone with 256, 512, 768 and 1,024
@@ -586,7 +587,7 @@ hipError_t launch_update_x(eolc_ctx *c, double h);
 
 int pcg_grid(int N);
 int patch_grid(int N, int rows);   // patches of at most `rows` vertices (a multiple of 8)
-int patch_rows(int N, int choice);   // rows per patch to try, in turn; 0: none left
+int patch_rows(int N, bool local, int choice);   // rows per patch to try, in turn; 0: none left
 int most_partials(int N);   // at most kMaxPartials on every mesh that set_topology accepts
 int vec_wg(int N);          // workgroup size and workgroups of the PCG's vector kernels
 int vec_grid(int N);

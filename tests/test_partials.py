@@ -12,7 +12,10 @@ LAST = 16384 * 1024   # the largest mesh
 
 
 def rule(name, *args):
-    return C.CDLL(eolc.LIB_PATH)[f"_ZN4eolc{len(name)}{name}E" + "i" * len(args)](*args)
+    sig = "".join("b" if isinstance(a, bool) else "i" for a in args)
+    f = C.CDLL(eolc.LIB_PATH)[f"_ZN4eolc{len(name)}{name}E" + sig]
+    f.argtypes = [C.c_bool if isinstance(a, bool) else C.c_int for a in args]
+    return f(*args)
 
 
 UP, MID, DOWN = [256, 512, 1024], [512, 1024, 256], [1024, 512, 256]
@@ -23,9 +26,12 @@ UP, MID, DOWN = [256, 512, 1024], [512, 1024, 256], [1024, 512, 256]
                                     (4194304, DOWN), (4194305, DOWN[:2]), (8388608, DOWN[:2]),
                                     (8388609, DOWN[:1]), (LAST, DOWN[:1])])
 def test_patches_fit_the_partial_sums(n, rows):
-    """The row counts tried on both sides of their lines, and the patches that they give."""
-    assert [rule("patch_rows", n, k) for k in range(4)] == rows + [0] * (4 - len(rows))
+    """The row counts tried on both sides of their lines, and the patches that they give;
+    a mesh in arbitrary vertex order starts with 512 rows instead of 1,024 while those fit."""
+    assert [rule("patch_rows", n, True, k) for k in range(4)] == rows + [0] * (4 - len(rows))
     assert all(rule("patch_grid", n, r) <= MOST for r in rows)
+    spread = [rule("patch_rows", n, False, k) for k in range(4)]
+    assert spread[0] == (512 if rows[:2] == [1024, 512] else rows[0]) and set(spread) == set(rows) | {0}
 
 
 def test_every_grid_fits_the_partial_sums():
@@ -36,6 +42,6 @@ def test_every_grid_fits_the_partial_sums():
     for n in sorted(sizes):
         most = rule("most_partials", n)
         grids = [rule("pcg_grid", n), rule("vec_grid", n)]
-        grids += [rule("patch_grid", n, r) for r in (rule("patch_rows", n, k) for k in range(4)) if r]
+        grids += [rule("patch_grid", n, r) for r in (rule("patch_rows", n, True, k) for k in range(4)) if r]
         assert most >= max(grids)
         assert (most <= MOST) == (n <= LAST), n   # set_topology refuses by this
