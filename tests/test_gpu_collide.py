@@ -4,6 +4,8 @@ restatement of btc::pointTriCollision and btc::boxTriCollision.
 Bar: bit-exact -- every field of every record (indices, types, and the FP64
 distances, normals, positions and weights compared by bit pattern), in the
 reference's order."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -124,7 +126,6 @@ def test_cd2_no_obstacles_and_far_obstacles(ctx):
 
 
 def test_overflow_reports_required_size(ctx):
-    import ctypes as C
     sc, pts, nrm, whd, E = thin_box_scene(48, 1e-3)
     ctx.set_topology(sc.X, sc.tri, sc.hinge)
     ctx.upload_state(sc.x0, np.zeros_like(sc.x0))
@@ -277,13 +278,16 @@ def test_kept_block_after_a_call_beyond_its_limit():
     each) leaves the block to the smaller queries after it: their memory (200,000 points)
     is held from the second one on, also over a new topology, and given back with the
     context."""
-    import torch
-
     sc, pts, nrm, _, _ = thin_box_scene(24, 1e-3)
     rng = np.random.default_rng(6)
     many = np.concatenate([rng.uniform(0.0, 1.0, (1_000_000, 2)), np.full((1_000_000, 1), 5.0)], axis=1)
     up = np.tile([0.0, 0.0, 1.0], (len(many), 1))
-    free = lambda: torch.cuda.mem_get_info(0)[0]
+
+    def free():
+        now, total = C.c_size_t(0), C.c_size_t(0)
+        assert C.CDLL(eolc.LIB_PATH).hipMemGetInfo(C.byref(now), C.byref(total)) == 0   # (the library's own runtime)
+        return now.value
+
     with eolc.Context(0) as c:
         for k in range(2):
             c.set_topology(sc.X, sc.tri, sc.hinge)
